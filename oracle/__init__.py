@@ -27,7 +27,7 @@ def build(with_reference: bool | None = None) -> None:
     """Compile liboracle.so and, where the reference sources exist, the reference build."""
     subprocess.check_call(["make", "-s", "-C", HERE, "oracle"])
     if with_reference is None:
-        with_reference = os.path.isdir(REFERENCE_ROOT)
+        with_reference = os.path.isdir(os.path.join(REFERENCE_ROOT, "lib"))
     if with_reference:
         subprocess.check_call(["make", "-s", "-j8", "-C", HERE, "ref"])
 
