@@ -6,12 +6,13 @@
 // label_propagation_refinement.cpp:21-155).
 //
 // A round is S sub-rounds; a node belongs to sub-round hash3(seed ^ kSubSalt, 0, v) % S. One
-// sub-round is four launches, all order-independent, so the result is bit-identical to the CPU
-// mirror of the same schedule whatever the thread interleaving:
+// sub-round is three or four launches (or a part of refine_tail, which runs the rounds of a small
+// refinement frontier in one workgroup), all order-independent, so the result is bit-identical to
+// the CPU mirror of the same schedule whatever the thread interleaving:
 //   propose  every node of the sub-round picks its best eligible neighbouring label from the
 //            label / weight snapshot; proposers append a mover record and add their weight and
 //            priority key to the target's inc / top (integer atomics: order-free);
-//   filter   (refinement) departures from overloaded blocks;
+//   filter   (refinement, while a block is overloaded) departures from overloaded blocks;
 //   admit    a proposal is admitted if all proposals into its target fit, or if it is the
 //            target's top-priority proposal and fits alone;
 //   apply    admitted moves update labels and label weights; scratch is reset.
@@ -19,6 +20,8 @@
 //   deg <= 8/16/32/64   G lanes per node, one edge per lane, shuffle aggregation (no LDS);
 //   deg <= 512          one wave per node, LDS hash table (open addressing, LDS atomics);
 //   larger              one workgroup per node, hash table in a pre-cleared global region.
+
+#include <atomic>
 
 #include <rocprim/device/device_scan.hpp>
 
@@ -241,8 +244,6 @@ __device__ __attribute__((always_inline)) inline void scan_wave_table(
 }
 
 // ---------------------------------------------------------------- G lanes per node (deg <= G)
-// dcount: the list's length on the device (the compacted frontier of a refinement round);
-// workgroups then stride over the list's virtual blocks, so a small frontier costs few of them.
 // A virtual block holds IT x (kBlock / G) nodes: every lane group serves IT nodes at once, whose
 // dependent loads (list, offsets, targets, labels, label weights) are issued together, so each
 // wave has that many chains in flight.
@@ -261,10 +262,6 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
         const long long gi = ((long long)vb * IT + i) * NB + threadIdx.x / G;
         valid[i] = gi < count;
         v[i] = valid[i] ? list[gi] : 0;
-    }
-    if (M == LpMode::Refine) {
-#pragma unroll
-        for (int i = 0; i < IT; ++i) valid[i] = valid[i] && a.active[v[i]] != 0;
     }
     // every lane of the group takes part in the shuffles below: no early exit
 #pragma unroll
@@ -385,12 +382,10 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
     __syncthreads();  // the LDS of this virtual block is read before the next one writes it
 }
 
-template <LpMode M, int G, int IT>
+template <int G, int IT>
 __global__ __launch_bounds__(kBlock) void propose_group(LpArgs a, const int* __restrict__ list,
-                                                        int count, const int* __restrict__ dcount) {
-    if (dcount) count = *dcount;
-    const int nvb = (int)(((long long)count + IT * (kBlock / G) - 1) / (IT * (kBlock / G)));
-    for (int vb = blockIdx.x; vb < nvb; vb += gridDim.x) group_vb<M, G, IT>(a, list, count, vb, vb);
+                                                        int count) {
+    group_vb<LpMode::Cluster, G, IT>(a, list, count, blockIdx.x, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- one wave per node
@@ -409,9 +404,8 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int gi = vb * (kBlock / 64) + wave;
-    bool valid = gi < count;
+    const bool valid = gi < count;
     const int v = valid ? list[gi] : 0;
-    if (M == LpMode::Refine && valid) valid = a.active[v] != 0;
     const int own = valid ? a.label[v] : -1;
     const int beg = valid ? a.xadj[v] : 0;
     const int deg = valid ? a.xadj[v + 1] - beg : 0;
@@ -489,14 +483,10 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
     __syncthreads();  // the LDS of this virtual block is read before the next one clears it
 }
 
-template <LpMode M, bool DENSE, int WCAP = kWaveCap>
+template <int WCAP = kWaveCap>
 __global__ __launch_bounds__(kBlock) void propose_wave(LpArgs a, const int* __restrict__ list,
-                                                       int count, int num_labels,
-                                                       const int* __restrict__ dcount) {
-    if (dcount) count = *dcount;
-    const int nvb = (count + kBlock / 64 - 1) / (kBlock / 64);
-    for (int vb = blockIdx.x; vb < nvb; vb += gridDim.x)
-        wave_vb<M, DENSE, WCAP>(a, list, count, num_labels, vb, vb);
+                                                       int count) {
+    wave_vb<LpMode::Cluster, false, WCAP>(a, list, count, 0, blockIdx.x, blockIdx.x);
 }
 
 // Refinement: the proposals of all degree lists of a sub-round in one launch. The lists are the
@@ -514,7 +504,6 @@ __device__ __attribute__((always_inline)) inline void hubcnt_vb(const LpArgs& a,
     const int gi = vb * (kBlock / 64) + wave;
     if (gi >= count) return;  // uniform per wave; no workgroup barrier below
     const int v = list[gi];
-    if (a.active[v] == 0) return;
     const int* cnt = a.hub_cnt + a.hub_slot[v];
     const int own = a.label[v];
     const int nw = a.vwgt[v];
@@ -1134,14 +1123,13 @@ __global__ __launch_bounds__(256) void apply_moves(LpArgs a, const int* __restri
 // grid-stride loop takes element i of the lists' concatenation.
 struct SubLists {
     const int* list[kNumBins];
-    const int* dcount[kNumBins];  // device-side length, or nullptr: hcount
-    int hcount[kNumBins];
+    const int* dcount[kNumBins];  // device-side length
 };
 __device__ inline int sub_lengths(const SubLists& L, int* cnt) {
     int total = 0;
 #pragma unroll
     for (int b = 0; b < kNumBins; ++b) {
-        cnt[b] = L.dcount[b] ? *L.dcount[b] : L.hcount[b];
+        cnt[b] = *L.dcount[b];
         total += cnt[b];
     }
     return total;
@@ -1217,6 +1205,349 @@ __global__ void set_hub_slots(const int* __restrict__ list, const int* __restric
     if (t >= n_multi) return;
     const int i = multi[t];
     hub_slot[list[i]] = dense_off[i];
+}
+
+// ---------------------------------------------------------------- refinement: small frontiers
+// After a few rounds the frontier of a refinement is a few hundred nodes (RGG 2^20, k = 2: 1 M
+// nodes in round 0, then 600, 88, 24, none), and a round over the grid is bound by its launches
+// (~3 us each, 14 a round) whatever the frontier. refine_tail runs the remaining rounds in one
+// workgroup: the frontier, the proposals, the label weights and the admission scratch live in
+// LDS, so a sub-round costs a few workgroup barriers, and the rounds end with the frontier. One
+// workgroup and not a grid with device-wide barriers: a barrier across the XCDs' L2s costs about
+// as much as a launch. The limits keep it to frontiers for which one CU is faster than the grid:
+// a pass of 64 nodes of <= 16 edges takes about 2 us, so kTailNodes / 4 nodes of a sub-round
+// stay at the cost of its launches. Larger frontiers (or labels beyond the LDS, or hubs among
+// the nodes) are left to the grid. Graphs within the limits start here without node lists.
+// Measured, calls of kahip_partition: RGG 2^10 k = 2 5.1 -> 2.2 ms (refinement 3.0 -> 0.3), RGG
+// 2^22 k = 2 32.3 -> 26.1 ms, R-MAT 2^17 k = 8 39.1 -> 36.8 ms (its coarse levels settle early).
+constexpr int kTailThreads = 1024;
+constexpr int kTailNodes = 2048;     // frontier nodes
+constexpr int kTailEdges = 1 << 15;  // edges of the frontier's rows
+constexpr int kTailLabels = 512;     // labels (blocks) held in LDS
+constexpr int kTailHash = 2 * kTailNodes;
+constexpr int kTailWaves = kTailThreads / 64;
+constexpr int kTailDegree = 512;     // largest degree (8 edges per lane of a wave)
+constexpr int kTailGroup = 16;       // lanes per node of degree <= 16
+
+// Runs rounds a.round.. while the frontier is small; *state receives the round to go on with
+// (`rounds`: all done), whose frontier is then flagged in a.next_active, or compacted already if
+// no round ran.
+__global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t) {
+    __shared__ int lsize[kTailLabels], linc[kTailLabels], lout[kTailLabels];
+    __shared__ unsigned long long ltop[kTailLabels], ldtop[kTailLabels];
+    __shared__ int conn_of[kTailWaves][kTailLabels];
+    __shared__ int raw[kTailNodes];   // the round's frontier, in any order
+    __shared__ int item[kTailNodes];  // ... grouped by (sub-round, degree class)
+    __shared__ int pt[kTailNodes], pg[kTailNodes];  // proposal of item i: target (-1 none), gain
+    __shared__ int mv[kTailNodes];    // items moved in the sub-round
+    __shared__ int hash[kTailHash];   // next frontier
+    __shared__ int seg[2 * kMaxSub + 1], cur[2 * kMaxSub];
+    __shared__ int pre[kMaxSub * kNumBins + 1];
+    // (nfront is written by wave 0 or counted below, after the barrier)
+    __shared__ int nfront, nnext, nedges, nmv, nmoves, over, spill, bad;
+    __shared__ unsigned long long trav;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int grp = tid / kTailGroup, gl = tid & (kTailGroup - 1);
+    const int k = t.num_labels;
+    if (tid == 0) {
+        nedges = over = bad = 0;
+        trav = 0ull;
+        if (!t.clists) nfront = 0;
+    }
+    if (t.clists && wave == 0) {  // list offsets in the frontier: nseg <= 48 lists, a lane each
+        static_assert(kMaxSub * kNumBins < 64, "one lane per list");
+        const int cnt = lane < t.nseg ? t.ccount[lane] : 0;
+        int incl = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        if (lane <= t.nseg) pre[lane] = incl - cnt;
+        if (lane == 63) nfront = incl;
+    }
+    __syncthreads();
+    for (int i = tid; i < t.nseg; i += kTailThreads)
+        if (t.cnext) t.cnext[i] = 0;
+    // the grid's filter launches are needed only while a block is overloaded: admitted moves
+    // never overload one
+    for (int b = tid; b < k; b += kTailThreads)
+        if (a.size[b] > bound_of(a, b)) over = 1;
+    if (t.clists) {
+        if (nfront <= kTailNodes)
+            for (int i = tid; i < nfront; i += kTailThreads) {
+                int lo = 0, hi = t.nseg - 1;  // last list starting at or before i
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (pre[mid] <= i) lo = mid; else hi = mid - 1;
+                }
+                raw[i] = t.clists[t.offsets[lo] + (i - pre[lo])];
+            }
+    } else {  // round 0 of a graph of at most kTailNodes nodes (host)
+        for (int v = tid; v < t.n; v += kTailThreads)
+            if (a.xadj[v + 1] > a.xadj[v]) raw[atomicAdd(&nfront, 1)] = v;
+    }
+    __syncthreads();
+    int r = t.round;
+    bool fits = nfront <= kTailNodes && k <= kTailLabels && !t.hubs;  // uniform
+    if (fits) {
+        for (int i = tid; i < nfront; i += kTailThreads) {
+            const int d = a.xadj[raw[i] + 1] - a.xadj[raw[i]];
+            atomicAdd(&nedges, min(d, kTailEdges));
+            if (d > kTailDegree) bad = 1;
+        }
+        __syncthreads();
+        fits = nedges <= kTailEdges && !bad;
+    }
+    if (fits && nfront > 0 && r < t.rounds) {
+        for (int b = tid; b < k; b += kTailThreads) {
+            lsize[b] = a.size[b];
+            linc[b] = lout[b] = 0;
+            ltop[b] = ldtop[b] = 0ull;
+            for (int w = 0; w < kTailWaves; ++w) conn_of[w][b] = 0;
+        }
+        for (int i = tid; i < kTailHash; i += kTailThreads) hash[i] = -1;
+        while (true) {  // one round; every branch below is uniform
+            if (tid < 2 * kMaxSub) cur[tid] = 0;
+            if (tid == 0) nmoves = nnext = nedges = spill = 0;
+            __syncthreads();
+            const int nf = nfront;
+            // items by (sub-round, class): class 0 has up to kTailGroup edges
+            int myc[kTailNodes / kTailThreads], myr[kTailNodes / kTailThreads];
+#pragma unroll
+            for (int j = 0; j < kTailNodes / kTailThreads; ++j) {
+                const int i = tid + j * kTailThreads;
+                myc[j] = -1;
+                if (i < nf) {
+                    const int v = raw[i];
+                    const int d = a.xadj[v + 1] - a.xadj[v];
+                    myc[j] = 2 * subround_of(t.seed, v, t.S) + (d > kTailGroup ? 1 : 0);
+                    myr[j] = atomicAdd(&cur[myc[j]], 1);
+                    atomicAdd(&trav, (unsigned long long)d);
+                }
+            }
+            __syncthreads();
+            if (wave == 0) {
+                const int cnt = lane < 2 * kMaxSub ? cur[lane] : 0;
+                int incl = cnt;
+#pragma unroll
+                for (int o = 1; o < 2 * kMaxSub; o <<= 1) {
+                    const int y = __shfl_up(incl, o, 64);
+                    if (lane >= o) incl += y;
+                }
+                if (lane <= 2 * kMaxSub) seg[lane] = lane < 2 * kMaxSub ? incl - cnt : nf;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < kTailNodes / kTailThreads; ++j)
+                if (myc[j] >= 0) {
+                    const int at = seg[myc[j]] + myr[j];
+                    item[at] = raw[tid + j * kTailThreads];
+                    pt[at] = -1;
+                }
+            __syncthreads();
+            const uint32_t tie_seed = tie_seed_of(t.seed, r);
+            for (int sr = 0; sr < t.S; ++sr) {
+                const int s0 = seg[2 * sr], s1 = seg[2 * sr + 1], s2 = seg[2 * sr + 2];
+                if (s0 == s2) continue;
+                if (tid == 0) nmv = 0;
+                // the proposal of item i (one lane calls it)
+                auto put = [&](int i, int v, int own, int w, int conn_own, const Cand& c) {
+                    if (c.conn < 0) return;
+                    const int so = lsize[own];
+                    const bool ovl = so > bound_of(a, own);
+                    if (!(c.conn > conn_own || ovl ||
+                          (c.conn == conn_own && (long long)c.size + 2LL * w <= (long long)so)))
+                        return;
+                    pt[i] = c.lab;
+                    pg[i] = c.conn - conn_own;
+                    const unsigned long long key = prio_key(c.conn - conn_own, v);
+                    atomicAdd(ovl ? &lout[own] : &linc[c.lab], w);
+                    atomicMax(ovl ? &ldtop[own] : &ltop[c.lab], key);
+                };
+                // kTailGroup lanes per node of up to kTailGroup edges
+                for (int base = s0; base < s1; base += kTailThreads / kTailGroup) {
+                    const int i = base + grp;
+                    const bool valid = i < s1;
+                    const int v = valid ? item[i] : 0;
+                    const int own = valid ? a.label[v] : -1;
+                    const int beg = valid ? a.xadj[v] : 0;
+                    const int deg = valid ? a.xadj[v + 1] - beg : 0;
+                    int lab = gl < deg ? a.adjncy[beg + gl] : -1;
+                    const int w = gl < deg ? a.adjwgt[beg + gl] : 0;
+                    if (lab >= 0) lab = a.label[lab];
+                    int conn = w;
+                    bool leader = lab >= 0;
+                    agg_rot<1>(lab, gl, lab, w, gl, conn, leader);
+                    const int conn_own =
+                        reduce_max<kTailGroup>((lab >= 0 && lab == own) ? conn : 0);
+                    const int nw = valid ? a.vwgt[v] : 0;
+                    Cand c{-1, 0u, 0x7fffffff, 0};
+                    if (leader && lab != own &&
+                        (long long)lsize[lab] + nw < (long long)bound_of(a, lab))
+                        c = Cand{conn, hash3(tie_seed, (uint32_t)v, (uint32_t)lab), lab,
+                                 lsize[lab]};
+                    reduce_cand<kTailGroup>(c);
+                    if (valid && gl == 0) put(i, v, own, nw, conn_own, c);
+                }
+                // one wave per larger node: a counter per label, summed with LDS atomics; every
+                // lane then tries the labels of its own edges (a label's candidate is the same
+                // whichever lane brings it)
+                for (int i = s1 + wave; i < s2; i += kTailWaves) {
+                    int* const V = conn_of[wave];
+                    const int v = item[i];
+                    const int own = a.label[v];
+                    const int beg = a.xadj[v], end = a.xadj[v + 1];
+                    constexpr int EPL = kTailDegree / 64;
+                    int labs[EPL], ws[EPL];
+#pragma unroll
+                    for (int j = 0; j < EPL; ++j) {
+                        const int e = beg + lane + 64 * j;
+                        labs[j] = e < end ? a.adjncy[e] : -1;
+                        ws[j] = e < end ? a.adjwgt[e] : 0;
+                    }
+#pragma unroll
+                    for (int j = 0; j < EPL; ++j)
+                        if (labs[j] >= 0) labs[j] = a.label[labs[j]];
+#pragma unroll
+                    for (int j = 0; j < EPL; ++j)
+                        if (labs[j] >= 0) atomicAdd(&V[labs[j]], ws[j]);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    const int nw = a.vwgt[v];
+                    int conn_own = 0;
+                    Cand c{-1, 0u, 0x7fffffff, 0};
+#pragma unroll
+                    for (int j = 0; j < EPL; ++j) {
+                        const int lab = labs[j];
+                        if (lab < 0) continue;
+                        const int conn = V[lab];
+                        if (lab == own) {
+                            conn_own = conn;
+                            continue;
+                        }
+                        if ((long long)lsize[lab] + nw >= (long long)bound_of(a, lab)) continue;
+                        const uint32_t tie = hash3(tie_seed, (uint32_t)v, (uint32_t)lab);
+                        if (better(conn, tie, lab, c.conn, c.tie, c.lab))
+                            c = Cand{conn, tie, lab, lsize[lab]};
+                    }
+                    conn_own = reduce_max<64>(conn_own);
+                    reduce_cand<64>(c);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int j = 0; j < EPL; ++j)
+                        if (labs[j] >= 0) V[labs[j]] = 0;
+                    if (lane == 0) put(i, v, own, nw, conn_own, c);
+                }
+                __syncthreads();
+                // filter, admit and apply as on the grid, a thread per item
+                constexpr int IPT = kTailNodes / kTailThreads;
+                int own[IPT], w[IPT];
+                bool ok[IPT];
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) {
+                    const int i = s0 + tid + j * kTailThreads;
+                    ok[j] = i < s2 && pt[i] >= 0;
+                    own[j] = ok[j] ? a.label[item[i]] : 0;
+                    w[j] = ok[j] ? a.vwgt[item[i]] : 0;
+                }
+                if (over) {
+#pragma unroll
+                    for (int j = 0; j < IPT; ++j) {
+                        const int i = s0 + tid + j * kTailThreads;
+                        if (!ok[j]) continue;
+                        const int so = lsize[own[j]], ub = bound_of(a, own[j]);
+                        if (so <= ub) continue;
+                        const unsigned long long key = prio_key(pg[i], item[i]);
+                        if ((long long)so - (long long)lout[own[j]] >= (long long)ub ||
+                            ldtop[own[j]] == key) {
+                            atomicAdd(&linc[pt[i]], w[j]);
+                            atomicMax(&ltop[pt[i]], key);
+                        } else {
+                            ok[j] = false;
+                        }
+                    }
+                    __syncthreads();
+                }
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) {
+                    const int i = s0 + tid + j * kTailThreads;
+                    if (!ok[j]) continue;
+                    const int to = pt[i];
+                    const long long st = lsize[to], bt = bound_of(a, to);
+                    ok[j] = st + (long long)linc[to] < bt ||
+                            (ltop[to] == prio_key(pg[i], item[i]) && st + w[j] < bt);
+                }
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) {
+                    const int i = s0 + tid + j * kTailThreads;
+                    if (i >= s2 || pt[i] < 0) continue;
+                    const int to = pt[i], v = item[i], from = a.label[v];
+                    linc[to] = 0;
+                    ltop[to] = 0ull;
+                    lout[from] = 0;
+                    ldtop[from] = 0ull;
+                    if (!ok[j]) continue;
+                    atomicSub(&lsize[from], w[j]);
+                    atomicAdd(&lsize[to], w[j]);
+                    a.label[v] = to;
+                    mv[atomicAdd(&nmv, 1)] = v;
+                }
+                __syncthreads();
+                // the moved nodes' neighbours form the next frontier: flagged for the grid and
+                // collected in the hash (a full hash only stops the collecting)
+                const int nm = nmv;
+                for (int m = wave; m < nm; m += kTailWaves) {
+                    const int v = mv[m];
+                    const int beg = a.xadj[v], end = a.xadj[v + 1];
+                    if (lane == 0) atomicAdd(&trav, (unsigned long long)(end - beg));
+                    for (int e = beg + lane; e < end; e += 64) {
+                        const int u = a.adjncy[e];
+                        a.next_active[u] = 1;
+                        bool fresh = false;
+                        if (!spill && probe_claim(hash, kTailHash, u, fresh) < 0) spill = 1;
+                        if (fresh && atomicAdd(&nnext, 1) >= kTailNodes) spill = 1;
+                    }
+                }
+                if (tid == 0) nmoves += nm;
+                __syncthreads();
+            }
+            if (tid == 0) {
+                t.moves[r] = nmoves;
+                nfront = 0;
+            }
+            ++r;
+            __syncthreads();
+            if (spill) break;
+            for (int i = tid; i < kTailHash; i += kTailThreads) {
+                const int u = hash[i];
+                if (u < 0) continue;
+                raw[atomicAdd(&nfront, 1)] = u;  // nnext <= kTailNodes
+                const int d = a.xadj[u + 1] - a.xadj[u];
+                atomicAdd(&nedges, min(d, kTailEdges));
+                if (d > kTailDegree) bad = 1;
+            }
+            __syncthreads();
+            if (nfront == 0 || nedges > kTailEdges || bad || r == t.rounds) break;
+            for (int i = tid; i < kTailHash; i += kTailThreads) {
+                if (hash[i] >= 0) a.next_active[hash[i]] = 0;
+                hash[i] = -1;
+            }
+            __syncthreads();
+        }
+        for (int b = tid; b < k; b += kTailThreads) a.size[b] = lsize[b];
+        if (tid == 0 && trav) atomicAdd(&a.trav[0], trav);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        const int next = nfront == 0 && !(r > t.round && spill) ? t.rounds : r;
+        t.state[1] = next;
+        t.state[2] = over;
+        __threadfence_system();
+        __hip_atomic_store(&t.state[0], t.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // ---------------------------------------------------------------- binning
@@ -1299,12 +1630,13 @@ __global__ void bin_scatter(int n, const int* __restrict__ xadj, uint32_t seed, 
 
 // Frontier of a refinement round: the active nodes of every non-hub list, compacted per list
 // into clists (same offsets as lists); ccount[l] receives list l's length. The order inside a
-// list is free: the synchronous schedule does not depend on it.
+// list is free: the synchronous schedule does not depend on it. clear: the flags are consumed, so
+// that the array serves as the next round's (unless a kernel of this round still reads them).
 constexpr int kCompactItems = 8;  // list entries per thread of compact_active
 __global__ __launch_bounds__(256) void compact_active(const int* __restrict__ lists,
                                                       const int* __restrict__ offsets, int nseg,
-                                                      int total, const uint8_t* __restrict__ active,
-                                                      int* __restrict__ ccount,
+                                                      int total, uint8_t* __restrict__ active,
+                                                      int clear, int* __restrict__ ccount,
                                                       int* __restrict__ clists) {
     __shared__ int off[kMaxSub * kNumBins];
     __shared__ int local[kMaxSub * kNumBins];
@@ -1336,6 +1668,7 @@ __global__ __launch_bounds__(256) void compact_active(const int* __restrict__ li
             }
             l[j] = lo;
             r[j] = atomicAdd(&local[lo], 1);
+            if (clear) active[v[j]] = 0;
         }
     }
     __syncthreads();
@@ -1444,25 +1777,15 @@ __global__ void block_weights_global(int n, const int* __restrict__ part,
 
 inline int grid_for(long long work, int block) { return (int)((work + block - 1) / block); }
 
-// The G-lane proposal kernel of one list with `items` nodes per lane group: clustering launches
-// one workgroup per virtual block, refinement strides over its device-side frontier count.
+// The clustering's G-lane proposal kernel of one list with `items` nodes per lane group, one
+// workgroup per virtual block.
 template <int G>
-void launch_group(bool cl, int items, const LpArgs& a, const int* lst, int cnt, const int* dc,
-                  hipStream_t s) {
-    const int g = grid_for((long long)cnt * G, kBlock * items);
-    const dim3 grid(cl ? g : std::min(g, kFrontierGrid));
+void launch_group(int items, const LpArgs& a, const int* lst, int cnt, hipStream_t s) {
+    const dim3 grid(grid_for((long long)cnt * G, kBlock * items));
     switch (items) {
-        case 1:
-            if (cl) hipLaunchKernelGGL((propose_group<LpMode::Cluster, G, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt, nullptr);
-            else hipLaunchKernelGGL((propose_group<LpMode::Refine, G, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt, dc);
-            break;
-        case 4:
-            if (cl) hipLaunchKernelGGL((propose_group<LpMode::Cluster, G, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt, nullptr);
-            else hipLaunchKernelGGL((propose_group<LpMode::Refine, G, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt, dc);
-            break;
-        default:
-            if (cl) hipLaunchKernelGGL((propose_group<LpMode::Cluster, G, 2>), grid, dim3(kBlock), 0, s, a, lst, cnt, nullptr);
-            else hipLaunchKernelGGL((propose_group<LpMode::Refine, G, 2>), grid, dim3(kBlock), 0, s, a, lst, cnt, dc);
+        case 1: hipLaunchKernelGGL((propose_group<G, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
+        case 4: hipLaunchKernelGGL((propose_group<G, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
+        default: hipLaunchKernelGGL((propose_group<G, 2>), grid, dim3(kBlock), 0, s, a, lst, cnt);
     }
 }
 
@@ -1514,13 +1837,31 @@ void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, u
     KH_REQUIRE(g.n < (1 << 30) && num_labels < (1 << 30), "labels must be below 2^30");
     subrounds_ = S;
     num_labels_ = num_labels;
+    moves_.reserve(kMaxRounds);
+    trav_.reserve(64);
+    err_.reserve(1);
+    if (mode == LpMode::Refine) {
+        active_.reserve(g.n);
+        next_active_.reserve(g.n);
+        tail_.init();
+    }
+    // a graph that refine_tail takes from round 0 needs no lists
+    small_ = mode == LpMode::Refine && !include && g.n <= kTailNodes && g.m2 <= kTailEdges &&
+             num_labels <= kTailLabels;
+    if (!small_) build_lists(mode, g, seed, s, include);
+}
+
+void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
+                              const uint8_t* include) {
+    const int S = subrounds_, num_labels = num_labels_;
+    const BinConfig& bins = bins_;
     dense_wave_ = mode == LpMode::Refine && num_labels <= kWaveDense;
     dense_hub_ = mode == LpMode::Refine && num_labels <= kHubDense;
     const int L = kMaxSub * kNumBins;
     lists_.reserve(g.n);
     if (mode == LpMode::Refine) {
         clists_.reserve(g.n);
-        ccount_.reserve(L);
+        ccount_.reserve(2 * L);
     }
     counts_.reserve(L + kMaxSub);
     cursor_.reserve(L + kMaxSub);
@@ -1529,17 +1870,12 @@ void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, u
     prop_t_.reserve(g.n);
     prop_gain_.reserve(g.n);
     prop_ok_.reserve(g.n);
-    moves_.reserve(kMaxRounds);
     inc_.reserve(num_labels);
     out_.reserve(num_labels);
     top_.reserve(num_labels);
     dtop_.reserve(num_labels);
-    active_.reserve(g.n);
-    next_active_.reserve(g.n);
     n_big_tasks_.reserve((long long)kMaxSub * kMaxRounds);
     n_mid_tasks_.reserve((long long)kMaxSub * kMaxRounds);
-    trav_.reserve(64);
-    err_.reserve(1);
 
     fill_async(counts_.p, L + kMaxSub, 0, s);
     fill_async(cursor_.p, L + kMaxSub, 0, s);
@@ -1816,16 +2152,10 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     const int S = subrounds_;
     const bool cl = mode == LpMode::Cluster;
     KH_REQUIRE(cl || !(dense_wave_ || dense_hub_) || num_labels_ > 0, "prepare() not called");
-    // no allocation here: prepare() sized everything
-    fill_async(n_big_tasks_.p, (long long)kMaxSub * kMaxRounds, 0, s);
-    fill_async(n_mid_tasks_.p, (long long)kMaxSub * kMaxRounds, 0, s);
     fill_async(moves_.p, kMaxRounds, 0, s);
     fill_async(trav_.p, 64, 0ull, s);
     fill_async(err_.p, 1, 0, s);
-    if (!cl) {
-        fill_async(active_.p, g.n, (uint8_t)1, s);
-        fill_async(next_active_.p, g.n, (uint8_t)0, s);
-    }
+    if (rounds == 0) return;
     LpArgs a{};
     a.xadj = g.xadj;
     a.adjncy = g.adjncy;
@@ -1835,6 +2165,26 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     a.size = size;
     a.bound = bound;
     a.lbound = lbound;
+    a.trav = trav_.p;
+    a.err = err_.p;
+    uint8_t* act = active_.p;
+    uint8_t* nxt = next_active_.p;
+    int r = 0;
+    bool filter = !cl;  // an overloaded block may exist
+    if (small_) {
+        // the whole refinement in one workgroup; the lists are built only if it stops early
+        fill_async(act, g.n, (uint8_t)0, s);
+        fill_async(nxt, g.n, (uint8_t)0, s);
+        a.next_active = nxt;
+        TailArgs t{};
+        t.n = g.n;
+        t.rounds = rounds;
+        t.seed = seed;
+        r = run_tail(a, t, s, &filter);
+        if (r >= rounds) return;
+        build_lists(mode, g, seed, s, nullptr);
+        std::swap(act, nxt);  // round r's frontier (r > 0)
+    }
     a.inc = inc_.p;
     a.top = top_.p;
     a.out = out_.p;
@@ -1842,18 +2192,18 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     a.prop_t = prop_t_.p;
     a.prop_gain = prop_gain_.p;
     a.prop_ok = prop_ok_.p;
-    a.trav = trav_.p;
-    a.err = err_.p;
+    if (cl || !dense_hub_) {
+        fill_async(n_big_tasks_.p, (long long)kMaxSub * kMaxRounds, 0, s);
+        fill_async(n_mid_tasks_.p, (long long)kMaxSub * kMaxRounds, 0, s);
+    }
     // Refinement hubs of more than one chunk keep per-block connection counters across the
     // rounds: one scan builds them, every applied move updates its hub neighbours' counters, and
     // the hubs then decide from the counters instead of rescanning their edges each round.
     const bool incremental = !cl && dense_hub_ && dense_total_ > 0;
     a.hub_slot = incremental ? hub_slot_.p : nullptr;
     a.hub_cnt = incremental ? dense_cnt_.p : nullptr;
-    uint8_t* act = active_.p;
-    uint8_t* nxt = next_active_.p;
     const std::string base = std::string(phase ? phase : (cl ? "lp_cluster" : "lp_refine"));
-    if (incremental && rounds > 0) {
+    if (incremental) {
         ProfScope ps(prof, base + "_hub_counters", 0.0, 0, s);
         fill_async(dense_cnt_.p, dense_total_, 0, s);
         const int copies = std::min(kHubDenseThreads / 64, kHubDenseSlots / num_labels_);
@@ -1868,17 +2218,54 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     const bool fused_hubs = incremental && dense_all_;
     const int nseg = S * kNumBins;
     const int listed = host_offsets[nseg - 1] + host_counts[nseg - 1];
-    for (int r = 0; r < rounds; ++r) {
+    int hubs = 0;
+    for (int sr = 0; sr < S; ++sr) hubs += host_counts[sr * kNumBins + kNumBins - 1];
+    // the compaction consumes the frontier flags unless hub kernels of the round read them
+    const bool keep_flags = hubs > 0 && !fused_hubs;
+    if (!cl) {
+        if (listed == 0) return;
+        if (r == 0) {
+            fill_async(act, g.n, (uint8_t)(keep_flags ? 1 : 0), s);
+            fill_async(nxt, g.n, (uint8_t)0, s);
+        }
+        fill_async(ccount_.p, 2 * nseg, 0, s);
+    }
+    int* cnow = ccount_.p;  // list lengths of the frontier, cleared by the tail before last
+    int* cnext = cnow + nseg;
+    while (r < rounds) {
+        // refinement: round 0 works on the whole lists, later rounds on the compacted frontier
+        const int* flists = lists_.p;
+        const int* fcount = counts_.p;
+        if (!cl && r > 0) {
+            ProfScope ps(prof, base + "_frontier", 0.0, 0, s);
+            std::swap(cnow, cnext);
+            hipLaunchKernelGGL(compact_active, dim3(grid_for(listed, 256 * kCompactItems)), dim3(256), 0, s,
+                               lists_.p, offsets_.p, nseg, listed, act, keep_flags ? 0 : 1, cnow, clists_.p);
+            a.next_active = nxt;
+            TailArgs t{};
+            t.clists = clists_.p;
+            t.offsets = offsets_.p;
+            t.ccount = cnow;
+            t.cnext = cnext;
+            t.nseg = nseg;
+            t.n = g.n;
+            t.round = r;
+            t.rounds = rounds;
+            t.seed = seed;
+            t.hubs = hubs;
+            const int next = run_tail(a, t, s, &filter);
+            if (next != r) {
+                r = next;
+                std::swap(act, nxt);
+                continue;
+            }
+            flists = clists_.p;
+            fcount = cnow;
+        }
         a.tie_seed = tie_seed_of(seed, r);
         a.moves = moves_.p + r;
         a.active = cl ? nullptr : act;
         a.next_active = cl ? nullptr : nxt;
-        if (!cl && listed > 0) {
-            ProfScope ps(prof, base + "_frontier", 0.0, 0, s);
-            fill_async(ccount_.p, nseg, 0, s);
-            hipLaunchKernelGGL(compact_active, dim3(grid_for(listed, 256 * kCompactItems)), dim3(256), 0, s,
-                               lists_.p, offsets_.p, nseg, listed, act, ccount_.p, clists_.p);
-        }
         for (int sr = 0; sr < S; ++sr) {
             int sub_total = 0;
             if (!cl) {
@@ -1889,8 +2276,8 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 for (int b = 0; b < kNumBins; ++b) {
                     const int l = sr * kNumBins + b;
                     const bool take = b < kNumBins - 1 || fused_hubs;
-                    F.list[b] = clists_.p + host_offsets[l];
-                    F.dcount[b] = take ? ccount_.p + l : nullptr;
+                    F.list[b] = flists + host_offsets[l];
+                    F.dcount[b] = take ? fcount + l : nullptr;
                     listed_sr += take ? host_counts[l] : 0;
                 }
                 if (listed_sr > 0)
@@ -1902,10 +2289,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 sub_total += cnt;
                 if (cnt == 0) continue;
                 if (!cl && (b < kNumBins - 1 || fused_hubs)) continue;  // in the frontier launch
-                // refinement: the round's frontier of the list (length on the device)
-                const bool fr = !cl && b < kNumBins - 1;
-                const int* lst = (fr ? clists_.p : lists_.p) + host_offsets[l];
-                const int* dc = fr ? ccount_.p + l : nullptr;
+                const int* lst = lists_.p + host_offsets[l];
                 // algorithmic bytes: 12 B per traversed edge (target, weight, label gather) and
                 // 16 B per node (two offsets, weight, own label); label weights are O(moved).
                 // (the hub list's mid-size hubs are timed in a scope of their own)
@@ -1915,24 +2299,21 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 const double bytes = cl ? 12.0 * (double)ledges + 16.0 * lnodes : 0.0;
                 ProfScope ps(prof, base + "_propose_" + kBinName[b], bytes, cl ? ledges : 0, s);
                 switch (b) {
-                    case 0: launch_group<8>(cl, bins_.group_items, a, lst, cnt, dc, s); break;
-                    case 1: launch_group<16>(cl, bins_.group_items, a, lst, cnt, dc, s); break;
-                    case 2: launch_group<32>(cl, bins_.group_items, a, lst, cnt, dc, s); break;
-                    case 3: launch_group<64>(cl, bins_.group_items, a, lst, cnt, dc, s); break;
-                    case 4:
-                        if (cl) {
-                            const int ns = host_wave_small_[sr];  // degree <= wave_small, first
-                            if (ns > 0) {
-                                const dim3 gs(grid_for(ns, kBlock / 64));
-                                if (bins_.wave_small == 64) hipLaunchKernelGGL((propose_wave<LpMode::Cluster, false, 128>), gs, dim3(kBlock), 0, s, a, lst, ns, nl, nullptr);
-                                else if (bins_.wave_small == 256) hipLaunchKernelGGL((propose_wave<LpMode::Cluster, false, 512>), gs, dim3(kBlock), 0, s, a, lst, ns, nl, nullptr);
-                                else hipLaunchKernelGGL((propose_wave<LpMode::Cluster, false, 256>), gs, dim3(kBlock), 0, s, a, lst, ns, nl, nullptr);
-                            }
-                            if (cnt > ns) hipLaunchKernelGGL((propose_wave<LpMode::Cluster, false>), dim3(grid_for(cnt - ns, kBlock / 64)), dim3(kBlock), 0, s, a, lst + ns, cnt - ns, nl, nullptr);
+                    case 0: launch_group<8>(bins_.group_items, a, lst, cnt, s); break;
+                    case 1: launch_group<16>(bins_.group_items, a, lst, cnt, s); break;
+                    case 2: launch_group<32>(bins_.group_items, a, lst, cnt, s); break;
+                    case 3: launch_group<64>(bins_.group_items, a, lst, cnt, s); break;
+                    case 4: {
+                        const int ns = host_wave_small_[sr];  // degree <= wave_small, first
+                        if (ns > 0) {
+                            const dim3 gs(grid_for(ns, kBlock / 64));
+                            if (bins_.wave_small == 64) hipLaunchKernelGGL(propose_wave<128>, gs, dim3(kBlock), 0, s, a, lst, ns);
+                            else if (bins_.wave_small == 256) hipLaunchKernelGGL(propose_wave<512>, gs, dim3(kBlock), 0, s, a, lst, ns);
+                            else hipLaunchKernelGGL(propose_wave<256>, gs, dim3(kBlock), 0, s, a, lst, ns);
                         }
-                        else if (dense_wave_) hipLaunchKernelGGL((propose_wave<LpMode::Refine, true>), dim3(std::min(grid_for(cnt, kBlock / 64), kFrontierGrid)), dim3(kBlock), 0, s, a, lst, cnt, nl, dc);
-                        else hipLaunchKernelGGL((propose_wave<LpMode::Refine, false>), dim3(std::min(grid_for(cnt, kBlock / 64), kFrontierGrid)), dim3(kBlock), 0, s, a, lst, cnt, nl, dc);
+                        if (cnt > ns) hipLaunchKernelGGL(propose_wave<>, dim3(grid_for(cnt - ns, kBlock / 64)), dim3(kBlock), 0, s, a, lst + ns, cnt - ns);
                         break;
+                    }
                     default: {
                         if (!cl && dense_hub_) {
                             const int4* cm = cmap_.p + cmap_base_[sr];
@@ -2010,22 +2391,69 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 for (int b = 0; b < kNumBins; ++b) {
                     const int l = sr * kNumBins + b;
                     // every list's compacted frontier (an inactive hub proposes nothing)
-                    L.list[b] = clists_.p + host_offsets[l];
-                    L.dcount[b] = ccount_.p + l;
-                    L.hcount[b] = host_counts[l];
+                    L.list[b] = flists + host_offsets[l];
+                    L.dcount[b] = fcount + l;
                 }
                 const int gs = std::min(gm, 1024);
-                hipLaunchKernelGGL(filter_departures_sub, dim3(gs), dim3(256), 0, s, a, L);
+                if (filter) hipLaunchKernelGGL(filter_departures_sub, dim3(gs), dim3(256), 0, s, a, L);
                 hipLaunchKernelGGL(admit_moves_sub, dim3(gs), dim3(256), 0, s, a, L);
                 hipLaunchKernelGGL(apply_moves_sub, dim3(gs), dim3(256), 0, s, a, L);
             }
         }
         if (!cl) {
             std::swap(act, nxt);
-            fill_async(nxt, g.n, (uint8_t)0, s);
+            if (keep_flags) fill_async(nxt, g.n, (uint8_t)0, s);
         }
+        ++r;
     }
     KH_CHECK(hipGetLastError());
+}
+
+// Launches refine_tail and waits for its answer: the round to go on with, and whether a block is
+// overloaded. The answer is polled in host memory, which takes about 5 us from the kernel's end
+// to the next launch (a stream synchronisation takes three times as long).
+int LpWorkspace::run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded) {
+    t.num_labels = num_labels_;
+    t.S = subrounds_;
+    t.moves = moves_.p;
+    t.state = tail_.dev;
+    t.seq = ++tail_.seq;
+    hipLaunchKernelGGL(refine_tail, dim3(1), dim3(kTailThreads), 0, s, a, t);
+    KH_CHECK(hipGetLastError());
+    tail_.wait(s);
+    *overloaded = tail_.host[2] != 0;
+    return tail_.host[1];
+}
+
+void TailState::init() {
+    if (host) return;
+    void* h = nullptr;
+    KH_CHECK(hipHostMalloc(&h, 64, hipHostMallocMapped | hipHostMallocCoherent));
+    host = static_cast<volatile int*>(h);
+    host[0] = 0;
+    void* d = nullptr;
+    KH_CHECK(hipHostGetDevicePointer(&d, h, 0));
+    dev = static_cast<int*>(d);
+}
+
+TailState::~TailState() {
+    if (host) (void)hipHostFree(const_cast<int*>(host));
+}
+
+void TailState::wait(hipStream_t s) const {
+    // the stream is asked now and then, so that a failed launch ends the wait
+    for (unsigned spin = 1; host[0] != seq; ++spin) {
+        __builtin_ia32_pause();
+        if (spin % (1u << 16)) continue;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();  // not an error of ours
+            continue;
+        }
+        KH_CHECK(e);
+        KH_REQUIRE(host[0] == seq, "label propagation: the refinement ended without its answer");
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
 }
 
 void LpWorkspace::read_moves(int rounds, int* out, hipStream_t s) {

@@ -39,8 +39,31 @@ struct LpArgs {
     int* err;  // device error flag (kErrProbe), cleared by run(), read by check()
 };
 
-struct LpStats {
-    int moves[kMaxRounds];
+// Arguments of refine_tail beyond LpArgs.
+struct TailArgs {
+    const int* clists;   // round `round`'s frontier, compacted per list; nullptr: every node
+    const int* offsets;  // list offsets
+    const int* ccount;   // list lengths
+    int* cnext;          // cleared for the next compaction (nseg entries)
+    int nseg, n, num_labels, S, round, rounds;
+    uint32_t seed;
+    int hubs;            // nodes of more than the wave bin's degree exist: never run here
+    int* moves;          // per round
+    int* state;          // host-visible {sequence number, next round, overloaded block exists}
+    int seq;
+};
+
+// Host memory in which refine_tail leaves its answer {sequence number, next round, overloaded}.
+struct TailState {
+    volatile int* host = nullptr;
+    int* dev = nullptr;
+    int seq = 0;
+    TailState() = default;
+    TailState(const TailState&) = delete;
+    TailState& operator=(const TailState&) = delete;
+    ~TailState();
+    void init();
+    void wait(hipStream_t s) const;  // for the answer with number seq
 };
 
 class LpWorkspace {
@@ -73,6 +96,11 @@ public:
     int host_offsets[kMaxSub * kNumBins] = {};
 
 private:
+    void build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
+                     const uint8_t* include);
+    int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
+    TailState tail_;
+    bool small_ = false;  // refinement that starts in refine_tail, without lists
     void build_chunk_maps(hipStream_t s);  // cmap_ of every sub-round (after chunk_prefix_)
     int subrounds_ = 1;
     int num_labels_ = 0;
