@@ -126,3 +126,24 @@ def test_autotune_bins_keeps_results():
     assert np.array_equal(q1, q2)
     g.free()
     b.free()
+
+
+@pytest.mark.parametrize("sizes", [[31] * 200, [1023, 1024, 1025, 2], [5000, 1, 1, 7000],
+                                   [9000]])
+def test_cuts_and_weights_around_the_tiles(sizes):
+    """Per-graph cuts and weights where a tile (1024 nodes, 4096 edges) lies in one graph, ends
+    with one, or spans many."""
+    gs = []
+    for i, n in enumerate(sizes):
+        x, a, _, _ = GR.gen_rgg(n, i + 1) if n > 2 else (np.zeros(n + 1, np.int32),
+                                                         np.zeros(0, np.int32), None, None)
+        vw = np.random.default_rng(i).integers(1, 9, n).astype(np.int32)
+        gs.append((x, a, vw, None))
+    b = K.Batch.from_graphs(gs)
+    part, cuts, mbw, _ = b.partition(k=2, seed=1)
+    off = b.info()["node_off"]
+    for g, (x, a, vw, _) in enumerate(gs):
+        p = part[off[g]:off[g + 1]]
+        assert cuts[g] == O.edge_cut(x, a, None, p)
+        assert mbw[g] == O.block_weights(vw, 2, p).max()
+    b.free()
