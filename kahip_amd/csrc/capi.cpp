@@ -784,6 +784,7 @@ int kahip_mlp_gradient(int count, const float* features, const float* labels,
                                 hipMemcpyHostToDevice, s));
         KH_CHECK(hipMemcpyAsync(y.p, labels, sizeof(float) * count, hipMemcpyHostToDevice, s));
         KH_CHECK(hipMemcpyAsync(w.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, s));
+        eng.rw.train_begin(w.p, s);
         eng.rw.train_step(f.p, y.p, count, w.p, nullptr, nullptr, g.p, 1, 0.f, l.p, s);
         float hl = 0;
         KH_CHECK(hipMemcpyAsync(grads, g.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, s));
@@ -816,6 +817,7 @@ int kahip_mlp_train(long long count, const float* features, const float* labels,
         std::vector<float> zeros(kMlpParams, 0.f), hl(steps_per_epoch);
         KH_CHECK(hipMemcpyAsync(m.p, zeros.data(), sizeof(float) * kMlpParams, hipMemcpyHostToDevice, s));
         KH_CHECK(hipMemcpyAsync(v.p, zeros.data(), sizeof(float) * kMlpParams, hipMemcpyHostToDevice, s));
+        eng.rw.train_begin(w.p, s);
         int step = 0;
         for (int ep = 0; ep < epochs; ++ep) {
             for (long long i = 0; i < steps_per_epoch; ++i) {

@@ -318,51 +318,123 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const IN* __restrict__
 // gradients and the loss are fp32 sums over the edges (lane shuffles, then the four waves in
 // order). Per-workgroup gradients go to `partial` and are summed in a fixed order, so training
 // is deterministic.
+//
+// A step of 4096 examples is 64 workgroups, a quarter of the chip, so it is bound by the latency
+// of one workgroup and by the launches: the BF16 operands of W1, W2 and W2^T come packed (TrainPack,
+// 16-byte loads; kept current by the update kernel) instead of about 200 scattered floats a lane,
+// the backward's LDS tiles are stored with the edges along the rows, so that an operand is one
+// 16-byte LDS read instead of eight 2-byte ones, and the sums over 16 lanes are DPP moves. Same
+// roundings, products and orders of summation as before: the same bits. Measured at batch 4096:
+// train_kernel 14.3 -> 6.7 us, gradient reduction + Adam 21.0 us in two launches -> 4.0 us
+// in one.
 constexpr int kTB = 64;  // examples per workgroup
+constexpr int kTBPad = kTB + 8;  // LDS row of a tile: 144 bytes, rows start in different banks
 
-__device__ inline float sum16(float x) {  // sum over the 16 lanes of a lane group (fixed tree)
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) x += __shfl_xor(x, o, 64);
+// BF16 operands of the training products, one 8-element vector per lane:
+//   [0, kPackA1 + kPackA2)  A1 and A2 as in the packed weights of mlp_forward_kernel
+//   then T2[kb][tk][lane]   W2[hid(kb, g, j)][16 tk + lane%16]
+constexpr int kPackT2 = 2 * 4 * 64 * 8;
+constexpr int kTrainPack = kPackBf16 + kPackT2;
+
+// (kb, g, j) of hidden unit h: the inverse of hid_of
+__device__ inline void hid_place(int h, int& kb, int& g, int& j) {
+    const int q = h >> 4;
+    kb = q >> 1;
+    g = (h >> 2) & 3;
+    j = ((q & 1) << 2) + (h & 3);
+}
+
+// Writes parameter p's value to its places in the pack (weights of W1 and W2 only).
+__device__ inline void pack_param(int p, float x, __bf16* __restrict__ pack) {
+    const __bf16 b = (__bf16)x;
+    int kb, g, j;
+    if (p < kOffB1) {
+        const int h = p / kFeatures, k = p % kFeatures;  // lane group 0: k < 8
+        pack[((h >> 4) * 64 + (h & 15)) * 8 + k] = b;
+    } else if (p >= kOffW2 && p < kOffB2) {
+        const int h = (p - kOffW2) / kHidden, c = (p - kOffW2) % kHidden;
+        hid_place(c, kb, g, j);
+        pack[kPackA1 + (((h >> 4) * 2 + kb) * 64 + g * 16 + (h & 15)) * 8 + j] = b;
+        hid_place(h, kb, g, j);
+        pack[kPackBf16 + ((kb * 4 + (c >> 4)) * 64 + g * 16 + (c & 15)) * 8 + j] = b;
+    }
+}
+
+__global__ void pack_train_kernel(const float* __restrict__ params, __bf16* __restrict__ pack) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    // A1 slots of lane groups 1..3 (k >= 8) are zero
+    if (i < kPackA1 && ((i >> 3) & 63) >= 16) pack[i] = (__bf16)0.f;
+    if (i < kMlpParams) pack_param(i, params[i], pack);
+}
+
+// Sum over the 16 lanes of a lane group, valid in its first lane (fixed tree: lane xor 1, 2, 4, 8;
+// for the lanes that reach the first one, a rotation by 12 is xor 4 and one by 8 is xor 8).
+template <int CTRL>
+__device__ inline float dpp(float x) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+}
+__device__ inline float sum16_tail(float x) {
+    x += dpp<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+    x += dpp<0x12C>(x);  // row_ror 12
+    x += dpp<0x128>(x);  // row_ror 8
     return x;
+}
+__device__ inline float sum16(float x) {
+    return sum16_tail(x + dpp<0xB1>(x));  // quad_perm [1, 0, 3, 2]
+}
+// ... of the products a * b; the first addition is fused with the product.
+__device__ inline float sum16(float a, float b) {
+    return sum16_tail(__builtin_fmaf(a, b, dpp<0xB1>(a * b)));
 }
 
 __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ feat,
                                                     const float* __restrict__ label, int batch,
                                                     const float* __restrict__ params,
+                                                    const __bf16* __restrict__ pack,
                                                     float* __restrict__ partial,
                                                     float* __restrict__ loss_out) {
-    __shared__ __bf16 Xs[kTB][16];          // features (columns 8..15 zero)
-    __shared__ __bf16 H1s[kTB][kHidden];    // layer-1 activations
-    __shared__ __bf16 D2s[kTB][kHidden];    // dL/dZ2
-    __shared__ __bf16 D1s[kTB][kHidden];    // dL/dZ1
+    // tiles with the workgroup's edges along the rows (16-byte aligned rows)
+    __shared__ __align__(16) __bf16 Xs[16][kTBPad];        // features (rows 8..15 zero)
+    __shared__ __align__(16) __bf16 H1s[kHidden][kTBPad];  // layer-1 activations
+    __shared__ __align__(16) __bf16 D2s[kHidden][kTBPad];  // dL/dZ2
+    __shared__ __align__(16) __bf16 D1s[kHidden][kTBPad];  // dL/dZ1
     __shared__ float red[4][3 * kHidden + 2];  // per-wave sums: dW3, db2, db1, db3, loss
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, col = lane & 15;
     const int le = wave * 16 + col;  // the lane's example within the workgroup
     const long long e = (long long)blockIdx.x * kTB + le;
     const bool valid = e < batch;
-    // A operands of the forward (as the packed weights of mlp_forward_kernel)
-    bf16x8 a1[4], a2[4][2];
+    const bf16x8* P = reinterpret_cast<const bf16x8*>(pack);
+    bf16x8 a1[4], a2[4][2], aw[2][4];
+    f32x4 b1[4], b2[4], w3v[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
+        a1[t] = P[t * 64 + lane];
+        b1[t] = *reinterpret_cast<const f32x4*>(params + kOffB1 + 16 * t + 4 * g);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = 8 * g + j;
-            a1[t][j] = (__bf16)(k < kFeatures ? params[kOffW1 + (16 * t + col) * kFeatures + k] : 0.f);
-        }
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                a2[t][kb][j] = (__bf16)params[kOffW2 + (16 * t + col) * kHidden + hid_of(kb, g, j)];
+        for (int kb = 0; kb < 2; ++kb) a2[t][kb] = P[kPackA1 / 8 + (t * 2 + kb) * 64 + lane];
     }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        b2[t] = *reinterpret_cast<const f32x4*>(params + kOffB2 + 16 * t + 4 * g);
+        w3v[t] = *reinterpret_cast<const f32x4*>(params + kOffW3 + 16 * t + 4 * g);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) aw[kb][t] = P[kPackBf16 / 8 + (kb * 4 + t) * 64 + lane];
+    }
+    const float y = valid ? label[e] : 0.f;
     // forward, layer 1: B = the 8 features of edge `col` in lane group 0
     bf16x8 xb = {};
     if (g == 0) {
+        f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+        if (valid) {  // rows of 32 bytes, aligned as the array
+            x0 = *reinterpret_cast<const f32x4*>(feat + e * kFeatures);
+            x1 = *reinterpret_cast<const f32x4*>(feat + e * kFeatures + 4);
+        }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xb[j] = (__bf16)(valid ? feat[e * kFeatures + j] : 0.f);
+        for (int j = 0; j < 8; ++j) xb[j] = (__bf16)(j < 4 ? x0[j & 3] : x1[j & 3]);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) Xs[le][j] = j < 8 ? xb[j] : (__bf16)0.f;
+        for (int j = 0; j < 16; ++j) Xs[j][le] = j < 8 ? xb[j & 7] : (__bf16)0.f;
     }
     f32x4 z1[4];  // Z1[16t + 4g + r][col]
 #pragma unroll
@@ -371,8 +443,8 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
         z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[t], xb, z, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            z1[t][r] = z[r] + params[kOffB1 + 16 * t + 4 * g + r];
-            H1s[le][16 * t + 4 * g + r] = (__bf16)fmaxf(z1[t][r], 0.f);
+            z1[t][r] = z[r] + b1[t][r];
+            H1s[16 * t + 4 * g + r][le] = (__bf16)fmaxf(z1[t][r], 0.f);
         }
     }
     // layer 2 (B operand: the lane's own layer-1 activations in the K order of hid_of)
@@ -388,16 +460,13 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
         for (int t = 0; t < 4; ++t)
             z2[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[t][kb], hb, z2[t], 0, 0, 0);
     }
-    float w3[4][4];
     float acc = 0.f;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int h = 16 * t + 4 * g + r;
-            z2[t][r] += params[kOffB2 + h];
-            w3[t][r] = params[kOffW3 + h];
-            acc += w3[t][r] * fmaxf(z2[t][r], 0.f);
+            z2[t][r] += b2[t][r];
+            acc += w3v[t][r] * fmaxf(z2[t][r], 0.f);
         }
     acc += __shfl_xor(acc, 16, 64);
     acc += __shfl_xor(acc, 32, 64);
@@ -405,7 +474,6 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
     // loss and dL/dz3 of the lane's edge (every lane group holds the same values)
     float d = 0.f, l = 0.f;
     if (valid) {
-        const float y = label[e];
         l = fmaxf(z3, 0.f) - z3 * y + log1pf(expf(-fabsf(z3)));  // BCE with logits, stable form
         d = (1.f / (1.f + expf(-z3)) - y) / (float)batch;
     }
@@ -416,9 +484,9 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            D2[t][r] = z2[t][r] > 0.f ? d * w3[t][r] : 0.f;
-            D2s[le][16 * t + 4 * g + r] = (__bf16)D2[t][r];
-            sw3[t][r] = sum16(d * fmaxf(z2[t][r], 0.f));
+            D2[t][r] = z2[t][r] > 0.f ? d * w3v[t][r] : 0.f;
+            D2s[16 * t + 4 * g + r][le] = (__bf16)D2[t][r];
+            sw3[t][r] = sum16(d, fmaxf(z2[t][r], 0.f));
             sb2[t][r] = sum16(D2[t][r]);
         }
     // dH1 = W2^T D2 (M = 64 inputs of layer 2 in 4 tiles, N = the wave's 16 edges, K = 64)
@@ -431,13 +499,8 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
 #pragma unroll
         for (int j = 0; j < 8; ++j) db[j] = (__bf16)D2[2 * kb + (j >> 2)][j & 3];
 #pragma unroll
-        for (int tk = 0; tk < 4; ++tk) {
-            bf16x8 aw;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                aw[j] = (__bf16)params[kOffW2 + hid_of(kb, g, j) * kHidden + 16 * tk + col];
-            D1[tk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw, db, D1[tk], 0, 0, 0);
-        }
+        for (int tk = 0; tk < 4; ++tk)
+            D1[tk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[kb][tk], db, D1[tk], 0, 0, 0);
     }
     float sb1[4][4];
 #pragma unroll
@@ -445,7 +508,7 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             D1[t][r] = z1[t][r] > 0.f ? D1[t][r] : 0.f;
-            D1s[le][16 * t + 4 * g + r] = (__bf16)D1[t][r];
+            D1s[16 * t + 4 * g + r][le] = (__bf16)D1[t][r];
             sb1[t][r] = sum16(D1[t][r]);
         }
     const float sd = sum16(d), sl = sum16(l);
@@ -466,19 +529,16 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
     }
     __syncthreads();
     float* out = partial + (long long)blockIdx.x * kMlpParams;
-    // dW2 rows 16 wave .. + 15 (A = D2^T from LDS, B = H1 from LDS, K = 64 edges)
+    // dW2 rows 16 wave .. + 15 (A = D2^T and B = H1 from LDS, K = 64 edges)
 #pragma unroll
     for (int tk = 0; tk < 4; ++tk) {
         f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-            bf16x8 a, b;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int ee = 32 * s2 + 8 * g + j;
-                a[j] = D2s[ee][16 * wave + col];
-                b[j] = H1s[ee][16 * tk + col];
-            }
+            const bf16x8 a =
+                *reinterpret_cast<const bf16x8*>(&D2s[16 * wave + col][32 * s2 + 8 * g]);
+            const bf16x8 b =
+                *reinterpret_cast<const bf16x8*>(&H1s[16 * tk + col][32 * s2 + 8 * g]);
             c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
         }
 #pragma unroll
@@ -490,13 +550,9 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
         f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-            bf16x8 a, b;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int ee = 32 * s2 + 8 * g + j;
-                a[j] = D1s[ee][16 * wave + col];
-                b[j] = Xs[ee][col];
-            }
+            const bf16x8 a =
+                *reinterpret_cast<const bf16x8*>(&D1s[16 * wave + col][32 * s2 + 8 * g]);
+            const bf16x8 b = *reinterpret_cast<const bf16x8*>(&Xs[col][32 * s2 + 8 * g]);
             c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
         }
         if (col < kFeatures)
@@ -519,30 +575,49 @@ __global__ __launch_bounds__(256) void train_kernel(const float* __restrict__ fe
     }
 }
 
-__global__ void reduce_grads(int blocks, int batch, const float* __restrict__ partial,
-                             const float* __restrict__ block_loss, float* __restrict__ grads,
-                             float* __restrict__ loss) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < kMlpParams) {
-        float s = 0.f;
-        for (int b = 0; b < blocks; ++b) s += partial[(long long)b * kMlpParams + p];
-        grads[p] = s;
-    } else if (p == kMlpParams && loss) {
-        float s = 0.f;
-        for (int b = 0; b < blocks; ++b) s += block_loss[b];
-        *loss = s / (float)batch;
+// Sum of x[b * stride], b = 0 .. blocks - 1 in order, 32 loads in flight at a time.
+__device__ inline float ordered_sum(const float* __restrict__ x, int blocks, int stride) {
+    constexpr int U = 32;
+    float s = 0.f;
+    int b = 0;
+    for (; b + U <= blocks; b += U) {
+        float v[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) v[j] = x[(long long)(b + j) * stride];
+#pragma unroll
+        for (int j = 0; j < U; ++j) s += v[j];
     }
+    for (; b < blocks; ++b) s += x[(long long)b * stride];
+    return s;
 }
 
-__global__ void adam_kernel(float* __restrict__ params, float* __restrict__ m,
-                            float* __restrict__ v, const float* __restrict__ g, float lr,
-                            float c1, float c2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+// The workgroups' gradients summed in order and, when lr > 0, the Adam update of the parameter
+// and of its packed copies. One thread per parameter in workgroups of one wave, so the 4802 sums
+// spread over 76 CUs.
+__global__ __launch_bounds__(64) void update_kernel(int blocks, int batch,
+                                                    const float* __restrict__ partial,
+                                                    const float* __restrict__ block_loss,
+                                                    float* __restrict__ grads,
+                                                    float* __restrict__ loss,
+                                                    float* __restrict__ params,
+                                                    float* __restrict__ m, float* __restrict__ v,
+                                                    __bf16* __restrict__ pack, float lr, float c1,
+                                                    float c2) {
+    const int p = blockIdx.x * 64 + threadIdx.x;
+    if (p == kMlpParams && loss) *loss = ordered_sum(block_loss, blocks, 1) / (float)batch;
     if (p >= kMlpParams) return;
+    const float g = ordered_sum(partial + p, blocks, kMlpParams);
+    grads[p] = g;
+    if (!(lr > 0.f)) return;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    m[p] = b1 * m[p] + (1.f - b1) * g[p];
-    v[p] = b2 * v[p] + (1.f - b2) * g[p] * g[p];
-    params[p] -= lr * (m[p] / c1) / (sqrtf(v[p] / c2) + eps);
+    // the fused operations are spelled out: their rounding is not left to the compiler's choice
+    const float mp = __builtin_fmaf(b1, m[p], (1.f - b1) * g);
+    const float vp = __builtin_fmaf(g, (1.f - b2) * g, b2 * v[p]);
+    m[p] = mp;
+    v[p] = vp;
+    const float x = params[p] - lr * (mp / c1) / (sqrtf(vp / c2) + eps);
+    params[p] = x;
+    pack_param(p, x, pack);
 }
 
 void pack_weights(const MlpWeights& w, std::vector<uint8_t>& out) {
@@ -696,23 +771,29 @@ void RatingWorkspace::scores(RatingMode mode, const DGraph& g, int bound, uint32
     KH_CHECK(hipGetLastError());
 }
 
+void RatingWorkspace::train_begin(const float* params, hipStream_t s) {
+    tpack_.reserve(kTrainPack);
+    const int threads = kMlpParams > kPackA1 ? kMlpParams : kPackA1;
+    hipLaunchKernelGGL(pack_train_kernel, dim3(grid_for(threads, 256)), dim3(256), 0, s, params,
+                       reinterpret_cast<__bf16*>(tpack_.p));
+    KH_CHECK(hipGetLastError());
+}
+
 void RatingWorkspace::train_step(const float* feat, const float* labels, int batch,
                                  float* params, float* m, float* v, float* grads, int step,
                                  float lr, float* loss, hipStream_t s) {
     KH_REQUIRE(batch > 0, "empty batch");
+    KH_REQUIRE(tpack_.p, "train_begin() not called");
     const int blocks = (batch + kTB - 1) / kTB;
     partial_.reserve((long long)blocks * kMlpParams);
     loss_.reserve(blocks);
+    __bf16* pack = reinterpret_cast<__bf16*>(tpack_.p);
     hipLaunchKernelGGL(train_kernel, dim3(blocks), dim3(256), 0, s, feat, labels, batch, params,
-                       partial_.p, loss_.p);
-    hipLaunchKernelGGL(reduce_grads, dim3(grid_for(kMlpParams + 1, 256)), dim3(256), 0, s, blocks,
-                       batch, partial_.p, loss_.p, grads, loss);
-    if (lr > 0) {
-        const float c1 = 1.f - std::pow(0.9f, (float)step);
-        const float c2 = 1.f - std::pow(0.999f, (float)step);
-        hipLaunchKernelGGL(adam_kernel, dim3(grid_for(kMlpParams, 256)), dim3(256), 0, s, params,
-                           m, v, grads, lr, c1, c2);
-    }
+                       pack, partial_.p, loss_.p);
+    const float c1 = 1.f - std::pow(0.9f, (float)step);
+    const float c2 = 1.f - std::pow(0.999f, (float)step);
+    hipLaunchKernelGGL(update_kernel, dim3(grid_for(kMlpParams + 1, 64)), dim3(64), 0, s, blocks,
+                       batch, partial_.p, loss_.p, grads, loss, params, m, v, pack, lr, c1, c2);
     KH_CHECK(hipGetLastError());
 }
 

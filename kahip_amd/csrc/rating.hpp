@@ -41,6 +41,8 @@ public:
     // score_shift(g) (at least 1) so that a node's score sum stays below 2^31.
     void scores(RatingMode mode, const DGraph& g, int bound, uint32_t seed, const MlpWeights* w,
                 int* score, hipStream_t s, LpWorkspace& lp, Profiler* prof);
+    // Packs params for train_step, which then keeps the pack current.
+    void train_begin(const float* params, hipStream_t s);
     // One optimisation step (Adam, step >= 1) of the mean binary cross-entropy of the MLP on
     // (features, labels); params / m / v / grads are FP32 device arrays of kMlpParams, grads
     // receives the mean gradient and *loss (device, may be null) the mean loss; lr = 0 only
@@ -59,7 +61,7 @@ private:
     DevBuf<unsigned long long> sig_;
     DevBuf<int> lab_, size_, map_, heavy_, rec_;
     DevBuf<float> feat_, logit_, partial_, loss_;
-    DevBuf<uint16_t> wpack_, featb_;
+    DevBuf<uint16_t> wpack_, featb_, tpack_;
 };
 
 // score = clamp(round(logit * 128) + 2048, 1, kScoreMax); the same formula on the host.

@@ -194,3 +194,33 @@ def test_rated_pipeline_learned_matches_mirror(graphs, name, k, seed, levels):
     assert st["level_n"] == info["level_n"]
     assert np.array_equal(part, want)
     assert st["ms_rating"] > 0
+
+
+@pytest.mark.parametrize("batch", [1, 63, 64, 65, 2048, 2049, 4161])
+def test_training_steps_match_single_gradients(batch):
+    """Two training steps against Adam on the gradients of mlp_gradient, which packs its operands
+    anew: the second step works on the copies that the first one's update left. Batches around the
+    workgroup of 64 examples and the 32 partial sums in flight."""
+    rng = np.random.default_rng(batch)
+    X = np.abs(rng.normal(size=(2 * batch, 8))).astype(np.float32) * 2
+    y = (rng.random(2 * batch) < 0.4).astype(np.float32)
+    w, lr = rand_params(batch).astype(np.float32), 1e-2
+    b1, b2 = float(np.float32(0.9)), float(np.float32(0.999))
+    a1 = float(np.float32(1) - np.float32(0.9))
+    a2 = float(np.float32(1) - np.float32(0.999))
+    m, v = np.zeros(len(w)), np.zeros(len(w))
+    got = w
+    for step in (1, 2):
+        lo = (step - 1) * batch
+        loss, g = K.mlp_gradient(X[lo:lo + batch], y[lo:lo + batch], got)
+        want_loss, want = R.mlp_loss_grad(X[lo:lo + batch], y[lo:lo + batch], got, bf16=True,
+                                          bf16_backward=True)
+        assert abs(loss - want_loss) <= 1e-5 * (1 + abs(want_loss))
+        assert np.linalg.norm(g - want) <= 2e-3 * np.linalg.norm(want)
+        g = g.astype(np.float64)
+        m, v = b1 * m + a1 * g, b2 * v + a2 * g * g
+        adam = got - lr * (m / (1 - b1 ** step)) / (np.sqrt(v / (1 - b2 ** step)) + 1e-8)
+        got, losses = K.mlp_train(X[:step * batch], y[:step * batch], w, batch=batch, epochs=1,
+                                  lr=lr)
+        # an update is at most lr / (sqrt(a2) ...) ~ 10 lr; fp32 Adam is good to 1e-5 of it
+        assert np.max(np.abs(got - adam)) <= 1e-3 * lr + 1e-6 * np.abs(w).max()
