@@ -1,8 +1,8 @@
 // extern "C" entry points of libkahip.so (declared in include/kaHIP_interface.h and
 // include/kahip_amd.h). Host arrays are copied to the GPU, the work runs on a stream, results
 // are copied back. State that survives a call: the thread-local last error and last profile
-// summary, and the partition entry points' cached engine per device (its stream and device
-// workspaces, reused by the next call on that device; kahip_release_workspaces frees them).
+// summary, and the cached engine per device (its stream and device workspaces, reused by the next
+// call on that device; kahip_release_workspaces frees them).
 
 #include <algorithm>
 #include <climits>
@@ -14,6 +14,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <optional>
 #include <queue>
 #include <sstream>
 #include <string>
@@ -56,9 +57,10 @@ int guarded(F&& f) {
     return 1;
 }
 
-// The partition entry points (kaffpa, kahip_partition, kahip_batch_partition) run on a cached
-// engine of the current device, so that a repeated call reuses the device workspaces sized by
-// the previous ones instead of allocating (and freeing) them inside the call; every workspace is
+// The entry points run on a cached engine of the current device, so that a repeated call reuses
+// the device workspaces sized by the previous ones instead of allocating (and freeing) them inside
+// the call (a stream, about 35 buffers and 6 of the 22 ms of kahip_contract on R-MAT 2^19); every
+// workspace is
 // re-initialised by the kernels that use it, exactly as between two levels of one call. A call
 // that finds the device's engine held by another thread runs on an engine of its own, and a call
 // that fails drops the cached engine. The cache is never destroyed at exit (its memory goes with
@@ -163,16 +165,65 @@ PartitionParams to_params(const kahip_params* q) {
     return p;
 }
 
-void check_csr(int n, const int* xadj, const int* adjncy) {
+// Whether every p[i] lies in [0, hi) (no early exit: the loop vectorises).
+bool in_range(const int* p, long long n, int hi) {
+    unsigned bad = 0;
+    for (long long i = 0; i < n; ++i) bad |= (unsigned)((unsigned)p[i] >= (unsigned)hi);
+    return bad == 0;
+}
+
+// The offsets of a host CSR; its targets are checked by check_targets or, on the GPU, by the
+// upload.
+void check_rows(int n, const int* xadj, const int* adjncy) {
     KH_REQUIRE(n >= 0, "n must be non-negative");
     KH_REQUIRE(xadj != nullptr, "xadj is NULL");
     KH_REQUIRE(xadj[0] == 0, "xadj[0] must be 0");
-    for (int v = 0; v < n; ++v) KH_REQUIRE(xadj[v + 1] >= xadj[v], "xadj must be non-decreasing");
-    const long long m2 = xadj[n];
-    KH_REQUIRE(m2 == 0 || adjncy != nullptr, "adjncy is NULL");
-    for (long long e = 0; e < m2; ++e)
-        KH_REQUIRE(adjncy[e] >= 0 && adjncy[e] < n, "adjncy entry out of range");
+    unsigned bad = 0;
+    for (int v = 0; v < n; ++v) bad |= (unsigned)(xadj[v + 1] < xadj[v]);
+    KH_REQUIRE(bad == 0, "xadj must be non-decreasing");
+    KH_REQUIRE(xadj[n] == 0 || adjncy != nullptr, "adjncy is NULL");
 }
+
+constexpr const char* kBadTarget = "adjncy entry out of range";
+
+void check_csr(int n, const int* xadj, const int* adjncy) {
+    check_rows(n, xadj, adjncy);
+    KH_REQUIRE(in_range(adjncy, xadj[n], n), kBadTarget);
+}
+
+// Runs f(engine, graph, stream) on the device's kept engine and the host CSR, uploaded into the
+// engine's graph, or into *own (then f only sees it uploaded). Refuses a bad CSR, then what
+// check() refuses, before f; the refusals do not depend on a GPU, and the engine stays kept.
+template <class C, class F>
+void with_host_graph(int n, const int* xadj, const int* adjncy, const int* vwgt,
+                     const int* adjwgt, OwnedGraph* own, C&& check, F&& f) {
+    check_rows(n, xadj, adjncy);
+    std::optional<EngineLease> lease;
+    try {
+        lease.emplace();
+    } catch (...) {
+        KH_REQUIRE(in_range(adjncy, xadj[n], n), kBadTarget);
+        check();
+        throw;
+    }
+    Engine& eng = **lease;
+    OwnedGraph& g = own ? *own : eng.io.in;
+    std::exception_ptr refused;
+    if (!upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, eng.stream(), &eng.io.bad)) {
+        refused = std::make_exception_ptr(Error(kBadTarget));
+    } else {
+        try {
+            check();
+        } catch (...) {
+            refused = std::current_exception();
+        }
+    }
+    if (!refused) f(eng, g.g, eng.stream());
+    lease.reset();
+    if (refused) std::rethrow_exception(refused);
+}
+
+constexpr auto kNoCheck = [] {};
 
 std::string profile_json(const Profiler& prof) {
     std::ostringstream os;
@@ -219,16 +270,16 @@ void fill_stats(const PartitionStats& s, kahip_stats* o) {
 int run_kaffpa(int n, const int* vwgt, const int* xadj, const int* adjcwgt, const int* adjncy,
                const kahip_params* params, int* edgecut, int* part, kahip_stats* stats) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        PartitionParams p = to_params(params);
-        EngineLease eng;
-        OwnedGraph g;
-        upload_graph(n, xadj, adjncy, vwgt, adjcwgt, g, eng->stream());
-        PartitionStats st;
-        eng->partition(g.g, p, part, &st);
-        if (p.profile) g_last_profile = profile_json(eng->prof);
-        if (edgecut) *edgecut = (int)st.cut;
-        fill_stats(st, stats);
+        PartitionParams p;
+        auto check = [&] { p = to_params(params); };
+        with_host_graph(n, xadj, adjncy, vwgt, adjcwgt, nullptr, check,
+                        [&](Engine& eng, DGraph& g, hipStream_t) {
+            PartitionStats st;
+            eng.partition(g, p, part, &st);
+            if (p.profile) g_last_profile = profile_json(eng.prof);
+            if (edgecut) *edgecut = (int)st.cut;
+            fill_stats(st, stats);
+        });
     });
 }
 
@@ -368,19 +419,10 @@ int kahip_rebalance(int n, const int* xadj, const int* adjncy, const int* vwgt,
 int kahip_graph_from_host(int n, const int* xadj, const int* adjncy, const int* vwgt,
                           const int* adjwgt, kahip_graph_t* out) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        auto* g = new kahip_graph();
-        hipStream_t s;
-        KH_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-        try {
-            upload_graph(n, xadj, adjncy, vwgt, adjwgt, g->og, s);
-        } catch (...) {
-            (void)hipStreamDestroy(s);
-            delete g;
-            throw;
-        }
-        KH_CHECK(hipStreamDestroy(s));
-        *out = g;
+        auto g = std::make_unique<kahip_graph>();
+        with_host_graph(n, xadj, adjncy, vwgt, adjwgt, &g->og, kNoCheck,
+                        [](Engine&, DGraph&, hipStream_t) {});
+        *out = g.release();
     });
 }
 
@@ -472,43 +514,39 @@ int kahip_lp_cluster(int n, const int* xadj, const int* adjncy, const int* vwgt,
                      const int* adjwgt, int bound, int rounds, int subrounds, unsigned seed,
                      int* cluster, int* num_clusters, int* moves_per_round) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        Engine eng;
-        hipStream_t s = eng.stream();
-        OwnedGraph g;
-        upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, s);
-        DevBuf<int> label, size, map;
-        label.reserve(n);
-        size.reserve(n);
-        map.reserve(n);
-        LpWorkspace::init_cluster_labels(g.g, label.p, size.p, s);
-        BinConfig bins;
-        eng.lp.prepare(LpMode::Cluster, g.g, n, subrounds, seed, bins, s);
-        eng.lp.run(LpMode::Cluster, g.g, label.p, size.p, bound, rounds, seed, s, nullptr,
-                   "lp_cluster");
-        eng.lp.check(s);
-        if (moves_per_round) eng.lp.read_moves(rounds, moves_per_round, s);
-        const int nc = eng.cw.remap(g.g, label.p, map.p, s, nullptr);
-        if (n) KH_CHECK(hipMemcpyAsync(cluster, map.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
-        if (num_clusters) *num_clusters = nc;
+        with_host_graph(n, xadj, adjncy, vwgt, adjwgt, nullptr, kNoCheck,
+                        [&](Engine& eng, DGraph& g, hipStream_t s) {
+            int* label = eng.io.i[0].reserve(n);
+            int* size = eng.io.i[1].reserve(n);
+            int* map = eng.io.i[2].reserve(n);
+            LpWorkspace::init_cluster_labels(g, label, size, s);
+            BinConfig bins;
+            eng.lp.prepare(LpMode::Cluster, g, n, subrounds, seed, bins, s);
+            eng.lp.run(LpMode::Cluster, g, label, size, bound, rounds, seed, s, nullptr,
+                       "lp_cluster");
+            eng.lp.check(s);
+            if (moves_per_round) eng.lp.read_moves(rounds, moves_per_round, s);
+            const int nc = eng.cw.remap(g, label, map, s, nullptr);
+            if (n) KH_CHECK(hipMemcpyAsync(cluster, map, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+            KH_CHECK(hipStreamSynchronize(s));
+            if (num_clusters) *num_clusters = nc;
+        });
     });
 }
 
 int kahip_remap(int n, const int* label, int* map, int* num_clusters) {
     return guarded([&] {
         KH_REQUIRE(n >= 0, "n must be non-negative");
-        for (int v = 0; v < n; ++v) KH_REQUIRE(label[v] >= 0 && label[v] < n, "label out of range");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        DevBuf<int> dl, dm;
-        dl.reserve(n);
-        dm.reserve(n);
-        if (n) KH_CHECK(hipMemcpyAsync(dl.p, label, sizeof(int) * n, hipMemcpyHostToDevice, s));
+        KH_REQUIRE(in_range(label, n, n), "label out of range");
+        EngineLease eng;
+        hipStream_t s = eng->stream();
+        int* dl = eng->io.i[0].reserve(n);
+        int* dm = eng->io.i[1].reserve(n);
+        if (n) KH_CHECK(hipMemcpyAsync(dl, label, sizeof(int) * n, hipMemcpyHostToDevice, s));
         DGraph g;
         g.n = n;
-        const int nc = eng.cw.remap(g, dl.p, dm.p, s, nullptr);
-        if (n) KH_CHECK(hipMemcpyAsync(map, dm.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+        const int nc = eng->cw.remap(g, dl, dm, s, nullptr);
+        if (n) KH_CHECK(hipMemcpyAsync(map, dm, sizeof(int) * n, hipMemcpyDeviceToHost, s));
         KH_CHECK(hipStreamSynchronize(s));
         if (num_clusters) *num_clusters = nc;
     });
@@ -517,24 +555,24 @@ int kahip_remap(int n, const int* label, int* map, int* num_clusters) {
 int kahip_contract(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
                    const int* map, int nc, int* cxadj, int* cadjncy, int* cadjwgt, int* cvwgt) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        KH_REQUIRE(nc >= 0 && (n == 0 || nc >= 1), "bad number of clusters");
-        for (int v = 0; v < n; ++v) KH_REQUIRE(map[v] >= 0 && map[v] < nc, "map out of range");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        OwnedGraph g, c;
-        upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, s);
-        DevBuf<int> dm;
-        dm.reserve(n);
-        if (n) KH_CHECK(hipMemcpyAsync(dm.p, map, sizeof(int) * n, hipMemcpyHostToDevice, s));
-        eng.cw.contract(g.g, dm.p, nc, c, s, nullptr);
-        KH_CHECK(hipMemcpyAsync(cxadj, c.g.xadj, sizeof(int) * (nc + 1), hipMemcpyDeviceToHost, s));
-        if (c.g.m2) {
-            KH_CHECK(hipMemcpyAsync(cadjncy, c.g.adjncy, sizeof(int) * c.g.m2, hipMemcpyDeviceToHost, s));
-            KH_CHECK(hipMemcpyAsync(cadjwgt, c.g.adjwgt, sizeof(int) * c.g.m2, hipMemcpyDeviceToHost, s));
-        }
-        if (nc) KH_CHECK(hipMemcpyAsync(cvwgt, c.g.vwgt, sizeof(int) * nc, hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
+        auto check = [&] {
+            KH_REQUIRE(nc >= 0 && (n == 0 || nc >= 1), "bad number of clusters");
+            KH_REQUIRE(in_range(map, n, nc), "map out of range");
+        };
+        with_host_graph(n, xadj, adjncy, vwgt, adjwgt, nullptr, check,
+                        [&](Engine& eng, DGraph& g, hipStream_t s) {
+            OwnedGraph& c = eng.io.out;
+            int* dm = eng.io.i[0].reserve(n);
+            if (n) KH_CHECK(hipMemcpyAsync(dm, map, sizeof(int) * n, hipMemcpyHostToDevice, s));
+            eng.cw.contract(g, dm, nc, c, s, nullptr);
+            KH_CHECK(hipMemcpyAsync(cxadj, c.g.xadj, sizeof(int) * (nc + 1), hipMemcpyDeviceToHost, s));
+            if (c.g.m2) {
+                KH_CHECK(hipMemcpyAsync(cadjncy, c.g.adjncy, sizeof(int) * c.g.m2, hipMemcpyDeviceToHost, s));
+                KH_CHECK(hipMemcpyAsync(cadjwgt, c.g.adjwgt, sizeof(int) * c.g.m2, hipMemcpyDeviceToHost, s));
+            }
+            if (nc) KH_CHECK(hipMemcpyAsync(cvwgt, c.g.vwgt, sizeof(int) * nc, hipMemcpyDeviceToHost, s));
+            KH_CHECK(hipStreamSynchronize(s));
+        });
     });
 }
 
@@ -542,40 +580,36 @@ int kahip_lp_refine(int n, const int* xadj, const int* adjncy, const int* vwgt,
                     const int* adjwgt, int k, int bound, int rounds, int subrounds, unsigned seed,
                     int* part, int* moves_per_round) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        KH_REQUIRE(k >= 1 && k <= 65536, "k must be in [1, 65536]");
-        for (int v = 0; v < n; ++v) KH_REQUIRE(part[v] >= 0 && part[v] < k, "part out of range");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        OwnedGraph g;
-        upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, s);
-        DevBuf<int> dp, W;
-        dp.reserve(n);
-        W.reserve(k);
-        if (n) KH_CHECK(hipMemcpyAsync(dp.p, part, sizeof(int) * n, hipMemcpyHostToDevice, s));
-        compute_block_weights(g.g, dp.p, k, W.p, s);
-        BinConfig bins;
-        eng.lp.prepare(LpMode::Refine, g.g, k, subrounds, seed, bins, s);
-        eng.lp.run(LpMode::Refine, g.g, dp.p, W.p, bound, rounds, seed, s, nullptr, "lp_refine");
-        eng.lp.check(s);
-        if (moves_per_round) eng.lp.read_moves(rounds, moves_per_round, s);
-        if (n) KH_CHECK(hipMemcpyAsync(part, dp.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
+        auto check = [&] {
+            KH_REQUIRE(k >= 1 && k <= 65536, "k must be in [1, 65536]");
+            KH_REQUIRE(in_range(part, n, k), "part out of range");
+        };
+        with_host_graph(n, xadj, adjncy, vwgt, adjwgt, nullptr, check,
+                        [&](Engine& eng, DGraph& g, hipStream_t s) {
+            int* dp = eng.io.i[0].reserve(n);
+            int* W = eng.io.i[1].reserve(k);
+            if (n) KH_CHECK(hipMemcpyAsync(dp, part, sizeof(int) * n, hipMemcpyHostToDevice, s));
+            compute_block_weights(g, dp, k, W, s);
+            BinConfig bins;
+            eng.lp.prepare(LpMode::Refine, g, k, subrounds, seed, bins, s);
+            eng.lp.run(LpMode::Refine, g, dp, W, bound, rounds, seed, s, nullptr, "lp_refine");
+            eng.lp.check(s);
+            if (moves_per_round) eng.lp.read_moves(rounds, moves_per_round, s);
+            if (n) KH_CHECK(hipMemcpyAsync(part, dp, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+            KH_CHECK(hipStreamSynchronize(s));
+        });
     });
 }
 
 int kahip_edge_cut(int n, const int* xadj, const int* adjncy, const int* adjwgt, const int* part,
                    long long* cut) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        Engine eng;
-        hipStream_t s = eng.stream();
-        OwnedGraph g;
-        upload_graph(n, xadj, adjncy, nullptr, adjwgt, g, s);
-        DevBuf<int> dp;
-        dp.reserve(n);
-        if (n) KH_CHECK(hipMemcpyAsync(dp.p, part, sizeof(int) * n, hipMemcpyHostToDevice, s));
-        *cut = eng.mw.edge_cut(g.g, dp.p, s, nullptr);
+        with_host_graph(n, xadj, adjncy, nullptr, adjwgt, nullptr, kNoCheck,
+                        [&](Engine& eng, DGraph& g, hipStream_t s) {
+            int* dp = eng.io.i[0].reserve(n);
+            if (n) KH_CHECK(hipMemcpyAsync(dp, part, sizeof(int) * n, hipMemcpyHostToDevice, s));
+            *cut = eng.mw.edge_cut(g, dp, s, nullptr);
+        });
     });
 }
 
@@ -591,29 +625,23 @@ int kahip_quality_noalloc(int n, long long m2, const int* xadj, const int* adjnc
 int kahip_block_weights(int n, const int* vwgt, int k, const int* part, long long* weights) {
     return guarded([&] {
         KH_REQUIRE(n >= 0 && k >= 1 && k <= 65536, "bad n or k");
-        for (int v = 0; v < n; ++v) KH_REQUIRE(part[v] >= 0 && part[v] < k, "part out of range");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        DevBuf<int> dp, dv, W;
-        dp.reserve(n);
-        dv.reserve(n);
-        W.reserve(k);
+        KH_REQUIRE(in_range(part, n, k), "part out of range");
+        EngineLease eng;
+        hipStream_t s = eng->stream();
+        int* dp = eng->io.i[0].reserve(n);
+        int* dv = eng->io.i[1].reserve(n);
+        int* W = eng->io.i[2].reserve(k);
         DGraph g;
         g.n = n;
-        g.vwgt = dv.p;
+        g.vwgt = dv;
         if (n) {
-            KH_CHECK(hipMemcpyAsync(dp.p, part, sizeof(int) * n, hipMemcpyHostToDevice, s));
-            if (vwgt) {
-                KH_CHECK(hipMemcpyAsync(dv.p, vwgt, sizeof(int) * n, hipMemcpyHostToDevice, s));
-            } else {
-                std::vector<int> ones(n, 1);
-                KH_CHECK(hipMemcpyAsync(dv.p, ones.data(), sizeof(int) * n, hipMemcpyHostToDevice, s));
-                KH_CHECK(hipStreamSynchronize(s));
-            }
+            KH_CHECK(hipMemcpyAsync(dp, part, sizeof(int) * n, hipMemcpyHostToDevice, s));
+            if (vwgt) KH_CHECK(hipMemcpyAsync(dv, vwgt, sizeof(int) * n, hipMemcpyHostToDevice, s));
+            else fill_async(dv, n, 1, s);
         }
-        compute_block_weights(g, dp.p, k, W.p, s);
+        compute_block_weights(g, dp, k, W, s);
         std::vector<int> h(k);
-        KH_CHECK(hipMemcpyAsync(h.data(), W.p, sizeof(int) * k, hipMemcpyDeviceToHost, s));
+        KH_CHECK(hipMemcpyAsync(h.data(), W, sizeof(int) * k, hipMemcpyDeviceToHost, s));
         KH_CHECK(hipStreamSynchronize(s));
         for (int b = 0; b < k; ++b) weights[b] = h[b];
     });
@@ -623,17 +651,16 @@ int kahip_project(int n_fine, const int* map, int n_coarse, const int* coarse_pa
                   int* fine_part) {
     return guarded([&] {
         KH_REQUIRE(n_fine >= 0 && n_coarse >= 0, "bad sizes");
-        for (int v = 0; v < n_fine; ++v) KH_REQUIRE(map[v] >= 0 && map[v] < n_coarse, "map out of range");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        DevBuf<int> dm, dc, df;
-        dm.reserve(n_fine);
-        dc.reserve(n_coarse);
-        df.reserve(n_fine);
-        if (n_fine) KH_CHECK(hipMemcpyAsync(dm.p, map, sizeof(int) * n_fine, hipMemcpyHostToDevice, s));
-        if (n_coarse) KH_CHECK(hipMemcpyAsync(dc.p, coarse_part, sizeof(int) * n_coarse, hipMemcpyHostToDevice, s));
-        project_partition(n_fine, dm.p, dc.p, df.p, s, nullptr);
-        if (n_fine) KH_CHECK(hipMemcpyAsync(fine_part, df.p, sizeof(int) * n_fine, hipMemcpyDeviceToHost, s));
+        KH_REQUIRE(in_range(map, n_fine, n_coarse), "map out of range");
+        EngineLease eng;
+        hipStream_t s = eng->stream();
+        int* dm = eng->io.i[0].reserve(n_fine);
+        int* dc = eng->io.i[1].reserve(n_coarse);
+        int* df = eng->io.i[2].reserve(n_fine);
+        if (n_fine) KH_CHECK(hipMemcpyAsync(dm, map, sizeof(int) * n_fine, hipMemcpyHostToDevice, s));
+        if (n_coarse) KH_CHECK(hipMemcpyAsync(dc, coarse_part, sizeof(int) * n_coarse, hipMemcpyHostToDevice, s));
+        project_partition(n_fine, dm, dc, df, s, nullptr);
+        if (n_fine) KH_CHECK(hipMemcpyAsync(fine_part, df, sizeof(int) * n_fine, hipMemcpyDeviceToHost, s));
         KH_CHECK(hipStreamSynchronize(s));
     });
 }
@@ -695,32 +722,28 @@ int kahip_fm_refine(int n, const int* xadj, const int* adjncy, const int* vwgt,
 int kahip_edge_features(int n, const int* xadj, const int* adjncy, const int* vwgt,
                         const int* adjwgt, int bound, unsigned seed, float* features) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        Engine eng;
-        hipStream_t s = eng.stream();
-        OwnedGraph g;
-        upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, s);
-        DevBuf<float> f;
-        f.reserve(std::max<long long>(g.g.m2 * kFeatures, 1));
-        eng.rw.features(g.g, bound, seed, f.p, s, eng.lp, nullptr);
-        if (g.g.m2)
-            KH_CHECK(hipMemcpyAsync(features, f.p, sizeof(float) * kFeatures * g.g.m2,
-                                    hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
+        with_host_graph(n, xadj, adjncy, vwgt, adjwgt, nullptr, kNoCheck,
+                        [&](Engine& eng, DGraph& g, hipStream_t s) {
+            float* f = eng.io.f[0].reserve(std::max<long long>(g.m2 * kFeatures, 1));
+            eng.rw.features(g, bound, seed, f, s, eng.lp, nullptr);
+            if (g.m2)
+                KH_CHECK(hipMemcpyAsync(features, f, sizeof(float) * kFeatures * g.m2,
+                                        hipMemcpyDeviceToHost, s));
+            KH_CHECK(hipStreamSynchronize(s));
+        });
     });
 }
 
 int kahip_graph_edge_features(kahip_graph_t g, int bound, unsigned seed, float* features) {
     return guarded([&] {
         KH_REQUIRE(g, "null graph");
-        Engine eng;
-        hipStream_t s = eng.stream();
+        EngineLease eng;
+        hipStream_t s = eng->stream();
         const DGraph& d = g->og.g;
-        DevBuf<float> f;
-        f.reserve(std::max<long long>(d.m2 * kFeatures, 1));
-        eng.rw.features(d, bound, seed, f.p, s, eng.lp, nullptr);
+        float* f = eng->io.f[0].reserve(std::max<long long>(d.m2 * kFeatures, 1));
+        eng->rw.features(d, bound, seed, f, s, eng->lp, nullptr);
         if (d.m2)
-            KH_CHECK(hipMemcpyAsync(features, f.p, sizeof(float) * kFeatures * d.m2,
+            KH_CHECK(hipMemcpyAsync(features, f, sizeof(float) * kFeatures * d.m2,
                                     hipMemcpyDeviceToHost, s));
         KH_CHECK(hipStreamSynchronize(s));
     });
@@ -731,18 +754,17 @@ int kahip_mlp_forward(long long count, const float* features, const float* param
     return guarded([&] {
         KH_REQUIRE(count >= 0, "count must be non-negative");
         KH_REQUIRE(params, "params is NULL");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        DevBuf<float> f, o;
-        f.reserve(std::max<long long>(count * kFeatures, 1));
-        o.reserve(std::max<long long>(count, 1));
+        EngineLease eng;
+        hipStream_t s = eng->stream();
+        float* f = eng->io.f[0].reserve(std::max<long long>(count * kFeatures, 1));
+        float* o = eng->io.f[1].reserve(std::max<long long>(count, 1));
         if (count)
-            KH_CHECK(hipMemcpyAsync(f.p, features, sizeof(float) * kFeatures * count,
+            KH_CHECK(hipMemcpyAsync(f, features, sizeof(float) * kFeatures * count,
                                     hipMemcpyHostToDevice, s));
-        eng.rw.mlp_forward(f.p, count, *reinterpret_cast<const MlpWeights*>(params), o.p, s,
-                           nullptr);
+        eng->rw.mlp_forward(f, count, *reinterpret_cast<const MlpWeights*>(params), o, s,
+                            nullptr);
         if (count)
-            KH_CHECK(hipMemcpyAsync(logits, o.p, sizeof(float) * count, hipMemcpyDeviceToHost, s));
+            KH_CHECK(hipMemcpyAsync(logits, o, sizeof(float) * count, hipMemcpyDeviceToHost, s));
         KH_CHECK(hipStreamSynchronize(s));
     });
 }
@@ -751,20 +773,19 @@ int kahip_edge_scores(int n, const int* xadj, const int* adjncy, const int* vwgt
                       const int* adjwgt, int rating, const float* params, int bound,
                       unsigned seed, int* scores) {
     return guarded([&] {
-        check_csr(n, xadj, adjncy);
-        KH_REQUIRE(rating == 1 || rating == 2, "rating must be EXPANSION_STAR2 or LEARNED");
-        KH_REQUIRE(rating != 2 || params, "learned rating needs params");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        OwnedGraph g;
-        upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, s);
-        DevBuf<int> o;
-        o.reserve(std::max<long long>(g.g.m2, 1));
-        eng.rw.scores((RatingMode)rating, g.g, bound, seed,
-                      reinterpret_cast<const MlpWeights*>(params), o.p, s, eng.lp, nullptr);
-        if (g.g.m2)
-            KH_CHECK(hipMemcpyAsync(scores, o.p, sizeof(int) * g.g.m2, hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
+        auto check = [&] {
+            KH_REQUIRE(rating == 1 || rating == 2, "rating must be EXPANSION_STAR2 or LEARNED");
+            KH_REQUIRE(rating != 2 || params, "learned rating needs params");
+        };
+        with_host_graph(n, xadj, adjncy, vwgt, adjwgt, nullptr, check,
+                        [&](Engine& eng, DGraph& g, hipStream_t s) {
+            int* o = eng.io.i[0].reserve(std::max<long long>(g.m2, 1));
+            eng.rw.scores((RatingMode)rating, g, bound, seed,
+                          reinterpret_cast<const MlpWeights*>(params), o, s, eng.lp, nullptr);
+            if (g.m2)
+                KH_CHECK(hipMemcpyAsync(scores, o, sizeof(int) * g.m2, hipMemcpyDeviceToHost, s));
+            KH_CHECK(hipStreamSynchronize(s));
+        });
     });
 }
 
@@ -772,9 +793,10 @@ int kahip_mlp_gradient(int count, const float* features, const float* labels,
                        const float* params, float* grads, double* loss) {
     return guarded([&] {
         KH_REQUIRE(count > 0, "count must be positive");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        DevBuf<float> f, y, w, g, l;
+        EngineLease eng;
+        hipStream_t s = eng->stream();
+        DevBuf<float>&f = eng->io.f[0], &y = eng->io.f[1], &w = eng->io.f[2], &g = eng->io.f[3],
+              &l = eng->io.f[4];
         f.reserve((long long)count * kFeatures);
         y.reserve(count);
         w.reserve(kMlpParams);
@@ -784,8 +806,8 @@ int kahip_mlp_gradient(int count, const float* features, const float* labels,
                                 hipMemcpyHostToDevice, s));
         KH_CHECK(hipMemcpyAsync(y.p, labels, sizeof(float) * count, hipMemcpyHostToDevice, s));
         KH_CHECK(hipMemcpyAsync(w.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, s));
-        eng.rw.train_begin(w.p, s);
-        eng.rw.train_step(f.p, y.p, count, w.p, nullptr, nullptr, g.p, 1, 0.f, l.p, s);
+        eng->rw.train_begin(w.p, s);
+        eng->rw.train_step(f.p, y.p, count, w.p, nullptr, nullptr, g.p, 1, 0.f, l.p, s);
         float hl = 0;
         KH_CHECK(hipMemcpyAsync(grads, g.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, s));
         KH_CHECK(hipMemcpyAsync(&hl, l.p, sizeof(float), hipMemcpyDeviceToHost, s));
@@ -799,9 +821,10 @@ int kahip_mlp_train(long long count, const float* features, const float* labels,
     return guarded([&] {
         KH_REQUIRE(count > 0 && batch > 0 && epochs >= 0, "bad count / batch / epochs");
         KH_REQUIRE(lr > 0, "lr must be positive");
-        Engine eng;
-        hipStream_t s = eng.stream();
-        DevBuf<float> f, y, w, m, v, g, l;
+        EngineLease eng;
+        hipStream_t s = eng->stream();
+        DevBuf<float>&f = eng->io.f[0], &y = eng->io.f[1], &w = eng->io.f[2], &g = eng->io.f[3],
+              &l = eng->io.f[4], &m = eng->io.f[5], &v = eng->io.f[6];
         f.reserve(count * kFeatures);
         y.reserve(count);
         w.reserve(kMlpParams);
@@ -817,13 +840,13 @@ int kahip_mlp_train(long long count, const float* features, const float* labels,
         std::vector<float> zeros(kMlpParams, 0.f), hl(steps_per_epoch);
         KH_CHECK(hipMemcpyAsync(m.p, zeros.data(), sizeof(float) * kMlpParams, hipMemcpyHostToDevice, s));
         KH_CHECK(hipMemcpyAsync(v.p, zeros.data(), sizeof(float) * kMlpParams, hipMemcpyHostToDevice, s));
-        eng.rw.train_begin(w.p, s);
+        eng->rw.train_begin(w.p, s);
         int step = 0;
         for (int ep = 0; ep < epochs; ++ep) {
             for (long long i = 0; i < steps_per_epoch; ++i) {
                 const long long lo = i * batch;
                 const int b = (int)std::min<long long>(batch, count - lo);
-                eng.rw.train_step(f.p + lo * kFeatures, y.p + lo, b, w.p, m.p, v.p, g.p, ++step,
+                eng->rw.train_step(f.p + lo * kFeatures, y.p + lo, b, w.p, m.p, v.p, g.p, ++step,
                                   lr, l.p + i, s);
             }
             KH_CHECK(hipMemcpyAsync(hl.data(), l.p, sizeof(float) * steps_per_epoch,

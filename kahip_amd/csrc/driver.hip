@@ -30,6 +30,24 @@ __global__ void fill_ones(int* p, long long n) {
     if (i < n) p[i] = 1;
 }
 
+// *bad = 1 if an entry lies outside [0, n). Bound by the read of a (a host loop over the entries
+// takes 0.35 ns each, 11 ms for 31 M; this 30 us). a is 16-byte aligned.
+__global__ __launch_bounds__(256) void check_targets(long long m, const int* __restrict__ a, int n,
+                                                     int* __restrict__ bad) {
+    const long long step = (long long)gridDim.x * 256;
+    const long long t0 = (long long)blockIdx.x * 256 + threadIdx.x;
+    const int4* a4 = reinterpret_cast<const int4*>(a);
+    const unsigned un = (unsigned)n;
+    bool b = false;
+    for (long long i = t0; i < m / 4; i += step) {
+        const int4 x = a4[i];
+        b |= (unsigned)x.x >= un || (unsigned)x.y >= un || (unsigned)x.z >= un ||
+             (unsigned)x.w >= un;
+    }
+    if (t0 < m % 4) b |= (unsigned)a[m - 1 - t0] >= un;
+    if (b) *bad = 1;
+}
+
 // keys[v] = (a[v] << 32) | b[v], ids[v] = v
 __global__ void pair_keys(int n, const int* __restrict__ a, const int* __restrict__ b,
                           unsigned long long* __restrict__ keys, int* __restrict__ ids) {
@@ -95,8 +113,8 @@ int ip_repetitions_for(int k) {
     return std::min(4, reps);
 }
 
-void upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
-                  OwnedGraph& out, hipStream_t s) {
+bool upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
+                  OwnedGraph& out, hipStream_t s, DevBuf<int>* bad) {
     KH_REQUIRE(n >= 0, "n must be non-negative");
     out.alloc_nodes(n);
     const long long m2 = n > 0 ? (long long)xadj[n] : 0;
@@ -104,6 +122,16 @@ void upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, co
     KH_CHECK(hipMemcpyAsync(out.g.xadj, xadj, sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
     if (m2 > 0)
         KH_CHECK(hipMemcpyAsync(out.g.adjncy, adjncy, sizeof(int) * m2, hipMemcpyHostToDevice, s));
+    int is_bad = 0;
+    if (bad && m2 > 0) {
+        bad->reserve(1);
+        fill_async(bad->p, 1, 0, s);
+        hipLaunchKernelGGL(check_targets, dim3(std::min(grid_for(m2, 1024), 2048)), dim3(256), 0, s,
+                           m2, out.g.adjncy, n, bad->p);
+        KH_CHECK(hipMemcpyAsync(&is_bad, bad->p, sizeof(int), hipMemcpyDeviceToHost, s));
+        KH_CHECK(hipStreamSynchronize(s));
+        if (is_bad) return false;
+    }
     long long total = 0;
     if (vwgt) {
         KH_CHECK(hipMemcpyAsync(out.g.vwgt, vwgt, sizeof(int) * n, hipMemcpyHostToDevice, s));
@@ -123,6 +151,7 @@ void upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, co
     out.g.total_vwgt = total;
     out.g.max_degree = maxdeg;
     KH_CHECK(hipStreamSynchronize(s));
+    return true;
 }
 
 void download_graph(const DGraph& g, HostGraph& out, hipStream_t s) {

@@ -115,6 +115,14 @@ public:
     ContractWorkspace cw;
     MetricsWorkspace mw;
     RatingWorkspace rw;
+    // device arrays of the entry points that take host arrays, kept between calls like the
+    // workspaces (grown, never shrunk; written before they are read within a call)
+    struct HostCallBuffers {
+        OwnedGraph in, out;
+        DevBuf<int> i[3];
+        DevBuf<float> f[7];
+        DevBuf<int> bad;
+    } io;
 
 private:
     hipStream_t s_ = nullptr;
@@ -133,9 +141,11 @@ private:
     } buf_;
 };
 
-// Uploads a host CSR (vwgt / adjwgt may be null: unit weights) into an owned device graph.
-void upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
-                  OwnedGraph& out, hipStream_t s);
+// Uploads a host CSR (vwgt / adjwgt may be null: unit weights) into an owned device graph; with
+// `bad` (scratch) the targets are checked on the GPU before anything reads them: false if one lies
+// outside [0, n), the graph is then not usable.
+bool upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
+                  OwnedGraph& out, hipStream_t s, DevBuf<int>* bad = nullptr);
 void download_graph(const DGraph& g, HostGraph& out, hipStream_t s);
 
 }  // namespace kahip
