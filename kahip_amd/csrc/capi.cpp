@@ -209,7 +209,7 @@ void with_host_graph(int n, const int* xadj, const int* adjncy, const int* vwgt,
     Engine& eng = **lease;
     OwnedGraph& g = own ? *own : eng.io.in;
     std::exception_ptr refused;
-    if (!upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, eng.stream(), &eng.io.bad)) {
+    if (!upload_graph(n, xadj, adjncy, vwgt, adjwgt, g, eng.stream(), &eng.io.bad, &eng.mw.mail)) {
         refused = std::make_exception_ptr(Error(kBadTarget));
     } else {
         try {
@@ -780,8 +780,9 @@ int kahip_edge_scores(int n, const int* xadj, const int* adjncy, const int* vwgt
         with_host_graph(n, xadj, adjncy, vwgt, adjwgt, nullptr, check,
                         [&](Engine& eng, DGraph& g, hipStream_t s) {
             int* o = eng.io.i[0].reserve(std::max<long long>(g.m2, 1));
-            eng.rw.scores((RatingMode)rating, g, bound, seed,
-                          reinterpret_cast<const MlpWeights*>(params), o, s, eng.lp, nullptr);
+            if (rating == 2)
+                eng.rw.upload_weights(*reinterpret_cast<const MlpWeights*>(params), s);
+            eng.rw.scores((RatingMode)rating, g, bound, seed, o, s, eng.lp, nullptr);
             if (g.m2)
                 KH_CHECK(hipMemcpyAsync(scores, o, sizeof(int) * g.m2, hipMemcpyDeviceToHost, s));
             KH_CHECK(hipStreamSynchronize(s));

@@ -101,7 +101,7 @@ struct DGraph {
     int* adjwgt = nullptr;
     int* vwgt = nullptr;
     int64_t total_vwgt = 0;
-    int max_degree = 0;
+    int max_degree = 0;  // 0: not known (coarse graphs)
 };
 
 // LP mode shared by clustering (labels = clusters, bound B) and refinement (labels = blocks,

@@ -75,18 +75,29 @@ __global__ void apply_newid(int n, const int* __restrict__ label, const int* __r
 
 __global__ void count_members(int n, const int* __restrict__ xadj, const int* __restrict__ vwgt,
                               const int* __restrict__ map, int* __restrict__ cnt,
-                              int* __restrict__ fdeg, int* __restrict__ cvwgt) {
+                              int* __restrict__ fdeg, int* __restrict__ cvwgt,
+                              int* __restrict__ iota) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= n) return;
+    iota[v] = v;
     const int p = map[v];
     atomicAdd(&cnt[p], 1);
     atomicAdd(&fdeg[p], xadj[v + 1] - xadj[v]);
     atomicAdd(&cvwgt[p], vwgt[v]);
 }
 
-__global__ void iota_kernel(int n, int* __restrict__ out) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) out[v] = v;
+// Per coarse node counters and weights, and the list lengths and error flag (ctl).
+__global__ void init_rows(int nc, int* __restrict__ cnt, int* __restrict__ fdeg,
+                          int* __restrict__ cdeg, int* __restrict__ cvwgt, int m,
+                          int* __restrict__ ctl) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= nc) {
+        cnt[i] = 0;
+        fdeg[i] = 0;
+        cdeg[i] = 0;
+    }
+    if (i < nc) cvwgt[i] = 0;
+    if (i < m) ctl[i] = 0;
 }
 
 // Rows by summed member degree fd (an upper bound of the row's distinct neighbours), so that no
@@ -900,14 +911,11 @@ int ContractWorkspace::remap(const DGraph& g, const int* label, int* map, hipStr
     hipLaunchKernelGGL(leader_min, dim3(grid_for(n, 256)), dim3(256), 0, s, n, label, leader_.p);
     hipLaunchKernelGGL(leader_flag, dim3(grid_for(n, 256)), dim3(256), 0, s, n, label, leader_.p,
                        flag_.p);
-    fill_async(flag_.p + n, 1, 0, s);
-    scan_i32(flag_.p, newid_.p, n + 1, s);
+    scan_i32(flag_.p, newid_.p, n + 1, s);  // newid_[n]: their number
     hipLaunchKernelGGL(apply_newid, dim3(grid_for(n, 256)), dim3(256), 0, s, n, label, leader_.p,
                        newid_.p, map);
-    int nc = 0;
-    KH_CHECK(hipMemcpyAsync(&nc, newid_.p + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
-    return nc;
+    mail_.post(s, {newid_.p + n, 1});
+    return mail_.wait(s)[0];
 }
 
 void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedGraph& out,
@@ -921,18 +929,19 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
     tpos_.reserve(nc + 1);
     cdeg_.reserve(nc + 1);
     members_.reserve(n);
-    fill_async(cnt_.p, nc + 1, 0, s);
-    fill_async(fdeg_.p, nc + 1, 0, s);
-    fill_async(cdeg_.p, nc + 1, 0, s);
-    fill_async(out.g.vwgt, nc, 0, s);
+    // ctl_: lengths of the five LDS tiers' row lists and of the global tier's, error flag
+    constexpr int kCtlGlobal = 5, kCtlErr = 6, kCtlInts = 7;
+    ctl_.reserve(kCtlInts);
+    int* const err = ctl_.p + kCtlErr;
+    hipLaunchKernelGGL(init_rows, dim3(grid_for(std::max(nc + 1, kCtlInts), 256)), dim3(256), 0, s,
+                       nc, cnt_.p, fdeg_.p, cdeg_.p, out.g.vwgt, kCtlInts, ctl_.p);
     if (n > 0) {
+        iota_.reserve(n);
         hipLaunchKernelGGL(count_members, dim3(grid_for(n, 256)), dim3(256), 0, s, n, g.xadj,
-                           g.vwgt, map, cnt_.p, fdeg_.p, out.g.vwgt);
+                           g.vwgt, map, cnt_.p, fdeg_.p, out.g.vwgt, iota_.p);
         // members grouped by cluster, ascending node id inside a group (a stable radix sort of
         // the node ids by cluster)
-        iota_.reserve(n);
         mkeys_.reserve(n);
-        hipLaunchKernelGGL(iota_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, iota_.p);
         int bits = 1;
         while (bits < 31 && (1LL << bits) < (long long)nc) ++bits;
         const unsigned* keys = reinterpret_cast<const unsigned*>(map);
@@ -950,23 +959,19 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
     tq_.reserve(m2);
     tw_.reserve(m2);
     ovl2_list_.reserve(nc);
-    ovl_count_.reserve(1);
-    fill_async(ovl_count_.p, 1, 0, s);
-    err_.reserve(1);
-    fill_async(err_.p, 1, 0, s);
+    int novl = 0;
     if (nc > 0) {
         // algorithmic bytes of the row pass: 12 B per fine edge (target, weight, cluster of
         // target), 12 B per fine node (offsets, member id), 8 B per coarse entry written
         const double bytes = 12.0 * (double)m2 + 12.0 * n;
         for (auto& l : rlist_) l.reserve(nc);
-        rcount_.reserve(5);
-        fill_async(rcount_.p, 5, 0, s);
         hipLaunchKernelGGL(row_bins, dim3(grid_for(nc, 256)), dim3(256), 0, s, nc, fdeg_.p,
                            rlist_[0].p, rlist_[1].p, rlist_[2].p, rlist_[3].p, rlist_[4].p,
-                           rcount_.p, ovl2_list_.p, ovl_count_.p);
-        int rc[3] = {0, 0, 0};
-        KH_CHECK(hipMemcpyAsync(rc, rcount_.p, sizeof(rc), hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
+                           ctl_.p, ovl2_list_.p, ctl_.p + kCtlGlobal);
+        mail_.post(s, {ctl_.p, kCtlErr});
+        const int* const got = mail_.wait(s);
+        const int rc[5] = {got[0], got[1], got[2], got[3], got[4]};
+        novl = got[kCtlGlobal];
         {
             ProfScope ps(prof, "contract_rows_lds", bytes, m2, s);
             if (rc[0] > 0)
@@ -976,29 +981,28 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
             if (rc[1] > 0)
                 hipLaunchKernelGGL((rows_wave<kWaveTierCap[0]>), dim3(rc[1]), dim3(64), 0, s,
                                    rlist_[1].p, rc[1], g.xadj, g.adjncy, g.adjwgt, map, moff_.p,
-                                   members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p, err_.p);
+                                   members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p, err);
             if (rc[2] > 0)
                 hipLaunchKernelGGL((rows_wave<kWaveTierCap[1]>), dim3(rc[2]), dim3(64), 0, s,
                                    rlist_[2].p, rc[2], g.xadj, g.adjncy, g.adjwgt, map, moff_.p,
-                                   members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p, err_.p);
+                                   members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p, err);
         }
         {
             // grid-stride over the device-side counts: five 256-thread workgroups per CU, one
             // 1024-thread workgroup per CU
             ProfScope ps(prof, "contract_rows_lds_big", 0.0, 0, s);
-            hipLaunchKernelGGL((rows_block<kMidThreads, kMidCap>), dim3(256 * 5),
-                               dim3(kMidThreads), 0, s, rlist_[3].p, rcount_.p + 3, g.xadj,
+            if (rc[3] > 0)
+                hipLaunchKernelGGL((rows_block<kMidThreads, kMidCap>), dim3(std::min(rc[3], 256 * 5)),
+                               dim3(kMidThreads), 0, s, rlist_[3].p, ctl_.p + 3, g.xadj,
                                g.adjncy, g.adjwgt, map, moff_.p, members_.p, fdeg_.p, tpos_.p,
-                               cdeg_.p, tq_.p, tw_.p, err_.p);
-            hipLaunchKernelGGL((rows_block<kBigThreads, kBigCap>), dim3(256), dim3(kBigThreads),
-                               0, s, rlist_[4].p, rcount_.p + 4, g.xadj, g.adjncy, g.adjwgt, map,
+                               cdeg_.p, tq_.p, tw_.p, err);
+            if (rc[4] > 0)
+                hipLaunchKernelGGL((rows_block<kBigThreads, kBigCap>), dim3(std::min(rc[4], 256)), dim3(kBigThreads),
+                               0, s, rlist_[4].p, ctl_.p + 4, g.xadj, g.adjncy, g.adjwgt, map,
                                moff_.p, members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p,
-                               err_.p);
+                               err);
         }
     }
-    int novl = 0;
-    KH_CHECK(hipMemcpyAsync(&novl, ovl_count_.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
     if (novl > 0) {
         ProfScope ps(prof, "contract_rows_global", 0.0, novl, s);
         ofd_.reserve(novl);
@@ -1053,13 +1057,11 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
         gpart_.reserve((long long)nchunks * kGChunk);
         gbig_.reserve(std::max(ntasks, 1));
         gnbig_.reserve(1);
-        fill_async(gcnt_.p + ct_total, 1, 0, s);  // sentinel
         fill_async(gnbig_.p, 1, 0, s);
         mdeg_.reserve((long long)n + 1);
         mpre_.reserve((long long)n + 1);
         hipLaunchKernelGGL(member_degrees, dim3(grid_for(n, 256)), dim3(256), 0, s, n,
                            members_.p, g.xadj, mdeg_.p);
-        fill_async(mdeg_.p + n, 1, 0, s);
         scan_i32(mdeg_.p, mpre_.p, n + 1, s);
         stage_q_.reserve(std::max<long long>(m2, 1));
         stage_w_.reserve(std::max<long long>(m2, 1));
@@ -1070,15 +1072,15 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
                            gdb_.p);
         hipLaunchKernelGGL(gchunk, dim3(nchunks), dim3(kGThreads), 0, s, gda_.p, gdb_.p, g.xadj,
                            g.adjncy, g.adjwgt, map, moff_.p, members_.p, mpre_.p, goffm_base_.p,
-                           goffm_.p, gct_base_.p, gcnt_.p, gpart_.p, stage_q_.p, err_.p);
+                           goffm_.p, gct_base_.p, gcnt_.p, gpart_.p, stage_q_.p, err);
         scan_i32(gcnt_.p, gpos_.p, (int)ct_total + 1, s);
         hipLaunchKernelGGL(gmerge, dim3(ntasks), dim3(kGMergeThreads), 0, s, gchunk_prefix_.p,
                            gtask_prefix_.p, gtrow_.p, ntasks, gct_base_.p, gpos_.p,
                            goffm_base_.p, goffm_.p, gpart_.p, stage_q_.p, stage_w_.p, gbig_.p,
-                           gnbig_.p, err_.p);
-        int nbig = 0;
-        KH_CHECK(hipMemcpyAsync(&nbig, gnbig_.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
+                           gnbig_.p, err);
+        mail_.post(s, {gnbig_.p, 1});
+        KH_CHECK(hipStreamSynchronize(s));  // the host vectors above must outlive their copies
+        const int nbig = mail_.wait(s)[0];
         if (nbig > 0) {
             // rare: a (row, bucket) range too large for LDS gets a private global table
             DevBuf<int> totals;
@@ -1114,13 +1116,12 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
             hipLaunchKernelGGL(gmerge_global, dim3(nbig), dim3(1024), 0, s, gbig_.p, nbig,
                                gchunk_prefix_.p, gtask_prefix_.p, gtrow_.p, gct_base_.p, gpos_.p,
                                goffm_base_.p, goffm_.p, gpart_.p, hoff_.p, hcap_.p, hk_.p, hv_.p,
-                               hm_.p, stage_q_.p, stage_w_.p, err_.p);
+                               hm_.p, stage_q_.p, stage_w_.p, err);
             KH_CHECK(hipStreamSynchronize(s));  // host vectors above must outlive the copies
         }
         // emission in f order: counts per chunk, a scan over the chunks, ordered writes
         ecnt_.reserve((long long)nchunks + 1);
         epos_.reserve((long long)nchunks + 1);
-        fill_async(ecnt_.p + nchunks, 1, 0, s);
         hipLaunchKernelGGL(gemit_count, dim3(nchunks), dim3(kEmitThreads), 0, s, gdb_.p,
                            stage_q_.p, ecnt_.p);
         scan_i32(ecnt_.p, epos_.p, nchunks + 1, s);
@@ -1128,11 +1129,10 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
                            stage_q_.p, stage_w_.p, epos_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p);
     }
     scan_i32(cdeg_.p, out.xadj_dev(), nc + 1, s);
-    int mc = 0, err = 0;
-    KH_CHECK(hipMemcpyAsync(&mc, out.xadj_dev() + nc, sizeof(int), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipMemcpyAsync(&err, err_.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
-    KH_REQUIRE(err == 0, "contraction: a hash table probe found no free slot (kernel table sizing "
+    mail_.post(s, {out.xadj_dev() + nc, 1}, {err, 1});
+    const int* const got = mail_.wait(s);
+    const int mc = got[0];
+    KH_REQUIRE(got[1] == 0, "contraction: a hash table probe found no free slot (kernel table sizing "
                          "invariant violated); the result is invalid");
     out.alloc_edges(mc);
     if (nc > 0) {

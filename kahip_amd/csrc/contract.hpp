@@ -3,6 +3,7 @@
 
 #include "common.hpp"
 #include "devbuf.hpp"
+#include "mail.hpp"
 
 namespace kahip {
 
@@ -38,8 +39,9 @@ private:
     DevBuf<int> leader_, flag_, newid_;
     DevBuf<int> cnt_, fdeg_, moff_, tpos_, cdeg_, members_, tq_, tw_;
     DevBuf<int> iota_, mkeys_;               // radix sort of the node ids by cluster
-    DevBuf<int> rlist_[5], rcount_;          // rows of the thread tier and the four LDS tiers
-    DevBuf<int> ovl2_list_, ovl_count_;      // rows of the global tier
+    DevBuf<int> rlist_[5];                   // rows of the thread tier and the four LDS tiers
+    DevBuf<int> ovl2_list_, ctl_;            // rows of the global tier; list lengths, error flag
+    Mail mail_;
     DevBuf<long long> hcap_, hoff_;
     DevBuf<int> gchunk_prefix_, mdeg_, mpre_, ofd_;
     DevBuf<int> hk_, hv_, hm_;
@@ -50,7 +52,6 @@ private:
     DevBuf<int4> gda_, gdb_;                 // per-chunk descriptors (gchunk_desc)
     DevBuf<int> stage_q_, stage_w_;          // merged entries at the f of their first edge
     DevBuf<int> ecnt_, epos_;                // staged entries per chunk and their scan
-    DevBuf<int> err_;  // device error flag (kErrProbe) of the last contract()
 };
 
 // fine_part[v] = coarse_part[map[v]] (reference: graph_hierarchy.cpp:54-58).

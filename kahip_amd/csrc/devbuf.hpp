@@ -31,13 +31,17 @@ struct DevBuf {
         return *this;
     }
     ~DevBuf() { free(); }
-    // Ensures room for n elements (contents are not preserved on growth).
+    // Ensures room for n elements (contents are not preserved on growth). A buffer that has to
+    // grow gets an eighth more than asked for: calls on graphs of about one size differ by a few
+    // percent in their edges, and without it most of them would free and allocate every buffer
+    // again (about 0.1 ms each).
     T* reserve(long long n) {
         if (n < 1) n = 1;
         if (n > cap) {
+            const long long room = cap > 0 ? n + n / 8 : n;
             free();
-            KH_CHECK(hipMalloc((void**)&p, sizeof(T) * n));
-            cap = n;
+            KH_CHECK(hipMalloc((void**)&p, sizeof(T) * room));
+            cap = room;
         }
         return p;
     }

@@ -68,15 +68,17 @@ __global__ void run_leaders(int n, const unsigned long long* __restrict__ skeys,
     for (int j = i; j < n && skeys[j] == skeys[i]; ++j) out[sids[j]] = lead;
 }
 
+// Time between two events; read once the stream has passed the second one.
 struct EventPair {
     hipEvent_t a = nullptr, b = nullptr;
     EventPair() {
         KH_CHECK(hipEventCreate(&a));
         KH_CHECK(hipEventCreate(&b));
     }
+    EventPair(EventPair&& o) noexcept : a(o.a), b(o.b) { o.a = o.b = nullptr; }
     ~EventPair() {
-        (void)hipEventDestroy(a);
-        (void)hipEventDestroy(b);
+        if (a) (void)hipEventDestroy(a);
+        if (b) (void)hipEventDestroy(b);
     }
     float ms() const {
         float t = 0;
@@ -84,6 +86,12 @@ struct EventPair {
         return t;
     }
 };
+
+float total_ms(const std::vector<EventPair>& ev) {
+    float t = 0;
+    for (const EventPair& e : ev) t += e.ms();
+    return t;
+}
 
 }  // namespace
 
@@ -114,7 +122,7 @@ int ip_repetitions_for(int k) {
 }
 
 bool upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
-                  OwnedGraph& out, hipStream_t s, DevBuf<int>* bad) {
+                  OwnedGraph& out, hipStream_t s, DevBuf<int>* bad, Mail* mail) {
     KH_REQUIRE(n >= 0, "n must be non-negative");
     out.alloc_nodes(n);
     const long long m2 = n > 0 ? (long long)xadj[n] : 0;
@@ -122,15 +130,13 @@ bool upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, co
     KH_CHECK(hipMemcpyAsync(out.g.xadj, xadj, sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
     if (m2 > 0)
         KH_CHECK(hipMemcpyAsync(out.g.adjncy, adjncy, sizeof(int) * m2, hipMemcpyHostToDevice, s));
-    int is_bad = 0;
-    if (bad && m2 > 0) {
+    const bool check = bad && m2 > 0;
+    if (check) {
         bad->reserve(1);
         fill_async(bad->p, 1, 0, s);
         hipLaunchKernelGGL(check_targets, dim3(std::min(grid_for(m2, 1024), 2048)), dim3(256), 0, s,
                            m2, out.g.adjncy, n, bad->p);
-        KH_CHECK(hipMemcpyAsync(&is_bad, bad->p, sizeof(int), hipMemcpyDeviceToHost, s));
-        KH_CHECK(hipStreamSynchronize(s));
-        if (is_bad) return false;
+        mail->post(s, {bad->p, 1});
     }
     long long total = 0;
     if (vwgt) {
@@ -150,16 +156,31 @@ bool upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, co
     for (int v = 0; v < n; ++v) maxdeg = std::max(maxdeg, xadj[v + 1] - xadj[v]);
     out.g.total_vwgt = total;
     out.g.max_degree = maxdeg;
-    KH_CHECK(hipStreamSynchronize(s));
-    return true;
+    KH_CHECK(hipStreamSynchronize(s));  // the copies from the host arrays have been taken
+    return !check || mail->wait(s)[0] == 0;
 }
 
-void download_graph(const DGraph& g, HostGraph& out, hipStream_t s) {
+void download_graph(const DGraph& g, HostGraph& out, hipStream_t s, Mail* mail) {
     out.n = g.n;
     out.xadj.resize(g.n + 1);
     out.adjncy.resize(g.m2);
     out.adjwgt.resize(g.m2);
     out.vwgt.resize(g.n);
+    const long long words = 2LL * g.n + 1 + 2 * g.m2;
+    if (mail && words <= Mail::kInts) {  // small: one kernel instead of four copies
+        const int m2 = (int)g.m2;
+        mail->post(s, {g.xadj, g.n + 1}, {g.adjncy, m2}, {g.adjwgt, m2}, {g.vwgt, g.n});
+        const int* w = mail->wait(s);
+        auto take = [&](std::vector<int>& v) {
+            std::copy(w, w + v.size(), v.begin());
+            w += v.size();
+        };
+        take(out.xadj);
+        take(out.adjncy);
+        take(out.adjwgt);
+        take(out.vwgt);
+        return;
+    }
     KH_CHECK(hipMemcpyAsync(out.xadj.data(), g.xadj, sizeof(int) * (g.n + 1), hipMemcpyDeviceToHost, s));
     if (g.m2 > 0) {
         KH_CHECK(hipMemcpyAsync(out.adjncy.data(), g.adjncy, sizeof(int) * g.m2, hipMemcpyDeviceToHost, s));
@@ -240,6 +261,7 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
                            oids2.p, lab);
         KH_CHECK(hipGetLastError());
     };
+    std::vector<EventPair> ev_rating, ev_refine;  // read at the end
     const unsigned num_stop = (unsigned)p.stop_factor * (unsigned)p.k;
     int level = 0;
     S.level_n[0] = g0.n;
@@ -255,14 +277,12 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         // The clustering sees the rating in place of the edge weights; contraction keeps them.
         DGraph rated = fine;
         if (p.rating != RatingMode::None && level < p.rating_levels && fine.m2 > 0) {
-            EventPair ev;
-            KH_CHECK(hipEventRecord(ev.a, s));
+            ev_rating.emplace_back();
+            KH_CHECK(hipEventRecord(ev_rating.back().a, s));
             score.reserve(fine.m2);
-            rw.scores(p.rating, fine, (int)B, rating_seed(p.seed, level), p.mlp, score.p, s, lp,
-                      prof);
-            KH_CHECK(hipEventRecord(ev.b, s));
-            KH_CHECK(hipEventSynchronize(ev.b));
-            S.ms_rating += ev.ms();
+            if (p.rating == RatingMode::Learned && level == 0) rw.upload_weights(*p.mlp, s);
+            rw.scores(p.rating, fine, (int)B, rating_seed(p.seed, level), score.p, s, lp, prof);
+            KH_CHECK(hipEventRecord(ev_rating.back().b, s));
             rated.adjwgt = score.p;
         }
         ProfScope ps_cluster(prof, "lp_cluster_total", 0.0, 0, s);  // the level's clustering
@@ -304,14 +324,12 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
     }
     S.levels = level;
     KH_CHECK(hipEventRecord(ev_coarsen.b, s));
-    KH_CHECK(hipStreamSynchronize(s));
-    S.ms_coarsen = ev_coarsen.ms();
 
     // ------------------------------------------------------------------ initial partitioning
     const DGraph& cg = level_graph(level);
     const auto t0 = std::chrono::steady_clock::now();
     HostGraph hg;
-    download_graph(cg, hg, s);
+    download_graph(cg, hg, s, &mw.mail);
     std::vector<int> hpart;
     IpParams ip;
     ip.k = p.k;
@@ -326,7 +344,6 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
     part_c.reserve(std::max(cg.n, 1));
     if (cg.n > 0)
         KH_CHECK(hipMemcpyAsync(part_c.p, hpart.data(), sizeof(int) * cg.n, hipMemcpyHostToDevice, s));
-    KH_CHECK(hipStreamSynchronize(s));
     S.ms_initial = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 
     // ------------------------------------------------------------------ uncoarsening
@@ -337,11 +354,10 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
     W.reserve(p.k);
     HostGraph hl;
     std::vector<int> hp;
-    S.ms_refine = 0;
     for (int l = level; l >= 0; --l) {
         const DGraph& gl = level_graph(l);
-        EventPair ev;
-        KH_CHECK(hipEventRecord(ev.a, s));
+        ev_refine.emplace_back();
+        KH_CHECK(hipEventRecord(ev_refine.back().a, s));
         int* part_l;
         if (l == level) {
             part_l = part_c.p;
@@ -357,10 +373,9 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         // the profiler times the clustering and contraction kernels, not the refinement rounds
         lp.run(LpMode::Refine, gl, part_l, W.p, (int)U, p.refine_rounds, rseed, s, nullptr,
                "lp_refine");
-        KH_CHECK(hipEventRecord(ev.b, s));
+        KH_CHECK(hipEventRecord(ev_refine.back().b, s));
         lp.check(s);
         S.edges_refine += lp.traversed(s);
-        S.ms_refine += ev.ms();
         if (p.fm_rounds > 0 && gl.n > 0) {
             const auto t1 = std::chrono::steady_clock::now();
             download_graph(gl, hl, s);
@@ -385,12 +400,11 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
     // ------------------------------------------------------------------ metrics
     EventPair ev_cut;
     KH_CHECK(hipEventRecord(ev_cut.a, s));
-    S.cut = mw.edge_cut(g0, part_c.p, s, prof);
+    const int* cut_words = mw.launch_edge_cut(g0, part_c.p, s, prof);
     KH_CHECK(hipEventRecord(ev_cut.b, s));
     S.edges_cut = g0.m2;
     compute_block_weights(g0, part_c.p, p.k, W.p, s);
-    std::vector<int> hw(p.k);
-    KH_CHECK(hipMemcpyAsync(hw.data(), W.p, sizeof(int) * p.k, hipMemcpyDeviceToHost, s));
+    mw.mail.post(s, {cut_words, 2}, {W.p, p.k});
     if (g0.n > 0) {
         const int* out_part = part_c.p;
         if (reorder) {
@@ -400,7 +414,13 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         }
         KH_CHECK(hipMemcpyAsync(part_out, out_part, sizeof(int) * g0.n, hipMemcpyDeviceToHost, s));
     }
+    const int* hw = mw.mail.wait(s);
+    S.cut = MetricsWorkspace::cut_of(hw);
+    hw += 2;
     KH_CHECK(hipStreamSynchronize(s));
+    S.ms_coarsen = ev_coarsen.ms();
+    S.ms_rating = total_ms(ev_rating);
+    S.ms_refine = total_ms(ev_refine);
     S.ms_cut = ev_cut.ms();
     long long mx = 0;
     for (int b = 0; b < p.k; ++b) mx = std::max(mx, (long long)hw[b]);

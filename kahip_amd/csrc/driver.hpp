@@ -142,10 +142,12 @@ private:
 };
 
 // Uploads a host CSR (vwgt / adjwgt may be null: unit weights) into an owned device graph; with
-// `bad` (scratch) the targets are checked on the GPU before anything reads them: false if one lies
+// `bad` (scratch) and `mail` the targets are checked on the GPU before anything reads them: false if one lies
 // outside [0, n), the graph is then not usable.
 bool upload_graph(int n, const int* xadj, const int* adjncy, const int* vwgt, const int* adjwgt,
-                  OwnedGraph& out, hipStream_t s, DevBuf<int>* bad = nullptr);
-void download_graph(const DGraph& g, HostGraph& out, hipStream_t s);
+                  OwnedGraph& out, hipStream_t s, DevBuf<int>* bad = nullptr,
+                  Mail* mail = nullptr);
+// mail (optional): small graphs come through it.
+void download_graph(const DGraph& g, HostGraph& out, hipStream_t s, Mail* mail = nullptr);
 
 }  // namespace kahip

@@ -21,7 +21,7 @@
 //   deg <= 512          one wave per node, LDS hash table (open addressing, LDS atomics);
 //   larger              one workgroup per node, hash table in a pre-cleared global region.
 
-#include <atomic>
+#include <cstring>
 
 #include <rocprim/device/device_scan.hpp>
 
@@ -73,6 +73,21 @@ struct Cand {
     int size;
 };
 static_assert(sizeof(Cand) == sizeof(int4), "bucket results are stored as int4");
+
+// The arguments of clustering blockIdx.y of a launch over several (uniform).
+__device__ inline void select_copy(LpArgs& a) {
+    const int y = blockIdx.y;
+    if (y == 0) return;
+    const long long o = y * a.copy_stride;
+    a.label += o;
+    a.size += o;
+    a.inc += o;
+    a.top += o;
+    a.prop_t += o;
+    a.prop_gain += o;
+    a.prop_ok += o;
+    a.tie_seed = y == 1 ? a.copy_tie1 : a.copy_tie2;
+}
 
 // Bucket of a label among P buckets of a hub (independent of the LDS slot hash).
 __device__ inline int bucket_of(int lab, int P) {
@@ -385,6 +400,7 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
 template <int G, int IT>
 __global__ __launch_bounds__(kBlock) void propose_group(LpArgs a, const int* __restrict__ list,
                                                         int count) {
+    select_copy(a);
     group_vb<LpMode::Cluster, G, IT>(a, list, count, blockIdx.x, blockIdx.x);
 }
 
@@ -486,6 +502,7 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
 template <int WCAP = kWaveCap>
 __global__ __launch_bounds__(kBlock) void propose_wave(LpArgs a, const int* __restrict__ list,
                                                        int count) {
+    select_copy(a);
     wave_vb<LpMode::Cluster, false, WCAP>(a, list, count, 0, blockIdx.x, blockIdx.x);
 }
 
@@ -1099,6 +1116,7 @@ __global__ void filter_departures(LpArgs a, const int* __restrict__ list, int co
 }
 
 __global__ void admit_moves(LpArgs a, const int* __restrict__ list, int count) {
+    select_copy(a);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < count) admit_one(a, list[i]);
 }
@@ -1106,6 +1124,7 @@ __global__ void admit_moves(LpArgs a, const int* __restrict__ list, int count) {
 template <LpMode M>
 __global__ __launch_bounds__(256) void apply_moves(LpArgs a, const int* __restrict__ list,
                                                    int count) {
+    select_copy(a);
     __shared__ int block_moves;
     if (threadIdx.x == 0) block_moves = 0;
     __syncthreads();
@@ -1598,12 +1617,26 @@ __global__ void bin_count(int n, const int* __restrict__ xadj, uint32_t seed, in
 // them, cursor slot L + sr), then the others.
 __global__ void bin_scatter(int n, const int* __restrict__ xadj, uint32_t seed, int S,
                             BinConfig cfg, const uint8_t* __restrict__ include, int split,
-                            const int* __restrict__ counts, const int* __restrict__ offsets,
+                            const int* __restrict__ counts, int* __restrict__ offsets,
                             int* __restrict__ cursor, int* __restrict__ lists) {
     constexpr int L = kMaxSub * kNumBins;
+    static_assert(L < 64, "one lane per list");
     __shared__ int local[L + kMaxSub];
     __shared__ int base[L + kMaxSub];
+    __shared__ int off[64];
     for (int i = threadIdx.x; i < L + kMaxSub; i += blockDim.x) local[i] = 0;
+    if (threadIdx.x < 64) {  // list offsets: the lists in order (workgroup 0 keeps them)
+        const int lane = threadIdx.x;
+        const int cnt = lane < L ? counts[lane] : 0;
+        int incl = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        off[lane] = incl - cnt;
+        if (blockIdx.x == 0 && lane < L) offsets[lane] = incl - cnt;
+    }
     __syncthreads();
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     int l = -1, slot = -1, r = 0, skip = 0;
@@ -1625,7 +1658,7 @@ __global__ void bin_scatter(int n, const int* __restrict__ xadj, uint32_t seed, 
     for (int i = threadIdx.x; i < L + kMaxSub; i += blockDim.x)
         base[i] = local[i] ? atomicAdd(&cursor[i], local[i]) : 0;
     __syncthreads();
-    if (l >= 0) lists[offsets[l] + skip + base[slot] + r] = v;
+    if (l >= 0) lists[off[l] + skip + base[slot] + r] = v;
 }
 
 // Frontier of a refinement round: the active nodes of every non-hub list, compacted per list
@@ -1748,12 +1781,41 @@ __global__ void fill_u8(uint8_t* p, long long n, uint8_t value) {
     if (i < n) p[i] = value;
 }
 
+// Admission scratch of a clustering (labels = nodes) or refinement.
+__global__ void init_scratch(long long n, int* __restrict__ prop_t, long long nl,
+                             int* __restrict__ inc, unsigned long long* __restrict__ top,
+                             int* __restrict__ out, unsigned long long* __restrict__ dtop) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) prop_t[i] = -1;
+    if (i < nl) {
+        inc[i] = 0;
+        top[i] = 0ull;
+        if (out) {
+            out[i] = 0;
+            dtop[i] = 0ull;
+        }
+    }
+}
+
+// Frontier flags and list lengths of a refinement.
+__global__ void init_frontier(int n, uint8_t* __restrict__ act, uint8_t value,
+                              uint8_t* __restrict__ nxt, int m, int* __restrict__ ccount) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        act[i] = value;
+        nxt[i] = 0;
+    }
+    if (i < m) ccount[i] = 0;
+}
+
+// (blockIdx.y: copies, one after the other)
 __global__ void init_labels(int n, int* __restrict__ label, int* __restrict__ size,
                             const int* __restrict__ vwgt) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    const long long o = (long long)blockIdx.y * n;
     if (v < n) {
-        label[v] = v;
-        size[v] = vwgt[v];
+        label[o + v] = v;
+        size[o + v] = vwgt[v];
     }
 }
 
@@ -1780,8 +1842,8 @@ inline int grid_for(long long work, int block) { return (int)((work + block - 1)
 // The clustering's G-lane proposal kernel of one list with `items` nodes per lane group, one
 // workgroup per virtual block.
 template <int G>
-void launch_group(int items, const LpArgs& a, const int* lst, int cnt, hipStream_t s) {
-    const dim3 grid(grid_for((long long)cnt * G, kBlock * items));
+void launch_group(int items, const LpArgs& a, const int* lst, int cnt, int copies, hipStream_t s) {
+    const dim3 grid(grid_for((long long)cnt * G, kBlock * items), copies);
     switch (items) {
         case 1: hipLaunchKernelGGL((propose_group<G, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
         case 4: hipLaunchKernelGGL((propose_group<G, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
@@ -1826,7 +1888,10 @@ void fill_async(long long* p, long long n, long long value, hipStream_t s) {
 }
 
 void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, uint32_t seed,
-                          const BinConfig& bins, hipStream_t s, const uint8_t* include) {
+                          const BinConfig& bins, hipStream_t s, const uint8_t* include,
+                          int copies) {
+    KH_REQUIRE(copies == 1 || (mode == LpMode::Cluster && S == 1 && copies <= kMaxCopies),
+               "copies are one-sub-round clusterings");
     KH_REQUIRE(S >= 1 && S <= kMaxSub, "sub-rounds must be in [1, 8]");
     KH_REQUIRE(bins.hi[kNumBins - 2] <= 512, "the wave bin holds degrees <= 512");
     KH_REQUIRE(bins.group_items == 1 || bins.group_items == 2 || bins.group_items == 4,
@@ -1837,23 +1902,23 @@ void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, u
     KH_REQUIRE(g.n < (1 << 30) && num_labels < (1 << 30), "labels must be below 2^30");
     subrounds_ = S;
     num_labels_ = num_labels;
-    moves_.reserve(kMaxRounds);
-    trav_.reserve(64);
-    err_.reserve(1);
+    ctl_.reserve(kCtlInts);
+    fill_async(ctl_.p, kCtlInts, 0, s);
     if (mode == LpMode::Refine) {
         active_.reserve(g.n);
         next_active_.reserve(g.n);
-        tail_.init();
     }
     // a graph that refine_tail takes from round 0 needs no lists
     small_ = mode == LpMode::Refine && !include && g.n <= kTailNodes && g.m2 <= kTailEdges &&
              num_labels <= kTailLabels;
-    if (!small_) build_lists(mode, g, seed, s, include);
+    if (!small_) build_lists(mode, g, seed, s, include, copies);
 }
 
 void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
-                              const uint8_t* include) {
-    const int S = subrounds_, num_labels = num_labels_;
+                              const uint8_t* include, int copies) {
+    const int S = subrounds_;
+    const long long num_labels = num_labels_, scratch_n = (long long)copies * g.n;
+    const long long scratch_l = copies * num_labels;
     const BinConfig& bins = bins_;
     dense_wave_ = mode == LpMode::Refine && num_labels <= kWaveDense;
     dense_hub_ = mode == LpMode::Refine && num_labels <= kHubDense;
@@ -1863,48 +1928,46 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
         clists_.reserve(g.n);
         ccount_.reserve(2 * L);
     }
-    counts_.reserve(L + kMaxSub);
-    cursor_.reserve(L + kMaxSub);
     offsets_.reserve(L);
-    edges_.reserve(L);
-    prop_t_.reserve(g.n);
-    prop_gain_.reserve(g.n);
-    prop_ok_.reserve(g.n);
-    inc_.reserve(num_labels);
-    out_.reserve(num_labels);
-    top_.reserve(num_labels);
-    dtop_.reserve(num_labels);
-    n_big_tasks_.reserve((long long)kMaxSub * kMaxRounds);
-    n_mid_tasks_.reserve((long long)kMaxSub * kMaxRounds);
+    // {edges per list (64 bit), counts per list and of the small wave nodes, cursors}
+    constexpr int kBinInts = 2 * kMaxSub * kNumBins + 2 * (kMaxSub * kNumBins + kMaxSub);
+    bin_.reserve(kBinInts);
+    unsigned long long* edges = reinterpret_cast<unsigned long long*>(bin_.p);
+    counts_ = bin_.p + 2 * L;
+    int* cursor = counts_ + L + kMaxSub;
+    prop_t_.reserve(scratch_n);
+    prop_gain_.reserve(scratch_n);
+    prop_ok_.reserve(scratch_n);
+    inc_.reserve(scratch_l);
+    top_.reserve(scratch_l);
+    if (mode == LpMode::Refine) {
+        out_.reserve(num_labels);
+        dtop_.reserve(num_labels);
+    }
 
-    fill_async(counts_.p, L + kMaxSub, 0, s);
-    fill_async(cursor_.p, L + kMaxSub, 0, s);
+    fill_async(bin_.p, kBinInts, 0, s);
     const int split = mode == LpMode::Cluster ? 1 : 0;  // small-degree wave kernel (clustering)
-    fill_async(edges_.p, L, 0ull, s);
-    fill_async(prop_t_.p, g.n, -1, s);
-    fill_async(inc_.p, num_labels, 0, s);
-    fill_async(out_.p, num_labels, 0, s);
-    fill_async(top_.p, num_labels, 0ull, s);
-    fill_async(dtop_.p, num_labels, 0ull, s);
+    const bool refine = mode == LpMode::Refine;
+    hipLaunchKernelGGL(init_scratch, dim3(std::max(grid_for(std::max(scratch_n, scratch_l), 256), 1)),
+                       dim3(256), 0, s, scratch_n, prop_t_.p, scratch_l, inc_.p, top_.p,
+                       refine ? out_.p : nullptr, refine ? dtop_.p : nullptr);
     if (g.n > 0)
         hipLaunchKernelGGL(bin_count, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n, g.xadj,
-                           seed, S, bins, include, split, counts_.p, edges_.p);
-    KH_CHECK(hipMemcpyAsync(host_counts, counts_.p, sizeof(int) * L, hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipMemcpyAsync(host_wave_small_, counts_.p + L, sizeof(int) * kMaxSub,
-                            hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipMemcpyAsync(host_edges, edges_.p, sizeof(long long) * L, hipMemcpyDeviceToHost,
-                            s));
-    KH_CHECK(hipStreamSynchronize(s));
+                           seed, S, bins, include, split, counts_, edges);
+    mail_.post(s, {bin_.p, 2 * L + L + kMaxSub});
+    if (g.n > 0)
+        hipLaunchKernelGGL(bin_scatter, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n, g.xadj,
+                           seed, S, bins, include, split, counts_, offsets_.p, cursor, lists_.p);
+    KH_CHECK(hipGetLastError());
+    const int* got = mail_.wait(s);  // (the scatter runs meanwhile)
+    std::memcpy(host_edges, got, sizeof(long long) * L);
+    std::memcpy(host_counts, got + 2 * L, sizeof(int) * L);
+    std::memcpy(host_wave_small_, got + 3 * L, sizeof(int) * kMaxSub);
     int acc = 0;
     for (int i = 0; i < L; ++i) {
         host_offsets[i] = acc;
-        acc += (i < S * kNumBins) ? host_counts[i] : 0;
+        acc += host_counts[i];
     }
-    KH_CHECK(hipMemcpyAsync(offsets_.p, host_offsets, sizeof(int) * L, hipMemcpyHostToDevice, s));
-    if (g.n > 0)
-        hipLaunchKernelGGL(bin_scatter, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n, g.xadj,
-                           seed, S, bins, include, split, counts_.p, offsets_.p, cursor_.p,
-                           lists_.p);
 
     // hubs (last bin): chunk prefix per sub-round list, global tables for multi-chunk hubs
     int hubs = 0;
@@ -2152,9 +2215,8 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     const int S = subrounds_;
     const bool cl = mode == LpMode::Cluster;
     KH_REQUIRE(cl || !(dense_wave_ || dense_hub_) || num_labels_ > 0, "prepare() not called");
-    fill_async(moves_.p, kMaxRounds, 0, s);
-    fill_async(trav_.p, 64, 0ull, s);
-    fill_async(err_.p, 1, 0, s);
+    fill_async(ctl_.p, kCtlErr, 0, s);  // the error flag is cleared by prepare()
+    fetched_ = false;
     if (rounds == 0) return;
     LpArgs a{};
     a.xadj = g.xadj;
@@ -2165,16 +2227,16 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     a.size = size;
     a.bound = bound;
     a.lbound = lbound;
-    a.trav = trav_.p;
-    a.err = err_.p;
+    a.trav = reinterpret_cast<unsigned long long*>(ctl_.p);
+    a.err = ctl_.p + kCtlErr;
     uint8_t* act = active_.p;
     uint8_t* nxt = next_active_.p;
     int r = 0;
     bool filter = !cl;  // an overloaded block may exist
     if (small_) {
         // the whole refinement in one workgroup; the lists are built only if it stops early
-        fill_async(act, g.n, (uint8_t)0, s);
-        fill_async(nxt, g.n, (uint8_t)0, s);
+        hipLaunchKernelGGL(init_frontier, dim3(std::max(grid_for(g.n, 256), 1)), dim3(256), 0, s,
+                           g.n, act, (uint8_t)0, nxt, 0, nullptr);
         a.next_active = nxt;
         TailArgs t{};
         t.n = g.n;
@@ -2182,7 +2244,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         t.seed = seed;
         r = run_tail(a, t, s, &filter);
         if (r >= rounds) return;
-        build_lists(mode, g, seed, s, nullptr);
+        build_lists(mode, g, seed, s, nullptr, 1);
         std::swap(act, nxt);  // round r's frontier (r > 0)
     }
     a.inc = inc_.p;
@@ -2192,10 +2254,6 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     a.prop_t = prop_t_.p;
     a.prop_gain = prop_gain_.p;
     a.prop_ok = prop_ok_.p;
-    if (cl || !dense_hub_) {
-        fill_async(n_big_tasks_.p, (long long)kMaxSub * kMaxRounds, 0, s);
-        fill_async(n_mid_tasks_.p, (long long)kMaxSub * kMaxRounds, 0, s);
-    }
     // Refinement hubs of more than one chunk keep per-block connection counters across the
     // rounds: one scan builds them, every applied move updates its hub neighbours' counters, and
     // the hubs then decide from the counters instead of rescanning their edges each round.
@@ -2224,18 +2282,16 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     const bool keep_flags = hubs > 0 && !fused_hubs;
     if (!cl) {
         if (listed == 0) return;
-        if (r == 0) {
-            fill_async(act, g.n, (uint8_t)(keep_flags ? 1 : 0), s);
-            fill_async(nxt, g.n, (uint8_t)0, s);
-        }
-        fill_async(ccount_.p, 2 * nseg, 0, s);
+        const int nf = r == 0 ? g.n : 0;  // else flagged by the tail
+        hipLaunchKernelGGL(init_frontier, dim3(grid_for(std::max(nf, 2 * nseg), 256)), dim3(256),
+                           0, s, nf, act, (uint8_t)(keep_flags ? 1 : 0), nxt, 2 * nseg, ccount_.p);
     }
     int* cnow = ccount_.p;  // list lengths of the frontier, cleared by the tail before last
     int* cnext = cnow + nseg;
     while (r < rounds) {
         // refinement: round 0 works on the whole lists, later rounds on the compacted frontier
         const int* flists = lists_.p;
-        const int* fcount = counts_.p;
+        const int* fcount = counts_;
         if (!cl && r > 0) {
             ProfScope ps(prof, base + "_frontier", 0.0, 0, s);
             std::swap(cnow, cnext);
@@ -2263,7 +2319,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
             fcount = cnow;
         }
         a.tie_seed = tie_seed_of(seed, r);
-        a.moves = moves_.p + r;
+        a.moves = ctl_.p + kCtlMoves + r;
         a.active = cl ? nullptr : act;
         a.next_active = cl ? nullptr : nxt;
         for (int sr = 0; sr < S; ++sr) {
@@ -2299,21 +2355,11 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 const double bytes = cl ? 12.0 * (double)ledges + 16.0 * lnodes : 0.0;
                 ProfScope ps(prof, base + "_propose_" + kBinName[b], bytes, cl ? ledges : 0, s);
                 switch (b) {
-                    case 0: launch_group<8>(bins_.group_items, a, lst, cnt, s); break;
-                    case 1: launch_group<16>(bins_.group_items, a, lst, cnt, s); break;
-                    case 2: launch_group<32>(bins_.group_items, a, lst, cnt, s); break;
-                    case 3: launch_group<64>(bins_.group_items, a, lst, cnt, s); break;
-                    case 4: {
-                        const int ns = host_wave_small_[sr];  // degree <= wave_small, first
-                        if (ns > 0) {
-                            const dim3 gs(grid_for(ns, kBlock / 64));
-                            if (bins_.wave_small == 64) hipLaunchKernelGGL(propose_wave<128>, gs, dim3(kBlock), 0, s, a, lst, ns);
-                            else if (bins_.wave_small == 256) hipLaunchKernelGGL(propose_wave<512>, gs, dim3(kBlock), 0, s, a, lst, ns);
-                            else hipLaunchKernelGGL(propose_wave<256>, gs, dim3(kBlock), 0, s, a, lst, ns);
-                        }
-                        if (cnt > ns) hipLaunchKernelGGL(propose_wave<>, dim3(grid_for(cnt - ns, kBlock / 64)), dim3(kBlock), 0, s, a, lst + ns, cnt - ns);
-                        break;
-                    }
+                    case 0:
+                    case 1:
+                    case 2:
+                    case 3:
+                    case 4: launch_proposals(b, sr, a, cnt, 1, s); break;
                     default: {
                         if (!cl && dense_hub_) {
                             const int4* cm = cmap_.p + cmap_base_[sr];
@@ -2360,9 +2406,9 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                             const int* pt = pos_t_.p;
                             const int* cp = chunk_prefix_.p + chunk_base_[sr];
                             int* bt = big_tasks_.p;
-                            int* nbt = n_big_tasks_.p + (r * S + sr);
+                            int* nbt = ctl_.p + kCtlBig + (r * S + sr);
                             int* mt = mid_tasks_.p;
-                            int* nmt = n_mid_tasks_.p + (r * S + sr);
+                            int* nmt = ctl_.p + kCtlMid + (r * S + sr);
                             if (cl) {
                                 hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
                                 hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
@@ -2409,71 +2455,111 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     KH_CHECK(hipGetLastError());
 }
 
+void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
+                             const uint32_t* seeds, int copies, hipStream_t s) {
+    if (g.n == 0) return;
+    hipLaunchKernelGGL(init_labels, dim3(grid_for(g.n, 256), copies), dim3(256), 0, s, g.n, label,
+                       size, g.vwgt);
+    if (host_counts[kNumBins - 1] > 0) {  // the hub kernels take one clustering at a time
+        for (int i = 0; i < copies; ++i)
+            run(LpMode::Cluster, g, label + (long long)i * g.n, size + (long long)i * g.n, bound, 1,
+                seeds[i], s, nullptr, "rating_sweep");
+        return;
+    }
+    fetched_ = false;
+    LpArgs a{};
+    a.xadj = g.xadj;
+    a.adjncy = g.adjncy;
+    a.adjwgt = g.adjwgt;
+    a.vwgt = g.vwgt;
+    a.label = label;
+    a.size = size;
+    a.bound = bound;
+    a.inc = inc_.p;
+    a.top = top_.p;
+    a.prop_t = prop_t_.p;
+    a.prop_gain = prop_gain_.p;
+    a.prop_ok = prop_ok_.p;
+    a.moves = ctl_.p + kCtlMoves;
+    a.err = ctl_.p + kCtlErr;
+    a.copy_stride = g.n;
+    static_assert(kMaxCopies == 3, "one tie seed per copy");
+    a.tie_seed = tie_seed_of(seeds[0], 0);
+    if (copies > 1) a.copy_tie1 = tie_seed_of(seeds[1], 0);
+    if (copies > 2) a.copy_tie2 = tie_seed_of(seeds[2], 0);
+    int total = 0;
+    for (int b = 0; b < kNumBins - 1; ++b) {
+        const int cnt = host_counts[b];
+        if (cnt > 0) launch_proposals(b, 0, a, cnt, copies, s);
+        total += cnt;
+    }
+    if (total == 0) return;
+    const dim3 grid(grid_for(total, 256), copies);
+    hipLaunchKernelGGL(admit_moves, grid, dim3(256), 0, s, a, lists_.p, total);
+    hipLaunchKernelGGL((apply_moves<LpMode::Cluster>), grid, dim3(256), 0, s, a, lists_.p, total);
+    KH_CHECK(hipGetLastError());
+}
+
+// The clustering proposals of list b (not the hub list) of sub-round sr.
+void LpWorkspace::launch_proposals(int b, int sr, const LpArgs& a, int cnt, int copies,
+                                   hipStream_t s) {
+    const int* lst = lists_.p + host_offsets[sr * kNumBins + b];
+    switch (b) {
+        case 0: launch_group<8>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 1: launch_group<16>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 2: launch_group<32>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 3: launch_group<64>(bins_.group_items, a, lst, cnt, copies, s); break;
+        default: {
+            const int ns = host_wave_small_[sr];  // degree <= wave_small, first
+            if (ns > 0) {
+                const dim3 gs(grid_for(ns, kBlock / 64), copies);
+                if (bins_.wave_small == 64) hipLaunchKernelGGL(propose_wave<128>, gs, dim3(kBlock), 0, s, a, lst, ns);
+                else if (bins_.wave_small == 256) hipLaunchKernelGGL(propose_wave<512>, gs, dim3(kBlock), 0, s, a, lst, ns);
+                else hipLaunchKernelGGL(propose_wave<256>, gs, dim3(kBlock), 0, s, a, lst, ns);
+            }
+            if (cnt > ns) hipLaunchKernelGGL(propose_wave<>, dim3(grid_for(cnt - ns, kBlock / 64), copies), dim3(kBlock), 0, s, a, lst + ns, cnt - ns);
+        }
+    }
+}
+
 // Launches refine_tail and waits for its answer: the round to go on with, and whether a block is
-// overloaded. The answer is polled in host memory, which takes about 5 us from the kernel's end
-// to the next launch (a stream synchronisation takes three times as long).
+// overloaded.
 int LpWorkspace::run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded) {
     t.num_labels = num_labels_;
     t.S = subrounds_;
-    t.moves = moves_.p;
-    t.state = tail_.dev;
-    t.seq = ++tail_.seq;
+    t.moves = ctl_.p + kCtlMoves;
+    t.state = mail_.box();
+    t.seq = mail_.next();
     hipLaunchKernelGGL(refine_tail, dim3(1), dim3(kTailThreads), 0, s, a, t);
     KH_CHECK(hipGetLastError());
-    tail_.wait(s);
-    *overloaded = tail_.host[2] != 0;
-    return tail_.host[1];
+    const int* answer = mail_.wait(s);
+    *overloaded = answer[1] != 0;
+    return answer[0];
 }
 
-void TailState::init() {
-    if (host) return;
-    void* h = nullptr;
-    KH_CHECK(hipHostMalloc(&h, 64, hipHostMallocMapped | hipHostMallocCoherent));
-    host = static_cast<volatile int*>(h);
-    host[0] = 0;
-    void* d = nullptr;
-    KH_CHECK(hipHostGetDevicePointer(&d, h, 0));
-    dev = static_cast<int*>(d);
-}
-
-TailState::~TailState() {
-    if (host) (void)hipHostFree(const_cast<int*>(host));
-}
-
-void TailState::wait(hipStream_t s) const {
-    // the stream is asked now and then, so that a failed launch ends the wait
-    for (unsigned spin = 1; host[0] != seq; ++spin) {
-        __builtin_ia32_pause();
-        if (spin % (1u << 16)) continue;
-        const hipError_t e = hipStreamQuery(s);
-        if (e == hipErrorNotReady) {
-            (void)hipGetLastError();  // not an error of ours
-            continue;
-        }
-        KH_CHECK(e);
-        KH_REQUIRE(host[0] == seq, "label propagation: the refinement ended without its answer");
-    }
-    std::atomic_thread_fence(std::memory_order_acquire);
+void LpWorkspace::fetch(hipStream_t s) {
+    if (fetched_) return;
+    mail_.post(s, {ctl_.p, kCtlBig}, {ctl_.p + kCtlErr, 1});
+    std::memcpy(host_ctl_, mail_.wait(s), sizeof(host_ctl_));
+    fetched_ = true;
 }
 
 void LpWorkspace::read_moves(int rounds, int* out, hipStream_t s) {
-    if (rounds <= 0) return;
-    KH_CHECK(hipMemcpyAsync(out, moves_.p, sizeof(int) * rounds, hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
+    fetch(s);
+    std::memcpy(out, host_ctl_ + kCtlMoves, sizeof(int) * std::max(rounds, 0));
 }
 
 void LpWorkspace::check(hipStream_t s) {
-    int e = 0;
-    KH_CHECK(hipMemcpyAsync(&e, err_.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
-    KH_REQUIRE(e == 0, "label propagation: a hash table probe found no free slot (kernel table "
-                       "sizing invariant violated); the result is invalid");
+    fetch(s);
+    KH_REQUIRE(host_ctl_[kCtlBig] == 0,
+               "label propagation: a hash table probe found no free slot (kernel table "
+               "sizing invariant violated); the result is invalid");
 }
 
 long long LpWorkspace::traversed(hipStream_t s) {
+    fetch(s);
     unsigned long long h[64];
-    KH_CHECK(hipMemcpyAsync(h, trav_.p, sizeof(h), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
+    std::memcpy(h, host_ctl_, sizeof(h));
     long long t = 0;
     for (int i = 0; i < 64; ++i) t += (long long)h[i];
     return t;

@@ -3,11 +3,13 @@
 
 #include "common.hpp"
 #include "devbuf.hpp"
+#include "mail.hpp"
 
 namespace kahip {
 
 constexpr int kMaxSub = 8;
 constexpr int kMaxRounds = 64;
+constexpr int kMaxCopies = 3;  // clusterings of run_copies()
 
 // Kernel arguments shared by the propose / filter / admit / apply launches of one sub-round.
 struct LpArgs {
@@ -36,7 +38,12 @@ struct LpArgs {
     // their hub neighbours.
     const int* hub_slot;
     int* hub_cnt;
-    int* err;  // device error flag (kErrProbe), cleared by run(), read by check()
+    int* err;  // device error flag (kErrProbe), cleared by prepare(), read by check()
+    // Independent clusterings of one graph in one launch (gridDim.y of them): clustering y has its
+    // arrays y * copy_stride further on and the tie seed tie_seed, copy_tie1, copy_tie2 (not an
+    // array: indexing a kernel argument by y would put all of them in scratch memory).
+    long long copy_stride;
+    uint32_t copy_tie1, copy_tie2;
 };
 
 // Arguments of refine_tail beyond LpArgs.
@@ -49,21 +56,8 @@ struct TailArgs {
     uint32_t seed;
     int hubs;            // nodes of more than the wave bin's degree exist: never run here
     int* moves;          // per round
-    int* state;          // host-visible {sequence number, next round, overloaded block exists}
+    int* state;          // mail: {number, next round, overloaded block exists}
     int seq;
-};
-
-// Host memory in which refine_tail leaves its answer {sequence number, next round, overloaded}.
-struct TailState {
-    volatile int* host = nullptr;
-    int* dev = nullptr;
-    int seq = 0;
-    TailState() = default;
-    TailState(const TailState&) = delete;
-    TailState& operator=(const TailState&) = delete;
-    ~TailState();
-    void init();
-    void wait(hipStream_t s) const;  // for the answer with number seq
 };
 
 class LpWorkspace {
@@ -71,8 +65,15 @@ public:
     // Bins the nodes of g into per-(sub-round, degree bin) lists and sizes the scratch for
     // num_labels labels. One small host readback.
     // Nodes with include[v] == 0 (include may be null) are left out: they never propose.
+    // copies > 1: for run_copies().
     void prepare(LpMode mode, const DGraph& g, int num_labels, int subrounds, uint32_t seed,
-                 const BinConfig& bins, hipStream_t s, const uint8_t* include = nullptr);
+                 const BinConfig& bins, hipStream_t s, const uint8_t* include = nullptr,
+                 int copies = 1);
+    // One round of `copies` clusterings from single nodes that differ in the seed (and so in the
+    // tie-breaking; the sub-rounds are prepare()'s, one): label receives copies x n labels, size
+    // (scratch) their weights.
+    void run_copies(const DGraph& g, int* label, int* size, int bound, const uint32_t* seeds,
+                    int copies, hipStream_t s);
     // Runs `rounds` synchronous rounds. label/size are device arrays (node -> label,
     // label -> weight). Refinement starts from an all-active frontier.
     // lbound (optional): the bound of each label, replacing `bound`.
@@ -81,13 +82,14 @@ public:
              const int* lbound = nullptr);
     // label[v] = v, size[v] = vwgt[v]
     static void init_cluster_labels(const DGraph& g, int* label, int* size, hipStream_t s);
-    // Moves per round of the last run (synchronises the stream).
+    // Moves per round of the last run (waits for it).
     void read_moves(int rounds, int* out, hipStream_t s);
-    // Directed edges read by the last refinement run (synchronises the stream): the rows scanned
+    // Directed edges read by the last refinement run (waits for it): the rows scanned
     // by the proposal kernels (hubs deciding from their kept counters read none) and the rows of
     // moved nodes scanned to mark their neighbours and update hub counters.
     long long traversed(hipStream_t s);
-    // Throws if a kernel of the last run() set the device error flag (synchronises the stream).
+    // Throws if a kernel of a run() since the last prepare() set the device error flag (waits for
+    // the last run).
     void check(hipStream_t s);
 
     int host_counts[kMaxSub * kNumBins] = {};
@@ -97,9 +99,19 @@ public:
 
 private:
     void build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
-                     const uint8_t* include);
+                     const uint8_t* include, int copies);
+    void launch_proposals(int b, int sr, const LpArgs& a, int cnt, int copies, hipStream_t s);
     int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
-    TailState tail_;
+    void fetch(hipStream_t s);  // host_ctl_ of the last run
+    Mail mail_;
+    // Counters of a run: {traversed edges in 64 spread 64-bit counters, moves per round, lengths
+    // of the hub merges' big and middle task queues per sub-round, error flag}
+    static constexpr int kCtlMoves = 128, kCtlBig = kCtlMoves + kMaxRounds,
+                         kCtlMid = kCtlBig + kMaxSub * kMaxRounds,
+                         kCtlErr = kCtlMid + kMaxSub * kMaxRounds, kCtlInts = kCtlErr + 1;
+    DevBuf<int> ctl_;
+    int host_ctl_[kCtlBig + 1] = {};  // the traversed edges, the moves, the error flag
+    bool fetched_ = false;
     bool small_ = false;  // refinement that starts in refine_tail, without lists
     void build_chunk_maps(hipStream_t s);  // cmap_ of every sub-round (after chunk_prefix_)
     int subrounds_ = 1;
@@ -129,25 +141,23 @@ private:
     DevBuf<int> ct_base_, cnt_t_, pos_t_;
     DevBuf<char> scan_tmp_;
     DevBuf<long long> offm_base_;
-    DevBuf<int> offm_, task_prefix_, bown_, big_tasks_, n_big_tasks_, mid_tasks_, n_mid_tasks_;
+    DevBuf<int> offm_, task_prefix_, bown_, big_tasks_, mid_tasks_;
     DevBuf<int4> bres_;
     DevBuf<int4> cmap_, tmap_, mmap_;  // hub-chunk, (hub, bucket) task, mid-size hub descriptors
     DevBuf<int> midpos_;
     DevBuf<int2> tsub_;  // (hub, bucket) task: {multi-chunk hub index, bucket | buckets << 16}
     DevBuf<uint8_t> fb_;
-    DevBuf<int> lists_, counts_, cursor_, offsets_;
+    DevBuf<int> lists_, bin_, offsets_;
+    int* counts_ = nullptr;  // in bin_: list lengths
     DevBuf<int> clists_, ccount_;  // refinement frontier per list (compacted each round)
-    DevBuf<unsigned long long> edges_;
-    DevBuf<int> prop_t_, prop_gain_, moves_;
+    DevBuf<int> prop_t_, prop_gain_;
     DevBuf<uint8_t> prop_ok_;
     DevBuf<int> inc_, out_;
-    DevBuf<unsigned long long> trav_;
     DevBuf<unsigned long long> top_, dtop_;
     DevBuf<uint8_t> active_, next_active_;
     DevBuf<int> hub_key_, hub_val_;
     DevBuf<int> dense_off_, dense_cnt_;  // chunked dense refinement hubs: per-hub counters
     DevBuf<int> hub_slot_;
-    DevBuf<int> err_;
     long long dense_total_ = 0;
     bool dense_all_ = false;
     long long hub_total_ = 0;

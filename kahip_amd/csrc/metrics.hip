@@ -6,6 +6,7 @@
 // per workgroup and added with one 64-bit atomic. Integer sums: any order gives the same bits.
 
 #include <algorithm>
+#include <cstring>
 #include <mutex>
 
 #include "common.hpp"
@@ -173,8 +174,8 @@ void quality_noalloc(int n, long long m2, const int* xadj, const int* adjncy, co
     KH_CHECK(hipGetLastError());
 }
 
-long long MetricsWorkspace::edge_cut(const DGraph& g, const int* part, hipStream_t s,
-                                     Profiler* prof) {
+const int* MetricsWorkspace::launch_edge_cut(const DGraph& g, const int* part, hipStream_t s,
+                                             Profiler* prof) {
     acc_.reserve(1);
     fill_async(acc_.p, 1, 0ull, s);
     if (g.m2 > 0) {
@@ -186,9 +187,18 @@ long long MetricsWorkspace::edge_cut(const DGraph& g, const int* part, hipStream
                            dim3(kBlock), 0, s, g.n, g.m2, g.xadj, g.adjncy, g.adjwgt, part,
                            acc_.p);
     }
-    unsigned long long h = 0;
-    KH_CHECK(hipMemcpyAsync(&h, acc_.p, sizeof(h), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
+    return reinterpret_cast<const int*>(acc_.p);
+}
+
+long long MetricsWorkspace::edge_cut(const DGraph& g, const int* part, hipStream_t s,
+                                     Profiler* prof) {
+    mail.post(s, {launch_edge_cut(g, part, s, prof), 2});
+    return cut_of(mail.wait(s));
+}
+
+long long MetricsWorkspace::cut_of(const int* words) {
+    unsigned long long h;
+    std::memcpy(&h, words, sizeof(h));
     return (long long)h / 2;
 }
 

@@ -3,6 +3,7 @@
 
 #include "common.hpp"
 #include "devbuf.hpp"
+#include "mail.hpp"
 
 namespace kahip {
 
@@ -10,6 +11,11 @@ class MetricsWorkspace {
 public:
     // Sum over directed edges with endpoints in different blocks, halved (one readback).
     long long edge_cut(const DGraph& g, const int* part, hipStream_t s, Profiler* prof);
+    // The same without the readback: the device words (two) that will hold the doubled cut, and
+    // the cut from their values.
+    const int* launch_edge_cut(const DGraph& g, const int* part, hipStream_t s, Profiler* prof);
+    static long long cut_of(const int* words);
+    Mail mail;
 
 private:
     DevBuf<unsigned long long> acc_;

@@ -656,7 +656,7 @@ void RatingWorkspace::sweeps_and_sketch(const DGraph& g, int bound, uint32_t see
                                         LpWorkspace& lp, Profiler* prof) {
     sig_.reserve(g.n);
     lab_.reserve(3LL * g.n);
-    size_.reserve(g.n);
+    size_.reserve(3LL * g.n);
     rec_.reserve((long long)g.n * (sizeof(NodeRec) / sizeof(int)));
     if (g.n == 0) return;
     {
@@ -665,21 +665,21 @@ void RatingWorkspace::sweeps_and_sketch(const DGraph& g, int bound, uint32_t see
         hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, s, heavy_.p);
         hipLaunchKernelGGL(sketch_light_kernel, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n,
                            g.xadj, g.adjncy, sig_.p, heavy_.p);
-        hipLaunchKernelGGL(sketch_heavy_kernel, dim3(kSketchHeavyGrid), dim3(256), 0, s, g.xadj,
-                           g.adjncy, heavy_.p, sig_.p);
+        if (g.max_degree == 0 || g.max_degree > kSketchLight)  // 0: not known
+            hipLaunchKernelGGL(sketch_heavy_kernel, dim3(kSketchHeavyGrid), dim3(256), 0, s, g.xadj,
+                               g.adjncy, heavy_.p, sig_.p);
     }
     {
         // three one-round sweeps with a single sub-round: the node lists do not depend on the
-        // seed then, so they are built once; the seeds only change the tie-breaking
+        // seed then, so they are built once and each launch covers all three sweeps; the seeds
+        // only change the tie-breaking
         ProfScope ps(prof, "rating_sweeps", 0.0, 3 * g.m2, s);
+        static_assert(kMaxCopies == 3, "three sweeps");
         BinConfig bins;
-        lp.prepare(LpMode::Cluster, g, g.n, 1, 0u, bins, s);
-        for (int i = 0; i < 3; ++i) {
-            int* lab = lab_.p + (long long)i * g.n;
-            const uint32_t sd = hash3(seed, 0xA6u, (uint32_t)i);
-            LpWorkspace::init_cluster_labels(g, lab, size_.p, s);
-            lp.run(LpMode::Cluster, g, lab, size_.p, bound, 1, sd, s, nullptr, "rating_sweep");
-        }
+        lp.prepare(LpMode::Cluster, g, g.n, 1, 0u, bins, s, nullptr, 3);
+        uint32_t seeds[3];
+        for (int i = 0; i < 3; ++i) seeds[i] = hash3(seed, 0xA6u, (uint32_t)i);
+        lp.run_copies(g, lab_.p, size_.p, bound, seeds, 3, s);
         lp.check(s);
     }
     hipLaunchKernelGGL(node_rec_kernel, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n, g.xadj,
@@ -722,14 +722,16 @@ void RatingWorkspace::mlp_forward(const float* feat, long long m, const MlpWeigh
 }
 
 int RatingWorkspace::score_shift(const DGraph& g, hipStream_t s) {
-    map_.reserve(1);
-    int* d = map_.p;
-    hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, s, d);
-    hipLaunchKernelGGL(max_degree_kernel, dim3(std::min(grid_for(g.n, 256), 1024)), dim3(256), 0, s,
-                       g.n, g.xadj, d);
-    int maxdeg = 0;
-    KH_CHECK(hipMemcpyAsync(&maxdeg, d, sizeof(int), hipMemcpyDeviceToHost, s));
-    KH_CHECK(hipStreamSynchronize(s));
+    int maxdeg = g.max_degree;
+    if (maxdeg == 0) {  // a coarse graph
+        map_.reserve(1);
+        int* d = map_.p;
+        hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, s, d);
+        hipLaunchKernelGGL(max_degree_kernel, dim3(std::min(grid_for(g.n, 256), 1024)), dim3(256), 0,
+                           s, g.n, g.xadj, d);
+        mail_.post(s, {d, 1});
+        maxdeg = mail_.wait(s)[0];
+    }
     int shift = 0;
     while (shift < 12 && (long long)maxdeg * (kScoreMax >> shift) >= (1LL << 31)) ++shift;
     KH_REQUIRE((long long)maxdeg * (kScoreMax >> shift) < (1LL << 31), "degree too large");
@@ -737,8 +739,7 @@ int RatingWorkspace::score_shift(const DGraph& g, hipStream_t s) {
 }
 
 void RatingWorkspace::scores(RatingMode mode, const DGraph& g, int bound, uint32_t seed,
-                             const MlpWeights* w, int* score, hipStream_t s, LpWorkspace& lp,
-                             Profiler* prof) {
+                             int* score, hipStream_t s, LpWorkspace& lp, Profiler* prof) {
     if (g.m2 == 0) return;
     const int shift = score_shift(g, s);
     if (mode == RatingMode::ExpansionStar2) {
@@ -748,10 +749,9 @@ void RatingWorkspace::scores(RatingMode mode, const DGraph& g, int bound, uint32
         KH_CHECK(hipGetLastError());
         return;
     }
-    KH_REQUIRE(mode == RatingMode::Learned && w, "learned rating needs MLP weights");
+    KH_REQUIRE(mode == RatingMode::Learned && wpack_.p, "learned rating needs MLP weights");
     // features rounded to BF16 (16 B per edge), then the MLP writes the quantised scores
     featb_.reserve(g.m2 * 8);
-    upload_weights(*w, s);
     sweeps_and_sketch(g, bound, seed, s, lp, prof);
     {
         ProfScope ps(prof, "rating_features", 0.0, g.m2, s);

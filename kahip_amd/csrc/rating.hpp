@@ -39,8 +39,10 @@ public:
                      hipStream_t s, Profiler* prof);
     // Integer scores of the chosen rating for every directed edge of g, shifted right by
     // score_shift(g) (at least 1) so that a node's score sum stays below 2^31.
-    void scores(RatingMode mode, const DGraph& g, int bound, uint32_t seed, const MlpWeights* w,
-                int* score, hipStream_t s, LpWorkspace& lp, Profiler* prof);
+    // Learned: with the weights of the last upload_weights().
+    void scores(RatingMode mode, const DGraph& g, int bound, uint32_t seed, int* score,
+                hipStream_t s, LpWorkspace& lp, Profiler* prof);
+    void upload_weights(const MlpWeights& w, hipStream_t s);
     // Packs params for train_step, which then keeps the pack current.
     void train_begin(const float* params, hipStream_t s);
     // One optimisation step (Adam, step >= 1) of the mean binary cross-entropy of the MLP on
@@ -57,11 +59,11 @@ public:
 private:
     void sweeps_and_sketch(const DGraph& g, int bound, uint32_t seed, hipStream_t s,
                            LpWorkspace& lp, Profiler* prof);
-    void upload_weights(const MlpWeights& w, hipStream_t s);
     DevBuf<unsigned long long> sig_;
     DevBuf<int> lab_, size_, map_, heavy_, rec_;
     DevBuf<float> feat_, logit_, partial_, loss_;
     DevBuf<uint16_t> wpack_, featb_, tpack_;
+    Mail mail_;
 };
 
 // score = clamp(round(logit * 128) + 2048, 1, kScoreMax); the same formula on the host.
