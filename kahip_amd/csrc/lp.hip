@@ -17,7 +17,7 @@
 //            target's top-priority proposal and fits alone;
 //   apply    admitted moves update labels and label weights; scratch is reset.
 // Nodes are binned by degree (per sub-round lists built once per call):
-//   deg <= 8/16/32/64   G lanes per node, one edge per lane, shuffle aggregation (no LDS);
+//   deg <= 8/16/32/64   8 or 16 lanes per node, 1 to 4 edges per lane, summed by DPP moves;
 //   deg <= 512          one wave per node, LDS hash table (open addressing, LDS atomics);
 //   larger              one workgroup per node, hash table in a pre-cleared global region.
 
@@ -132,26 +132,119 @@ __device__ inline void reduce_cand(Cand& c) {
     }
 }
 
-// Rotation within each row of 16 lanes (DPP row_ror: a full-rate VALU move, no LDS crossbar).
-template <int R>
-__device__ inline int row_ror(int x) {
-    if constexpr (R == 0) return x;
-    else return __builtin_amdgcn_update_dpp(0, x, 0x120 + R, 0xF, 0xF, false);
+// ---- lane groups of 8 and 16 (DPP: full-rate VALU moves, no LDS crossbar)
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppXor3 = 0x1B;  // quad_perm
+constexpr int kDppRor = 0x120;                                    // row_ror: + 1 .. 15
+constexpr int kDppMirror = 0x140, kDppHalfMirror = 0x141;         // lane xor 15, xor 7
+template <int CTRL>
+__device__ inline int dpp(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true);
 }
 
-// Adds, for rotations R..15 of (l0, w0, i0) within the lane's row, the weight w0 of every lane
-// whose label l0 equals lab; a lane of lower id i0 with the same label clears leader. The ids are
-// rotated with the values, so the result does not depend on the rotation's direction.
-template <int R>
-__device__ inline void agg_rot(int lab, int gl, int l0, int w0, int i0, int& conn, bool& leader) {
-    if constexpr (R < 16) {
-        const int lr = row_ror<R>(l0), wr = row_ror<R>(w0), ir = row_ror<R>(i0);
-        if (lr == lab) {
-            conn += wr;
-            if (ir < gl) leader = false;
-        }
-        agg_rot<R + 1>(lab, gl, l0, w0, i0, conn, leader);
+// Maximum / minimum over the 8 or 16 lanes of a group, in every lane. After two steps the lanes
+// of a quad agree, so the mirrors pair the quads and then the halves.
+template <int W, class F>
+__device__ inline int group_fold(int x, F f) {
+    static_assert(W == 8 || W == 16, "lane groups of 8 or 16");
+    x = f(x, dpp<kDppXor1>(x));
+    x = f(x, dpp<kDppXor2>(x));
+    x = f(x, dpp<kDppHalfMirror>(x));
+    if constexpr (W == 16) x = f(x, dpp<kDppMirror>(x));
+    return x;
+}
+template <int W>
+__device__ inline int group_max(int x) {
+    return group_fold<W>(x, [](int a, int b) { return max(a, b); });
+}
+template <int W>
+__device__ inline uint32_t group_umax(uint32_t x) {
+    return (uint32_t)group_fold<W>(
+        (int)x, [](int a, int b) { return (int)max((uint32_t)a, (uint32_t)b); });
+}
+template <int W>
+__device__ inline int group_min(int x) {
+    return group_fold<W>(x, [](int a, int b) { return min(a, b); });
+}
+
+// conn[j] += the weights of the entries that CTRL brings from another lane and whose label is
+// lab[j].
+template <int CTRL, int E>
+__device__ inline void add_equal(const int (&lab)[E], const int (&l)[E], const int (&w)[E],
+                                 int (&conn)[E]) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+        const int lr = dpp<CTRL>(l[k]), wr = dpp<CTRL>(w[k]);
+#pragma unroll
+        for (int j = 0; j < E; ++j) conn[j] += lr == lab[j] ? wr : 0;
     }
+}
+template <int R, int E>
+__device__ inline void add_rotations(const int (&lab)[E], const int (&w)[E], int (&conn)[E]) {
+    if constexpr (R < 16) {
+        add_equal<kDppRor + R>(lab, lab, w, conn);
+        add_rotations<R + 1>(lab, w, conn);
+    }
+}
+
+// conn[j] = summed weight of the entries of the lane group (E per lane) with the label of the
+// lane's entry j; absent entries have label -1 and weight 0. Every other lane is visited once: 8
+// lanes by lane xor 1..7 (xor 4..7 through one half mirror), 16 lanes by rotations.
+template <int W, int E>
+__device__ inline void group_sums(const int (&lab)[E], const int (&w)[E], int (&conn)[E]) {
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        conn[j] = w[j];
+#pragma unroll
+        for (int k = 0; k < E; ++k)
+            if (k != j) conn[j] += lab[k] == lab[j] ? w[k] : 0;
+    }
+    if constexpr (W == 16) {
+        add_rotations<1>(lab, w, conn);
+    } else {
+        int hl[E], hw[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            hl[k] = dpp<kDppHalfMirror>(lab[k]);
+            hw[k] = dpp<kDppHalfMirror>(w[k]);
+#pragma unroll
+            for (int j = 0; j < E; ++j) conn[j] += hl[k] == lab[j] ? hw[k] : 0;
+        }
+        add_equal<kDppXor1>(lab, lab, w, conn);
+        add_equal<kDppXor2>(lab, lab, w, conn);
+        add_equal<kDppXor3>(lab, lab, w, conn);
+        add_equal<kDppXor1>(lab, hl, hw, conn);
+        add_equal<kDppXor2>(lab, hl, hw, conn);
+        add_equal<kDppXor3>(lab, hl, hw, conn);
+    }
+}
+
+// Best candidate of a lane group: entry j of a lane brings (conn[j], lab[j], size[j]) if conn[j]
+// >= 0 (entries of one label bring the same candidate). The maximum of better() is taken field by
+// field, one fold each, instead of by exchanging whole candidates. conn = -1 if there is none.
+template <int W, int E>
+__device__ inline Cand group_best(uint32_t tie_seed, int v, const int (&conn)[E],
+                                  const int (&lab)[E], const int (&size)[E]) {
+    Cand c{-1, 0u, 0x7fffffff, 0};
+#pragma unroll
+    for (int j = 0; j < E; ++j) c.conn = max(c.conn, conn[j]);
+    c.conn = group_max<W>(c.conn);
+    uint32_t tie[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        tie[j] = 0u;
+        if (conn[j] == c.conn) tie[j] = hash3(tie_seed, (uint32_t)v, (uint32_t)lab[j]);
+        c.tie = max(c.tie, tie[j]);
+    }
+    c.tie = group_umax<W>(c.tie);
+#pragma unroll
+    for (int j = 0; j < E; ++j)
+        if (conn[j] == c.conn && tie[j] == c.tie) c.lab = min(c.lab, lab[j]);
+    c.lab = group_min<W>(c.lab);
+#pragma unroll
+    for (int j = 0; j < E; ++j)
+        if (lab[j] == c.lab) c.size = max(c.size, size[j]);
+    c.size = group_max<W>(c.size);
+    return c;
 }
 
 template <int W>
@@ -258,27 +351,34 @@ __device__ __attribute__((always_inline)) inline void scan_wave_table(
     }
 }
 
-// ---------------------------------------------------------------- G lanes per node (deg <= G)
-// A virtual block holds IT x (kBlock / G) nodes: every lane group serves IT nodes at once, whose
+// ---------------------------------------------------------------- W lanes per node, E edges per lane
+// Nodes of up to W x E edges: 8 lanes x 1 or 2, 16 lanes x 2 or 4. Bound by vector instructions
+// (RGG 2^22, 12 to 20 edges a node: the time of a launch is its instruction count over the SIMDs'
+// rate), so the labels are summed by comparing every entry with every other one by DPP moves, four
+// instructions a pair of lanes, without finding a leader per label (entries of one label bring the
+// same candidate); several entries per lane share the rest of the work among fewer lanes.
+// Measured per launch at RGG 2^22 against one entry per lane, leaders and whole candidates
+// exchanged through the LDS crossbar: degree 9..16 102 -> 68 us, 17..32 105 -> 52 us.
+// A virtual block holds IT x (kBlock / W) nodes: every lane group serves IT nodes at once, whose
 // dependent loads (list, offsets, targets, labels, label weights) are issued together, so each
 // wave has that many chains in flight.
-// One virtual block (IT x kBlock / G nodes of the list) of the G-lane kernel; every thread of
-// the workgroup calls it (it synchronises the workgroup). `salt` picks the traversal counter.
-template <LpMode M, int G, int IT>
+// One virtual block (IT x kBlock / W nodes of the list); every thread of the workgroup calls it
+// (it synchronises the workgroup). `salt` picks the traversal counter.
+template <LpMode M, int W, int E, int IT>
 __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
                                                                const int* __restrict__ list,
                                                                int count, int vb, int salt) {
-    constexpr int NB = kBlock / G;  // nodes per item and workgroup
-    const int gl = threadIdx.x & (G - 1);
-    int v[IT], own[IT], beg[IT], deg[IT], lab[IT], w[IT];
+    constexpr int NB = kBlock / W;  // nodes per item and workgroup
+    const int gl = threadIdx.x & (W - 1);
+    int v[IT], own[IT], beg[IT], deg[IT], lab[IT][E], w[IT][E];
     bool valid[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        const long long gi = ((long long)vb * IT + i) * NB + threadIdx.x / G;
+        const long long gi = ((long long)vb * IT + i) * NB + threadIdx.x / W;
         valid[i] = gi < count;
         v[i] = valid[i] ? list[gi] : 0;
     }
-    // every lane of the group takes part in the shuffles below: no early exit
+    // every lane of the group takes part in the exchanges below: no early exit
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         own[i] = valid[i] ? a.label[v[i]] : -1;
@@ -286,67 +386,63 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
         deg[i] = valid[i] ? a.xadj[v[i] + 1] - beg[i] : 0;
     }
 #pragma unroll
-    for (int i = 0; i < IT; ++i) {
-        if constexpr (G >= 16) {  // rows of 9..64 entries: streamed (non-temporal)
-            lab[i] = gl < deg[i] ? __builtin_nontemporal_load(a.adjncy + beg[i] + gl) : -1;
-            w[i] = gl < deg[i] ? __builtin_nontemporal_load(a.adjwgt + beg[i] + gl) : 0;
-        } else {
-            lab[i] = gl < deg[i] ? a.adjncy[beg[i] + gl] : -1;
-            w[i] = gl < deg[i] ? a.adjwgt[beg[i] + gl] : 0;
-        }
-    }
-#pragma unroll
     for (int i = 0; i < IT; ++i)
-        if (lab[i] >= 0) lab[i] = a.label[lab[i]];
-    // conn = summed weight of the group's lanes with this lane's label; leader = the lowest of
-    // them. Groups of 16, 32 and 64 lanes are whole DPP rows: rotations within the row, then
-    // within each other row of the group after one swap (xor 16, 32, 48), visit every lane of
-    // the group once.
-    int conn[IT];
-    bool leader[IT];
 #pragma unroll
-    for (int i = 0; i < IT; ++i) {
-        conn[i] = 0;
-        leader[i] = lab[i] >= 0;
-        if constexpr (G >= 16) {
-            conn[i] = w[i];
-            agg_rot<1>(lab[i], gl, lab[i], w[i], gl, conn[i], leader[i]);
-#pragma unroll
-            for (int x = 16; x < G; x += 16)
-                agg_rot<0>(lab[i], gl, __shfl_xor(lab[i], x, G), __shfl_xor(w[i], x, G), gl ^ x,
-                           conn[i], leader[i]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < G; ++j) {
-                const int lj = __shfl(lab[i], j, G);
-                const int wj = __shfl(w[i], j, G);
-                if (lj == lab[i]) {
-                    conn[i] += wj;
-                    if (j < gl) leader[i] = false;
-                }
+        for (int j = 0; j < E; ++j) {
+            const int e = gl + j * W;
+            lab[i][j] = -1;
+            w[i][j] = 0;
+            if (e >= deg[i]) continue;
+            if constexpr (W * E > 8) {  // rows of 9..64 entries: streamed (non-temporal)
+                lab[i][j] = __builtin_nontemporal_load(a.adjncy + beg[i] + e);
+                w[i][j] = __builtin_nontemporal_load(a.adjwgt + beg[i] + e);
+            } else {
+                lab[i][j] = a.adjncy[beg[i] + e];
+                w[i][j] = a.adjwgt[beg[i] + e];
             }
         }
-    }
-    int conn_own[IT], nw[IT], sz[IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            if (lab[i][j] >= 0) lab[i][j] = a.label[lab[i][j]];
+    int nw[IT], sz[IT][E], lb[IT][E];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        conn_own[i] = reduce_max<G>((lab[i] >= 0 && lab[i] == own[i]) ? conn[i] : 0);
         nw[i] = valid[i] ? a.vwgt[v[i]] : 0;
-        sz[i] = (leader[i] && lab[i] != own[i]) ? a.size[lab[i]] : 0;
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            sz[i][j] = lab[i][j] >= 0 && lab[i][j] != own[i] ? a.size[lab[i][j]] : 0;
+    }
+    if (a.lbound) {  // uniform
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+#pragma unroll
+            for (int j = 0; j < E; ++j)
+                lb[i][j] = lab[i][j] >= 0 && lab[i][j] != own[i] ? a.lbound[lab[i][j]] : 0;
+    } else {
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+#pragma unroll
+            for (int j = 0; j < E; ++j) lb[i][j] = a.bound;
     }
     Contrib r[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        Cand c{-1, 0u, 0x7fffffff, 0};
-        if (leader[i] && lab[i] != own[i] &&
-            (long long)sz[i] + nw[i] < (long long)bound_of(a, lab[i])) {
-            c.conn = conn[i];
-            c.tie = hash3(a.tie_seed, (uint32_t)v[i], (uint32_t)lab[i]);
-            c.lab = lab[i];
-            c.size = sz[i];
+        int conn[E], conn_own = 0;
+        group_sums<W>(lab[i], w[i], conn);
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const int l = lab[i][j];
+            conn_own = max(conn_own, (l >= 0) & (l == own[i]) ? conn[j] : 0);
+            // candidates: other labels with room for the node (a select without branches: hipcc
+            // 7.2 lost the -1 of a lane in the branching form)
+            const bool room = (long long)sz[i][j] + nw[i] < (long long)lb[i][j];
+            conn[j] = (l >= 0) & (l != own[i]) & room ? conn[j] : -1;
         }
-        reduce_cand<G>(c);
-        r[i] = (valid[i] && gl == 0) ? propose<M>(a, v[i], own[i], nw[i], conn_own[i], c)
+        conn_own = group_max<W>(conn_own);
+        const Cand c = group_best<W>(a.tie_seed, v[i], conn, lab[i], sz[i]);
+        r[i] = (valid[i] && gl == 0) ? propose<M>(a, v[i], own[i], nw[i], conn_own, c)
                                      : Contrib{-1, 0, 0ull, false};
     }
     // The block's proposals are combined per (target, kind) in an LDS hash before the atomics:
@@ -355,7 +451,7 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
     constexpr int HC = 2 * IT * NB;  // slots (load <= 1/2)
     // probed with a mask: a size that is not a power of two leaves slots unreachable and the
     // probe loop below would never end
-    static_assert((HC & (HC - 1)) == 0, "IT x kBlock / G must be a power of two");
+    static_assert((HC & (HC - 1)) == 0, "IT x kBlock / W must be a power of two");
     __shared__ int h_tag[HC];        // (label << 1) | departure, -1: empty
     __shared__ int h_w[HC];
     __shared__ unsigned long long h_key[HC];
@@ -397,11 +493,11 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
     __syncthreads();  // the LDS of this virtual block is read before the next one writes it
 }
 
-template <int G, int IT>
+template <int W, int E, int IT>
 __global__ __launch_bounds__(kBlock) void propose_group(LpArgs a, const int* __restrict__ list,
                                                         int count) {
     select_copy(a);
-    group_vb<LpMode::Cluster, G, IT>(a, list, count, blockIdx.x, blockIdx.x);
+    group_vb<LpMode::Cluster, W, E, IT>(a, list, count, blockIdx.x, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- one wave per node
@@ -508,7 +604,7 @@ __global__ __launch_bounds__(kBlock) void propose_wave(LpArgs a, const int* __re
 
 // Refinement: the proposals of all degree lists of a sub-round in one launch. The lists are the
 // round's compacted frontier (lengths on the device); the workgroups stride over the virtual
-// blocks of the five lists in order (G = 8, 16, 32, 64 lanes per node, then a wave per node), so a
+// blocks of the five lists in order (8 or 16 lanes per node, then a wave per node), so a
 // sub-round costs one launch instead of five. Same per-node code as the per-list kernels.
 // Refinement hubs with kept per-block counters (every hub of the level has them when their
 // counters fit): one wave per active hub decides from its k counters (as hub_dense_decide does
@@ -550,8 +646,8 @@ struct FrontierLists {
 template <int IT, bool DENSE, int DCAP = kWaveDense>
 __global__ __launch_bounds__(kBlock) void propose_frontier(LpArgs a, FrontierLists F,
                                                            int num_labels) {
-    constexpr int NPB[kNumBins] = {IT * (kBlock / 8), IT * (kBlock / 16), IT * (kBlock / 32),
-                                   IT * (kBlock / 64), kBlock / 64, kBlock / 64};
+    constexpr int NPB[kNumBins] = {IT * (kBlock / 8), IT * (kBlock / 8), IT * (kBlock / 16),
+                                   IT * (kBlock / 16), kBlock / 64, kBlock / 64};
     int cnt[kNumBins], nvb[kNumBins], total = 0;
 #pragma unroll
     for (int b = 0; b < kNumBins; ++b) {
@@ -568,10 +664,10 @@ __global__ __launch_bounds__(kBlock) void propose_frontier(LpArgs a, FrontierLis
                 b = k + 1;
             }
         switch (b) {
-            case 0: group_vb<LpMode::Refine, 8, IT>(a, F.list[0], cnt[0], vb, t); break;
-            case 1: group_vb<LpMode::Refine, 16, IT>(a, F.list[1], cnt[1], vb, t); break;
-            case 2: group_vb<LpMode::Refine, 32, IT>(a, F.list[2], cnt[2], vb, t); break;
-            case 3: group_vb<LpMode::Refine, 64, IT>(a, F.list[3], cnt[3], vb, t); break;
+            case 0: group_vb<LpMode::Refine, 8, 1, IT>(a, F.list[0], cnt[0], vb, t); break;
+            case 1: group_vb<LpMode::Refine, 8, 2, IT>(a, F.list[1], cnt[1], vb, t); break;
+            case 2: group_vb<LpMode::Refine, 16, 2, IT>(a, F.list[2], cnt[2], vb, t); break;
+            case 3: group_vb<LpMode::Refine, 16, 4, IT>(a, F.list[3], cnt[3], vb, t); break;
             case 4:
                 wave_vb<LpMode::Refine, DENSE, kWaveCap, DCAP>(a, F.list[4], cnt[4], num_labels,
                                                                 vb, t);
@@ -1392,21 +1488,18 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
                     const int own = valid ? a.label[v] : -1;
                     const int beg = valid ? a.xadj[v] : 0;
                     const int deg = valid ? a.xadj[v + 1] - beg : 0;
-                    int lab = gl < deg ? a.adjncy[beg + gl] : -1;
-                    const int w = gl < deg ? a.adjwgt[beg + gl] : 0;
-                    if (lab >= 0) lab = a.label[lab];
-                    int conn = w;
-                    bool leader = lab >= 0;
-                    agg_rot<1>(lab, gl, lab, w, gl, conn, leader);
-                    const int conn_own =
-                        reduce_max<kTailGroup>((lab >= 0 && lab == own) ? conn : 0);
+                    int lab[1] = {gl < deg ? a.adjncy[beg + gl] : -1};
+                    const int w[1] = {gl < deg ? a.adjwgt[beg + gl] : 0};
+                    if (lab[0] >= 0) lab[0] = a.label[lab[0]];
                     const int nw = valid ? a.vwgt[v] : 0;
-                    Cand c{-1, 0u, 0x7fffffff, 0};
-                    if (leader && lab != own &&
-                        (long long)lsize[lab] + nw < (long long)bound_of(a, lab))
-                        c = Cand{conn, hash3(tie_seed, (uint32_t)v, (uint32_t)lab), lab,
-                                 lsize[lab]};
-                    reduce_cand<kTailGroup>(c);
+                    int conn[1], size[1] = {lab[0] >= 0 ? lsize[lab[0]] : 0};
+                    group_sums<kTailGroup>(lab, w, conn);
+                    const int conn_own =
+                        group_max<kTailGroup>(lab[0] >= 0 && lab[0] == own ? conn[0] : 0);
+                    const int lb = a.lbound ? (lab[0] >= 0 ? a.lbound[lab[0]] : 0) : a.bound;
+                    const bool room = (long long)size[0] + nw < (long long)lb;
+                    conn[0] = (lab[0] >= 0) & (lab[0] != own) & room ? conn[0] : -1;
+                    const Cand c = group_best<kTailGroup>(tie_seed, v, conn, lab, size);
                     if (valid && gl == 0) put(i, v, own, nw, conn_own, c);
                 }
                 // one wave per larger node: a counter per label, summed with LDS atomics; every
@@ -1839,15 +1932,15 @@ __global__ void block_weights_global(int n, const int* __restrict__ part,
 
 inline int grid_for(long long work, int block) { return (int)((work + block - 1) / block); }
 
-// The clustering's G-lane proposal kernel of one list with `items` nodes per lane group, one
+// The clustering's lane-group proposal kernel of one list with `items` nodes per lane group, one
 // workgroup per virtual block.
-template <int G>
+template <int W, int E>
 void launch_group(int items, const LpArgs& a, const int* lst, int cnt, int copies, hipStream_t s) {
-    const dim3 grid(grid_for((long long)cnt * G, kBlock * items), copies);
+    const dim3 grid(grid_for((long long)cnt * W, kBlock * items), copies);
     switch (items) {
-        case 1: hipLaunchKernelGGL((propose_group<G, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
-        case 4: hipLaunchKernelGGL((propose_group<G, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
-        default: hipLaunchKernelGGL((propose_group<G, 2>), grid, dim3(kBlock), 0, s, a, lst, cnt);
+        case 1: hipLaunchKernelGGL((propose_group<W, E, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
+        case 4: hipLaunchKernelGGL((propose_group<W, E, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
+        default: hipLaunchKernelGGL((propose_group<W, E, 2>), grid, dim3(kBlock), 0, s, a, lst, cnt);
     }
 }
 
@@ -2505,10 +2598,10 @@ void LpWorkspace::launch_proposals(int b, int sr, const LpArgs& a, int cnt, int 
                                    hipStream_t s) {
     const int* lst = lists_.p + host_offsets[sr * kNumBins + b];
     switch (b) {
-        case 0: launch_group<8>(bins_.group_items, a, lst, cnt, copies, s); break;
-        case 1: launch_group<16>(bins_.group_items, a, lst, cnt, copies, s); break;
-        case 2: launch_group<32>(bins_.group_items, a, lst, cnt, copies, s); break;
-        case 3: launch_group<64>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 0: launch_group<8, 1>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 1: launch_group<8, 2>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 2: launch_group<16, 2>(bins_.group_items, a, lst, cnt, copies, s); break;
+        case 3: launch_group<16, 4>(bins_.group_items, a, lst, cnt, copies, s); break;
         default: {
             const int ns = host_wave_small_[sr];  // degree <= wave_small, first
             if (ns > 0) {
