@@ -468,6 +468,10 @@ void partition_batch(Engine& eng, const DGraph& g0, int G, const int* node_off,
         for (int i = 0; i < G; ++i)
             if (S.coarsest_level[i] == l) todo.push_back(i);
         if (todo.empty()) continue;
+        // the largest graphs first, so that none of them is left for one thread at the end
+        std::stable_sort(todo.begin(), todo.end(), [&](int a, int b) {
+            return S.coarsest_n[a] > S.coarsest_n[b];
+        });
         HostGraph hg;
         download_graph(level_graph(l), hg, s);
         const std::vector<int>& o = offs[l];

@@ -14,6 +14,7 @@
 #include "initial_partition.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <exception>
 #include <functional>
@@ -59,70 +60,117 @@ uint64_t stream_seed(uint64_t seed, uint64_t a, uint64_t b) {
     return r.next();
 }
 
+// ------------------------------------------------------------------ graphs of the bisections
+// Target and weight of an edge side by side: every loop below reads both.
+struct Edge {
+    int to, w;
+};
+struct Graph {
+    int n = 0;
+    std::vector<int> xadj, vwgt;
+    std::vector<Edge> edges;
+    long long total_weight() const {
+        long long t = 0;
+        for (int v = 0; v < n; ++v) t += vwgt[v];
+        return t;
+    }
+};
+
+// Graphs of more nodes than this miss the near caches when they are walked in random order; the
+// walks then fetch the rows and labels of the nodes ahead (RGG 2^22, k = 64: clustering in the
+// bisections 1.7 -> 1.1 s of thread time).
+constexpr int kPrefetchNodes = 4096;
+
 // ------------------------------------------------------------------ coarsening for bisection
 // Sequential size-constrained LP in a random order (the reference's IP uses the same clustering
 // with factor 12 inside the bisection hierarchy). Returns the number of clusters; label is
 // renumbered to 0..nc-1 in first-appearance order.
-int lp_cluster(const HostGraph& g, long long bound, int iters, Rng& rng, std::vector<int>& label) {
+int lp_cluster(const Graph& g, long long bound, int iters, Rng& rng, std::vector<int>& label_out) {
     const int n = g.n;
-    label.resize(n);
+    label_out.resize(n);
     // int32 sizes and connection sums: the library keeps total node and edge weight below 2^31
-    std::vector<int> size(n);
-    std::vector<int> order(n);
+    int max_row = 0;
+    for (int v = 0; v < n; ++v) max_row = std::max(max_row, g.xadj[v + 1] - g.xadj[v]);
+    std::vector<int> size_v(g.vwgt), order_v(n), acc_v(n, 0), touched_v(max_row + 1);
+    int* const label = label_out.data();
+    int* const size = size_v.data();
+    int* const order = order_v.data();
+    int* const acc = acc_v.data();
+    int* const touched = touched_v.data();
+    const int* const xadj = g.xadj.data();
+    const int* const vwgt = g.vwgt.data();
+    const Edge* const edges = g.edges.data();
     for (int v = 0; v < n; ++v) {
         label[v] = v;
-        size[v] = g.vwgt[v];
         order[v] = v;
     }
     for (int i = n - 1; i > 0; --i) std::swap(order[i], order[rng.below(i + 1)]);
-    std::vector<int> acc(n, 0);
-    std::vector<int> touched;
+    const bool far = n > kPrefetchNodes;
+    constexpr int kFar = 24, kMid = 12, kNear = 6, kRow = 16;
     for (int it = 0; it < iters; ++it) {
         int moved = 0;
-        for (int v : order) {
+        for (int i = 0; i < n; ++i) {
+            if (far) {
+                if (i + kFar < n) {
+                    __builtin_prefetch(xadj + order[i + kFar]);
+                    __builtin_prefetch(label + order[i + kFar]);
+                }
+                if (i + kMid < n) __builtin_prefetch(edges + xadj[order[i + kMid]]);
+                if (i + kNear < n) {
+                    const int u = order[i + kNear];
+                    const int e1 = std::min(xadj[u + 1], xadj[u] + kRow);
+                    for (int e = xadj[u]; e < e1; ++e) __builtin_prefetch(label + edges[e].to);
+                }
+            }
+            const int v = order[i];
             const int own = label[v];
-            for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
-                const int c = label[g.adjncy[e]];
-                if (acc[c] == 0) touched.push_back(c);
-                acc[c] += g.adjwgt[e];
+            int cnt = 0;
+            for (int e = xadj[v], e1 = xadj[v + 1]; e < e1; ++e) {
+                const int c = label[edges[e].to];
+                const int old = acc[c];
+                touched[cnt] = c;
+                cnt += old == 0;
+                acc[c] = old + edges[e].w;
             }
             int best = own;
             int bv = acc[own];
-            for (int c : touched) {
+            for (int t = 0; t < cnt; ++t) {
+                const int c = touched[t];
+                const int ac = acc[c];
                 // the connection test first: it rejects most candidates without reading size[c]
-                if (c == own || acc[c] < bv) continue;
-                if ((long long)size[c] + g.vwgt[v] >= bound) continue;
-                if (acc[c] > bv || rng.coin()) {
+                if (c == own || ac < bv) continue;
+                if ((long long)size[c] + vwgt[v] >= bound) continue;
+                if (ac > bv || rng.coin()) {
                     best = c;
-                    bv = acc[c];
+                    bv = ac;
                 }
             }
-            for (int c : touched) acc[c] = 0;
-            touched.clear();
+            for (int t = 0; t < cnt; ++t) acc[touched[t]] = 0;
             if (best != own) {
-                size[own] -= g.vwgt[v];
-                size[best] += g.vwgt[v];
+                size[own] -= vwgt[v];
+                size[best] += vwgt[v];
                 label[v] = best;
                 ++moved;
             }
         }
         if (moved == 0) break;
     }
-    std::vector<int> remap(n, -1);
+    std::fill(acc, acc + n, -1);  // now: new id of a label
     int nc = 0;
     for (int v = 0; v < n; ++v) {
-        int& r = remap[label[v]];
+        int& r = acc[label[v]];
         if (r < 0) r = nc++;
         label[v] = r;
     }
     return nc;
 }
 
-HostGraph contract(const HostGraph& g, const std::vector<int>& label, int nc) {
-    HostGraph c;
+Graph contract(const Graph& g, const std::vector<int>& label_v, int nc) {
+    Graph c;
     c.n = nc;
     c.vwgt.assign(nc, 0);
     c.xadj.assign(nc + 1, 0);
+    const int* const label = label_v.data();
     std::vector<int> start(nc + 1, 0), members(g.n);
     for (int v = 0; v < g.n; ++v) {
         c.vwgt[label[v]] += g.vwgt[v];
@@ -131,27 +179,37 @@ HostGraph contract(const HostGraph& g, const std::vector<int>& label, int nc) {
     for (int p = 0; p < nc; ++p) start[p + 1] += start[p];
     std::vector<int> pos(start.begin(), start.end() - 1);
     for (int v = 0; v < g.n; ++v) members[pos[label[v]]++] = v;
-    std::vector<int> acc(nc, 0);
-    std::vector<int> touched;
-    c.adjncy.reserve(g.adjncy.size() / 2);
-    c.adjwgt.reserve(g.adjncy.size() / 2);
+    std::vector<int> acc_v(nc, 0), touched;
+    int* const acc = acc_v.data();
+    const int* const xadj = g.xadj.data();
+    const Edge* const edges = g.edges.data();
+    c.edges.reserve(g.edges.size() / 2);
+    const bool far = g.n > kPrefetchNodes;
+    constexpr int kMid = 12, kNear = 6, kRow = 16;
     for (int p = 0; p < nc; ++p) {
         for (int i = start[p]; i < start[p + 1]; ++i) {
+            if (far) {
+                if (i + kMid < g.n) __builtin_prefetch(edges + xadj[members[i + kMid]]);
+                if (i + kNear < g.n) {
+                    const int u = members[i + kNear];
+                    const int e1 = std::min(xadj[u + 1], xadj[u] + kRow);
+                    for (int e = xadj[u]; e < e1; ++e) __builtin_prefetch(label + edges[e].to);
+                }
+            }
             const int v = members[i];
-            for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
-                const int q = label[g.adjncy[e]];
+            for (int e = xadj[v], e1 = xadj[v + 1]; e < e1; ++e) {
+                const int q = label[edges[e].to];
                 if (q == p) continue;
                 if (acc[q] == 0) touched.push_back(q);
-                acc[q] += g.adjwgt[e];
+                acc[q] += edges[e].w;
             }
         }
         for (int q : touched) {
-            c.adjncy.push_back(q);
-            c.adjwgt.push_back(acc[q]);
+            c.edges.push_back({q, acc[q]});
             acc[q] = 0;
         }
         touched.clear();
-        c.xadj[p + 1] = (int)c.adjncy.size();
+        c.xadj[p + 1] = (int)c.edges.size();
     }
     return c;
 }
@@ -161,266 +219,257 @@ struct Bisection {
     std::vector<char> side;
     long long w[2] = {0, 0};
     long long cut = 0;
+    bool counted = true;  // false: cut is not known yet, the first FM pass counts it
 };
-
-long long bis_cut(const HostGraph& g, const std::vector<char>& side) {
-    long long c = 0;
-    for (int v = 0; v < g.n; ++v)
-        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e)
-            if (side[v] != side[g.adjncy[e]]) c += g.adjwgt[e];
-    return c / 2;
-}
 
 inline long long overload(const long long w[2], const long long maxw[2]) {
     return std::max(0LL, w[0] - maxw[0]) + std::max(0LL, w[1] - maxw[1]);
 }
 
-// Addressable binary max-heap of the FM queue of one side: one entry per node, ordered by
-// (gain, random tiebreak, node). A gain change draws a new tiebreak and moves the entry in place.
-struct FmHeap {
-    std::vector<int> h;  // node ids in heap order
-    int* pos = nullptr;  // pos[v]: index of v in h, -1 if absent (shared by both sides)
-    const long long* gain = nullptr;
-    const uint64_t* key = nullptr;  // tie << 32 | node
-    bool less(int a, int b) const {
-        return gain[a] < gain[b] || (gain[a] == gain[b] && key[a] < key[b]);
+// What a move reads and writes of a neighbour.
+struct FmNode {
+    long long gain;
+    int pos;  // index in its side's heap, -1: not in it
+    char side, locked;
+};
+
+// Addressable 4-ary max-heap of the FM queue of one side: one entry per node, ordered by (gain,
+// random tiebreak, node), a total order, so the order of the pops does not depend on the shape of
+// the heap. Entries carry their keys: a sift reads four neighbouring entries instead of keys
+// scattered over the nodes. A gain change draws a new tiebreak and moves the entry in place.
+struct FmEntry {
+    long long gain;
+    uint64_t key;  // tie << 32 | node
+    int node() const { return (int)(uint32_t)key; }
+    unsigned __int128 order() const {  // one comparison without branches
+        return ((unsigned __int128)((uint64_t)gain ^ (1ull << 63)) << 64) | key;
     }
-    void up(int i) {
-        const int v = h[i];
+    bool operator<(const FmEntry& o) const {
+        return order() < o.order();
+    }
+};
+struct FmHeap {
+    FmEntry* h = nullptr;
+    int size = 0;
+    FmNode* node = nullptr;
+    void put(int i, const FmEntry& e) {
+        h[i] = e;
+        node[e.node()].pos = i;
+    }
+    void up(int i, const FmEntry& e) {
         while (i > 0) {
-            const int p = (i - 1) >> 1;
-            if (!less(h[p], v)) break;
-            h[i] = h[p];
-            pos[h[i]] = i;
+            const int p = (i - 1) >> 2;
+            if (!(h[p] < e)) break;
+            put(i, h[p]);
             i = p;
         }
-        h[i] = v;
-        pos[v] = i;
+        put(i, e);
     }
-    void down(int i) {
-        const int v = h[i];
-        const int sz = (int)h.size();
+    void down(int i, const FmEntry& e) {
         while (true) {
-            int c = 2 * i + 1;
-            if (c >= sz) break;
-            if (c + 1 < sz && less(h[c], h[c + 1])) ++c;
-            if (!less(v, h[c])) break;
-            h[i] = h[c];
-            pos[h[i]] = i;
+            const int c0 = 4 * i + 1;
+            if (c0 >= size) break;
+            const int c1 = std::min(c0 + 4, size);
+            int c = c0;
+            if (c1 - c0 == 4) {
+                const int x = c0 + (h[c0] < h[c0 + 1]), y = c0 + 2 + (h[c0 + 2] < h[c0 + 3]);
+                c = h[x] < h[y] ? y : x;
+            } else {
+                for (int j = c0 + 1; j < c1; ++j)
+                    if (h[c] < h[j]) c = j;
+            }
+            if (!(e < h[c])) break;
+            put(i, h[c]);
             i = c;
         }
-        h[i] = v;
-        pos[v] = i;
+        put(i, e);
     }
-    void insert(int v) {
-        h.push_back(v);
-        up((int)h.size() - 1);
+    void append(const FmEntry& e) { h[size++] = e; }  // before heapify()
+    void heapify() {
+        for (int i = 0; i < size; ++i) node[h[i].node()].pos = i;
+        for (int i = (size - 2) >> 2; i >= 0 && size > 1; --i) down(i, FmEntry(h[i]));
     }
-    void update(int v) {  // after key/gain of v changed
-        const int i = pos[v];
-        up(i);
-        down(pos[v]);
+    void insert(const FmEntry& e) { up(size++, e); }
+    void update(int i, const FmEntry& e) {
+        if (i > 0 && h[(i - 1) >> 2] < e) up(i, e);
+        else down(i, e);
     }
     void pop() {
-        const int v = h[0];
-        pos[v] = -1;
-        const int last = h.back();
-        h.pop_back();
-        if (!h.empty()) {
-            h[0] = last;
-            pos[last] = 0;
-            down(0);
-        }
+        node[h[0].node()].pos = -1;
+        const FmEntry last = h[--size];
+        if (size > 0) down(0, last);
     }
 };
 
 // Buffers of fm_pass, kept per thread across calls (the tries call it thousands of times on
 // graphs of a few hundred nodes, where allocation would dominate).
 struct FmScratch {
-    std::vector<long long> gain;
-    std::vector<uint64_t> key;
-    std::vector<int> pos, moved;
-    std::vector<char> locked;
-    std::vector<int> heap[2];
+    std::vector<FmNode> node;
+    std::vector<FmEntry> heap[2];
+    std::vector<int> moved;
 };
 
 // One FM pass with rollback to the best prefix. State order: lower overload first, then lower
 // cut. Returns true when the state improved. Queues: boundary nodes of each side by gain; a node
 // enters its queue when it first has a moved neighbour or at the start if it is on the boundary.
-bool fm_pass(const HostGraph& g, Bisection& b, const long long maxw[2], int stall_limit,
+bool fm_pass(const Graph& g, Bisection& b, const long long maxw[2], int stall_limit,
              int stall_pct, Rng& rng) {
     static thread_local FmScratch sc;
     const int n = g.n;
-    // moved into locals for the pass (and back at the end), so that the compiler can keep their
-    // data pointers in registers across the char stores into b.side
-    std::vector<long long> gain = std::move(sc.gain);
-    std::vector<uint64_t> key = std::move(sc.key);
-    std::vector<int> pos = std::move(sc.pos);
-    std::vector<int> moved = std::move(sc.moved);
-    std::vector<char> locked = std::move(sc.locked);
-    FmHeap pq[2];
-    pq[0].h = std::move(sc.heap[0]);
-    pq[1].h = std::move(sc.heap[1]);
-    gain.assign(n, 0);
-    key.resize(n);
-    pos.assign(n, -1);
-    locked.assign(n, 0);
-    moved.clear();
-    for (int s = 0; s < 2; ++s) {
-        pq[s].h.clear();
-        pq[s].pos = pos.data();
-        pq[s].gain = gain.data();
-        pq[s].key = key.data();
+    if ((int)sc.node.size() < n) {
+        sc.node.resize(n);
+        sc.heap[0].resize(n);
+        sc.heap[1].resize(n);
+        sc.moved.resize(n);
     }
+    FmNode* const node = sc.node.data();
+    int* const moved = sc.moved.data();
+    FmHeap pq[2];
+    pq[0].h = sc.heap[0].data();
+    pq[1].h = sc.heap[1].data();
+    pq[0].node = pq[1].node = node;
+    const int* const xadj = g.xadj.data();
+    const int* const vwgt = g.vwgt.data();
+    const Edge* const edges = g.edges.data();
+    char* const side = b.side.data();
     int nb = 0;
+    long long ext2 = 0;  // twice the cut
     for (int v = 0; v < n; ++v) {
-        long long gv = 0;
+        const char sv = side[v];
+        long long ext = 0, all = 0;
         bool bnd = false;
-        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
-            if (b.side[g.adjncy[e]] != b.side[v]) {
-                gv += g.adjwgt[e];
-                bnd = true;
-            } else {
-                gv -= g.adjwgt[e];
-            }
+        for (int e = xadj[v], e1 = xadj[v + 1]; e < e1; ++e) {
+            const bool other = side[edges[e].to] != sv;
+            const long long w = edges[e].w;
+            all += w;
+            ext += other ? w : 0;
+            bnd |= other;
         }
-        gain[v] = gv;
+        ext2 += ext;
+        node[v] = FmNode{2 * ext - all, -1, sv, 0};
         if (bnd) {
-            key[v] = ((uint64_t)(uint32_t)rng.next() << 32) | (uint32_t)v;
-            pq[(int)b.side[v]].insert(v);
+            pq[(int)sv].append({2 * ext - all, ((uint64_t)(uint32_t)rng.next() << 32) | (uint32_t)v});
             ++nb;
         }
     }
+    if (!b.counted) b.cut = ext2 / 2;
+    b.counted = true;
+    pq[0].heapify();
+    pq[1].heapify();
     if (stall_pct > 0) stall_limit = std::max(15, (int)((long long)stall_pct * nb / 100));
     long long cut = b.cut, w[2] = {b.w[0], b.w[1]};
     long long best_cut = cut, best_over = overload(w, maxw);
-    size_t best_len = 0;
+    int n_moved = 0, best_len = 0;
     int since_best = 0;
     while (true) {
-        const int v0 = pq[0].h.empty() ? -1 : pq[0].h[0];
-        const int v1 = pq[1].h.empty() ? -1 : pq[1].h[0];
         // a move from s to 1-s is allowed if the target stays within its bound or the source
         // is overloaded
-        auto ok = [&](int v, int s) {
-            if (v < 0) return false;
+        auto ok = [&](int s) {
+            if (pq[s].size == 0) return false;
             const int t = 1 - s;
-            return w[t] + g.vwgt[v] <= maxw[t] || w[s] > maxw[s];
+            return w[t] + vwgt[pq[s].h[0].node()] <= maxw[t] || w[s] > maxw[s];
         };
-        const bool a0 = ok(v0, 0), a1 = ok(v1, 1);
-        int v = -1, s = 0;
+        const bool a0 = ok(0), a1 = ok(1);
+        int s;
         if (a0 && a1) {
-            if (gain[v0] > gain[v1] || (gain[v0] == gain[v1] && w[0] >= w[1])) {
-                v = v0;
-                s = 0;
-            } else {
-                v = v1;
-                s = 1;
-            }
+            const long long g0 = pq[0].h[0].gain, g1 = pq[1].h[0].gain;
+            s = g0 > g1 || (g0 == g1 && w[0] >= w[1]) ? 0 : 1;
         } else if (a0) {
-            v = v0;
             s = 0;
         } else if (a1) {
-            v = v1;
             s = 1;
+        } else {
+            break;
         }
-        if (v < 0) break;
+        const int v = pq[s].h[0].node();
+        const long long gv = pq[s].h[0].gain;
         pq[s].pop();
-        const long long gv = gain[v];
-        b.side[v] = (char)(1 - s);
-        locked[v] = 1;
-        w[s] -= g.vwgt[v];
-        w[1 - s] += g.vwgt[v];
+        node[v].side = (char)(1 - s);
+        node[v].locked = 1;
+        w[s] -= vwgt[v];
+        w[1 - s] += vwgt[v];
         cut -= gv;
-        moved.push_back(v);
-        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
-            const int u = g.adjncy[e];
-            if (locked[u]) continue;
+        moved[n_moved++] = v;
+        for (int e = xadj[v], e1 = xadj[v + 1]; e < e1; ++e) {
+            const int u = edges[e].to;
+            FmNode& nu = node[u];
+            if (nu.locked) continue;
             // v left u's side (if u on s) or joined u's side (if u on 1-s)
-            const long long d = 2LL * g.adjwgt[e];
-            if (b.side[u] == s)
-                gain[u] += d;
-            else
-                gain[u] -= d;
-            key[u] = ((uint64_t)(uint32_t)rng.next() << 32) | (uint32_t)u;
-            if (pos[u] < 0)
-                pq[(int)b.side[u]].insert(u);
-            else
-                pq[(int)b.side[u]].update(u);
+            const long long d = 2LL * edges[e].w;
+            nu.gain += nu.side == s ? d : -d;
+            const FmEntry en{nu.gain, ((uint64_t)(uint32_t)rng.next() << 32) | (uint32_t)u};
+            FmHeap& q = pq[(int)nu.side];
+            if (nu.pos < 0) q.insert(en);
+            else q.update(nu.pos, en);
         }
         const long long ov = overload(w, maxw);
         if (ov < best_over || (ov == best_over && cut < best_cut)) {
             best_over = ov;
             best_cut = cut;
-            best_len = moved.size();
+            best_len = n_moved;
             since_best = 0;
         } else if (++since_best > stall_limit) {
             break;
         }
     }
-    // roll back to the best prefix
-    for (size_t i = moved.size(); i > best_len; --i) {
+    // keep the best prefix
+    for (int i = n_moved; i > best_len; --i) {
         const int v = moved[i - 1];
-        const int s = b.side[v];
-        b.side[v] = (char)(1 - s);
-        w[s] -= g.vwgt[v];
-        w[1 - s] += g.vwgt[v];
+        const int s = node[v].side;
+        w[s] -= vwgt[v];
+        w[1 - s] += vwgt[v];
     }
+    for (int i = 0; i < best_len; ++i) side[moved[i]] = node[moved[i]].side;
     const long long old_over = overload(b.w, maxw);
     const bool improved = best_over < old_over || (best_over == old_over && best_cut < b.cut);
     b.w[0] = w[0];
     b.w[1] = w[1];
     b.cut = best_cut;
-    sc.gain = std::move(gain);
-    sc.key = std::move(key);
-    sc.pos = std::move(pos);
-    sc.moved = std::move(moved);
-    sc.locked = std::move(locked);
-    sc.heap[0] = std::move(pq[0].h);
-    sc.heap[1] = std::move(pq[1].h);
     return improved;
 }
 
-void fm_refine(const HostGraph& g, Bisection& b, const long long maxw[2], int stall, int pct,
+void fm_refine(const Graph& g, Bisection& b, const long long maxw[2], int stall, int pct,
                Rng& rng) {
     for (int pass = 0; pass < 8; ++pass)
         if (!fm_pass(g, b, maxw, stall, pct, rng)) break;
 }
 
-// BFS growing of side 0 from random starts until it reaches target0.
-Bisection grow(const HostGraph& g, long long target0, Rng& rng) {
-    Bisection b;
+// BFS growing of side 0 from random starts until it reaches target0 (the cut is left to the
+// first FM pass).
+void grow(const Graph& g, long long total, long long target0, Rng& rng, Bisection& b,
+          std::vector<char>& seen_v, std::vector<int>& queue_v) {
     b.side.assign(g.n, 1);
+    seen_v.assign(g.n, 0);
+    queue_v.resize(g.n);
+    char* const seen = seen_v.data();
+    int* const queue = queue_v.data();
+    const int* const xadj = g.xadj.data();
+    const Edge* const edges = g.edges.data();
     long long w0 = 0;
-    std::vector<char> seen(g.n, 0);
-    std::vector<int> queue;
-    queue.reserve(g.n);
-    size_t head = 0;
+    int head = 0, tail = 0;
     int remaining = g.n;
     while (w0 < target0 && remaining > 0) {
-        if (head == queue.size()) {
+        if (head == tail) {
             int s = (int)rng.below((uint32_t)g.n);
             while (seen[s]) s = (s + 1) % g.n;
             seen[s] = 1;
-            queue.push_back(s);
+            queue[tail++] = s;
         }
         const int v = queue[head++];
         --remaining;
         b.side[v] = 0;
         w0 += g.vwgt[v];
-        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
-            const int u = g.adjncy[e];
+        for (int e = xadj[v], e1 = xadj[v + 1]; e < e1; ++e) {
+            const int u = edges[e].to;
             if (!seen[u]) {
                 seen[u] = 1;
-                queue.push_back(u);
+                queue[tail++] = u;
             }
         }
     }
-    long long total = 0;
-    for (int v = 0; v < g.n; ++v) total += g.vwgt[v];
     b.w[0] = w0;
     b.w[1] = total - w0;
-    b.cut = bis_cut(g, b.side);
-    return b;
+    b.counted = false;
 }
 
 bool better_bis(const Bisection& a, const Bisection& b, const long long maxw[2]) {
@@ -429,82 +478,93 @@ bool better_bis(const Bisection& a, const Bisection& b, const long long maxw[2])
 }
 
 // Multilevel bisection of g. side[v] = 0 for the first part.
-std::vector<char> ml_bisect(const HostGraph& g, long long target0, const long long maxw[2],
+std::vector<char> ml_bisect(const Graph& g, long long target0, const long long maxw[2],
                             const IpParams& p, Rng& rng) {
-    std::vector<HostGraph> levels;
+    std::vector<Graph> levels;
     std::vector<std::vector<int>> maps;
-    const HostGraph* cur = &g;
+    const Graph* cur = &g;
     const long long cbound = std::max(1LL, (std::min(maxw[0], maxw[1]) + p.coarsen_factor - 1) /
                                                p.coarsen_factor);
     while (cur->n > p.stop_nodes) {
         std::vector<int> label;
         const int nc = lp_cluster(*cur, cbound, 3, rng, label);
         if ((double)cur->n / (double)nc < 1.1) break;
-        HostGraph c = contract(*cur, label, nc);
+        Graph c = contract(*cur, label, nc);
         maps.push_back(std::move(label));
         levels.push_back(std::move(c));
         cur = &levels.back();
     }
-    Bisection best;
+    Bisection best, b;
     bool have = false;
+    std::vector<char> seen;
+    std::vector<int> queue;
+    const long long total = cur->total_weight();
     for (int t = 0; t < p.bisection_tries; ++t) {
-        Bisection b = grow(*cur, target0, rng);
+        grow(*cur, total, target0, rng, b, seen, queue);
         fm_refine(*cur, b, maxw, p.fm_stall, p.fm_pct_coarsest, rng);
         if (!have || better_bis(b, best, maxw)) {
-            best = std::move(b);
+            std::swap(best, b);
             have = true;
         }
     }
     for (int l = (int)levels.size() - 1; l >= 0; --l) {
-        const HostGraph& fine = l == 0 ? g : levels[l - 1];
+        const Graph& fine = l == 0 ? g : levels[l - 1];
         const std::vector<int>& map = maps[l];
-        Bisection b;
         b.side.resize(fine.n);
         for (int v = 0; v < fine.n; ++v) b.side[v] = best.side[map[v]];
         b.w[0] = best.w[0];
         b.w[1] = best.w[1];
         b.cut = best.cut;
         fm_refine(fine, b, maxw, p.fm_stall, p.fm_pct_levels, rng);
-        best = std::move(b);
+        std::swap(best, b);
     }
-    return best.side;
+    return std::move(best.side);
 }
 
-HostGraph extract(const HostGraph& g, const std::vector<char>& side, char which,
-                  std::vector<int>& ids) {
-    std::vector<int> local(g.n, -1);
-    ids.clear();
-    for (int v = 0; v < g.n; ++v)
-        if (side[v] == which) {
-            local[v] = (int)ids.size();
-            ids.push_back(v);
-        }
-    HostGraph s;
-    s.n = (int)ids.size();
-    s.xadj.assign(s.n + 1, 0);
-    s.vwgt.resize(s.n);
-    for (int i = 0; i < s.n; ++i) {
-        const int v = ids[i];
-        s.vwgt[i] = g.vwgt[v];
-        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
-            const int u = local[g.adjncy[e]];
-            if (u < 0) continue;
-            s.adjncy.push_back(u);
-            s.adjwgt.push_back(g.adjwgt[e]);
-        }
-        s.xadj[i + 1] = (int)s.adjncy.size();
+// Both sides of g as graphs of their own; ids[s][i] = node of g.
+void extract(const Graph& g, const std::vector<char>& side, Graph out[2], std::vector<int> ids[2]) {
+    std::vector<int> local(g.n);
+    int cnt[2] = {0, 0};
+    for (int v = 0; v < g.n; ++v) local[v] = cnt[(int)side[v]]++;
+    for (int s = 0; s < 2; ++s) {
+        out[s].n = cnt[s];
+        out[s].xadj.resize(cnt[s] + 1);
+        out[s].xadj[0] = 0;
+        out[s].vwgt.resize(cnt[s]);
+        out[s].edges.reserve(g.edges.size() / 2);
+        ids[s].resize(cnt[s]);
     }
-    return s;
+    for (int v = 0; v < g.n; ++v) {
+        const int s = side[v];
+        Graph& o = out[s];
+        const int i = local[v];
+        ids[s][i] = v;
+        o.vwgt[i] = g.vwgt[v];
+        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e) {
+            const int u = g.edges[e].to;
+            if (side[u] == s) o.edges.push_back({local[u], g.edges[e].w});
+        }
+        o.xadj[i + 1] = (int)o.edges.size();
+    }
 }
 
 struct RecCtx {
     const IpParams* p;
     uint64_t rep_seed;
-    std::atomic<int> spawn_budget{0};
+    std::atomic<int>* idle;  // threads not in use, shared by the repetitions
 };
+constexpr int kSpawnNodes = 1000;  // halves of fewer nodes are not worth a thread
+
+// Takes a thread if one is idle.
+bool take_thread(std::atomic<int>& idle) {
+    int have = idle.load();
+    while (have > 0)
+        if (idle.compare_exchange_weak(have, have - 1)) return true;
+    return false;
+}
 
 // Partitions g into blocks lb..ub; part receives block ids for g's nodes.
-void recurse(const HostGraph& g, int lb, int ub, RecCtx& ctx, std::vector<int>& part) {
+void recurse(const Graph& g, int lb, int ub, RecCtx& ctx, std::vector<int>& part) {
     part.assign(g.n, lb);
     const int kk = ub - lb + 1;
     if (kk <= 1 || g.n == 0) return;
@@ -525,22 +585,28 @@ void recurse(const HostGraph& g, int lb, int ub, RecCtx& ctx, std::vector<int>& 
     } else {
         side = ml_bisect(g, target0, maxw, *ctx.p, rng);
     }
-    std::vector<int> ids0, ids1;
-    HostGraph g0 = extract(g, side, 0, ids0);
-    HostGraph g1 = extract(g, side, 1, ids1);
+    std::vector<int> ids[2];
+    Graph half[2];
+    extract(g, side, half, ids);
     std::vector<int> p0, p1;
     bool spawned = false;
     std::future<void> fut;
-    if (k1 > 1 && k2 > 1 && g.n > 20000 && ctx.spawn_budget.fetch_sub(1) > 0) {
-        fut = std::async(std::launch::async, [&] { recurse(g0, lb, mid, ctx, p0); });
+    if (k1 > 1 && k2 > 1 && g.n > kSpawnNodes && take_thread(*ctx.idle)) {
+        fut = std::async(std::launch::async, [&] {
+            struct Back {  // the thread is idle again, also after an exception
+                std::atomic<int>* idle;
+                ~Back() { ++*idle; }
+            } back{ctx.idle};
+            recurse(half[0], lb, mid, ctx, p0);
+        });
         spawned = true;
     } else {
-        recurse(g0, lb, mid, ctx, p0);
+        recurse(half[0], lb, mid, ctx, p0);
     }
-    recurse(g1, mid + 1, ub, ctx, p1);
+    recurse(half[1], mid + 1, ub, ctx, p1);
     if (spawned) fut.get();
-    for (size_t i = 0; i < ids0.size(); ++i) part[ids0[i]] = p0[i];
-    for (size_t i = 0; i < ids1.size(); ++i) part[ids1[i]] = p1[i];
+    for (size_t i = 0; i < ids[0].size(); ++i) part[ids[0][i]] = p0[i];
+    for (size_t i = 0; i < ids[1].size(); ++i) part[ids[1][i]] = p1[i];
 }
 
 // Moves nodes out of blocks heavier than `bound` until none is (or no move is possible): nodes
@@ -611,32 +677,48 @@ void initial_partition(const HostGraph& g, const IpParams& p, std::vector<int>& 
     part.assign(g.n, 0);
     if (k == 1 || g.n == 0) return;
     // split off isolated nodes
-    std::vector<int> core_ids, iso_ids;
-    for (int v = 0; v < g.n; ++v)
-        (g.xadj[v + 1] > g.xadj[v] ? core_ids : iso_ids).push_back(v);
-    std::vector<char> all_core(g.n, 0);
-    for (int v : core_ids) all_core[v] = 1;
-    std::vector<int> ids;
-    HostGraph core = extract(g, all_core, 1, ids);
+    std::vector<int> ids, iso_ids, local(g.n, -1);
+    for (int v = 0; v < g.n; ++v) {
+        if (g.xadj[v + 1] > g.xadj[v]) {
+            local[v] = (int)ids.size();
+            ids.push_back(v);
+        } else {
+            iso_ids.push_back(v);
+        }
+    }
+    Graph core;
+    core.n = (int)ids.size();
+    core.xadj.assign(core.n + 1, 0);
+    core.vwgt.resize(core.n);
+    core.edges.reserve(g.adjncy.size());
+    for (int i = 0; i < core.n; ++i) {
+        const int v = ids[i];
+        core.vwgt[i] = g.vwgt[v];
+        for (int e = g.xadj[v]; e < g.xadj[v + 1]; ++e)
+            if (local[g.adjncy[e]] >= 0) core.edges.push_back({local[g.adjncy[e]], g.adjwgt[e]});
+        core.xadj[i + 1] = (int)core.edges.size();
+    }
     unsigned hw = std::thread::hardware_concurrency();
     int threads = p.threads > 0 ? p.threads : (int)std::min(16u, hw ? hw : 1u);
     const int reps = std::max(1, p.repetitions);
 
     std::vector<std::vector<int>> results(reps);
     std::vector<long long> cuts(reps, 0);
+    std::atomic<int> idle{std::max(0, threads - reps)};
     auto run_rep = [&](int r) {
         RecCtx ctx;
         ctx.p = &p;
         ctx.rep_seed = stream_seed(p.seed, 0x1e5u, (uint64_t)r);
-        ctx.spawn_budget = std::max(0, threads / reps - 1);
+        ctx.idle = &idle;
         std::vector<int> cp;
         recurse(core, 0, k - 1, ctx, cp);
         results[r] = std::move(cp);
-        std::vector<int> full(core.n);
-        cuts[r] = 0;
+        const std::vector<int>& part_r = results[r];
+        long long cut = 0;
         for (int v = 0; v < core.n; ++v)
             for (int e = core.xadj[v]; e < core.xadj[v + 1]; ++e)
-                if (results[r][v] != results[r][core.adjncy[e]]) cuts[r] += core.adjwgt[e];
+                if (part_r[v] != part_r[core.edges[e].to]) cut += core.edges[e].w;
+        cuts[r] = cut;
     };
     if (threads <= 1) {  // the caller parallelises (e.g. over the graphs of a batch)
         for (int r = 0; r < reps; ++r) run_rep(r);
@@ -651,6 +733,7 @@ void initial_partition(const HostGraph& g, const IpParams& p, std::vector<int>& 
                 } catch (...) {
                     err[r] = std::current_exception();
                 }
+                ++idle;
             });
         for (auto& t : pool) t.join();
         for (auto& e : err)
