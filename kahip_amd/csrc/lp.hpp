@@ -28,7 +28,8 @@ struct LpArgs {
     unsigned long long* top;   // per label: top proposal priority into it
     int* out;                  // per label: summed weight of departures (refinement)
     unsigned long long* dtop;  // per label: top departure priority (refinement)
-    int* prop_t;               // per node: proposed label, -1 outside propose..apply
+    int base;                  // list position of the launch's first list entry
+    int* prop_t;               // per list position: proposed label, -1 outside propose..apply
     int* prop_gain;
     uint8_t* prop_ok;
     int* moves;
@@ -100,7 +101,7 @@ public:
 private:
     void build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
                      const uint8_t* include, int copies);
-    void launch_proposals(int b, int sr, const LpArgs& a, int cnt, int copies, hipStream_t s);
+    void launch_proposals(int b, int sr, LpArgs a, int cnt, int copies, hipStream_t s);
     int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
     void fetch(hipStream_t s);  // host_ctl_ of the last run
     Mail mail_;
