@@ -148,7 +148,7 @@ private:
     DevBuf<int> midpos_;
     DevBuf<int2> tsub_;  // (hub, bucket) task: {multi-chunk hub index, bucket | buckets << 16}
     DevBuf<uint8_t> fb_;
-    DevBuf<int> lists_, bin_, offsets_;
+    DevBuf<int> lists_, bin_, bin_blocks_, offsets_;
     int* counts_ = nullptr;  // in bin_: list lengths
     DevBuf<int> clists_, ccount_;  // refinement frontier per list (compacted each round)
     DevBuf<int> prop_t_, prop_gain_;
