@@ -783,6 +783,7 @@ int kahip_edge_scores(int n, const int* xadj, const int* adjncy, const int* vwgt
             if (rating == 2)
                 eng.rw.upload_weights(*reinterpret_cast<const MlpWeights*>(params), s);
             eng.rw.scores((RatingMode)rating, g, bound, seed, o, s, eng.lp, nullptr);
+            if (rating == (int)RatingMode::Learned && g.m2 > 0) eng.lp.check(s);
             if (g.m2)
                 KH_CHECK(hipMemcpyAsync(scores, o, sizeof(int) * g.m2, hipMemcpyDeviceToHost, s));
             KH_CHECK(hipStreamSynchronize(s));

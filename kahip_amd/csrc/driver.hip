@@ -220,6 +220,8 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
     S.upper_bound = U;
     S.cluster_bound = B;
 
+    if (p.rating == RatingMode::Learned) rw.upload_weights(*p.mlp, s);
+
     // ------------------------------------------------------------------ coarsening
     // Skewed graphs are renumbered by degree first (part of the coarsening time); the pipeline
     // runs on the renumbered graph and the partition is mapped back at the end.
@@ -280,7 +282,6 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
             ev_rating.emplace_back();
             KH_CHECK(hipEventRecord(ev_rating.back().a, s));
             score.reserve(fine.m2);
-            if (p.rating == RatingMode::Learned && level == 0) rw.upload_weights(*p.mlp, s);
             rw.scores(p.rating, fine, (int)B, rating_seed(p.seed, level), score.p, s, lp, prof);
             KH_CHECK(hipEventRecord(ev_rating.back().b, s));
             rated.adjwgt = score.p;

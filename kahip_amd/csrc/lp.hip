@@ -1958,11 +1958,15 @@ __global__ void fill_u8(uint8_t* p, long long n, uint8_t value) {
     if (i < n) p[i] = value;
 }
 
-// Admission scratch of a clustering (labels = nodes) or refinement.
+// Admission scratch of a clustering (labels = nodes) or refinement, the binning's counters and the
+// error flag (if err).
 __global__ void init_scratch(long long n, int* __restrict__ prop_t, long long nl,
                              int* __restrict__ inc, unsigned long long* __restrict__ top,
-                             int* __restrict__ out, unsigned long long* __restrict__ dtop) {
+                             int* __restrict__ out, unsigned long long* __restrict__ dtop, int nbin,
+                             int* __restrict__ bin, int* __restrict__ err) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nbin) bin[i] = 0;
+    if (i == 0 && err) *err = 0;
     if (i < n) prop_t[i] = -1;
     if (i < nl) {
         inc[i] = 0;
@@ -2080,7 +2084,8 @@ void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, u
     subrounds_ = S;
     num_labels_ = num_labels;
     ctl_.reserve(kCtlInts);
-    fill_async(ctl_.p, kCtlInts, 0, s);
+    clear_err_ = !keep_err_;  // (run() clears the other counters)
+    keep_err_ = false;
     if (mode == LpMode::Refine) {
         active_.reserve(g.n);
         next_active_.reserve(g.n);
@@ -2089,6 +2094,8 @@ void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, u
     small_ = mode == LpMode::Refine && !include && g.n <= kTailNodes && g.m2 <= kTailEdges &&
              num_labels <= kTailLabels;
     if (!small_) build_lists(mode, g, seed, s, include, copies);
+    else if (clear_err_) fill_async(ctl_.p + kCtlErr, 1, 0, s);
+    clear_err_ = false;  // (run() may build the lists later on)
 }
 
 void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
@@ -2122,16 +2129,17 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
         dtop_.reserve(num_labels);
     }
 
-    fill_async(bin_.p, kBinInts, 0, s);
     // a span of nodes per binning workgroup: one pass of its threads up to kBinGrid workgroups
     const int span = std::max(grid_for(grid_for(g.n, kBinGrid), kBinThreads), 1) * kBinThreads;
     const int bin_grid = grid_for(g.n, span);
     bin_blocks_.reserve((long long)bin_grid * kBinSlots);
     const int split = mode == LpMode::Cluster ? 1 : 0;  // small-degree wave kernel (clustering)
     const bool refine = mode == LpMode::Refine;
-    hipLaunchKernelGGL(init_scratch, dim3(std::max(grid_for(std::max(scratch_n, scratch_l), 256), 1)),
-                       dim3(256), 0, s, scratch_n, prop_t_.p, scratch_l, inc_.p, top_.p,
-                       refine ? out_.p : nullptr, refine ? dtop_.p : nullptr);
+    const long long init_n = std::max<long long>({scratch_n, scratch_l, kBinInts});
+    hipLaunchKernelGGL(init_scratch, dim3(grid_for(init_n, 256)), dim3(256), 0, s, scratch_n,
+                       prop_t_.p, scratch_l, inc_.p, top_.p, refine ? out_.p : nullptr,
+                       refine ? dtop_.p : nullptr, kBinInts, bin_.p,
+                       clear_err_ ? ctl_.p + kCtlErr : nullptr);
     if (g.n > 0)
         hipLaunchKernelGGL(bin_count, dim3(bin_grid), dim3(kBinThreads), 0, s, g.n, span, g.xadj,
                            seed, S, bins, include, split, counts_, edges, bin_blocks_.p);
@@ -2741,6 +2749,7 @@ void LpWorkspace::read_moves(int rounds, int* out, hipStream_t s) {
 }
 
 void LpWorkspace::check(hipStream_t s) {
+    keep_err_ = false;
     fetch(s);
     KH_REQUIRE(host_ctl_[kCtlBig] == 0,
                "label propagation: a hash table probe found no free slot (kernel table "

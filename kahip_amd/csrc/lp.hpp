@@ -92,6 +92,8 @@ public:
     // Throws if a kernel of a run() since the last prepare() set the device error flag (waits for
     // the last run).
     void check(hipStream_t s);
+    // Leaves that to the next check(): the next prepare() keeps the flag.
+    void check_later() { keep_err_ = true; }
 
     int host_counts[kMaxSub * kNumBins] = {};
     int host_wave_small_[kMaxSub] = {};  // clustering: wave-list nodes of the small-LDS kernel
@@ -113,6 +115,7 @@ private:
     DevBuf<int> ctl_;
     int host_ctl_[kCtlBig + 1] = {};  // the traversed edges, the moves, the error flag
     bool fetched_ = false;
+    bool keep_err_ = false, clear_err_ = false;
     bool small_ = false;  // refinement that starts in refine_tail, without lists
     void build_chunk_maps(hipStream_t s);  // cmap_ of every sub-round (after chunk_prefix_)
     int subrounds_ = 1;

@@ -28,19 +28,21 @@ __global__ __launch_bounds__(kMailThreads) void send_mail(Pieces m, int* box, in
 
 }  // namespace
 
-void Mail::init() {
-    if (host_) return;
-    void* h = nullptr;
-    KH_CHECK(hipHostMalloc(&h, sizeof(int) * (kInts + 1), hipHostMallocMapped | hipHostMallocCoherent));
-    host_ = static_cast<volatile int*>(h);
-    host_[0] = 0;
-    void* d = nullptr;
-    KH_CHECK(hipHostGetDevicePointer(&d, h, 0));
-    dev_ = static_cast<int*>(d);
+void MappedBuf::alloc(size_t bytes) {
+    KH_CHECK(hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    KH_CHECK(hipHostGetDevicePointer(&dev, p, 0));
 }
 
-Mail::~Mail() {
-    if (host_) (void)hipHostFree(const_cast<int*>(host_));
+MappedBuf::~MappedBuf() {
+    if (p) (void)hipHostFree(p);
+}
+
+void Mail::init() {
+    if (host_) return;
+    buf_.alloc(sizeof(int) * (kInts + 1));
+    dev_ = static_cast<int*>(buf_.dev);
+    host_ = static_cast<volatile int*>(buf_.p);
+    host_[0] = 0;
 }
 
 int* Mail::box() {

@@ -6,6 +6,17 @@
 
 namespace kahip {
 
+// Host memory that kernels read and write in place.
+struct MappedBuf {
+    void* p = nullptr;    // for the host
+    void* dev = nullptr;  // for kernels
+    MappedBuf() = default;
+    MappedBuf(const MappedBuf&) = delete;
+    MappedBuf& operator=(const MappedBuf&) = delete;
+    ~MappedBuf();
+    void alloc(size_t bytes);
+};
+
 // A kernel writes a few words into mapped host memory, then their sequence number; the host polls
 // for it. The answer is there about 6 us after the kernels before it; a pageable
 // device-to-host copy and its synchronisation take 20 to 40 us (blit kernel, signal, wake-up), and
@@ -20,9 +31,6 @@ public:
     static constexpr int kMaxPieces = 4;
 
     Mail() = default;
-    Mail(const Mail&) = delete;
-    Mail& operator=(const Mail&) = delete;
-    ~Mail();
     // Enqueues the sending of the pieces, one after the other, on s.
     void post(hipStream_t s, Piece a, Piece b = {nullptr, 0}, Piece c = {nullptr, 0},
               Piece d = {nullptr, 0});
@@ -35,6 +43,7 @@ public:
 
 private:
     void init();
+    MappedBuf buf_;
     volatile int* host_ = nullptr;
     int* dev_ = nullptr;
     int seq_ = 0;

@@ -620,34 +620,24 @@ __global__ __launch_bounds__(64) void update_kernel(int blocks, int batch,
     pack_param(p, x, pack);
 }
 
-void pack_weights(const MlpWeights& w, std::vector<uint8_t>& out) {
-    out.assign(kPackBytes, 0);
-    uint16_t* bf = reinterpret_cast<uint16_t*>(out.data());
-    for (int t = 0; t < 4; ++t)
-        for (int lane = 0; lane < 64; ++lane) {
-            const int g = lane >> 4, row = lane & 15;
-            for (int j = 0; j < 8; ++j) {
-                const int k = 8 * g + j;
-                const float x = k < kFeatures ? w.p[kOffW1 + (16 * t + row) * kFeatures + k] : 0.f;
-                bf[(t * 64 + lane) * 8 + j] = f2bf(x);
-            }
-        }
-    for (int t = 0; t < 4; ++t)
-        for (int kb = 0; kb < 2; ++kb)
-            for (int lane = 0; lane < 64; ++lane) {
-                const int g = lane >> 4, row = lane & 15;
-                for (int j = 0; j < 8; ++j) {
-                    const float x = w.p[kOffW2 + (16 * t + row) * kHidden + hid_of(kb, g, j)];
-                    bf[kPackA1 + ((t * 2 + kb) * 64 + lane) * 8 + j] = f2bf(x);
-                }
-            }
-    float* tail = reinterpret_cast<float*>(bf + kPackBf16);
-    for (int h = 0; h < kHidden; ++h) {
-        tail[h] = w.p[kOffB1 + h];
-        tail[64 + h] = w.p[kOffB2 + h];
-        tail[128 + h] = w.p[kOffW3 + h];
+// Weights p in the layout of mlp_forward_kernel, a thread per packed value. p is mapped host
+// memory (19 KB), read once.
+__global__ __launch_bounds__(256) void pack_weights(const float* __restrict__ p,
+                                                    uint16_t* __restrict__ pack) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= kPackBf16 + kPackFloats) return;
+    const int j = i & 7, lane = (i >> 3) & 63, g = lane >> 4, row = lane & 15;
+    if (i < kPackA1) {
+        const int t = i >> 9, k = 8 * g + j;
+        pack[i] = f2bf(k < kFeatures ? p[kOffW1 + (16 * t + row) * kFeatures + k] : 0.f);
+    } else if (i < kPackBf16) {
+        const int tk = (i - kPackA1) >> 9;  // 2 t + kb
+        pack[i] = f2bf(p[kOffW2 + (16 * (tk >> 1) + row) * kHidden + hid_of(tk & 1, g, j)]);
+    } else {
+        const int f = i - kPackBf16, h = f & 63;
+        const int from = f < 64 ? kOffB1 : f < 128 ? kOffB2 : f < 192 ? kOffW3 : kOffB3;
+        reinterpret_cast<float*>(pack + kPackBf16)[f] = p[from + h];
     }
-    tail[192] = w.p[kOffB3];
 }
 
 }  // namespace
@@ -680,7 +670,7 @@ void RatingWorkspace::sweeps_and_sketch(const DGraph& g, int bound, uint32_t see
         uint32_t seeds[3];
         for (int i = 0; i < 3; ++i) seeds[i] = hash3(seed, 0xA6u, (uint32_t)i);
         lp.run_copies(g, lab_.p, size_.p, bound, seeds, 3, s);
-        lp.check(s);
+        lp.check_later();
     }
     hipLaunchKernelGGL(node_rec_kernel, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n, g.xadj,
                        g.vwgt, sig_.p, lab_.p, lab_.p + g.n, lab_.p + 2LL * g.n,
@@ -691,6 +681,7 @@ void RatingWorkspace::sweeps_and_sketch(const DGraph& g, int bound, uint32_t see
 void RatingWorkspace::features(const DGraph& g, int bound, uint32_t seed, float* out,
                                hipStream_t s, LpWorkspace& lp, Profiler* prof) {
     sweeps_and_sketch(g, bound, seed, s, lp, prof);
+    if (g.n > 0) lp.check(s);
     ProfScope ps(prof, "rating_features", 0.0, g.m2, s);
     if (g.m2 > 0)
         hipLaunchKernelGGL(features_kernel<float>, dim3(grid_for((g.m2 + 7) / 8, 256)), dim3(256),
@@ -700,11 +691,15 @@ void RatingWorkspace::features(const DGraph& g, int bound, uint32_t seed, float*
 }
 
 void RatingWorkspace::upload_weights(const MlpWeights& w, hipStream_t s) {
-    std::vector<uint8_t> host;
-    pack_weights(w, host);
+    // Through mapped host memory and packed by a kernel: packing on the host, a pageable copy and
+    // its synchronisation were 0.05 ms of every call with the learned rating.
     wpack_.reserve(kPackBytes / 2);
-    KH_CHECK(hipMemcpyAsync(wpack_.p, host.data(), kPackBytes, hipMemcpyHostToDevice, s));
-    KH_CHECK(hipStreamSynchronize(s));  // `host` must outlive the copy
+    if (!wmap_.p) wmap_.alloc(sizeof(w.p));
+    KH_CHECK(hipStreamSynchronize(s));  // an earlier pack has been read (idle between calls)
+    std::memcpy(wmap_.p, w.p, sizeof(w.p));
+    hipLaunchKernelGGL(pack_weights, dim3(grid_for(kPackBf16 + kPackFloats, 256)), dim3(256), 0, s,
+                       static_cast<const float*>(wmap_.dev), wpack_.p);
+    KH_CHECK(hipGetLastError());
 }
 
 void RatingWorkspace::mlp_forward(const float* feat, long long m, const MlpWeights& w,

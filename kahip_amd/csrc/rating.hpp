@@ -39,7 +39,8 @@ public:
                      hipStream_t s, Profiler* prof);
     // Integer scores of the chosen rating for every directed edge of g, shifted right by
     // score_shift(g) (at least 1) so that a node's score sum stays below 2^31.
-    // Learned: with the weights of the last upload_weights().
+    // Learned: with the weights of the last upload_weights(); a failed sweep shows at lp's next
+    // check().
     void scores(RatingMode mode, const DGraph& g, int bound, uint32_t seed, int* score,
                 hipStream_t s, LpWorkspace& lp, Profiler* prof);
     void upload_weights(const MlpWeights& w, hipStream_t s);
@@ -63,6 +64,7 @@ private:
     DevBuf<int> lab_, size_, map_, heavy_, rec_;
     DevBuf<float> feat_, logit_, partial_, loss_;
     DevBuf<uint16_t> wpack_, featb_, tpack_;
+    MappedBuf wmap_;  // weights on their way to wpack_
     Mail mail_;
 };
 
