@@ -46,8 +46,8 @@ typedef struct {
                             profiler; non-zero is rejected with an error */
     int group_items;     /* tile shape: nodes per lane group in flight in the 8..64-lane LP
                             kernels, 1, 2 (default) or 4 */
-    int wave_small;      /* tile shape: clustering wave-bin nodes up to this degree use the
-                            small-table wave kernel, 64, 128 (default) or 256 */
+    int wave_small;      /* tile shape: wave-bin nodes up to this degree use the wave variant of
+                            half the edges per lane, 64, 128 (default) or 256 */
 } kahip_params;
 
 /* Edge ratings of the clustering. NONE uses the edge weights (the FASTSOCIAL preset);

@@ -225,7 +225,7 @@ BinConfig autotune_bins(const DGraph& g, const PartitionParams& p, bool shapes, 
         return t;
     };
     // coordinate descent: the wave bin's upper degree, then (with shapes) the group kernels'
-    // items per lane group, then the small wave kernel's degree limit
+    // items per lane group, then the small wave variant's degree limit
     BinConfig best = p.bins;
     float best_ms = 1e30f;
     for (int c = 0; c < kAutotuneCandidates; ++c) {

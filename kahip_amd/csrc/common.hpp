@@ -116,8 +116,8 @@ struct BinConfig {
     // Launch (tile) shapes of the LP kernels; the synchronous schedule makes the result
     // independent of them.
     int group_items = 2;   // nodes per lane group in flight in the 8..64-lane kernels: 1, 2 or 4
-    int wave_small = 128;  // clustering: wave-bin nodes up to this degree use the small-table wave
-                           // kernel (2 x wave_small LDS slots per wave): 64, 128 or 256
+    int wave_small = 128;  // wave-bin nodes up to this degree use the variant of four edges per
+                           // lane instead of eight: 64, 128 or 256
 };
 
 inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }

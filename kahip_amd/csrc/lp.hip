@@ -19,6 +19,7 @@
 // Nodes are binned by degree (per sub-round lists built once per call):
 //   deg <= 8/16/32/64   8 or 16 lanes per node, 1 to 4 edges per lane, summed by DPP moves;
 //   deg <= 512          one wave per node, LDS hash table (open addressing, LDS atomics);
+//                       one launch of a sub-round serves all of these lists;
 //   larger              one workgroup per node, hash table in a pre-cleared global region.
 
 #include <cstring>
@@ -33,15 +34,12 @@ namespace kahip {
 namespace {
 
 constexpr int kWaveCap = 1024;    // LDS hash slots per wave (degree <= 512 => load <= 1/2)
-static_assert(kWaveCap == 1024, "propose_wave loads up to kWaveCap / 2 edges per wave");
+static_assert(kWaveCap == 1024, "wave_vb loads up to kWaveCap / 2 edges per wave");
 constexpr int kWaveDense = 2048;  // dense LDS counters per wave (refinement, k <= 2048)
 constexpr int kWaveDenseSmall = 512;  // the frontier kernel's counters for k <= 512 (less LDS)
-// Clustering splits the wave list: nodes of degree <= BinConfig::wave_small (64, 128 or 256)
-// come first and use a kernel of 2 x wave_small slots per wave (8 KB of LDS per workgroup at 128
-// instead of 32 KB, so more waves per CU).
 constexpr int kBlock = 256;
 constexpr int kFrontierGrid = 2048;  // workgroups of a refinement list kernel (grid-stride)
-// nodes per lane group in flight in propose_group: BinConfig::group_items (1, 2 or 4)
+// nodes per lane group in flight in group_vb: BinConfig::group_items (1, 2 or 4)
 constexpr int kHubChunk = 4096;   // hub edges per workgroup
 constexpr int kHubCap = 8192;     // LDS hash slots per hub chunk (load <= 1/2)
 constexpr int kHubThreads = 1024;      // clustering hub chunks (4 edges per thread)
@@ -505,62 +503,45 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
     __syncthreads();  // the LDS of this virtual block is read before the next one writes it
 }
 
-template <int W, int E, int IT>
-__global__ __launch_bounds__(kBlock) void propose_group(LpArgs a, const int* __restrict__ list,
-                                                        int count) {
-    select_copy(a);
-    unsigned long long edges = 0;
-    group_vb<LpMode::Cluster, W, E, IT>(a, list, a.base, count, blockIdx.x, edges);
-}
-
 // ---------------------------------------------------------------- one wave per node
 // Labels are aggregated in LDS: a hash table (open addressing, LDS atomics) in general, or a
 // dense counter per label when the labels are the k blocks of the refinement and k is small.
-// One virtual block (kBlock / 64 nodes of the list, a wave each) of the wave kernel; every thread
-// of the workgroup calls it.
-template <LpMode M, bool DENSE, int WCAP, int DCAP = kWaveDense>
-__device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
-                                                              const int* __restrict__ list,
-                                                              int base, int count, int num_labels,
-                                                              int vb, unsigned long long& edges) {
-    static_assert(!DENSE || WCAP == kWaveCap, "the dense variant serves every wave degree");
-    __shared__ int skey[kBlock / 64][DENSE ? 1 : WCAP];
-    __shared__ int sval[kBlock / 64][DENSE ? DCAP : WCAP];  // dense: num_labels <= DCAP
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int gi = vb * (kBlock / 64) + wave;
-    const bool valid = gi < count;
-    const int v = valid ? list[gi] : 0;
-    const int own = valid ? a.label[v] : -1;
-    const int beg = valid ? a.xadj[v] : 0;
-    const int deg = valid ? a.xadj[v + 1] - beg : 0;
+// The node's table belongs to its wave, whose LDS operations are in order: no barriers.
+constexpr int kWaveEdges = kWaveCap / 2 / 64;  // edges per lane at the largest degree
+__device__ __attribute__((always_inline)) inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// EPL: edges per lane, 64 x EPL >= degree.
+template <LpMode M, bool DENSE, int EPL>
+__device__ __attribute__((always_inline)) inline void wave_node(const LpArgs& a, int pos, int v,
+                                                                int beg, int deg, int num_labels,
+                                                                int lane, int* K, int* V) {
+    const int own = a.label[v];
     int cap = 64;
     if (DENSE) {
         cap = num_labels;
     } else {
-        while (cap < 2 * deg) cap <<= 1;  // deg <= WCAP / 2 => cap <= WCAP
+        while (cap < 2 * deg) cap <<= 1;  // deg <= kWaveCap / 2 => cap <= kWaveCap
     }
-    int* K = skey[wave];
-    int* V = sval[wave];
-    for (int i = lane; i < cap; i += 64) {
-        if (!DENSE) K[i] = -1;
-        V[i] = 0;
-    }
-    __syncthreads();
-    // All of a lane's (<= 8) edges are loaded first so that their label gathers are in flight
-    // together; the LDS insertions follow.
-    constexpr int EPL = WCAP / 2 / 64;  // edges per lane at the maximum degree (WCAP / 2)
+    // All of a lane's edges are loaded first so that their label gathers are in flight together;
+    // the LDS insertions follow.
     int labs[EPL], ws[EPL];
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
         const int e = beg + lane + 64 * j;
-        // a row of up to WCAP / 2 edges, read once per sub-round: streamed (non-temporal)
+        // a row read once per sub-round: streamed (non-temporal)
         labs[j] = e < beg + deg ? __builtin_nontemporal_load(a.adjncy + e) : -1;
         ws[j] = e < beg + deg ? __builtin_nontemporal_load(a.adjwgt + e) : 0;
+    }
+    for (int i = lane; i < cap; i += 64) {
+        if (!DENSE) K[i] = -1;
+        V[i] = 0;
     }
 #pragma unroll
     for (int j = 0; j < EPL; ++j)
         if (labs[j] >= 0) labs[j] = a.label[labs[j]];
+    wave_lds_order();
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
         const int lab = labs[j];
@@ -577,14 +558,13 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
         }
         atomicAdd(&V[h], w);
     }
-    __syncthreads();
-    const int nw = valid ? a.vwgt[v] : 0;
+    wave_lds_order();
+    const int nw = a.vwgt[v];
     int conn_own = 0;
     Cand c{-1, 0u, 0x7fffffff, 0};
-    if (valid && !DENSE) {
-        constexpr int SL = WCAP / 64 < 8 ? WCAP / 64 : 8;
-        scan_wave_table<SL>(a, K, V, cap, lane, v, own, nw, conn_own, c);
-    } else if (valid) {
+    if (!DENSE) {
+        scan_wave_table<EPL < 8 ? 2 * EPL : 8>(a, K, V, cap, lane, v, own, nw, conn_own, c);
+    } else {
         for (int i = lane; i < cap; i += 64) {
             const int lab = V[i] ? i : -1;
             if (lab < 0) continue;
@@ -601,19 +581,73 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
     }
     conn_own = reduce_max<64>(conn_own);
     reduce_cand<64>(c);
-    if (valid && lane == 0) {
-        decide<M>(a, base + gi, v, own, nw, conn_own, c);
-        if (M == LpMode::Refine) edges += (unsigned long long)deg;
-    }
-    __syncthreads();  // the LDS of this virtual block is read before the next one clears it
+    if (lane == 0) decide<M>(a, pos, v, own, nw, conn_own, c);
+    wave_lds_order();  // the table is read before the wave's next node clears it
 }
 
-template <int WCAP = kWaveCap>
-__global__ __launch_bounds__(kBlock) void propose_wave(LpArgs a, const int* __restrict__ list,
-                                                       int count) {
+// One virtual block: kBlock / 64 nodes of the list, a wave each. DCAP: dense counters per wave
+// (num_labels <= DCAP). Rows of up to LpArgs::wave_small edges take the variant with half the
+// registers and predicated loads.
+template <LpMode M, bool DENSE, int DCAP = kWaveDense>
+__device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
+                                                              const int* __restrict__ list,
+                                                              int base, int count, int num_labels,
+                                                              int vb, unsigned long long& edges) {
+    __shared__ int skey[kBlock / 64][DENSE ? 1 : kWaveCap];
+    __shared__ int sval[kBlock / 64][DENSE ? DCAP : kWaveCap];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int gi = vb * (kBlock / 64) + wave;
+    if (gi >= count) return;
+    const int v = list[gi];
+    const int beg = a.xadj[v], deg = a.xadj[v + 1] - beg;
+    if (deg <= a.wave_small)
+        wave_node<M, DENSE, kWaveEdges / 2>(a, base + gi, v, beg, deg, num_labels, lane,
+                                            skey[wave], sval[wave]);
+    else
+        wave_node<M, DENSE, kWaveEdges>(a, base + gi, v, beg, deg, num_labels, lane, skey[wave],
+                                        sval[wave]);
+    if (M == LpMode::Refine && lane == 0) edges += (unsigned long long)deg;
+}
+
+// Clustering: the proposals of a sub-round's lists in one launch, the longest rows first, one
+// workgroup per virtual block. A launch per list left the chip idle at the end of each, six times
+// a sub-round. WAVES = false, for sub-rounds of lane groups only, needs no table (6 KB of LDS
+// instead of 38).
+// Measured, kahip_partition: R-MAT 2^17 k = 8 23.9 -> 20.8 ms, 2^13 k = 6 10.2 -> 9.0 ms,
+// kahip_lp_cluster of R-MAT 2^20 18.5 -> 17.2 ms, of 2^15 3.3 -> 2.0 ms; meshes of 2^22 nodes,
+// whose lists fill the chip, the same.
+struct ClusterLists {
+    const int* list[kNumBins - 1];
+    int base[kNumBins - 1];  // list positions of their first entries
+    int count[kNumBins - 1];
+};
+template <int IT, bool WAVES>
+__global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F) {
     select_copy(a);
+    constexpr LpMode C = LpMode::Cluster;
+    constexpr int N = kNumBins - 1;
+    constexpr int NPB[N] = {IT * (kBlock / 8), IT * (kBlock / 8), IT * (kBlock / 16),
+                            IT * (kBlock / 16), kBlock / 64};
+    int vb = blockIdx.x, b = N - 1;  // uniform per workgroup
+#pragma unroll
+    for (int k = N - 1; k > 0; --k) {
+        const int nvb = (F.count[k] + NPB[k] - 1) / NPB[k];
+        if (b == k && vb >= nvb) {
+            vb -= nvb;
+            b = k - 1;
+        }
+    }
     unsigned long long edges = 0;
-    wave_vb<LpMode::Cluster, false, WCAP>(a, list, a.base, count, 0, blockIdx.x, edges);
+    switch (b) {
+        case 0: group_vb<C, 8, 1, IT>(a, F.list[0], F.base[0], F.count[0], vb, edges); break;
+        case 1: group_vb<C, 8, 2, IT>(a, F.list[1], F.base[1], F.count[1], vb, edges); break;
+        case 2: group_vb<C, 16, 2, IT>(a, F.list[2], F.base[2], F.count[2], vb, edges); break;
+        case 3: group_vb<C, 16, 4, IT>(a, F.list[3], F.base[3], F.count[3], vb, edges); break;
+        default:
+            if constexpr (WAVES)
+                wave_vb<C, false>(a, F.list[4], F.base[4], F.count[4], 0, vb, edges);
+    }
 }
 
 // Refinement: the proposals of all degree lists of a sub-round in one launch. The lists are the
@@ -685,8 +719,8 @@ __global__ __launch_bounds__(kBlock) void propose_frontier(LpArgs a, FrontierLis
             case 2: group_vb<LpMode::Refine, 16, 2, IT>(a, F.list[2], F.base[2], cnt[2], vb, edges); break;
             case 3: group_vb<LpMode::Refine, 16, 4, IT>(a, F.list[3], F.base[3], cnt[3], vb, edges); break;
             case 4:
-                wave_vb<LpMode::Refine, DENSE, kWaveCap, DCAP>(a, F.list[4], F.base[4], cnt[4], num_labels,
-                                                                vb, edges);
+                wave_vb<LpMode::Refine, DENSE, DCAP>(a, F.list[4], F.base[4], cnt[4], num_labels, vb,
+                                                      edges);
                 break;
             default: hubcnt_vb(a, F.list[5], F.base[5], cnt[5], num_labels, vb);
         }
@@ -1736,31 +1770,22 @@ constexpr int kBinThreads = 512;
 constexpr int kBinGrid = 512;
 constexpr int kBinItems = 4;  // nodes per thread in flight
 constexpr int kBinLists = kMaxSub * kNumBins;
-constexpr int kBinSlots = kBinLists + kMaxSub;  // lists, then the small wave nodes of a sub-round
 
-// List slot of node v (-1: in none): its list, or the small part of its sub-round's wave list.
-__device__ inline int bin_slot(const BinConfig& cfg, const uint8_t* __restrict__ include,
-                               uint32_t seed, int S, int split, int v, int deg) {
+// List of node v (-1: in none).
+__device__ inline int list_of(const BinConfig& cfg, const uint8_t* __restrict__ include,
+                              uint32_t seed, int S, int v, int deg) {
     if (deg <= 0 || (include && !include[v])) return -1;
-    const int sr = subround_of(seed, v, S);
-    const int b = bin_of(cfg, deg);
-    return split && b == kNumBins - 2 && deg <= cfg.wave_small ? kBinLists + sr
-                                                               : sr * kNumBins + b;
+    return subround_of(seed, v, S) * kNumBins + bin_of(cfg, deg);
 }
 
-__device__ inline int bin_list(int slot) {
-    return slot < kBinLists ? slot : (slot - kBinLists) * kNumBins + kNumBins - 2;
-}
-
-// counts[l] / edges[l]: nodes and edges of list l = sub-round * kNumBins + bin; with split,
-// counts[kBinLists + sr] also receives the wave-bin nodes of degree <= cfg.wave_small.
-// blocks[workgroup][slot]: the workgroup's nodes per slot.
+// counts[l] / edges[l]: nodes and edges of list l = sub-round * kNumBins + bin.
+// blocks[workgroup][l]: the workgroup's nodes per list.
 __global__ __launch_bounds__(kBinThreads) void bin_count(
     int n, int span, const int* __restrict__ xadj, uint32_t seed, int S, BinConfig cfg,
-    const uint8_t* __restrict__ include, int split, int* __restrict__ counts,
+    const uint8_t* __restrict__ include, int* __restrict__ counts,
     unsigned long long* __restrict__ edges, int* __restrict__ blocks) {
-    __shared__ unsigned long long local[kBinSlots];  // {edges, nodes}: both below 2^31
-    for (int i = threadIdx.x; i < kBinSlots; i += kBinThreads) local[i] = 0ull;
+    __shared__ unsigned long long local[kBinLists];  // {edges, nodes}: both below 2^31
+    for (int i = threadIdx.x; i < kBinLists; i += kBinThreads) local[i] = 0ull;
     __syncthreads();
     const unsigned lo = blockIdx.x * span, hi = lo + min(span, (int)(n - lo));
     for (unsigned v0 = lo + threadIdx.x; v0 < hi; v0 += kBinItems * kBinThreads) {
@@ -1773,31 +1798,28 @@ __global__ __launch_bounds__(kBinThreads) void bin_count(
 #pragma unroll
         for (int j = 0; j < kBinItems; ++j) {
             const int v = (int)(v0 + j * kBinThreads);
-            const int slot = bin_slot(cfg, include, seed, S, split, v, deg[j]);
-            if (slot >= 0) atomicAdd(&local[slot], ((unsigned long long)deg[j] << 32) | 1ull);
+            const int l = list_of(cfg, include, seed, S, v, deg[j]);
+            if (l >= 0) atomicAdd(&local[l], ((unsigned long long)deg[j] << 32) | 1ull);
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < kBinSlots; i += kBinThreads) {
+    for (int i = threadIdx.x; i < kBinLists; i += kBinThreads) {
         const int c = (int)(unsigned)local[i];
-        blocks[blockIdx.x * kBinSlots + i] = c;
+        blocks[blockIdx.x * kBinLists + i] = c;
         if (c) {
-            const int l = bin_list(i);
-            atomicAdd(&counts[l], c);
-            atomicAdd(&edges[l], local[i] >> 32);
-            if (i >= kBinLists) atomicAdd(&counts[i], c);
+            atomicAdd(&counts[i], c);
+            atomicAdd(&edges[i], local[i] >> 32);
         }
     }
 }
 
-// With split, a wave list holds its nodes of degree <= cfg.wave_small first, then the others.
 __global__ __launch_bounds__(kBinThreads) void bin_scatter(
     int n, int span, const int* __restrict__ xadj, uint32_t seed, int S, BinConfig cfg,
-    const uint8_t* __restrict__ include, int split, const int* __restrict__ counts,
+    const uint8_t* __restrict__ include, const int* __restrict__ counts,
     const int* __restrict__ blocks, int* __restrict__ offsets, int* __restrict__ cursor,
     int* __restrict__ lists) {
     static_assert(kBinLists < 64, "one lane per list");
-    __shared__ int next[kBinSlots];  // the workgroup's next free entry per slot
+    __shared__ int next[kBinLists];  // the workgroup's next free entry per list
     __shared__ int off[64];
     if (threadIdx.x < 64) {  // list offsets: the lists in order (workgroup 0 keeps them)
         const int lane = threadIdx.x;
@@ -1812,13 +1834,9 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter(
         if (blockIdx.x == 0 && lane < kBinLists) offsets[lane] = incl - cnt;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < kBinSlots; i += kBinThreads) {
-        const int c = blocks[blockIdx.x * kBinSlots + i];
-        const int l = bin_list(i);
-        // (slot kBinLists + sr counts the front part of its wave list: 0 without split)
-        const int skip = i < kBinLists && l % kNumBins == kNumBins - 2
-                             ? counts[kBinLists + l / kNumBins] : 0;
-        next[i] = c ? off[l] + skip + atomicAdd(&cursor[i], c) : 0;
+    for (int i = threadIdx.x; i < kBinLists; i += kBinThreads) {
+        const int c = blocks[blockIdx.x * kBinLists + i];
+        next[i] = c ? off[i] + atomicAdd(&cursor[i], c) : 0;
     }
     __syncthreads();
     const unsigned lo = blockIdx.x * span, hi = lo + min(span, (int)(n - lo));
@@ -1832,8 +1850,8 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter(
 #pragma unroll
         for (int j = 0; j < kBinItems; ++j) {
             const int v = (int)(v0 + j * kBinThreads);
-            const int slot = bin_slot(cfg, include, seed, S, split, v, deg[j]);
-            if (slot >= 0) lists[atomicAdd(&next[slot], 1)] = v;
+            const int l = list_of(cfg, include, seed, S, v, deg[j]);
+            if (l >= 0) lists[atomicAdd(&next[l], 1)] = v;
         }
     }
 }
@@ -2020,18 +2038,6 @@ __global__ void block_weights_global(int n, const int* __restrict__ part,
 
 inline int grid_for(long long work, int block) { return (int)((work + block - 1) / block); }
 
-// The clustering's lane-group proposal kernel of one list with `items` nodes per lane group, one
-// workgroup per virtual block.
-template <int W, int E>
-void launch_group(int items, const LpArgs& a, const int* lst, int cnt, int copies, hipStream_t s) {
-    const dim3 grid(grid_for((long long)cnt * W, kBlock * items), copies);
-    switch (items) {
-        case 1: hipLaunchKernelGGL((propose_group<W, E, 1>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
-        case 4: hipLaunchKernelGGL((propose_group<W, E, 4>), grid, dim3(kBlock), 0, s, a, lst, cnt); break;
-        default: hipLaunchKernelGGL((propose_group<W, E, 2>), grid, dim3(kBlock), 0, s, a, lst, cnt);
-    }
-}
-
 void launch_frontier(int items, bool dense, const LpArgs& a, const FrontierLists& F, int nl,
                      int listed, hipStream_t s) {
     // virtual blocks of at least 4 nodes: a listed count bounds the grid
@@ -2113,12 +2119,12 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
         ccount_.reserve(2 * L);
     }
     offsets_.reserve(L);
-    // {edges per list (64 bit), counts per list and of the small wave nodes, cursors}
-    constexpr int kBinInts = 2 * kMaxSub * kNumBins + 2 * (kMaxSub * kNumBins + kMaxSub);
+    // {edges per list (64 bit), counts per list, cursors}
+    constexpr int kBinInts = 4 * kMaxSub * kNumBins;
     bin_.reserve(kBinInts);
     unsigned long long* edges = reinterpret_cast<unsigned long long*>(bin_.p);
     counts_ = bin_.p + 2 * L;
-    int* cursor = counts_ + L + kMaxSub;
+    int* cursor = counts_ + L;
     prop_t_.reserve(scratch_n);
     prop_gain_.reserve(scratch_n);
     prop_ok_.reserve(scratch_n);
@@ -2132,8 +2138,7 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
     // a span of nodes per binning workgroup: one pass of its threads up to kBinGrid workgroups
     const int span = std::max(grid_for(grid_for(g.n, kBinGrid), kBinThreads), 1) * kBinThreads;
     const int bin_grid = grid_for(g.n, span);
-    bin_blocks_.reserve((long long)bin_grid * kBinSlots);
-    const int split = mode == LpMode::Cluster ? 1 : 0;  // small-degree wave kernel (clustering)
+    bin_blocks_.reserve((long long)bin_grid * kBinLists);
     const bool refine = mode == LpMode::Refine;
     const long long init_n = std::max<long long>({scratch_n, scratch_l, kBinInts});
     hipLaunchKernelGGL(init_scratch, dim3(grid_for(init_n, 256)), dim3(256), 0, s, scratch_n,
@@ -2142,17 +2147,16 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
                        clear_err_ ? ctl_.p + kCtlErr : nullptr);
     if (g.n > 0)
         hipLaunchKernelGGL(bin_count, dim3(bin_grid), dim3(kBinThreads), 0, s, g.n, span, g.xadj,
-                           seed, S, bins, include, split, counts_, edges, bin_blocks_.p);
-    mail_.post(s, {bin_.p, 2 * L + L + kMaxSub});
+                           seed, S, bins, include, counts_, edges, bin_blocks_.p);
+    mail_.post(s, {bin_.p, 2 * L + L});
     if (g.n > 0)
         hipLaunchKernelGGL(bin_scatter, dim3(bin_grid), dim3(kBinThreads), 0, s, g.n, span, g.xadj,
-                           seed, S, bins, include, split, counts_, bin_blocks_.p, offsets_.p, cursor,
+                           seed, S, bins, include, counts_, bin_blocks_.p, offsets_.p, cursor,
                            lists_.p);
     KH_CHECK(hipGetLastError());
     const int* got = mail_.wait(s);  // (the scatter runs meanwhile)
     std::memcpy(host_edges, got, sizeof(long long) * L);
     std::memcpy(host_counts, got + 2 * L, sizeof(int) * L);
-    std::memcpy(host_wave_small_, got + 3 * L, sizeof(int) * kMaxSub);
     int acc = 0;
     for (int i = 0; i < L; ++i) {
         host_offsets[i] = acc;
@@ -2396,8 +2400,6 @@ void LpWorkspace::build_chunk_maps(hipStream_t s) {
     }
 }
 
-static const char* kBinName[kNumBins] = {"g8", "g16", "g32", "g64", "wave", "hub"};
-
 void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int bound, int rounds,
                       uint32_t seed, hipStream_t s, Profiler* prof, const char* phase,
                       const int* lbound) {
@@ -2417,6 +2419,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     a.size = size;
     a.bound = bound;
     a.lbound = lbound;
+    a.wave_small = bins_.wave_small;
     a.trav = reinterpret_cast<unsigned long long*>(ctl_.p);
     a.err = ctl_.p + kCtlErr;
     uint8_t* act = active_.p;
@@ -2529,94 +2532,20 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 }
                 if (listed_sr > 0)
                     launch_frontier(bins_.group_items, dense_wave_, a, F, nl, listed_sr, s);
-            }
-            for (int b = 0; b < kNumBins; ++b) {
-                const int l = sr * kNumBins + b;
-                const int cnt = host_counts[l];
-                sub_total += cnt;
-                if (cnt == 0) continue;
-                if (!cl && (b < kNumBins - 1 || fused_hubs)) continue;  // in the frontier launch
-                const int* lst = lists_.p + host_offsets[l];
-                a.base = host_offsets[l];
+            } else {
+                long long ledges = 0, lnodes = 0;
+                for (int b = 0; b < kNumBins - 1; ++b) {
+                    ledges += host_edges[sr * kNumBins + b];
+                    lnodes += host_counts[sr * kNumBins + b];
+                }
                 // algorithmic bytes: 12 B per traversed edge (target, weight, label gather) and
                 // 16 B per node (two offsets, weight, own label); label weights are O(moved).
-                // (the hub list's mid-size hubs are timed in a scope of their own)
-                const bool hub = b == kNumBins - 1;
-                const long long ledges = host_edges[l] - (hub ? mid_edges_[sr] : 0);
-                const int lnodes = cnt - (hub ? mid_n_[sr] : 0);
-                const double bytes = cl ? 12.0 * (double)ledges + 16.0 * lnodes : 0.0;
-                ProfScope ps(prof, base + "_propose_" + kBinName[b], bytes, cl ? ledges : 0, s);
-                switch (b) {
-                    case 0:
-                    case 1:
-                    case 2:
-                    case 3:
-                    case 4: launch_proposals(b, sr, a, cnt, 1, s); break;
-                    default: {
-                        if (!cl && dense_hub_) {
-                            const int4* cm = cmap_.p + cmap_base_[sr];
-                            const int* dof = dense_off_.p + hub_base_[sr];
-                            const int copies = std::min(kHubDenseThreads / 64, kHubDenseSlots / nl);
-                            const size_t lds = sizeof(int) * (size_t)copies * nl;
-                            if (!(incremental && dense_all_))  // otherwise every hub decides from counters
-                                hipLaunchKernelGGL(propose_hub_dense_chunk, dim3(hub_chunks_[sr]), dim3(kHubDenseThreads), lds, s, a, cm, nl, dof, dense_cnt_.p, 0, incremental ? 1 : 0);
-                            ps.close();
-                            if (hub_multi_n_[sr] > 0) {
-                                ProfScope pf(prof, base + "_propose_hub_merge", 0.0, hub_multi_n_[sr], s);
-                                hipLaunchKernelGGL(hub_dense_decide, dim3(hub_multi_n_[sr]), dim3(256), 0, s, a, lst, multi_.p + multi_base_[sr], hub_multi_n_[sr], nl, dof, dense_cnt_.p, incremental ? 1 : 0);
-                            }
-                            break;
-                        }
-                        const int4* cm = cmap_.p + cmap_base_[sr];
-                        const long long* to = tab_off_.p + hub_base_[sr];
-                        const long long* ob = offm_base_.p + hub_base_[sr];
-                        const int* ctb = ct_base_.p + hub_base_[sr];
-                        if (hub_chunks_[sr] > 0) {
-                            if (cl) hipLaunchKernelGGL((propose_hub_chunk<LpMode::Cluster, kHubThreads, kHubChunk>), dim3(hub_chunks_[sr]), dim3(kHubThreads), 0, s, a, cm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
-                            else hipLaunchKernelGGL((propose_hub_chunk<LpMode::Refine, kHubThreads, kHubChunk>), dim3(hub_chunks_[sr]), dim3(kHubThreads), 0, s, a, cm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
-                        }
-                        ps.close();  // the hub scope times the chunked kernel alone
-                        if (mid_n_[sr] > 0) {
-                            const double mb = cl ? 12.0 * (double)mid_edges_[sr] + 16.0 * mid_n_[sr] : 0.0;
-                            ProfScope pm(prof, base + "_propose_hub_mid", mb, cl ? mid_edges_[sr] : 0, s);
-                            const int4* mm = mmap_.p + mid_base_[sr];
-                            if (cl) hipLaunchKernelGGL((propose_hub_chunk<LpMode::Cluster, kMidThreads, kMidChunk>), dim3(mid_n_[sr]), dim3(kMidThreads), 0, s, a, mm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
-                            else hipLaunchKernelGGL((propose_hub_chunk<LpMode::Refine, kMidThreads, kMidChunk>), dim3(mid_n_[sr]), dim3(kMidThreads), 0, s, a, mm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
-                        }
-                        if (hub_multi_n_[sr] > 0) {
-                            ProfScope pf(prof, base + "_propose_hub_merge", 0.0, hub_tasks_[sr], s);
-                            const int* ml = multi_.p + multi_base_[sr];
-                            const int* tp = task_prefix_.p + task_base_[sr];
-                            const int4* tm = tmap_.p + tmap_base_[sr];
-                            const int2* tsb = tsub_.p + tmap_base_[sr];
-                            const int nm = hub_multi_n_[sr];
-                            Cand* br = reinterpret_cast<Cand*>(bres_.p);
-                            const int nt = hub_tasks_[sr];
-                            // bucket-major positions, relative to this sub-round's block of counts
-                            size_t sb = scan_tmp_bytes_;
-                            KH_CHECK(rocprim::exclusive_scan(scan_tmp_.p, sb, cnt_t_.p + ct_sr_base_[sr], pos_t_.p + ct_sr_base_[sr], 0, (size_t)ct_sr_size_[sr] + 1, rocprim::plus<int>(), s));
-                            const int* pt = pos_t_.p;
-                            const int* cp = chunk_prefix_.p + chunk_base_[sr];
-                            int* bt = big_tasks_.p;
-                            int* nbt = ctl_.p + kCtlBig + (r * S + sr);
-                            int* mt = mid_tasks_.p;
-                            int* nmt = ctl_.p + kCtlMid + (r * S + sr);
-                            if (cl) {
-                                hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
-                                hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
-                                hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 2>), dim3(std::min(nt, 256)), dim3(kFinThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, bt, nbt, nullptr, nullptr);
-                                hipLaunchKernelGGL((hub_decide<LpMode::Cluster>), dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
-                            } else {
-                                hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
-                                hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
-                                hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 2>), dim3(std::min(nt, 256)), dim3(kFinThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, bt, nbt, nullptr, nullptr);
-                                hipLaunchKernelGGL((hub_decide<LpMode::Refine>), dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
-                            }
-                        }
-                        break;
-                    }
-                }
+                ProfScope ps(prof, base + "_propose_lists", 12.0 * (double)ledges + 16.0 * (double)lnodes, ledges, s);
+                launch_lists(a, sr, 1, s);
             }
+            const int cnt = host_counts[sr * kNumBins + kNumBins - 1];
+            for (int b = 0; b < kNumBins; ++b) sub_total += host_counts[sr * kNumBins + b];
+            if (cnt > 0 && !fused_hubs) propose_hubs(mode, a, r, sr, incremental, s, prof, base);
             if (sub_total == 0) continue;
             const int gm = grid_for(sub_total, 256);
             const int* sub_list = lists_.p + host_offsets[sr * kNumBins];  // bins are contiguous
@@ -2651,6 +2580,81 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     KH_CHECK(hipGetLastError());
 }
 
+// The proposals of sub-round sr's hub list.
+void LpWorkspace::propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool incremental, hipStream_t s,
+                               Profiler* prof, const std::string& base) {
+    const bool cl = mode == LpMode::Cluster;
+    const int S = subrounds_, nl = num_labels_;
+    const int l = sr * kNumBins + kNumBins - 1;
+    const int* lst = lists_.p + host_offsets[l];
+    a.base = host_offsets[l];
+    // (the list's mid-size hubs are timed in a scope of their own)
+    const long long ledges = host_edges[l] - mid_edges_[sr];
+    const int lnodes = host_counts[l] - mid_n_[sr];
+    const double bytes = cl ? 12.0 * (double)ledges + 16.0 * lnodes : 0.0;
+    ProfScope ps(prof, base + "_propose_hub", bytes, cl ? ledges : 0, s);
+    if (!cl && dense_hub_) {
+        const int4* cm = cmap_.p + cmap_base_[sr];
+        const int* dof = dense_off_.p + hub_base_[sr];
+        const int copies = std::min(kHubDenseThreads / 64, kHubDenseSlots / nl);
+        const size_t lds = sizeof(int) * (size_t)copies * nl;
+        if (!(incremental && dense_all_))  // otherwise every hub decides from counters
+            hipLaunchKernelGGL(propose_hub_dense_chunk, dim3(hub_chunks_[sr]), dim3(kHubDenseThreads), lds, s, a, cm, nl, dof, dense_cnt_.p, 0, incremental ? 1 : 0);
+        ps.close();
+        if (hub_multi_n_[sr] > 0) {
+            ProfScope pf(prof, base + "_propose_hub_merge", 0.0, hub_multi_n_[sr], s);
+            hipLaunchKernelGGL(hub_dense_decide, dim3(hub_multi_n_[sr]), dim3(256), 0, s, a, lst, multi_.p + multi_base_[sr], hub_multi_n_[sr], nl, dof, dense_cnt_.p, incremental ? 1 : 0);
+        }
+        return;
+    }
+    const int4* cm = cmap_.p + cmap_base_[sr];
+    const long long* to = tab_off_.p + hub_base_[sr];
+    const long long* ob = offm_base_.p + hub_base_[sr];
+    const int* ctb = ct_base_.p + hub_base_[sr];
+    if (hub_chunks_[sr] > 0) {
+        if (cl) hipLaunchKernelGGL((propose_hub_chunk<LpMode::Cluster, kHubThreads, kHubChunk>), dim3(hub_chunks_[sr]), dim3(kHubThreads), 0, s, a, cm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
+        else hipLaunchKernelGGL((propose_hub_chunk<LpMode::Refine, kHubThreads, kHubChunk>), dim3(hub_chunks_[sr]), dim3(kHubThreads), 0, s, a, cm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
+    }
+    ps.close();  // the hub scope times the chunked kernel alone
+    if (mid_n_[sr] > 0) {
+        const double mb = cl ? 12.0 * (double)mid_edges_[sr] + 16.0 * mid_n_[sr] : 0.0;
+        ProfScope pm(prof, base + "_propose_hub_mid", mb, cl ? mid_edges_[sr] : 0, s);
+        const int4* mm = mmap_.p + mid_base_[sr];
+        if (cl) hipLaunchKernelGGL((propose_hub_chunk<LpMode::Cluster, kMidThreads, kMidChunk>), dim3(mid_n_[sr]), dim3(kMidThreads), 0, s, a, mm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
+        else hipLaunchKernelGGL((propose_hub_chunk<LpMode::Refine, kMidThreads, kMidChunk>), dim3(mid_n_[sr]), dim3(kMidThreads), 0, s, a, mm, partials_.p, ob, offm_.p, ctb, cnt_t_.p);
+    }
+    if (hub_multi_n_[sr] > 0) {
+        ProfScope pf(prof, base + "_propose_hub_merge", 0.0, hub_tasks_[sr], s);
+        const int* ml = multi_.p + multi_base_[sr];
+        const int* tp = task_prefix_.p + task_base_[sr];
+        const int4* tm = tmap_.p + tmap_base_[sr];
+        const int2* tsb = tsub_.p + tmap_base_[sr];
+        const int nm = hub_multi_n_[sr];
+        Cand* br = reinterpret_cast<Cand*>(bres_.p);
+        const int nt = hub_tasks_[sr];
+        // bucket-major positions, relative to this sub-round's block of counts
+        size_t sb = scan_tmp_bytes_;
+        KH_CHECK(rocprim::exclusive_scan(scan_tmp_.p, sb, cnt_t_.p + ct_sr_base_[sr], pos_t_.p + ct_sr_base_[sr], 0, (size_t)ct_sr_size_[sr] + 1, rocprim::plus<int>(), s));
+        const int* pt = pos_t_.p;
+        const int* cp = chunk_prefix_.p + chunk_base_[sr];
+        int* bt = big_tasks_.p;
+        int* nbt = ctl_.p + kCtlBig + (r * S + sr);
+        int* mt = mid_tasks_.p;
+        int* nmt = ctl_.p + kCtlMid + (r * S + sr);
+        if (cl) {
+            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
+            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
+            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 2>), dim3(std::min(nt, 256)), dim3(kFinThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, bt, nbt, nullptr, nullptr);
+            hipLaunchKernelGGL((hub_decide<LpMode::Cluster>), dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
+        } else {
+            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
+            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
+            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 2>), dim3(std::min(nt, 256)), dim3(kFinThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, bt, nbt, nullptr, nullptr);
+            hipLaunchKernelGGL((hub_decide<LpMode::Refine>), dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
+        }
+    }
+}
+
 void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
                              const uint32_t* seeds, int copies, hipStream_t s) {
     if (g.n == 0) return;
@@ -2671,6 +2675,7 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
     a.label = label;
     a.size = size;
     a.bound = bound;
+    a.wave_small = bins_.wave_small;
     a.inc = inc_.p;
     a.top = top_.p;
     a.prop_t = prop_t_.p;
@@ -2684,12 +2689,9 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
     if (copies > 1) a.copy_tie1 = tie_seed_of(seeds[1], 0);
     if (copies > 2) a.copy_tie2 = tie_seed_of(seeds[2], 0);
     int total = 0;
-    for (int b = 0; b < kNumBins - 1; ++b) {
-        const int cnt = host_counts[b];
-        if (cnt > 0) launch_proposals(b, 0, a, cnt, copies, s);
-        total += cnt;
-    }
+    for (int b = 0; b < kNumBins - 1; ++b) total += host_counts[b];
     if (total == 0) return;
+    launch_lists(a, 0, copies, s);
     const dim3 grid(grid_for(total, 256), copies);
     hipLaunchKernelGGL(admit_moves, grid, dim3(256), 0, s, a, lists_.p, total);
     hipLaunchKernelGGL(apply_moves, dim3(std::min(grid_for(total, kApplyThreads), kApplyGrid), copies),
@@ -2697,27 +2699,32 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
     KH_CHECK(hipGetLastError());
 }
 
-// The clustering proposals of list b (not the hub list) of sub-round sr.
-void LpWorkspace::launch_proposals(int b, int sr, LpArgs a, int cnt, int copies,
-                                   hipStream_t s) {
-    a.base = host_offsets[sr * kNumBins + b];
-    const int* lst = lists_.p + a.base;
-    switch (b) {
-        case 0: launch_group<8, 1>(bins_.group_items, a, lst, cnt, copies, s); break;
-        case 1: launch_group<8, 2>(bins_.group_items, a, lst, cnt, copies, s); break;
-        case 2: launch_group<16, 2>(bins_.group_items, a, lst, cnt, copies, s); break;
-        case 3: launch_group<16, 4>(bins_.group_items, a, lst, cnt, copies, s); break;
-        default: {
-            const int ns = host_wave_small_[sr];  // degree <= wave_small, first
-            if (ns > 0) {
-                const dim3 gs(grid_for(ns, kBlock / 64), copies);
-                if (bins_.wave_small == 64) hipLaunchKernelGGL(propose_wave<128>, gs, dim3(kBlock), 0, s, a, lst, ns);
-                else if (bins_.wave_small == 256) hipLaunchKernelGGL(propose_wave<512>, gs, dim3(kBlock), 0, s, a, lst, ns);
-                else hipLaunchKernelGGL(propose_wave<256>, gs, dim3(kBlock), 0, s, a, lst, ns);
-            }
-            a.base += ns;
-            if (cnt > ns) hipLaunchKernelGGL(propose_wave<>, dim3(grid_for(cnt - ns, kBlock / 64), copies), dim3(kBlock), 0, s, a, lst + ns, cnt - ns);
-        }
+// The clustering proposals of sub-round sr's lists (not the hub list).
+void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, hipStream_t s) {
+    ClusterLists F{};
+    const int items = bins_.group_items;
+    int blocks = 0;
+    for (int b = 0; b < kNumBins - 1; ++b) {
+        const int l = sr * kNumBins + b;
+        F.list[b] = lists_.p + host_offsets[l];
+        F.base[b] = host_offsets[l];
+        F.count[b] = host_counts[l];
+        const int per = b < 2 ? items * (kBlock / 8) : b < 4 ? items * (kBlock / 16) : kBlock / 64;
+        blocks += grid_for(host_counts[l], per);
+    }
+    if (blocks == 0) return;
+    const dim3 grid(blocks, copies);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, a, F);
+    };
+    const bool waves = F.count[kNumBins - 2] > 0;
+    switch (items * 2 + (waves ? 1 : 0)) {
+        case 2: launch(propose_lists<1, false>); break;
+        case 3: launch(propose_lists<1, true>); break;
+        case 8: launch(propose_lists<4, false>); break;
+        case 9: launch(propose_lists<4, true>); break;
+        case 5: launch(propose_lists<2, true>); break;
+        default: launch(propose_lists<2, false>);
     }
 }
 

@@ -21,6 +21,7 @@ struct LpArgs {
     int* size;         // weight of each label
     int bound;         // admission bound: size + w < bound
     const int* lbound; // per-label bounds (a disjoint union of graphs), nullptr: `bound` for all
+    int wave_small;    // one-wave nodes up to this degree: half the edges per lane
     uint32_t tie_seed;
     const uint8_t* active;  // refinement frontier (nullptr for clustering)
     uint8_t* next_active;
@@ -96,14 +97,15 @@ public:
     void check_later() { keep_err_ = true; }
 
     int host_counts[kMaxSub * kNumBins] = {};
-    int host_wave_small_[kMaxSub] = {};  // clustering: wave-list nodes of the small-LDS kernel
     long long host_edges[kMaxSub * kNumBins] = {};
     int host_offsets[kMaxSub * kNumBins] = {};
 
 private:
     void build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
                      const uint8_t* include, int copies);
-    void launch_proposals(int b, int sr, LpArgs a, int cnt, int copies, hipStream_t s);
+    void launch_lists(const LpArgs& a, int sr, int copies, hipStream_t s);
+    void propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool incremental, hipStream_t s,
+                      Profiler* prof, const std::string& base);
     int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
     void fetch(hipStream_t s);  // host_ctl_ of the last run
     Mail mail_;
