@@ -327,12 +327,13 @@ __device__ inline void decide(const LpArgs& a, int pos, int v, int own, int w, i
 // own label. A pass takes SLOTS slots per lane: it reads their keys and values, then issues the
 // label-weight (and per-label bound) gathers of all of them, then evaluates, so a lane waits for
 // one gather latency per pass instead of one per slot. Candidates compare by the total order of
-// better(), so the result does not depend on the scan order. (The workgroup-per-hub kernels keep
-// the slot-by-slot scan: there the batched form measured slower.)
+// better(), so the result does not depend on the scan order. `other` receives the lane's largest
+// weight towards another label, eligible or not. (The workgroup-per-hub kernels keep the
+// slot-by-slot scan: there the batched form measured slower.)
 template <int SLOTS>
 __device__ __attribute__((always_inline)) inline void scan_wave_table(
     const LpArgs& a, const int* K, const int* V, int cap, int lane, int v, int own, int nw,
-    int& conn_own, Cand& c) {
+    int& conn_own, Cand& c, int& other) {
     for (int base = lane; base < cap; base += SLOTS * 64) {
         int lk[SLOTS], lv[SLOTS], ls[SLOTS], lb[SLOTS];
 #pragma unroll
@@ -359,6 +360,7 @@ __device__ __attribute__((always_inline)) inline void scan_wave_table(
                 conn_own = lv[j];
                 continue;
             }
+            other = max(other, lv[j]);
             if ((long long)ls[j] + nw >= (long long)lb[j] || lv[j] < c.conn) continue;
             const uint32_t t = hash3(a.tie_seed, (uint32_t)v, (uint32_t)lab);
             if (better(lv[j], t, lab, c.conn, c.tie, c.lab)) c = Cand{lv[j], t, lab, ls[j]};
@@ -379,7 +381,8 @@ __device__ __attribute__((always_inline)) inline void scan_wave_table(
 // wave has that many chains in flight.
 // One virtual block (IT x kBlock / W nodes of the list); every thread of the workgroup calls it
 // (it synchronises the workgroup). `edges` adds up the traversed edges (refinement).
-template <LpMode M, int W, int E, int IT>
+// SETTLE: also flags the nodes that are not settled (kSettleRound).
+template <LpMode M, int W, int E, int IT, bool SETTLE = false>
 __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
                                                                const int* __restrict__ list,
                                                                int base, int count, int vb,
@@ -445,7 +448,7 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
     Contrib r[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-        int conn[E], conn_own = 0;
+        int conn[E], conn_own = 0, other = -1;
         group_sums<W>(lab[i], w[i], conn);
 #pragma unroll
         for (int j = 0; j < E; ++j) {
@@ -454,9 +457,14 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
             // candidates: other labels with room for the node (a select without branches: hipcc
             // 7.2 lost the -1 of a lane in the branching form)
             const bool room = (long long)sz[i][j] + nw[i] < (long long)lb[i][j];
+            if (SETTLE) other = max(other, (l >= 0) & (l != own[i]) ? conn[j] : -1);
             conn[j] = (l >= 0) & (l != own[i]) & room ? conn[j] : -1;
         }
         conn_own = group_max<W>(conn_own);
+        if (SETTLE) {
+            other = group_max<W>(other);
+            if (valid[i] && gl == 0) a.next_active[v[i]] = other >= conn_own;
+        }
         const Cand c = group_best<W>(a.tie_seed, v[i], conn, lab[i], sz[i]);
         const int pos = base + (int)(((long long)vb * IT + i) * NB) + threadIdx.x / W;
         r[i] = (valid[i] && gl == 0) ? propose<M>(a, pos, v[i], own[i], nw[i], conn_own, c)
@@ -513,7 +521,7 @@ __device__ __attribute__((always_inline)) inline void wave_lds_order() {
     __builtin_amdgcn_wave_barrier();
 }
 // EPL: edges per lane, 64 x EPL >= degree.
-template <LpMode M, bool DENSE, int EPL>
+template <LpMode M, bool DENSE, int EPL, bool SETTLE>
 __device__ __attribute__((always_inline)) inline void wave_node(const LpArgs& a, int pos, int v,
                                                                 int beg, int deg, int num_labels,
                                                                 int lane, int* K, int* V) {
@@ -560,10 +568,10 @@ __device__ __attribute__((always_inline)) inline void wave_node(const LpArgs& a,
     }
     wave_lds_order();
     const int nw = a.vwgt[v];
-    int conn_own = 0;
+    int conn_own = 0, other = -1;
     Cand c{-1, 0u, 0x7fffffff, 0};
     if (!DENSE) {
-        scan_wave_table<EPL < 8 ? 2 * EPL : 8>(a, K, V, cap, lane, v, own, nw, conn_own, c);
+        scan_wave_table<EPL < 8 ? 2 * EPL : 8>(a, K, V, cap, lane, v, own, nw, conn_own, c, other);
     } else {
         for (int i = lane; i < cap; i += 64) {
             const int lab = V[i] ? i : -1;
@@ -581,6 +589,10 @@ __device__ __attribute__((always_inline)) inline void wave_node(const LpArgs& a,
     }
     conn_own = reduce_max<64>(conn_own);
     reduce_cand<64>(c);
+    if (SETTLE) {
+        other = reduce_max<64>(other);
+        if (lane == 0) a.next_active[v] = other >= conn_own;
+    }
     if (lane == 0) decide<M>(a, pos, v, own, nw, conn_own, c);
     wave_lds_order();  // the table is read before the wave's next node clears it
 }
@@ -588,7 +600,7 @@ __device__ __attribute__((always_inline)) inline void wave_node(const LpArgs& a,
 // One virtual block: kBlock / 64 nodes of the list, a wave each. DCAP: dense counters per wave
 // (num_labels <= DCAP). Rows of up to LpArgs::wave_small edges take the variant with half the
 // registers and predicated loads.
-template <LpMode M, bool DENSE, int DCAP = kWaveDense>
+template <LpMode M, bool DENSE, int DCAP = kWaveDense, bool SETTLE = false>
 __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
                                                               const int* __restrict__ list,
                                                               int base, int count, int num_labels,
@@ -602,11 +614,11 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
     const int v = list[gi];
     const int beg = a.xadj[v], deg = a.xadj[v + 1] - beg;
     if (deg <= a.wave_small)
-        wave_node<M, DENSE, kWaveEdges / 2>(a, base + gi, v, beg, deg, num_labels, lane,
+        wave_node<M, DENSE, kWaveEdges / 2, SETTLE>(a, base + gi, v, beg, deg, num_labels, lane,
                                             skey[wave], sval[wave]);
     else
-        wave_node<M, DENSE, kWaveEdges>(a, base + gi, v, beg, deg, num_labels, lane, skey[wave],
-                                        sval[wave]);
+        wave_node<M, DENSE, kWaveEdges, SETTLE>(a, base + gi, v, beg, deg, num_labels, lane,
+                                                skey[wave], sval[wave]);
     if (M == LpMode::Refine && lane == 0) edges += (unsigned long long)deg;
 }
 
@@ -621,34 +633,59 @@ struct ClusterLists {
     const int* list[kNumBins - 1];
     int base[kNumBins - 1];  // list positions of their first entries
     int count[kNumBins - 1];
+    const int* dcount;  // lengths on the device (a compacted sub-round), else nullptr
 };
-template <int IT, bool WAVES>
+template <int IT, bool WAVES, bool SETTLE>
 __global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F) {
     select_copy(a);
     constexpr LpMode C = LpMode::Cluster;
     constexpr int N = kNumBins - 1;
     constexpr int NPB[N] = {IT * (kBlock / 8), IT * (kBlock / 8), IT * (kBlock / 16),
                             IT * (kBlock / 16), kBlock / 64};
-    int vb = blockIdx.x, b = N - 1;  // uniform per workgroup
+    int cnt[N], nvb[N], total = 0;
 #pragma unroll
-    for (int k = N - 1; k > 0; --k) {
-        const int nvb = (F.count[k] + NPB[k] - 1) / NPB[k];
-        if (b == k && vb >= nvb) {
-            vb -= nvb;
-            b = k - 1;
-        }
+    for (int b = 0; b < N; ++b) {
+        cnt[b] = SETTLE && F.dcount ? F.dcount[b] : F.count[b];
+        nvb[b] = (cnt[b] + NPB[b] - 1) / NPB[b];
+        total += nvb[b];
     }
     unsigned long long edges = 0;
-    switch (b) {
-        case 0: group_vb<C, 8, 1, IT>(a, F.list[0], F.base[0], F.count[0], vb, edges); break;
-        case 1: group_vb<C, 8, 2, IT>(a, F.list[1], F.base[1], F.count[1], vb, edges); break;
-        case 2: group_vb<C, 16, 2, IT>(a, F.list[2], F.base[2], F.count[2], vb, edges); break;
-        case 3: group_vb<C, 16, 4, IT>(a, F.list[3], F.base[3], F.count[3], vb, edges); break;
-        default:
-            if constexpr (WAVES)
-                wave_vb<C, false>(a, F.list[4], F.base[4], F.count[4], 0, vb, edges);
+    for (int t = blockIdx.x; t < total; t += gridDim.x) {  // one pass over whole lists
+        int vb = t, b = N - 1;  // uniform per workgroup
+#pragma unroll
+        for (int k = N - 1; k > 0; --k)
+            if (b == k && vb >= nvb[k]) {
+                vb -= nvb[k];
+                b = k - 1;
+            }
+        switch (b) {
+            case 0: group_vb<C, 8, 1, IT, SETTLE>(a, F.list[0], F.base[0], cnt[0], vb, edges); break;
+            case 1: group_vb<C, 8, 2, IT, SETTLE>(a, F.list[1], F.base[1], cnt[1], vb, edges); break;
+            case 2: group_vb<C, 16, 2, IT, SETTLE>(a, F.list[2], F.base[2], cnt[2], vb, edges); break;
+            case 3: group_vb<C, 16, 4, IT, SETTLE>(a, F.list[3], F.base[3], cnt[3], vb, edges); break;
+            default:
+                if constexpr (WAVES)
+                    wave_vb<C, false, kWaveDense, SETTLE>(a, F.list[4], F.base[4], cnt[4], 0, vb,
+                                                          edges);
+        }
     }
 }
+
+// ---------------------------------------------------------------- clustering: settled nodes
+// A node whose weight towards its own cluster exceeds that towards every other one does not
+// propose, whatever the clusters' sizes and the tie-breaking, until it is moved or a neighbour
+// moves into another cluster than the node's own. On a mesh that is most of the nodes after two
+// rounds (RGG 2^18: 87 % after two, 92 % after three, 97 % after ten), so from round kSettleRound
+// on a proposing kernel also flags the nodes that are not settled, an application flags the moved
+// nodes and those neighbours, and from the round after it a sub-round first compacts its lists to
+// the flagged nodes (right before it, as the earlier sub-rounds' moves unsettle nodes of this one).
+// Earlier, most nodes move and flag all of their neighbours: measured, RGG 2^22, k = 2, coarsening
+// from round 1 9.3, from 2 8.9, from 3 9.0 ms, without 10.1 ms. For large graphs only: at
+// kSettleEdges edges and below a sub-round is bound by its launches, and the compaction is one
+// more (RGG of 60 001 nodes: 0.80 -> 1.12 ms, of 1 000 003: 3.8 -> 3.2 ms). Not for graphs
+// with hubs: on R-MAT graphs 14 to 18 % of the nodes settle and hardly fewer edges are read.
+constexpr int kSettleRound = 2;
+constexpr long long kSettleEdges = 1LL << 21;
 
 // Refinement: the proposals of all degree lists of a sub-round in one launch. The lists are the
 // round's compacted frontier (lengths on the device); the workgroups stride over the virtual
@@ -1322,7 +1359,11 @@ __global__ __launch_bounds__(256) void admit_moves_sub(LpArgs a, SubLists L) {
 // of three gathers: neighbour, hub slot, counter): with a lane per row, a row of 64 entries was
 // 64 such chains one after the other. Measured, R-MAT 2^20, k = 16: 58 -> 37 us
 // on average (the rest: the atomics on the hubs' counters), R-MAT 2^17 16 -> 10 us.
+// Clustering: flags the moved nodes and those neighbours that a move may unsettle (a neighbour in
+// the target cluster stays settled, unless the edge's weight is negative). A neighbour moved by
+// the same launch is flagged by its own move, so it does not matter which of its labels is read.
 constexpr int kApplyEdges = 4;
+template <LpMode M>
 __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) {
     __shared__ int block_moves;
     __shared__ unsigned long long claimed;  // {movers, their edges} of the step
@@ -1343,7 +1384,8 @@ __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) 
         if (t >= 0) {
             const int v = list[index];
             int from;
-            if (apply_one<LpMode::Refine>(a, pos, v, t, &from)) {
+            if (apply_one<M>(a, pos, v, t, &from)) {
+                if (M == LpMode::Cluster) a.next_active[v] = 1;
                 const int beg = a.xadj[v], deg = a.xadj[v + 1] - beg;
                 // index and first edge from one atomic: the movers' edges ascend with k
                 const unsigned long long at =
@@ -1381,6 +1423,16 @@ __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) 
                     u[j] = a.adjncy[e[j]];
                 }
             }
+            if constexpr (M == LpMode::Cluster) {
+                int lab[kApplyEdges];
+#pragma unroll
+                for (int j = 0; j < kApplyEdges; ++j) lab[j] = e[j] >= 0 ? a.label[u[j]] : 0;
+#pragma unroll
+                for (int j = 0; j < kApplyEdges; ++j)
+                    if (e[j] >= 0 && (lab[j] != row_to[k[j]] || a.adjwgt[e[j]] < 0))
+                        a.next_active[u[j]] = 1;
+                continue;
+            }
             int slot[kApplyEdges];
 #pragma unroll
             for (int j = 0; j < kApplyEdges; ++j) {
@@ -1400,7 +1452,7 @@ __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) 
         }
         __syncthreads();  // the step's rows are done before the movers are reset
     }
-    count_traversed(a, edges);
+    if (M == LpMode::Refine) count_traversed(a, edges);
     if (threadIdx.x == 0 && block_moves) atomicAdd(a.moves, block_moves);
 }
 
@@ -1856,14 +1908,15 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter(
     }
 }
 
-// Frontier of a refinement round: the active nodes of every non-hub list, compacted per list
-// into clists (same offsets as lists); ccount[l] receives list l's length. The order inside a
+// Frontier of a refinement round, or the nodes that a clustering sub-round looks at: the active
+// nodes of the lists in entries [first, first + total), compacted per list into clists (same offsets as lists); ccount[l] receives list l's length. The order inside a
 // list is free: the synchronous schedule does not depend on it. clear: the flags are consumed, so
 // that the array serves as the next round's (unless a kernel of this round still reads them).
 constexpr int kCompactItems = 8;  // list entries per thread of compact_active
 __global__ __launch_bounds__(256) void compact_active(const int* __restrict__ lists,
                                                       const int* __restrict__ offsets, int nseg,
-                                                      int total, uint8_t* __restrict__ active,
+                                                      int first, int total,
+                                                      uint8_t* __restrict__ active,
                                                       int clear, int* __restrict__ ccount,
                                                       int* __restrict__ clists) {
     __shared__ int off[kMaxSub * kNumBins];
@@ -1876,12 +1929,12 @@ __global__ __launch_bounds__(256) void compact_active(const int* __restrict__ li
     __syncthreads();
     // kCompactItems entries per thread, 256 apart (coalesced), their flag gathers in flight
     // together; one global count update per list and workgroup
-    const int i0 = blockIdx.x * 256 * kCompactItems + threadIdx.x;
+    const int i0 = first + blockIdx.x * 256 * kCompactItems + threadIdx.x;
     int v[kCompactItems], l[kCompactItems], r[kCompactItems];
 #pragma unroll
     for (int j = 0; j < kCompactItems; ++j) {
         const int i = i0 + 256 * j;
-        v[j] = i < total ? lists[i] : -1;
+        v[j] = i < first + total ? lists[i] : -1;
     }
 #pragma unroll
     for (int j = 0; j < kCompactItems; ++j) {
@@ -2479,6 +2532,14 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         hipLaunchKernelGGL(init_frontier, dim3(grid_for(std::max(nf, 2 * nseg), 256)), dim3(256),
                            0, s, nf, act, (uint8_t)(keep_flags ? 1 : 0), nxt, 2 * nseg, ccount_.p);
     }
+    const bool settle = cl && hubs == 0 && rounds > kSettleRound + 1 && g.m2 > kSettleEdges;
+    if (settle) {
+        active_.reserve(g.n);
+        clists_.reserve(g.n);
+        ccount_.reserve(rounds * nseg);  // list lengths per round
+        fill_async(ccount_.p, rounds * nseg, 0, s);
+        act = active_.p;
+    }
     int* cnow = ccount_.p;  // list lengths of the frontier, cleared by the tail before last
     int* cnext = cnow + nseg;
     while (r < rounds) {
@@ -2489,7 +2550,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
             ProfScope ps(prof, base + "_frontier", 0.0, 0, s);
             std::swap(cnow, cnext);
             hipLaunchKernelGGL(compact_active, dim3(grid_for(listed, 256 * kCompactItems)), dim3(256), 0, s,
-                               lists_.p, offsets_.p, nseg, listed, act, keep_flags ? 0 : 1, cnow, clists_.p);
+                               lists_.p, offsets_.p, nseg, 0, listed, act, keep_flags ? 0 : 1, cnow, clists_.p);
             a.next_active = nxt;
             TailArgs t{};
             t.clists = clists_.p;
@@ -2515,6 +2576,14 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         a.moves = ctl_.p + kCtlMoves + r;
         a.active = cl ? nullptr : act;
         a.next_active = cl ? nullptr : nxt;
+        if (settle && r >= kSettleRound) {
+            ProfScope ps(prof, base + "_settled", 0.0, 0, s);
+            a.next_active = act;
+            for (int sr = 0; sr < S; ++sr)
+                settled_subround(a, sr, r == kSettleRound ? nullptr : ccount_.p + r * nseg + sr * kNumBins, s);
+            ++r;
+            continue;
+        }
         for (int sr = 0; sr < S; ++sr) {
             int sub_total = 0;
             if (!cl) {
@@ -2541,7 +2610,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 // algorithmic bytes: 12 B per traversed edge (target, weight, label gather) and
                 // 16 B per node (two offsets, weight, own label); label weights are O(moved).
                 ProfScope ps(prof, base + "_propose_lists", 12.0 * (double)ledges + 16.0 * (double)lnodes, ledges, s);
-                launch_lists(a, sr, 1, s);
+                launch_lists(a, sr, 1, nullptr, false, s);
             }
             const int cnt = host_counts[sr * kNumBins + kNumBins - 1];
             for (int b = 0; b < kNumBins; ++b) sub_total += host_counts[sr * kNumBins + b];
@@ -2568,7 +2637,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 const int gs = std::min(gm, 1024);
                 if (filter) hipLaunchKernelGGL(filter_departures_sub, dim3(gs), dim3(256), 0, s, a, L);
                 hipLaunchKernelGGL(admit_moves_sub, dim3(gs), dim3(256), 0, s, a, L);
-                hipLaunchKernelGGL(apply_moves_sub, dim3(gs), dim3(kBlock), 0, s, a, L);
+                hipLaunchKernelGGL(apply_moves_sub<LpMode::Refine>, dim3(gs), dim3(kBlock), 0, s, a, L);
             }
         }
         if (!cl) {
@@ -2691,7 +2760,7 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
     int total = 0;
     for (int b = 0; b < kNumBins - 1; ++b) total += host_counts[b];
     if (total == 0) return;
-    launch_lists(a, 0, copies, s);
+    launch_lists(a, 0, copies, nullptr, false, s);
     const dim3 grid(grid_for(total, 256), copies);
     hipLaunchKernelGGL(admit_moves, grid, dim3(256), 0, s, a, lists_.p, total);
     hipLaunchKernelGGL(apply_moves, dim3(std::min(grid_for(total, kApplyThreads), kApplyGrid), copies),
@@ -2699,33 +2768,65 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
     KH_CHECK(hipGetLastError());
 }
 
-// The clustering proposals of sub-round sr's lists (not the hub list).
-void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, hipStream_t s) {
+// The clustering proposals of sub-round sr's lists (not the hub list); dcount: compacted to these
+// lengths; settle: also flag the nodes that are not settled.
+void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, const int* dcount, bool settle,
+                               hipStream_t s) {
     ClusterLists F{};
+    F.dcount = dcount;
     const int items = bins_.group_items;
     int blocks = 0;
     for (int b = 0; b < kNumBins - 1; ++b) {
         const int l = sr * kNumBins + b;
-        F.list[b] = lists_.p + host_offsets[l];
+        F.list[b] = (dcount ? clists_.p : lists_.p) + host_offsets[l];
         F.base[b] = host_offsets[l];
         F.count[b] = host_counts[l];
         const int per = b < 2 ? items * (kBlock / 8) : b < 4 ? items * (kBlock / 16) : kBlock / 64;
         blocks += grid_for(host_counts[l], per);
     }
     if (blocks == 0) return;
-    const dim3 grid(blocks, copies);
+    const dim3 grid(dcount ? std::min(blocks, kFrontierGrid) : blocks, copies);
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, a, F);
     };
     const bool waves = F.count[kNumBins - 2] > 0;
-    switch (items * 2 + (waves ? 1 : 0)) {
-        case 2: launch(propose_lists<1, false>); break;
-        case 3: launch(propose_lists<1, true>); break;
-        case 8: launch(propose_lists<4, false>); break;
-        case 9: launch(propose_lists<4, true>); break;
-        case 5: launch(propose_lists<2, true>); break;
-        default: launch(propose_lists<2, false>);
+    switch (items * 4 + (waves ? 1 : 0) + (settle ? 2 : 0)) {
+        case 4: launch(propose_lists<1, false, false>); break;
+        case 5: launch(propose_lists<1, true, false>); break;
+        case 6: launch(propose_lists<1, false, true>); break;
+        case 7: launch(propose_lists<1, true, true>); break;
+        case 16: launch(propose_lists<4, false, false>); break;
+        case 17: launch(propose_lists<4, true, false>); break;
+        case 18: launch(propose_lists<4, false, true>); break;
+        case 19: launch(propose_lists<4, true, true>); break;
+        case 9: launch(propose_lists<2, true, false>); break;
+        case 10: launch(propose_lists<2, false, true>); break;
+        case 11: launch(propose_lists<2, true, true>); break;
+        default: launch(propose_lists<2, false, false>);
     }
+}
+
+// Sub-round sr of a clustering from round kSettleRound on: over the whole lists (dcount nullptr)
+// or over their nodes that are not settled (dcount: their lengths, zero on entry).
+void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s) {
+    const int l0 = sr * kNumBins;
+    int total = 0;
+    for (int b = 0; b < kNumBins; ++b) total += host_counts[l0 + b];
+    if (total == 0) return;
+    if (dcount)
+        hipLaunchKernelGGL(compact_active, dim3(grid_for(total, 256 * kCompactItems)), dim3(256), 0,
+                           s, lists_.p, offsets_.p + l0, kNumBins, host_offsets[l0], total,
+                           a.next_active, 1, dcount, clists_.p);
+    launch_lists(a, sr, 1, dcount, true, s);
+    SubLists L{};
+    for (int b = 0; b < kNumBins; ++b) {
+        L.list[b] = (dcount ? clists_.p : lists_.p) + host_offsets[l0 + b];
+        L.base[b] = host_offsets[l0 + b];
+        L.dcount[b] = (dcount ? dcount : counts_ + l0) + b;
+    }
+    const int gs = std::min(grid_for(total, 256), 1024);
+    hipLaunchKernelGGL(admit_moves_sub, dim3(gs), dim3(256), 0, s, a, L);
+    hipLaunchKernelGGL(apply_moves_sub<LpMode::Cluster>, dim3(gs), dim3(kBlock), 0, s, a, L);
 }
 
 // Launches refine_tail and waits for its answer: the round to go on with, and whether a block is

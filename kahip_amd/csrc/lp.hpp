@@ -24,7 +24,7 @@ struct LpArgs {
     int wave_small;    // one-wave nodes up to this degree: half the edges per lane
     uint32_t tie_seed;
     const uint8_t* active;  // refinement frontier (nullptr for clustering)
-    uint8_t* next_active;
+    uint8_t* next_active;  // clustering: nodes that are not settled
     int* inc;                  // per label: summed weight of proposals into it
     unsigned long long* top;   // per label: top proposal priority into it
     int* out;                  // per label: summed weight of departures (refinement)
@@ -103,7 +103,9 @@ public:
 private:
     void build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
                      const uint8_t* include, int copies);
-    void launch_lists(const LpArgs& a, int sr, int copies, hipStream_t s);
+    void launch_lists(const LpArgs& a, int sr, int copies, const int* dcount, bool settle,
+                      hipStream_t s);
+    void settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s);
     void propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool incremental, hipStream_t s,
                       Profiler* prof, const std::string& base);
     int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
@@ -155,7 +157,7 @@ private:
     DevBuf<uint8_t> fb_;
     DevBuf<int> lists_, bin_, bin_blocks_, offsets_;
     int* counts_ = nullptr;  // in bin_: list lengths
-    DevBuf<int> clists_, ccount_;  // refinement frontier per list (compacted each round)
+    DevBuf<int> clists_, ccount_;  // frontier (or nodes not settled) per list, compacted
     DevBuf<int> prop_t_, prop_gain_;
     DevBuf<uint8_t> prop_ok_;
     DevBuf<int> inc_, out_;
