@@ -22,6 +22,7 @@
 //                       one launch of a sub-round serves all of these lists;
 //   larger              one workgroup per node, hash table in a pre-cleared global region.
 
+#include <algorithm>
 #include <cstring>
 
 #include <rocprim/device/device_scan.hpp>
@@ -53,15 +54,16 @@ constexpr int kFinThreads = 1024;  // hub_bucket_merge workgroup
 constexpr int kFinCap = 16384;     // LDS hash slots of hub_bucket_merge (128 KB)
 constexpr int kFinLds = 8192;      // buckets up to this many entries merge in LDS
 constexpr int kMaxBuckets = 2048;  // buckets per hub: min(kBucketsPerChunk x chunks, kMaxBuckets)
-constexpr int kBucketsPerChunk = 4;  // ~1000 entries per (hub, bucket): the small merge kernel takes most
-constexpr int kTinyThreads = 256;    // tiny bucket merge: <= kTinyMax entries in 16 KB of LDS
-constexpr int kTinyCap = 2048;
-constexpr int kTinyMax = 1024;
+constexpr int kBucketsPerChunk = 4;  // ~1000 entries per (hub, bucket)
 constexpr int kSmallThreads = 512;   // small bucket merge: <= kSmallMax entries in 32 KB of LDS
 constexpr int kSmallCap = 4096;
 constexpr int kSmallMax = 2048;
-constexpr int kHubStage = 256;       // merge tasks of hubs of at most this many chunks stage the
-                                     // chunks' segment offsets in LDS
+// Sub-rounds of at most kHubJoin chunks and mid-size hubs (two workgroups of kHubThreads per CU)
+// take the mid-size hubs along in the chunk kernel's launch.
+constexpr int kHubJoin = 512;
+constexpr int kHubStage = 256;       // merge tasks of hubs of at most this many chunks sum the
+                                     // chunks' entry counts themselves and keep the offsets in LDS
+static_assert(kHubStage <= kSmallThreads, "a thread per chunk");
 
 struct Cand {
     int conn;
@@ -1035,33 +1037,38 @@ __global__ __launch_bounds__(THREADS) void propose_hub_chunk(
 }
 
 // Merge of one (multi-chunk hub, bucket) task: the bucket's entries of all chunks of the hub are
-// summed in an LDS hash (or, past kFinLds entries, in the hub's global table, filtering by
-// bucket); the bucket's best candidate and, for the bucket of the own label, conn(own) are left
-// in bres / bown. Three sizes: LEVEL 0 (256 threads, 16 KB of LDS, eight per CU) takes every
-// task of the sub-round and queues those of more than kTinyMax entries for LEVEL 1 (512 threads,
-// 32 KB), which queues those of more than kSmallMax for LEVEL 2 (1024 threads, 128 KB); the
-// queued levels grid-stride over their queue.
-template <LpMode M, int LEVEL>
-__global__ __launch_bounds__(LEVEL == 0 ? kTinyThreads : (LEVEL == 1 ? kSmallThreads : kFinThreads))
+// summed in an LDS hash (or in the hub's global table, filtering by bucket); the bucket's best
+// candidate and, for the bucket of the own label, conn(own) are left in bres / bown. The small
+// form (512 threads, 32 KB of LDS, four per CU) takes every task of the sub-round; those of more
+// than kSmallMax entries use the global table, or are queued for the big form (1024 threads,
+// 128 KB, up to kFinLds entries, grid-stride over the queue) where a hub's buckets have reached
+// kMaxBuckets, so that tasks are larger than ~1000 entries by size and not by bad luck.
+// One launch where there were four (a scan of the counts over all tasks, 256-thread merges, 512
+// and 1024-thread merges of their queues): measured in kahip_partition, together with the
+// mid-size hubs' place in the chunk launch: R-MAT 2^17, k = 8 20.8 -> 19.0 ms (coarsening 9.1 -> 7.3),
+// R-MAT 2^20, k = 16 coarsening 24.4 -> 22.8 ms.
+template <LpMode M, bool BIG>
+__global__ __launch_bounds__(BIG ? kFinThreads : kSmallThreads)
 void hub_bucket_merge(
     LpArgs a, int n_tasks, const int4* __restrict__ tmap, const int2* __restrict__ tsub,
-    const int* __restrict__ posT, const int* __restrict__ chunk_prefix,
-    const long long* __restrict__ offm_base, const int* __restrict__ offm,
-    const int2* __restrict__ partials, const long long* __restrict__ tab_off,
-    int* __restrict__ gkey, int* __restrict__ gval, Cand* __restrict__ bres,
-    int* __restrict__ bown, uint8_t* __restrict__ fb, const int* __restrict__ in_q,
-    const int* __restrict__ in_n, int* __restrict__ out_q, int* __restrict__ out_n) {
-    constexpr int THREADS = LEVEL == 0 ? kTinyThreads : (LEVEL == 1 ? kSmallThreads : kFinThreads);
-    constexpr int CAP = LEVEL == 0 ? kTinyCap : (LEVEL == 1 ? kSmallCap : kFinCap);
-    constexpr int MAXE = LEVEL == 0 ? kTinyMax : kSmallMax;  // queued beyond (levels 0, 1)
-    static_assert(2 * MAXE <= CAP && 2 * kFinLds <= kFinCap, "merge tables fill at most half");
+    const int* __restrict__ cntT, const int* __restrict__ posT,
+    const int* __restrict__ chunk_prefix, const long long* __restrict__ offm_base,
+    const int* __restrict__ offm, const int2* __restrict__ partials,
+    const long long* __restrict__ tab_off, int* __restrict__ gkey, int* __restrict__ gval,
+    Cand* __restrict__ bres, int* __restrict__ bown, uint8_t* __restrict__ fb,
+    int* __restrict__ queue, int* __restrict__ queued) {
+    constexpr int THREADS = BIG ? kFinThreads : kSmallThreads;
+    constexpr int CAP = BIG ? kFinCap : kSmallCap;
+    constexpr int MAXE = BIG ? kFinLds : kSmallMax;
+    static_assert(2 * MAXE <= CAP, "merge tables fill at most half");
     __shared__ int K[CAP];
     __shared__ int V[CAP];
     __shared__ int spre[kHubStage + 1];  // task offsets of the chunks' bucket segments
     __shared__ int sstart[kHubStage];    // the segments' starts in their chunks' partials
-    const int n_iter = LEVEL == 0 ? n_tasks : *in_n;
+    __shared__ int wsum[kHubStage / 64];
+    const int n_iter = BIG ? *queued : n_tasks;
     for (int it = blockIdx.x; it < n_iter; it += gridDim.x) {
-        const int task = LEVEL == 0 ? it : in_q[it];
+        const int task = BIG ? queue[it] : it;
         const int4 tm = tmap[task];  // {first count index, one past the last, hub index, node}
         const int2 ts = tsub[task];  // {multi-chunk hub index, bucket | buckets << 16}
         const int mi = ts.x;
@@ -1073,29 +1080,45 @@ void hub_bucket_merge(
         }
         const int P = ts.y >> 16;
         const int b = ts.y & 0xffff;
-        const int r0 = posT[tm.x];
-        const int r1 = posT[tm.y];
-        const int total = r1 - r0;
-        if (LEVEL < 2 && total > MAXE) {
-            if (threadIdx.x == 0) out_q[atomicAdd(out_n, 1)] = task;
+        const int nch = tm.y - tm.x;
+        const int* offs = offm + offm_base[gi] + b;
+        const bool staged = nch <= kHubStage;  // uniform
+        int r0 = 0, total;
+        if (staged) {
+            const int c = threadIdx.x;
+            const int cnt = c < nch ? cntT[tm.x + c] : 0;
+            if (c < nch) sstart[c] = offs[(long long)c * (P + 1)];
+            int incl = cnt;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(incl, o, 64);
+                if ((c & 63) >= o) incl += y;
+            }
+            if (c < kHubStage && (c & 63) == 63) wsum[c >> 6] = incl;
+            __syncthreads();
+            if (c < nch) {
+                for (int w = 0; w < c >> 6; ++w) incl += wsum[w];
+                spre[c + 1] = incl;
+            }
+            if (c == 0) spre[0] = 0;
+            __syncthreads();
+            total = spre[nch];
+        } else {  // the sub-round's scan of the counts
+            r0 = posT[tm.x];
+            total = posT[tm.y] - r0;
+        }
+        if (!BIG && total > MAXE && queue) {
+            if (threadIdx.x == 0) queue[atomicAdd(queued, 1)] = task;
             __syncthreads();
             continue;
         }
-        const bool in_lds = LEVEL < 2 || total <= kFinLds;
+        const bool in_lds = total <= MAXE;
         const int deg = a.xadj[v + 1] - a.xadj[v];
         // The task's entries are read where the hub's chunks wrote them: chunk c holds entries
-        // [pre(c), pre(c + 1)) of the task, pre(c) = posT[tm.x + c] - r0, in its partials at
+        // [pre(c), pre(c + 1)) of the task, pre the prefix of their counts, in its partials at
         // offm[offm_base[gi] + c (P + 1) + b]; the chunk of entry i is the largest c with
         // pre(c) <= i (empty segments are skipped).
-        const int nch = tm.y - tm.x;
         const long long c0 = chunk_prefix[gi];
-        const int* offs = offm + offm_base[gi] + b;
-        const bool staged = nch <= kHubStage;  // uniform
-        if (staged)
-            for (int c = threadIdx.x; c <= nch; c += THREADS) {
-                spre[c] = posT[tm.x + c] - r0;
-                if (c < nch) sstart[c] = offs[(long long)c * (P + 1)];
-            }
         long long cap = CAP;
         int* TK = K;
         int* TV = V;
@@ -2308,13 +2331,17 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
         multi_base_[sr] = (int)multi.size();
         task_base_[sr] = (int)tasks.size();
         int c = 0, t = 0;
-        (void)0;
         mid_base_[sr] = mids;
         mid_edges_[sr] = 0;
+        hub_wide_[sr] = hub_capped_[sr] = false;
+        long long units = 0;  // chunks and mid-size hubs
+        for (int i = 0; i < hub_n_[sr]; ++i)
+            units += (deg[hub_base_[sr] + i] + kHubChunk - 1) / kHubChunk;
+        const bool join = units <= kHubJoin;
         for (int i = 0; i < hub_n_[sr]; ++i) {
             const int d = deg[hub_base_[sr] + i];
             prefix.push_back(c);
-            if (d <= kMidChunk) {  // the mid-size kernel, no chunk of the big one
+            if (d <= kMidChunk && !join) {  // the mid-size kernel, no chunk of the big one
                 midpos[hub_base_[sr] + i] = mids++ - mid_base_[sr];
                 mid_edges_[sr] += d;
                 continue;
@@ -2323,6 +2350,8 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
             c += nch;
             if (nch > 1) {
                 const int P = std::min(kBucketsPerChunk * nch, kMaxBuckets);
+                hub_wide_[sr] |= nch > kHubStage;
+                hub_capped_[sr] |= P < kBucketsPerChunk * nch;
                 long long cap = 64;
                 while (cap < 2LL * d) cap <<= 1;
                 toff[hub_base_[sr] + i] = hub_total_;
@@ -2361,12 +2390,14 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
     ct_base_.reserve(hubs);
     cnt_t_.reserve(ct_total);
     pos_t_.reserve(ct_total);
-    fill_async(cnt_t_.p, ct_total, 0, s);  // sentinels stay zero
+    if (std::any_of(hub_wide_, hub_wide_ + S, [](bool w) { return w; }))
+        fill_async(cnt_t_.p, ct_total, 0, s);  // sentinels stay zero
     KH_CHECK(hipMemcpyAsync(ct_base_.p, ctb.data(), sizeof(int) * hubs, hipMemcpyHostToDevice,
                             s));
     {
         size_t bytes = 0, need = 0;
         for (int sr = 0; sr < S; ++sr) {
+            if (!hub_wide_[sr]) continue;
             KH_CHECK(rocprim::exclusive_scan(nullptr, bytes, cnt_t_.p, pos_t_.p, 0,
                                              (size_t)ct_sr_size_[sr] + 1, rocprim::plus<int>(), s));
             need = std::max(need, bytes);
@@ -2377,7 +2408,6 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
     bres_.reserve(max_tasks);
     bown_.reserve(max_tasks);
     big_tasks_.reserve(max_tasks);
-    mid_tasks_.reserve(max_tasks);
     fb_.reserve(max_multi);
     fill_async(fb_.p, max_multi, (uint8_t)0, s);
     KH_CHECK(hipMemcpyAsync(chunk_prefix_.p, prefix.data(), sizeof(int) * prefix.size(),
@@ -2701,25 +2731,29 @@ void LpWorkspace::propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool increm
         const int nm = hub_multi_n_[sr];
         Cand* br = reinterpret_cast<Cand*>(bres_.p);
         const int nt = hub_tasks_[sr];
-        // bucket-major positions, relative to this sub-round's block of counts
-        size_t sb = scan_tmp_bytes_;
-        KH_CHECK(rocprim::exclusive_scan(scan_tmp_.p, sb, cnt_t_.p + ct_sr_base_[sr], pos_t_.p + ct_sr_base_[sr], 0, (size_t)ct_sr_size_[sr] + 1, rocprim::plus<int>(), s));
-        const int* pt = pos_t_.p;
+        if (hub_wide_[sr]) {
+            // bucket-major positions, relative to this sub-round's block of counts
+            size_t sb = scan_tmp_bytes_;
+            KH_CHECK(rocprim::exclusive_scan(scan_tmp_.p, sb, cnt_t_.p + ct_sr_base_[sr], pos_t_.p + ct_sr_base_[sr], 0, (size_t)ct_sr_size_[sr] + 1, rocprim::plus<int>(), s));
+        }
         const int* cp = chunk_prefix_.p + chunk_base_[sr];
-        int* bt = big_tasks_.p;
-        int* nbt = ctl_.p + kCtlBig + (r * S + sr);
-        int* mt = mid_tasks_.p;
-        int* nmt = ctl_.p + kCtlMid + (r * S + sr);
+        int* queue = hub_capped_[sr] ? big_tasks_.p : nullptr;
+        int* queued = ctl_.p + kCtlBig + (r * S + sr);
+        const auto merge = [&](auto kernel, int grid, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, a, nt, tm, tsb, cnt_t_.p, pos_t_.p, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, queue, queued);
+        };
+        const auto decide = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
+        };
+        const int big = std::min(nt, 256);
         if (cl) {
-            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
-            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
-            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Cluster, 2>), dim3(std::min(nt, 256)), dim3(kFinThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, bt, nbt, nullptr, nullptr);
-            hipLaunchKernelGGL((hub_decide<LpMode::Cluster>), dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
+            merge(hub_bucket_merge<LpMode::Cluster, false>, nt, kSmallThreads);
+            if (queue) merge(hub_bucket_merge<LpMode::Cluster, true>, big, kFinThreads);
+            decide(hub_decide<LpMode::Cluster>);
         } else {
-            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 0>), dim3(nt), dim3(kTinyThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, nullptr, nullptr, mt, nmt);
-            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 1>), dim3(std::min(nt, 1024)), dim3(kSmallThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, mt, nmt, bt, nbt);
-            hipLaunchKernelGGL((hub_bucket_merge<LpMode::Refine, 2>), dim3(std::min(nt, 256)), dim3(kFinThreads), 0, s, a, nt, tm, tsb, pt, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, bt, nbt, nullptr, nullptr);
-            hipLaunchKernelGGL((hub_decide<LpMode::Refine>), dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
+            merge(hub_bucket_merge<LpMode::Refine, false>, nt, kSmallThreads);
+            if (queue) merge(hub_bucket_merge<LpMode::Refine, true>, big, kFinThreads);
+            decide(hub_decide<LpMode::Refine>);
         }
     }
 }

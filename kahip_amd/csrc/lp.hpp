@@ -112,10 +112,9 @@ private:
     void fetch(hipStream_t s);  // host_ctl_ of the last run
     Mail mail_;
     // Counters of a run: {traversed edges in 64 spread 64-bit counters, moves per round, lengths
-    // of the hub merges' big and middle task queues per sub-round, error flag}
+    // of the hub merges' big task queues per sub-round, error flag}
     static constexpr int kCtlMoves = 128, kCtlBig = kCtlMoves + kMaxRounds,
-                         kCtlMid = kCtlBig + kMaxSub * kMaxRounds,
-                         kCtlErr = kCtlMid + kMaxSub * kMaxRounds, kCtlInts = kCtlErr + 1;
+                         kCtlErr = kCtlBig + kMaxSub * kMaxRounds, kCtlInts = kCtlErr + 1;
     DevBuf<int> ctl_;
     int host_ctl_[kCtlBig + 1] = {};  // the traversed edges, the moves, the error flag
     bool fetched_ = false;
@@ -142,6 +141,8 @@ private:
     int hub_tasks_[kMaxSub] = {};   // (hub, bucket) tasks per sub-round
     int ct_sr_base_[kMaxSub] = {};  // bucket-major count block of each sub-round
     int ct_sr_size_[kMaxSub] = {};
+    bool hub_wide_[kMaxSub] = {};    // a hub of more than kHubStage chunks: the counts are scanned
+    bool hub_capped_[kMaxSub] = {};  // a hub at kMaxBuckets: large tasks go to the big merge
     size_t scan_tmp_bytes_ = 0;
     DevBuf<int> hub_deg_, chunk_prefix_, multi_;
     DevBuf<long long> tab_off_, tab_cap_;
@@ -149,7 +150,7 @@ private:
     DevBuf<int> ct_base_, cnt_t_, pos_t_;
     DevBuf<char> scan_tmp_;
     DevBuf<long long> offm_base_;
-    DevBuf<int> offm_, task_prefix_, bown_, big_tasks_, mid_tasks_;
+    DevBuf<int> offm_, task_prefix_, bown_, big_tasks_;
     DevBuf<int4> bres_;
     DevBuf<int4> cmap_, tmap_, mmap_;  // hub-chunk, (hub, bucket) task, mid-size hub descriptors
     DevBuf<int> midpos_;
