@@ -637,8 +637,12 @@ struct ClusterLists {
     int count[kNumBins - 1];
     const int* dcount;  // lengths on the device (a compacted sub-round), else nullptr
 };
+// Turnover of a sub-round without an admission launch (kTurnNodes): the workgroups past the lists'
+// copy the label weights to the array that the application updates and clear the next sub-round's
+// admission scratch, kTurnItems labels a thread.
+constexpr int kTurnItems = 4;
 template <int IT, bool WAVES, bool SETTLE>
-__global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F) {
+__global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F, Turnover T) {
     select_copy(a);
     constexpr LpMode C = LpMode::Cluster;
     constexpr int N = kNumBins - 1;
@@ -650,6 +654,18 @@ __global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F
         cnt[b] = SETTLE && F.dcount ? F.dcount[b] : F.count[b];
         nvb[b] = (cnt[b] + NPB[b] - 1) / NPB[b];
         total += nvb[b];
+    }
+    if (!SETTLE && (int)blockIdx.x >= total) {  // uniform
+        const int i0 = ((int)blockIdx.x - total) * kBlock * kTurnItems + threadIdx.x;
+#pragma unroll
+        for (int j = 0; j < kTurnItems; ++j) {
+            const int i = i0 + j * kBlock;
+            if (i >= T.n) break;
+            T.size[i] = a.size[i];
+            T.inc[i] = 0;
+            T.top[i] = 0ull;
+        }
+        return;
     }
     unsigned long long edges = 0;
     for (int t = blockIdx.x; t < total; t += gridDim.x) {  // one pass over whole lists
@@ -1305,6 +1321,42 @@ __global__ __launch_bounds__(kApplyThreads) void apply_moves(LpArgs a,
         const int t = a.prop_t[a.base + i];
         int from;
         if (t >= 0) mine += apply_one<LpMode::Cluster>(a, a.base + i, list[i], t, &from);
+    }
+    if (mine) atomicAdd(&block_moves, mine);
+    __syncthreads();
+    if (threadIdx.x == 0 && block_moves) atomicAdd(a.moves, block_moves);
+}
+
+// Admission and application in one launch: the weights that admission reads (a.size, a.inc, a.top)
+// stay as they are, the moves go to the next sub-round's label weights (`size`, a copy of a.size),
+// and the scratch is cleared by the next sub-round's proposals (Turnover). For graphs of up to
+// kTurnNodes nodes, whose sub-rounds are bound by their launches: copying and clearing 20 bytes a
+// label takes as long as the launch beyond (R-MAT 2^20: the same either way). Measured: RGG 2^22,
+// k = 2 13.55 -> 13.17 ms (its coarse levels), R-MAT 2^17, k = 8 18.7 -> 18.3 ms, kahip_lp_cluster of
+// R-MAT 2^15 1.97 -> 1.88 ms.
+constexpr int kTurnNodes = 1 << 18;
+__global__ __launch_bounds__(kApplyThreads) void admit_apply(LpArgs a, int* __restrict__ size,
+                                                             const int* __restrict__ list,
+                                                             int count) {
+    __shared__ int block_moves;
+    if (threadIdx.x == 0) block_moves = 0;
+    __syncthreads();
+    int mine = 0;
+    for (unsigned i = blockIdx.x * kApplyThreads + threadIdx.x; i < (unsigned)count;
+         i += gridDim.x * kApplyThreads) {
+        const int pos = a.base + i;
+        const int t = a.prop_t[pos];
+        if (t < 0) continue;
+        const int v = list[i], w = a.vwgt[v], own = a.label[v];
+        const long long st = a.size[t], bt = bound_of(a, t);
+        a.prop_t[pos] = -1;
+        if (st + (long long)a.inc[t] < bt ||
+            (a.top[t] == prio_key(a.prop_gain[pos], v) && st + w < bt)) {
+            atomicSub(&size[own], w);
+            atomicAdd(&size[t], w);
+            a.label[v] = t;
+            ++mine;
+        }
     }
     if (mine) atomicAdd(&block_moves, mine);
     __syncthreads();
@@ -2037,6 +2089,11 @@ __global__ void fill_i32(int* p, long long n, int value) {
     if (i < n) p[i] = value;
 }
 
+__global__ void copy_i32(int* __restrict__ to, const int* __restrict__ from, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) to[i] = from[i];
+}
+
 __global__ void fill_u64(unsigned long long* p, long long n, unsigned long long value) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = value;
@@ -2570,6 +2627,17 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         fill_async(ccount_.p, rounds * nseg, 0, s);
         act = active_.p;
     }
+    // admission and application in one launch; the label weights change places each sub-round
+    // (run_copies() runs single rounds one after the other on one preparation's scratch)
+    const bool turn = cl && !settle && rounds > 1 && g.n <= kTurnNodes;
+    int* turn_size = nullptr;
+    int* turn_inc = nullptr;
+    unsigned long long* turn_top = nullptr;
+    if (turn) {
+        turn_size = size2_.reserve(g.n);
+        turn_inc = inc2_.reserve(g.n);
+        turn_top = top2_.reserve(g.n);
+    }
     int* cnow = ccount_.p;  // list lengths of the frontier, cleared by the tail before last
     int* cnext = cnow + nseg;
     while (r < rounds) {
@@ -2640,16 +2708,26 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
                 // algorithmic bytes: 12 B per traversed edge (target, weight, label gather) and
                 // 16 B per node (two offsets, weight, own label); label weights are O(moved).
                 ProfScope ps(prof, base + "_propose_lists", 12.0 * (double)ledges + 16.0 * (double)lnodes, ledges, s);
-                launch_lists(a, sr, 1, nullptr, false, s);
+                for (int b = 0; b < kNumBins; ++b) sub_total += host_counts[sr * kNumBins + b];
+                if (sub_total == 0) continue;
+                const Turnover T{turn ? g.n : 0, turn_size, turn_inc, turn_top};
+                launch_lists(a, sr, 1, nullptr, false, T, s);
             }
             const int cnt = host_counts[sr * kNumBins + kNumBins - 1];
-            for (int b = 0; b < kNumBins; ++b) sub_total += host_counts[sr * kNumBins + b];
+            if (!cl)
+                for (int b = 0; b < kNumBins; ++b) sub_total += host_counts[sr * kNumBins + b];
             if (cnt > 0 && !fused_hubs) propose_hubs(mode, a, r, sr, incremental, s, prof, base);
             if (sub_total == 0) continue;
             const int gm = grid_for(sub_total, 256);
             const int* sub_list = lists_.p + host_offsets[sr * kNumBins];  // bins are contiguous
             ProfScope ps(prof, base + "_admit_apply", 0.0, 0, s);
-            if (cl) {
+            if (turn) {
+                a.base = host_offsets[sr * kNumBins];
+                hipLaunchKernelGGL(admit_apply, dim3(std::min(grid_for(sub_total, kApplyThreads), kApplyGrid)), dim3(kApplyThreads), 0, s, a, turn_size, sub_list, sub_total);
+                std::swap(a.size, turn_size);
+                std::swap(a.inc, turn_inc);
+                std::swap(a.top, turn_top);
+            } else if (cl) {
                 a.base = host_offsets[sr * kNumBins];
                 hipLaunchKernelGGL(admit_moves, dim3(gm), dim3(256), 0, s, a, sub_list, sub_total);
                 hipLaunchKernelGGL(apply_moves, dim3(std::min(grid_for(sub_total, kApplyThreads), kApplyGrid)), dim3(kApplyThreads), 0, s, a, sub_list, sub_total);
@@ -2676,6 +2754,8 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         }
         ++r;
     }
+    if (a.size != size)  // an odd number of turnovers
+        hipLaunchKernelGGL(copy_i32, dim3(grid_for(g.n, 256)), dim3(256), 0, s, size, a.size, g.n);
     KH_CHECK(hipGetLastError());
 }
 
@@ -2794,7 +2874,7 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
     int total = 0;
     for (int b = 0; b < kNumBins - 1; ++b) total += host_counts[b];
     if (total == 0) return;
-    launch_lists(a, 0, copies, nullptr, false, s);
+    launch_lists(a, 0, copies, nullptr, false, Turnover{}, s);
     const dim3 grid(grid_for(total, 256), copies);
     hipLaunchKernelGGL(admit_moves, grid, dim3(256), 0, s, a, lists_.p, total);
     hipLaunchKernelGGL(apply_moves, dim3(std::min(grid_for(total, kApplyThreads), kApplyGrid), copies),
@@ -2805,7 +2885,7 @@ void LpWorkspace::run_copies(const DGraph& g, int* label, int* size, int bound,
 // The clustering proposals of sub-round sr's lists (not the hub list); dcount: compacted to these
 // lengths; settle: also flag the nodes that are not settled.
 void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, const int* dcount, bool settle,
-                               hipStream_t s) {
+                               const Turnover& T, hipStream_t s) {
     ClusterLists F{};
     F.dcount = dcount;
     const int items = bins_.group_items;
@@ -2818,10 +2898,11 @@ void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, const int* d
         const int per = b < 2 ? items * (kBlock / 8) : b < 4 ? items * (kBlock / 16) : kBlock / 64;
         blocks += grid_for(host_counts[l], per);
     }
+    blocks += grid_for(T.n, kBlock * kTurnItems);
     if (blocks == 0) return;
     const dim3 grid(dcount ? std::min(blocks, kFrontierGrid) : blocks, copies);
     const auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, a, F);
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, a, F, T);
     };
     const bool waves = F.count[kNumBins - 2] > 0;
     switch (items * 4 + (waves ? 1 : 0) + (settle ? 2 : 0)) {
@@ -2851,7 +2932,7 @@ void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStre
         hipLaunchKernelGGL(compact_active, dim3(grid_for(total, 256 * kCompactItems)), dim3(256), 0,
                            s, lists_.p, offsets_.p + l0, kNumBins, host_offsets[l0], total,
                            a.next_active, 1, dcount, clists_.p);
-    launch_lists(a, sr, 1, dcount, true, s);
+    launch_lists(a, sr, 1, dcount, true, Turnover{}, s);
     SubLists L{};
     for (int b = 0; b < kNumBins; ++b) {
         L.list[b] = (dcount ? clists_.p : lists_.p) + host_offsets[l0 + b];

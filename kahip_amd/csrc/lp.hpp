@@ -62,6 +62,14 @@ struct TailArgs {
     int seq;
 };
 
+// Arrays of the next clustering sub-round that a proposal launch makes ready.
+struct Turnover {
+    int n = 0;  // labels; 0: none
+    int* size = nullptr;
+    int* inc = nullptr;
+    unsigned long long* top = nullptr;
+};
+
 class LpWorkspace {
 public:
     // Bins the nodes of g into per-(sub-round, degree bin) lists and sizes the scratch for
@@ -104,7 +112,7 @@ private:
     void build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipStream_t s,
                      const uint8_t* include, int copies);
     void launch_lists(const LpArgs& a, int sr, int copies, const int* dcount, bool settle,
-                      hipStream_t s);
+                      const Turnover& T, hipStream_t s);
     void settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s);
     void propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool incremental, hipStream_t s,
                       Profiler* prof, const std::string& base);
@@ -163,6 +171,8 @@ private:
     DevBuf<uint8_t> prop_ok_;
     DevBuf<int> inc_, out_;
     DevBuf<unsigned long long> top_, dtop_;
+    DevBuf<int> size2_, inc2_;  // of every other sub-round of a clustering with turnover
+    DevBuf<unsigned long long> top2_;
     DevBuf<uint8_t> active_, next_active_;
     DevBuf<int> hub_key_, hub_val_;
     DevBuf<int> dense_off_, dense_cnt_;  // chunked dense refinement hubs: per-hub counters

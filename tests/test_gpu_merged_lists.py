@@ -54,3 +54,15 @@ def test_tile_shapes(items, small):
                           wave_small=small)
     want, _ = mirror_partition(x, a, vw, ew, 4, 0.03, 2, stop_factor=50)
     assert np.array_equal(part, want)
+
+
+@pytest.mark.parametrize("n", [262142, 262144, 262146])
+@pytest.mark.parametrize("rounds,subrounds", [(1, 1), (2, 1), (3, 1), (3, 3), (2, 8)])
+def test_turnover(n, rounds, subrounds):
+    """Around the largest graph whose admission and application share a launch, with odd and even
+    numbers of sub-rounds."""
+    x, a, vw, ew = regular(n, 6, 3, 3)
+    got = K.lp_cluster(x, a, vw, ew, 30, rounds, subrounds, 4)
+    want = O.lp_cluster_sync(x, a, vw, ew, 30, rounds, subrounds, 4)
+    assert np.array_equal(got[2], want[2][:rounds]) and got[1] == want[1]
+    assert np.array_equal(got[0], want[0])
