@@ -68,6 +68,14 @@ __device__ inline I probe_claim(int* K, I cap, int key) {
     return probe_claim(K, cap, key, fresh);
 }
 
+#ifdef __HIP__
+// LDS accesses of a wave before this are done, for its lanes, before those after it.
+__device__ __attribute__((always_inline)) inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+#endif
+
 // Device error flags (one int per workspace, cleared before its kernels run, read by the host
 // after them).
 constexpr int kErrProbe = 1;  // a hash table probe found no slot (sizing invariant broken)

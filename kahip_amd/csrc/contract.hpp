@@ -37,13 +37,15 @@ private:
     void scan_i32(const int* in, int* out, int n, hipStream_t s);
     DevBuf<char> scan_tmp_;
     DevBuf<int> leader_, flag_, newid_;
-    DevBuf<int> cnt_, fdeg_, moff_, tpos_, cdeg_, members_, tq_, tw_;
-    DevBuf<int> iota_, mkeys_;               // radix sort of the node ids by cluster
+    DevBuf<int> fdeg_, moff_, tpos_, cdeg_, members_, tq_, tw_;
+    DevBuf<int> mkeys_;                      // sorted clusters of the members
+    DevBuf<unsigned long long> mrec_, mpre_; // members' {degree, weight} and their scan
+    DevBuf<int> over_;                       // rows left over by rows_few
     DevBuf<int> rlist_[5];                   // rows of the thread tier and the four LDS tiers
     DevBuf<int> ovl2_list_, ctl_;            // rows of the global tier; list lengths, error flag
     Mail mail_;
     DevBuf<long long> hcap_, hoff_;
-    DevBuf<int> gchunk_prefix_, mdeg_, mpre_, ofd_;
+    DevBuf<int> gchunk_prefix_, ofd_;
     DevBuf<int> hk_, hv_, hm_;
     DevBuf<int> gtask_prefix_, goffm_, gcnt_, gpos_, gbig_, gnbig_;
     DevBuf<long long> goffm_base_, gct_base_;

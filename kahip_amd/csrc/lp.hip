@@ -518,10 +518,6 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
 // dense counter per label when the labels are the k blocks of the refinement and k is small.
 // The node's table belongs to its wave, whose LDS operations are in order: no barriers.
 constexpr int kWaveEdges = kWaveCap / 2 / 64;  // edges per lane at the largest degree
-__device__ __attribute__((always_inline)) inline void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 // EPL: edges per lane, 64 x EPL >= degree.
 template <LpMode M, bool DENSE, int EPL, bool SETTLE>
 __device__ __attribute__((always_inline)) inline void wave_node(const LpArgs& a, int pos, int v,
@@ -1742,8 +1738,7 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
 #pragma unroll
                     for (int j = 0; j < EPL; ++j)
                         if (labs[j] >= 0) atomicAdd(&V[labs[j]], ws[j]);
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
+                    wave_lds_order();
                     const int nw = a.vwgt[v];
                     int conn_own = 0;
                     Cand c{-1, 0u, 0x7fffffff, 0};
@@ -1763,8 +1758,7 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
                     }
                     conn_own = reduce_max<64>(conn_own);
                     reduce_cand<64>(c);
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
+                    wave_lds_order();
 #pragma unroll
                     for (int j = 0; j < EPL; ++j)
                         if (labs[j] >= 0) V[labs[j]] = 0;
