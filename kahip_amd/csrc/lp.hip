@@ -47,6 +47,7 @@ constexpr int kHubThreads = 1024;      // clustering hub chunks (4 edges per thr
 constexpr int kMidThreads = 256;       // hubs of kMidChunk edges or fewer (4 edges per thread)
 constexpr int kMidChunk = 1024;
 constexpr int kHubDenseThreads = 512;  // refinement hub chunks (8 edges per thread)
+constexpr int kLongRow = 1024;    // refinement: moved rows beyond are marked by all workgroups
 constexpr int kHubDense = 4096;   // dense LDS counters per hub (refinement, k <= 4096)
 constexpr long long kAllHubCounters = 1LL << 28;  // counters (ints) for incremental hubs
 constexpr int kHubDenseSlots = 12288;  // dynamic LDS counters (48 KB): min(8, slots / k) copies
@@ -1259,14 +1260,15 @@ __device__ inline void filter_one(const LpArgs& a, int pos, int v, int t) {
     }
 }
 
-__device__ inline void admit_one(const LpArgs& a, int pos, int v, int t) {
-    if (!a.prop_ok[pos]) return;
+__device__ inline bool admit_one(const LpArgs& a, int pos, int v, int t) {
+    if (!a.prop_ok[pos]) return false;
     const int w = a.vwgt[v];
     const long long st = a.size[t];
     const long long bt = bound_of(a, t);
     const bool ok = st + (long long)a.inc[t] < bt ||
                     (a.top[t] == prio_key(a.prop_gain[pos], v) && st + w < bt);
     if (!ok) a.prop_ok[pos] = 0;
+    return ok;
 }
 
 // Applies the proposal of list position pos (node v to label t) if it is admitted and clears its
@@ -1412,6 +1414,7 @@ __global__ __launch_bounds__(256) void filter_departures_sub(LpArgs a, SubLists 
     }
 }
 
+// (also lists the admitted moves of long rows, a.big)
 __global__ __launch_bounds__(256) void admit_moves_sub(LpArgs a, SubLists L) {
     int cnt[kNumBins];
     const int total = sub_lengths(L, cnt);
@@ -1420,7 +1423,11 @@ __global__ __launch_bounds__(256) void admit_moves_sub(LpArgs a, SubLists L) {
         int index;
         const int pos = sub_entry(L, cnt, i, &list, &index);
         const int t = a.prop_t[pos];
-        if (t >= 0) admit_one(a, pos, list[index], t);
+        if (t < 0) continue;
+        const int v = list[index];
+        if (!admit_one(a, pos, v, t) || !a.big) continue;
+        const int beg = a.xadj[v], deg = a.xadj[v + 1] - beg;
+        if (deg > kLongRow) a.big[atomicAdd(a.n_big, 1)] = make_int4(beg, deg, a.label[v], t);
     }
 }
 
@@ -1428,12 +1435,17 @@ __global__ __launch_bounds__(256) void admit_moves_sub(LpArgs a, SubLists L) {
 // hub neighbours with kept counters have them moved along. The rows of a step's movers are one
 // range of edges over the workgroup's threads, kApplyEdges apiece in flight (an edge is a chain
 // of three gathers: neighbour, hub slot, counter): with a lane per row, a row of 64 entries was
-// 64 such chains one after the other. Measured, R-MAT 2^20, k = 16: 58 -> 37 us
-// on average (the rest: the atomics on the hubs' counters), R-MAT 2^17 16 -> 10 us.
+// 64 such chains one after the other. Measured, R-MAT 2^20, k = 16: 58 -> 37 us on average, R-MAT
+// 2^17 16 -> 10 us.
 // Clustering: flags the moved nodes and those neighbours that a move may unsettle (a neighbour in
 // the target cluster stays settled, unless the edge's weight is negative). A neighbour moved by
 // the same launch is flagged by its own move, so it does not matter which of its labels is read.
+// Rows of more than kLongRow edges (one pass of the workgroup) are listed by the admission and
+// spread over all workgroups in pieces: a moved hub's row, up to 100 passes one after the other, was
+// the launch's time. Measured, R-MAT 2^20, k = 16: 26 -> 12 us on average, 2^17 10.7 -> 9.0 us.
+// (Summing the counter updates per workgroup in LDS first: 30 us; they do not wait for each other.)
 constexpr int kApplyEdges = 4;
+static_assert(kLongRow == kApplyEdges * kBlock, "a piece of a long row is a pass of the workgroup");
 template <LpMode M>
 __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) {
     __shared__ int block_moves;
@@ -1444,6 +1456,26 @@ __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) 
     int cnt[kNumBins];
     const int total = sub_lengths(L, cnt);
     unsigned long long edges = 0;
+    // neighbours u at entries e (-1: none) of rows moved between the labels
+    const auto mark = [&](const int (&e)[kApplyEdges], const int (&u)[kApplyEdges],
+                          const int (&from)[kApplyEdges], const int (&to)[kApplyEdges]) {
+        int slot[kApplyEdges];
+#pragma unroll
+        for (int j = 0; j < kApplyEdges; ++j) {
+            slot[j] = -1;
+            if (e[j] >= 0) {
+                a.next_active[u[j]] = 1;
+                if (a.hub_cnt) slot[j] = a.hub_slot[u[j]];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kApplyEdges; ++j)
+            if (slot[j] >= 0) {
+                const int w = a.adjwgt[e[j]];
+                atomicSub(&a.hub_cnt[slot[j] + from[j]], w);
+                atomicAdd(&a.hub_cnt[slot[j] + to[j]], w);
+            }
+    };
     for (int base = blockIdx.x * kBlock; base < total; base += gridDim.x * kBlock) {  // uniform
         if (threadIdx.x == 0) claimed = 0ull;
         __syncthreads();
@@ -1457,7 +1489,10 @@ __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) 
             int from;
             if (apply_one<M>(a, pos, v, t, &from)) {
                 if (M == LpMode::Cluster) a.next_active[v] = 1;
-                const int beg = a.xadj[v], deg = a.xadj[v + 1] - beg;
+                const int beg = a.xadj[v], row = a.xadj[v + 1] - beg;
+                const bool lng = M == LpMode::Refine && row > kLongRow;
+                if (lng) edges += (unsigned long long)row;
+                const int deg = lng ? 0 : row;  // a long row is marked below
                 // index and first edge from one atomic: the movers' edges ascend with k
                 const unsigned long long at =
                     atomicAdd(&claimed, (1ull << 32) | (unsigned long long)deg);
@@ -1504,24 +1539,54 @@ __global__ __launch_bounds__(kBlock) void apply_moves_sub(LpArgs a, SubLists L) 
                         a.next_active[u[j]] = 1;
                 continue;
             }
-            int slot[kApplyEdges];
+            int from[kApplyEdges], to[kApplyEdges];
 #pragma unroll
             for (int j = 0; j < kApplyEdges; ++j) {
-                slot[j] = -1;
-                if (e[j] >= 0) {
-                    a.next_active[u[j]] = 1;
-                    if (a.hub_cnt) slot[j] = a.hub_slot[u[j]];
-                }
+                from[j] = row_from[k[j]];
+                to[j] = row_to[k[j]];
             }
-#pragma unroll
-            for (int j = 0; j < kApplyEdges; ++j)
-                if (slot[j] >= 0) {
-                    const int w = a.adjwgt[e[j]];
-                    atomicSub(&a.hub_cnt[slot[j] + row_from[k[j]]], w);
-                    atomicAdd(&a.hub_cnt[slot[j] + row_to[k[j]]], w);
-                }
+            mark(e, u, from, to);
         }
         __syncthreads();  // the step's rows are done before the movers are reset
+    }
+    if (M == LpMode::Refine && a.big) {
+        __shared__ int piece[kBlock];  // first piece past row i of the batch
+        __shared__ int wave_pieces[kBlock / 64];
+        const int n_big = *a.n_big;
+        for (int b0 = 0; b0 < n_big; b0 += kBlock) {  // uniform
+            const int i = b0 + (int)threadIdx.x;
+            int incl = i < n_big ? (a.big[i].y + kLongRow - 1) / kLongRow : 0;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(incl, o, 64);
+                if ((int)(threadIdx.x & 63) >= o) incl += y;
+            }
+            if ((threadIdx.x & 63) == 63) wave_pieces[threadIdx.x >> 6] = incl;
+            __syncthreads();
+            for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) incl += wave_pieces[w];
+            piece[threadIdx.x] = incl;
+            __syncthreads();
+            const int pieces = piece[kBlock - 1];
+            for (int p = blockIdx.x; p < pieces; p += gridDim.x) {
+                int lo = 0, hi = kBlock - 1;  // first row that ends past p
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (piece[mid] > p) hi = mid; else lo = mid + 1;
+                }
+                const int4 r = a.big[b0 + lo];
+                const int e0 = (p - (lo ? piece[lo - 1] : 0)) * kLongRow + (int)threadIdx.x;
+                int e[kApplyEdges], u[kApplyEdges], from[kApplyEdges], to[kApplyEdges];
+#pragma unroll
+                for (int j = 0; j < kApplyEdges; ++j) {
+                    e[j] = e0 + j * kBlock < r.y ? r.x + e0 + j * kBlock : -1;
+                    u[j] = e[j] >= 0 ? a.adjncy[e[j]] : 0;
+                    from[j] = r.z;
+                    to[j] = r.w;
+                }
+                mark(e, u, from, to);
+            }
+            __syncthreads();  // `piece` is rewritten by the next batch
+        }
     }
     if (M == LpMode::Refine) count_traversed(a, edges);
     if (threadIdx.x == 0 && block_moves) atomicAdd(a.moves, block_moves);
@@ -2634,6 +2699,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     }
     int* cnow = ccount_.p;  // list lengths of the frontier, cleared by the tail before last
     int* cnext = cnow + nseg;
+    if (!cl && hubs > 0) a.big = big_.reserve(g.m2 / kLongRow + 1);
     while (r < rounds) {
         // refinement: round 0 works on the whole lists, later rounds on the compacted frontier
         const int* flists = lists_.p;
@@ -2679,6 +2745,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         for (int sr = 0; sr < S; ++sr) {
             int sub_total = 0;
             if (!cl) {
+                if (a.big) a.n_big = ctl_.p + kCtlLong + (r * S + sr);
                 // refinement: the five degree lists' proposals in one launch over the frontier,
                 // and the hubs' decisions from their kept counters when every hub has them
                 FrontierLists F{};

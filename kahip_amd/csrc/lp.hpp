@@ -40,6 +40,10 @@ struct LpArgs {
     // their hub neighbours.
     const int* hub_slot;
     int* hub_cnt;
+    // Refinement of a graph with hubs (nullptr otherwise): admitted moves of rows of more than
+    // kLongRow edges, {first edge, edges, old label, new label}, and their number (zero on entry).
+    int4* big;
+    int* n_big;
     int* err;  // device error flag (kErrProbe), cleared by prepare(), read by check()
     // Independent clusterings of one graph in one launch (gridDim.y of them): clustering y has its
     // arrays y * copy_stride further on and the tie seed tie_seed, copy_tie1, copy_tie2 (not an
@@ -120,9 +124,10 @@ private:
     void fetch(hipStream_t s);  // host_ctl_ of the last run
     Mail mail_;
     // Counters of a run: {traversed edges in 64 spread 64-bit counters, moves per round, lengths
-    // of the hub merges' big task queues per sub-round, error flag}
+    // of the hub merges' big task queues and of the long moved rows per sub-round, error flag}
     static constexpr int kCtlMoves = 128, kCtlBig = kCtlMoves + kMaxRounds,
-                         kCtlErr = kCtlBig + kMaxSub * kMaxRounds, kCtlInts = kCtlErr + 1;
+                         kCtlLong = kCtlBig + kMaxSub * kMaxRounds,
+                         kCtlErr = kCtlLong + kMaxSub * kMaxRounds, kCtlInts = kCtlErr + 1;
     DevBuf<int> ctl_;
     int host_ctl_[kCtlBig + 1] = {};  // the traversed edges, the moves, the error flag
     bool fetched_ = false;
@@ -159,7 +164,7 @@ private:
     DevBuf<char> scan_tmp_;
     DevBuf<long long> offm_base_;
     DevBuf<int> offm_, task_prefix_, bown_, big_tasks_;
-    DevBuf<int4> bres_;
+    DevBuf<int4> bres_, big_;
     DevBuf<int4> cmap_, tmap_, mmap_;  // hub-chunk, (hub, bucket) task, mid-size hub descriptors
     DevBuf<int> midpos_;
     DevBuf<int2> tsub_;  // (hub, bucket) task: {multi-chunk hub index, bucket | buckets << 16}
