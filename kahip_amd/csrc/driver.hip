@@ -355,6 +355,7 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
     W.reserve(p.k);
     HostGraph hl;
     std::vector<int> hp;
+    DevBuf<uint8_t>& border = buf_.border;  // of the level before
     for (int l = level; l >= 0; --l) {
         const DGraph& gl = level_graph(l);
         ev_refine.emplace_back();
@@ -364,6 +365,10 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
             part_l = part_c.p;
         } else {
             part_f.reserve(std::max(gl.n, 1));
+            // A node whose coarse node had no neighbour in another block has none either and
+            // cannot move before one of its neighbours does: on a mesh that is nearly every node.
+            border.reserve(level_graph(l + 1).n);
+            LpWorkspace::border(level_graph(l + 1), part_c.p, border.p, s);
             project_partition(gl.n, maps[l].p, part_c.p, part_f.p, s, prof);
             std::swap(part_c, part_f);
             part_l = part_c.p;
@@ -372,8 +377,10 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         const uint32_t rseed = refine_seed(p.seed, l);
         lp.prepare(LpMode::Refine, gl, p.k, p.subrounds, rseed, p.bins, s);
         // the profiler times the clustering and contraction kernels, not the refinement rounds
+        const bool from_border = l < level && !lp.has_hubs();
         lp.run(LpMode::Refine, gl, part_l, W.p, (int)U, p.refine_rounds, rseed, s, nullptr,
-               "lp_refine");
+               "lp_refine", nullptr, from_border ? maps[l].p : nullptr,
+               from_border ? border.p : nullptr);
         KH_CHECK(hipEventRecord(ev_refine.back().b, s));
         lp.check(s);
         S.edges_refine += lp.traversed(s);

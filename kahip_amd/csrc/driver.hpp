@@ -135,6 +135,7 @@ private:
         std::vector<std::unique_ptr<OwnedGraph>> coarse;  // coarse[l] = level l+1
         std::vector<DevBuf<int>> maps;                     // maps[l]: level l -> level l+1
         DevBuf<int> label, size, score, elabel, part_c, part_f, W;
+        DevBuf<uint8_t> border;
         DevBuf<unsigned long long> okeys, okeys2;
         DevBuf<int> oids, oids2;
         DevBuf<char> otmp;

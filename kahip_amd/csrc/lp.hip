@@ -2188,15 +2188,29 @@ __global__ void init_scratch(long long n, int* __restrict__ prop_t, long long nl
     }
 }
 
-// Frontier flags and list lengths of a refinement.
+// Frontier flags (value, or those of start at map[i]) and list lengths of a refinement.
 __global__ void init_frontier(int n, uint8_t* __restrict__ act, uint8_t value,
+                              const int* __restrict__ map, const uint8_t* __restrict__ start,
                               uint8_t* __restrict__ nxt, int m, int* __restrict__ ccount) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
-        act[i] = value;
+        act[i] = start ? start[map[i]] : value;
         nxt[i] = 0;
     }
     if (i < m) ccount[i] = 0;
+}
+
+// Nodes with a neighbour in another block.
+__global__ __launch_bounds__(256) void border_nodes(int n, const int* __restrict__ xadj,
+                                                    const int* __restrict__ adjncy,
+                                                    const int* __restrict__ part,
+                                                    uint8_t* __restrict__ border) {
+    const int v = blockIdx.x * 256 + threadIdx.x;
+    if (v >= n) return;
+    const int own = part[v], end = xadj[v + 1];
+    uint8_t b = 0;
+    for (int e = xadj[v]; e < end && !b; ++e) b = part[adjncy[e]] != own;
+    border[v] = b;
 }
 
 // (blockIdx.y: copies, one after the other)
@@ -2601,7 +2615,7 @@ void LpWorkspace::build_chunk_maps(hipStream_t s) {
 
 void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int bound, int rounds,
                       uint32_t seed, hipStream_t s, Profiler* prof, const char* phase,
-                      const int* lbound) {
+                      const int* lbound, const int* map, const uint8_t* start) {
     KH_REQUIRE(rounds >= 0 && rounds <= kMaxRounds, "LP rounds must be in [0, 64]");
     const int S = subrounds_;
     const bool cl = mode == LpMode::Cluster;
@@ -2628,7 +2642,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     if (small_) {
         // the whole refinement in one workgroup; the lists are built only if it stops early
         hipLaunchKernelGGL(init_frontier, dim3(std::max(grid_for(g.n, 256), 1)), dim3(256), 0, s,
-                           g.n, act, (uint8_t)0, nxt, 0, nullptr);
+                           g.n, act, (uint8_t)0, nullptr, nullptr, nxt, 0, nullptr);
         a.next_active = nxt;
         TailArgs t{};
         t.n = g.n;
@@ -2636,6 +2650,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         t.seed = seed;
         r = run_tail(a, t, s, &filter);
         if (r >= rounds) return;
+        start = nullptr;  // (r > 0: the tail starts from every node)
         build_lists(mode, g, seed, s, nullptr, 1);
         std::swap(act, nxt);  // round r's frontier (r > 0)
     }
@@ -2676,7 +2691,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         if (listed == 0) return;
         const int nf = r == 0 ? g.n : 0;  // else flagged by the tail
         hipLaunchKernelGGL(init_frontier, dim3(grid_for(std::max(nf, 2 * nseg), 256)), dim3(256),
-                           0, s, nf, act, (uint8_t)(keep_flags ? 1 : 0), nxt, 2 * nseg, ccount_.p);
+                           0, s, nf, act, (uint8_t)(keep_flags ? 1 : 0), map, start, nxt, 2 * nseg, ccount_.p);
     }
     const bool settle = cl && hubs == 0 && rounds > kSettleRound + 1 && g.m2 > kSettleEdges;
     if (settle) {
@@ -2701,10 +2716,11 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     int* cnext = cnow + nseg;
     if (!cl && hubs > 0) a.big = big_.reserve(g.m2 / kLongRow + 1);
     while (r < rounds) {
-        // refinement: round 0 works on the whole lists, later rounds on the compacted frontier
+        // refinement: round 0 works on the whole lists (unless its frontier is given), later rounds
+        // on the compacted frontier
         const int* flists = lists_.p;
         const int* fcount = counts_;
-        if (!cl && r > 0) {
+        if (!cl && (r > 0 || start)) {
             ProfScope ps(prof, base + "_frontier", 0.0, 0, s);
             std::swap(cnow, cnext);
             hipLaunchKernelGGL(compact_active, dim3(grid_for(listed, 256 * kCompactItems)), dim3(256), 0, s,
@@ -3047,6 +3063,19 @@ long long LpWorkspace::traversed(hipStream_t s) {
     long long t = 0;
     for (int i = 0; i < 64; ++i) t += (long long)h[i];
     return t;
+}
+
+void LpWorkspace::border(const DGraph& g, const int* part, uint8_t* flags, hipStream_t s) {
+    if (g.n > 0)
+        hipLaunchKernelGGL(border_nodes, dim3(grid_for(g.n, 256)), dim3(256), 0, s, g.n, g.xadj,
+                           g.adjncy, part, flags);
+    KH_CHECK(hipGetLastError());
+}
+
+bool LpWorkspace::has_hubs() const {
+    for (int sr = 0; sr < subrounds_; ++sr)
+        if (!small_ && host_counts[sr * kNumBins + kNumBins - 1] > 0) return true;
+    return false;
 }
 
 void LpWorkspace::init_cluster_labels(const DGraph& g, int* label, int* size, hipStream_t s) {

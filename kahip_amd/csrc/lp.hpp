@@ -91,9 +91,16 @@ public:
     // Runs `rounds` synchronous rounds. label/size are device arrays (node -> label,
     // label -> weight). Refinement starts from an all-active frontier.
     // lbound (optional): the bound of each label, replacing `bound`.
+    // start (optional): the refinement starts from the nodes v with start[map[v]] set instead;
+    // the others must have no neighbour in another block (they cannot move then).
     void run(LpMode mode, const DGraph& g, int* label, int* size, int bound, int rounds,
              uint32_t seed, hipStream_t s, Profiler* prof, const char* phase,
-             const int* lbound = nullptr);
+             const int* lbound = nullptr, const int* map = nullptr,
+             const uint8_t* start = nullptr);
+    // flags[v] = 1 if v has a neighbour in another block, else 0
+    static void border(const DGraph& g, const int* part, uint8_t* flags, hipStream_t s);
+    // Whether the graph of the last prepare() has hubs.
+    bool has_hubs() const;
     // label[v] = v, size[v] = vwgt[v]
     static void init_cluster_labels(const DGraph& g, int* label, int* size, hipStream_t s);
     // Moves per round of the last run (waits for it).
