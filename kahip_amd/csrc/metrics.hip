@@ -1,9 +1,14 @@
 // Partition quality on gfx950: edge cut (reference: lib/tools/quality_metrics.cpp:23-37) and
 // block weights (quality_metrics.cpp:265-288 uses them for balance).
 //
-// Edge cut is edge-parallel: each thread owns kChunk consecutive directed edges, finds the
-// source of its first edge by binary search in xadj and walks forward; partial sums are reduced
-// per workgroup and added with one 64-bit atomic. Integer sums: any order gives the same bits.
+// Edge cut is edge-parallel, in tiles of kTile consecutive directed edges. The block of every
+// edge's source goes through LDS: a thread finds the sources of kChunk consecutive edges (by a search
+// that gallops from the tile's first source, then forward) and writes their blocks, so that the
+// targets and weights can be read by consecutive threads. With kChunk consecutive edges read by each
+// thread, a load touched 32 cache lines, and the address units were the bound. A workgroup owns
+// a range of tiles and searches all of xadj for its first one only; one 64-bit atomic per workgroup.
+// Measured: RGG 2^22 (61 M directed edges) 269 -> 199 us, R-MAT 2^20 (31 M, random targets) 286 -> 198
+// us. Integer sums: any order gives the same bits.
 
 #include <algorithm>
 #include <cstring>
@@ -19,6 +24,8 @@ namespace {
 
 constexpr int kChunk = 8;
 constexpr int kBlock = 256;
+constexpr int kTile = kChunk * kBlock;
+constexpr int kCutGrid = 2048;
 
 __device__ inline int source_of(const int* __restrict__ xadj, int n, long long e) {
     // largest u with xadj[u] <= e (and xadj[u+1] > e for a non-empty row)
@@ -42,22 +49,57 @@ __global__ __launch_bounds__(kBlock) void edge_cut_kernel(int n, long long m2,
                                                           const int* __restrict__ part,
                                                           unsigned long long* __restrict__ out) {
     __shared__ long long red[kBlock / 64];
-    const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-    const long long e0 = t * kChunk;
+    __shared__ int first;       // source of the tile's first edge
+    __shared__ __align__(16) int own[kTile];  // block of every edge's source
+    static_assert(kChunk == 8, "two 16-byte stores");
     long long acc = 0;
-    if (e0 < m2) {
-        int u = source_of(xadj, n, e0);
-        long long next = xadj[u + 1];
-        int pu = part[u];
-        const long long e1 = e0 + kChunk < m2 ? e0 + kChunk : m2;
-        for (long long e = e0; e < e1; ++e) {
-            while (e >= next) {
-                ++u;
-                next = xadj[u + 1];
-                pu = part[u];
-            }
-            if (part[adjncy[e]] != pu) acc += UNIT ? 1 : adjwgt[e];
+    const long long tiles = (m2 + kTile - 1) / kTile;
+    const long long per = (tiles + gridDim.x - 1) / gridDim.x;
+    const long long end = min(m2, (blockIdx.x + 1) * per * kTile);
+    long long base = blockIdx.x * per * kTile;
+    if (threadIdx.x == 0 && base < end) first = source_of(xadj, n, base);
+    for (; base < end; base += kTile) {  // uniform
+        int q[kChunk], w[kChunk];
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+            const long long e = base + threadIdx.x + j * kBlock;
+            q[j] = e < m2 ? adjncy[e] : -1;
+            w[j] = UNIT ? 1 : e < m2 ? adjwgt[e] : 0;
         }
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j)
+            if (q[j] >= 0) q[j] = part[q[j]];
+            else w[j] = 0;
+        __syncthreads();
+        int u = first;
+        const long long e0 = base + threadIdx.x * kChunk;
+        if (e0 < m2) {
+            long long hop = 1;  // u + hop: past the source once xadj[u + hop] > e0
+            while (u + hop < n && (long long)xadj[u + hop] <= e0) {
+                u += (int)hop;
+                hop *= 2;
+            }
+            u += source_of(xadj + u, (int)min(hop, (long long)n - u), e0);
+            long long next = xadj[u + 1];
+            int pu = part[u], of[kChunk];
+#pragma unroll
+            for (int j = 0; j < kChunk; ++j) {
+                while (e0 + j >= next && e0 + j < m2) {
+                    ++u;
+                    next = xadj[u + 1];
+                    pu = part[u];
+                }
+                of[j] = pu;
+            }
+            int4* const to = reinterpret_cast<int4*>(own + threadIdx.x * kChunk);
+            to[0] = make_int4(of[0], of[1], of[2], of[3]);
+            to[1] = make_int4(of[4], of[5], of[6], of[7]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j)
+            if (q[j] != own[threadIdx.x + j * kBlock]) acc += w[j];
+        if (threadIdx.x == kBlock - 1) first = u;  // at or before the next tile's source
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
@@ -156,7 +198,7 @@ void quality_noalloc(int n, long long m2, const int* xadj, const int* adjncy, co
     fill_async(sc, 2LL + k, 0ull, s);  // a fill kernel: the call stays capturable
     if (m2 > 0) {
         const long long threads = (m2 + kChunk - 1) / kChunk;
-        const dim3 grid((unsigned)((threads + kBlock - 1) / kBlock));
+        const dim3 grid((unsigned)std::min<long long>((threads + kBlock - 1) / kBlock, kCutGrid));
         if (adjwgt)
             hipLaunchKernelGGL(edge_cut_kernel<false>, grid, dim3(kBlock), 0, s, n, m2, xadj,
                                adjncy, adjwgt, part, sc);
@@ -183,9 +225,9 @@ const int* MetricsWorkspace::launch_edge_cut(const DGraph& g, const int* part, h
         // algorithmic bytes: 12 B per directed edge (target, weight, block of target) and
         // 12 B per node (offset, block of source, block weight read in the balance pass)
         ProfScope ps(prof, "edge_cut", 12.0 * (double)g.m2 + 12.0 * g.n, g.m2, s);
-        hipLaunchKernelGGL(edge_cut_kernel<false>, dim3((unsigned)((threads + kBlock - 1) / kBlock)),
-                           dim3(kBlock), 0, s, g.n, g.m2, g.xadj, g.adjncy, g.adjwgt, part,
-                           acc_.p);
+        const long long grid = std::min<long long>((threads + kBlock - 1) / kBlock, kCutGrid);
+        hipLaunchKernelGGL(edge_cut_kernel<false>, dim3((unsigned)grid), dim3(kBlock), 0, s, g.n,
+                           g.m2, g.xadj, g.adjncy, g.adjwgt, part, acc_.p);
     }
     return reinterpret_cast<const int*>(acc_.p);
 }
