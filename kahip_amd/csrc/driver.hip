@@ -365,10 +365,6 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
             part_l = part_c.p;
         } else {
             part_f.reserve(std::max(gl.n, 1));
-            // A node whose coarse node had no neighbour in another block has none either and
-            // cannot move before one of its neighbours does: on a mesh that is nearly every node.
-            border.reserve(level_graph(l + 1).n);
-            LpWorkspace::border(level_graph(l + 1), part_c.p, border.p, s);
             project_partition(gl.n, maps[l].p, part_c.p, part_f.p, s, prof);
             std::swap(part_c, part_f);
             part_l = part_c.p;
@@ -376,8 +372,14 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         compute_block_weights(gl, part_l, p.k, W.p, s);
         const uint32_t rseed = refine_seed(p.seed, l);
         lp.prepare(LpMode::Refine, gl, p.k, p.subrounds, rseed, p.bins, s);
+        // A node whose coarse node has no neighbour in another block has none either and cannot
+        // move before one of its neighbours does: on a mesh that is nearly every node.
+        const bool from_border = l < level && lp.takes_start();
+        if (from_border) {
+            border.reserve(level_graph(l + 1).n);
+            LpWorkspace::border(level_graph(l + 1), part_f.p, border.p, s);  // (before projection)
+        }
         // the profiler times the clustering and contraction kernels, not the refinement rounds
-        const bool from_border = l < level && !lp.has_hubs();
         lp.run(LpMode::Refine, gl, part_l, W.p, (int)U, p.refine_rounds, rseed, s, nullptr,
                "lp_refine", nullptr, from_border ? maps[l].p : nullptr,
                from_border ? border.p : nullptr);

@@ -2200,16 +2200,18 @@ __global__ void init_frontier(int n, uint8_t* __restrict__ act, uint8_t value,
     if (i < m) ccount[i] = 0;
 }
 
-// Nodes with a neighbour in another block.
+// Nodes that may have a neighbour in another block: those with one among their first
+// kBorderEdges, and those of longer rows (one thread per row: a long one would keep the launch).
+constexpr int kBorderEdges = 64;
 __global__ __launch_bounds__(256) void border_nodes(int n, const int* __restrict__ xadj,
                                                     const int* __restrict__ adjncy,
                                                     const int* __restrict__ part,
                                                     uint8_t* __restrict__ border) {
     const int v = blockIdx.x * 256 + threadIdx.x;
     if (v >= n) return;
-    const int own = part[v], end = xadj[v + 1];
-    uint8_t b = 0;
-    for (int e = xadj[v]; e < end && !b; ++e) b = part[adjncy[e]] != own;
+    const int own = part[v], beg = xadj[v], end = xadj[v + 1];
+    uint8_t b = end - beg > kBorderEdges;
+    for (int e = beg; e < end && !b; ++e) b = part[adjncy[e]] != own;
     border[v] = b;
 }
 
@@ -3072,10 +3074,11 @@ void LpWorkspace::border(const DGraph& g, const int* part, uint8_t* flags, hipSt
     KH_CHECK(hipGetLastError());
 }
 
-bool LpWorkspace::has_hubs() const {
+bool LpWorkspace::takes_start() const {
+    if (small_) return false;
     for (int sr = 0; sr < subrounds_; ++sr)
-        if (!small_ && host_counts[sr * kNumBins + kNumBins - 1] > 0) return true;
-    return false;
+        if (host_counts[sr * kNumBins + kNumBins - 1] > 0) return false;
+    return true;
 }
 
 void LpWorkspace::init_cluster_labels(const DGraph& g, int* label, int* size, hipStream_t s) {

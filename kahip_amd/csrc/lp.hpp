@@ -97,10 +97,11 @@ public:
              uint32_t seed, hipStream_t s, Profiler* prof, const char* phase,
              const int* lbound = nullptr, const int* map = nullptr,
              const uint8_t* start = nullptr);
-    // flags[v] = 1 if v has a neighbour in another block, else 0
+    // flags[v] = 1 if v may have a neighbour in another block, else 0
     static void border(const DGraph& g, const int* part, uint8_t* flags, hipStream_t s);
-    // Whether the graph of the last prepare() has hubs.
-    bool has_hubs() const;
+    // Whether `start` is of use on the graph of the last prepare(): it has no hubs and is not
+    // refined by one workgroup from its first round on.
+    bool takes_start() const;
     // label[v] = v, size[v] = vwgt[v]
     static void init_cluster_labels(const DGraph& g, int* label, int* size, hipStream_t s);
     // Moves per round of the last run (waits for it).

@@ -52,7 +52,8 @@ int* Mail::box() {
 
 int Mail::next() {
     init();
-    return ++seq_;
+    seq_ = (int)((unsigned)seq_ + 1u);  // (wraps)
+    return seq_;
 }
 
 void Mail::post(hipStream_t s, Piece a, Piece b, Piece c, Piece d) {

@@ -32,3 +32,31 @@ def test_disconnected(degrees):
         part, _ = K.partition(*g, k=k, seed=1, stop_factor=10)
         want, _ = mirror_partition(*g, k, 0.03, 1, stop_factor=10)
         assert np.array_equal(part, want)
+
+
+@pytest.mark.parametrize("row", [63, 64, 65, 3000])
+def test_long_coarse_rows(row):
+    """Coarse rows around the length that the border scan reads: a ring of `row` clusters of five
+    nodes, each also joined to one cluster in the middle."""
+    n = 5 * (row + 1)
+    c = np.arange(1, row + 1)
+    u, v, w = [], [], []
+    for j in range(4):  # heavy paths inside the clusters
+        u.append(5 * np.arange(row + 1) + j)
+        v.append(5 * np.arange(row + 1) + j + 1)
+        w.append(np.full(row + 1, 50))
+    u.append(5 * c)  # to the middle cluster, spread over its members
+    v.append(c % 5)
+    w.append(np.ones(row, np.int64))
+    u.append(5 * c[:-1] + 2)
+    v.append(5 * c[1:] + 3)
+    w.append(np.full(row - 1, 2))
+    u, v, w = np.concatenate(u), np.concatenate(v), np.concatenate(w)
+    a, b, w = np.concatenate([u, v]), np.concatenate([v, u]), np.concatenate([w, w])
+    order = np.argsort(a, kind="stable")
+    x = np.concatenate([[0], np.cumsum(np.bincount(a, minlength=n))]).astype(np.int32)
+    g = (x, b[order].astype(np.int32), np.ones(n, np.int32), w[order].astype(np.int32))
+    for k in (2, 5):
+        part, _ = K.partition(*g, k=k, seed=3, stop_factor=5, cluster_factor=2, reorder=0)
+        want, _ = mirror_partition(*g, k, 0.03, 3, stop_factor=5, cluster_factor=2, reorder=0)
+        assert np.array_equal(part, want)
