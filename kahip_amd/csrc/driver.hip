@@ -372,8 +372,8 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         compute_block_weights(gl, part_l, p.k, W.p, s);
         const uint32_t rseed = refine_seed(p.seed, l);
         lp.prepare(LpMode::Refine, gl, p.k, p.subrounds, rseed, p.bins, s);
-        // A node whose coarse node has no neighbour in another block has none either and cannot
-        // move before one of its neighbours does: on a mesh that is nearly every node.
+        // A node whose coarse node has no neighbour in another block has none either, and no
+        // candidate before one of its neighbours moves: on a mesh that is nearly every node.
         const bool from_border = l < level && lp.takes_start();
         if (from_border) {
             border.reserve(level_graph(l + 1).n);

@@ -91,16 +91,17 @@ public:
     // Runs `rounds` synchronous rounds. label/size are device arrays (node -> label,
     // label -> weight). Refinement starts from an all-active frontier.
     // lbound (optional): the bound of each label, replacing `bound`.
-    // start (optional): the refinement starts from the nodes v with start[map[v]] set instead;
-    // the others must have no neighbour in another block (they cannot move then).
+    // start (optional): the first round starts from the nodes v with start[map[v]] set; the others
+    // must have no neighbour in another block, so that they have no candidate until a neighbour
+    // moves, and enter the round's later sub-rounds when one does. Same result as from all nodes.
     void run(LpMode mode, const DGraph& g, int* label, int* size, int bound, int rounds,
              uint32_t seed, hipStream_t s, Profiler* prof, const char* phase,
              const int* lbound = nullptr, const int* map = nullptr,
              const uint8_t* start = nullptr);
     // flags[v] = 1 if v may have a neighbour in another block, else 0
     static void border(const DGraph& g, const int* part, uint8_t* flags, hipStream_t s);
-    // Whether `start` is of use on the graph of the last prepare(): it has no hubs and is not
-    // refined by one workgroup from its first round on.
+    // Whether `start` is of use on the graph of the last prepare(): it is large, has no hubs and is
+    // not refined by one workgroup from its first round on.
     bool takes_start() const;
     // label[v] = v, size[v] = vwgt[v]
     static void init_cluster_labels(const DGraph& g, int* label, int* size, hipStream_t s);
