@@ -56,15 +56,20 @@ constexpr int kFinCap = 16384;     // LDS hash slots of hub_bucket_merge (128 KB
 constexpr int kFinLds = 8192;      // buckets up to this many entries merge in LDS
 constexpr int kMaxBuckets = 2048;  // buckets per hub: min(kBucketsPerChunk x chunks, kMaxBuckets)
 constexpr int kBucketsPerChunk = 4;  // ~1000 entries per (hub, bucket)
+constexpr int kTinyThreads = 256;    // tiny bucket merge: <= kTinyMax entries in 16 KB of LDS
+constexpr int kTinyCap = 2048;
+constexpr int kTinyMax = 1024;
+constexpr int kTinyTasks = 2048;     // sub-rounds of more merge tasks start with it
 constexpr int kSmallThreads = 512;   // small bucket merge: <= kSmallMax entries in 32 KB of LDS
 constexpr int kSmallCap = 4096;
 constexpr int kSmallMax = 2048;
+constexpr int kSmallGrid = 1024;     // its workgroups over a queue (four per CU)
 // Sub-rounds of at most kHubJoin chunks and mid-size hubs (two workgroups of kHubThreads per CU)
 // take the mid-size hubs along in the chunk kernel's launch.
 constexpr int kHubJoin = 512;
 constexpr int kHubStage = 256;       // merge tasks of hubs of at most this many chunks sum the
                                      // chunks' entry counts themselves and keep the offsets in LDS
-static_assert(kHubStage <= kSmallThreads, "a thread per chunk");
+static_assert(kHubStage <= kTinyThreads, "a thread per chunk");
 
 struct Cand {
     int conn;
@@ -1051,17 +1056,24 @@ __global__ __launch_bounds__(THREADS) void propose_hub_chunk(
 
 // Merge of one (multi-chunk hub, bucket) task: the bucket's entries of all chunks of the hub are
 // summed in an LDS hash (or in the hub's global table, filtering by bucket); the bucket's best
-// candidate and, for the bucket of the own label, conn(own) are left in bres / bown. The small
-// form (512 threads, 32 KB of LDS, four per CU) takes every task of the sub-round; those of more
-// than kSmallMax entries use the global table, or are queued for the big form (1024 threads,
-// 128 KB, up to kFinLds entries, grid-stride over the queue) where a hub's buckets have reached
-// kMaxBuckets, so that tasks are larger than ~1000 entries by size and not by bad luck.
-// One launch where there were four (a scan of the counts over all tasks, 256-thread merges, 512
-// and 1024-thread merges of their queues): measured in kahip_partition, together with the
-// mid-size hubs' place in the chunk launch: R-MAT 2^17, k = 8 20.8 -> 19.0 ms (coarsening 9.1 -> 7.3),
-// R-MAT 2^20, k = 16 coarsening 24.4 -> 22.8 ms.
-template <LpMode M, bool BIG>
-__global__ __launch_bounds__(BIG ? kFinThreads : kSmallThreads)
+// candidate and, for the bucket of the own label, conn(own) are left in bres / bown. LEVEL 1 (512
+// threads, 32 KB of LDS, four per CU) takes every task of the sub-round; those of more than
+// kSmallMax entries use the global table, or are queued for LEVEL 2 (1024 threads, 128 KB, up to
+// kFinLds entries, grid-stride over the queue) where a hub's buckets have reached kMaxBuckets, so
+// that tasks are larger than ~1000 entries by size and not by bad luck.
+// One launch where there were four (a scan of the counts over all tasks, and a launch per level):
+// measured in kahip_partition, together with the mid-size hubs' place in the chunk launch: R-MAT
+// 2^17, k = 8 20.8 -> 19.0 ms (coarsening 9.1 -> 7.3), R-MAT 2^20, k = 16 coarsening 24.4 -> 22.8 ms.
+// Sub-rounds of more than kTinyTasks tasks fill the chip many times over, a launch more is nothing
+// there and a task's latency (chunk counts, table, reduction) is the bound: LEVEL 0 (256 threads,
+// 16 KB, eight per CU) takes every task and queues those of more than kTinyMax entries for LEVEL 1.
+// Eight waves per SIMD need at most 96 SGPRs (by launch_bounds; 106 without). Measured, merges of a
+// clustering: R-MAT 2^24 (38 600 tasks a sub-round) 42.4 -> 27.8 ms, 2^22 (6 650) 7.1 -> 5.2, 2^21
+// (3 950) 2.26 -> 1.85, 2^18 with 64 samples a node (2 390) 2.73 -> 2.62; LEVEL 0 below the limit:
+// 2^20 (730) 2.13 -> 2.61, 2^17 (40) 0.64 -> 0.77 ms.
+template <LpMode M, int LEVEL>
+__global__ __launch_bounds__(LEVEL == 0 ? kTinyThreads : (LEVEL == 1 ? kSmallThreads : kFinThreads),
+                             LEVEL == 2 ? 4 : 8)
 void hub_bucket_merge(
     LpArgs a, int n_tasks, const int4* __restrict__ tmap, const int2* __restrict__ tsub,
     const int* __restrict__ cntT, const int* __restrict__ posT,
@@ -1069,19 +1081,20 @@ void hub_bucket_merge(
     const int* __restrict__ offm, const int2* __restrict__ partials,
     const long long* __restrict__ tab_off, int* __restrict__ gkey, int* __restrict__ gval,
     Cand* __restrict__ bres, int* __restrict__ bown, uint8_t* __restrict__ fb,
-    int* __restrict__ queue, int* __restrict__ queued) {
-    constexpr int THREADS = BIG ? kFinThreads : kSmallThreads;
-    constexpr int CAP = BIG ? kFinCap : kSmallCap;
-    constexpr int MAXE = BIG ? kFinLds : kSmallMax;
+    const int* __restrict__ in_q, const int* __restrict__ in_n, int* __restrict__ out_q,
+    int* __restrict__ out_n) {
+    constexpr int THREADS = LEVEL == 0 ? kTinyThreads : (LEVEL == 1 ? kSmallThreads : kFinThreads);
+    constexpr int CAP = LEVEL == 0 ? kTinyCap : (LEVEL == 1 ? kSmallCap : kFinCap);
+    constexpr int MAXE = LEVEL == 0 ? kTinyMax : (LEVEL == 1 ? kSmallMax : kFinLds);
     static_assert(2 * MAXE <= CAP, "merge tables fill at most half");
     __shared__ int K[CAP];
     __shared__ int V[CAP];
     __shared__ int spre[kHubStage + 1];  // task offsets of the chunks' bucket segments
     __shared__ int sstart[kHubStage];    // the segments' starts in their chunks' partials
     __shared__ int wsum[kHubStage / 64];
-    const int n_iter = BIG ? *queued : n_tasks;
+    const int n_iter = LEVEL > 0 && in_q ? *in_n : n_tasks;
     for (int it = blockIdx.x; it < n_iter; it += gridDim.x) {
-        const int task = BIG ? queue[it] : it;
+        const int task = LEVEL > 0 && in_q ? in_q[it] : it;
         const int4 tm = tmap[task];  // {first count index, one past the last, hub index, node}
         const int2 ts = tsub[task];  // {multi-chunk hub index, bucket | buckets << 16}
         const int mi = ts.x;
@@ -1120,8 +1133,8 @@ void hub_bucket_merge(
             r0 = posT[tm.x];
             total = posT[tm.y] - r0;
         }
-        if (!BIG && total > MAXE && queue) {
-            if (threadIdx.x == 0) queue[atomicAdd(queued, 1)] = task;
+        if (LEVEL < 2 && total > MAXE && out_q) {
+            if (threadIdx.x == 0) out_q[atomicAdd(out_n, 1)] = task;
             __syncthreads();
             continue;
         }
@@ -2548,6 +2561,7 @@ void LpWorkspace::build_lists(LpMode mode, const DGraph& g, uint32_t seed, hipSt
     bres_.reserve(max_tasks);
     bown_.reserve(max_tasks);
     big_tasks_.reserve(max_tasks);
+    if (max_tasks > kTinyTasks) mid_tasks_.reserve(max_tasks);
     fb_.reserve(max_multi);
     fill_async(fb_.p, max_multi, (uint8_t)0, s);
     KH_CHECK(hipMemcpyAsync(chunk_prefix_.p, prefix.data(), sizeof(int) * prefix.size(),
@@ -2916,22 +2930,27 @@ void LpWorkspace::propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool increm
             KH_CHECK(rocprim::exclusive_scan(scan_tmp_.p, sb, cnt_t_.p + ct_sr_base_[sr], pos_t_.p + ct_sr_base_[sr], 0, (size_t)ct_sr_size_[sr] + 1, rocprim::plus<int>(), s));
         }
         const int* cp = chunk_prefix_.p + chunk_base_[sr];
+        const bool tiny = nt > kTinyTasks;
+        int* mid = tiny ? mid_tasks_.p : nullptr;
         int* queue = hub_capped_[sr] ? big_tasks_.p : nullptr;
+        int* n_mid = ctl_.p + kCtlMid + (r * S + sr);
         int* queued = ctl_.p + kCtlBig + (r * S + sr);
-        const auto merge = [&](auto kernel, int grid, int threads) {
-            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, a, nt, tm, tsb, cnt_t_.p, pos_t_.p, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, queue, queued);
+        const auto merge = [&](auto kernel, int grid, int threads, const int* in_q, const int* in_n, int* out_q, int* out_n) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, a, nt, tm, tsb, cnt_t_.p, pos_t_.p, cp, ob, offm_.p, partials_.p, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p, in_q, in_n, out_q, out_n);
+        };
+        const auto merges = [&](auto k0, auto k1, auto k2) {
+            if (tiny) merge(k0, nt, kTinyThreads, nullptr, nullptr, mid, n_mid);
+            merge(k1, tiny ? kSmallGrid : nt, kSmallThreads, mid, n_mid, queue, queued);
+            if (queue) merge(k2, std::min(nt, 256), kFinThreads, queue, queued, nullptr, nullptr);
         };
         const auto decide = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(nm), dim3(256), 0, s, a, lst, ml, nm, tp, to, hub_key_.p, hub_val_.p, br, bown_.p, fb_.p);
         };
-        const int big = std::min(nt, 256);
         if (cl) {
-            merge(hub_bucket_merge<LpMode::Cluster, false>, nt, kSmallThreads);
-            if (queue) merge(hub_bucket_merge<LpMode::Cluster, true>, big, kFinThreads);
+            merges(hub_bucket_merge<LpMode::Cluster, 0>, hub_bucket_merge<LpMode::Cluster, 1>, hub_bucket_merge<LpMode::Cluster, 2>);
             decide(hub_decide<LpMode::Cluster>);
         } else {
-            merge(hub_bucket_merge<LpMode::Refine, false>, nt, kSmallThreads);
-            if (queue) merge(hub_bucket_merge<LpMode::Refine, true>, big, kFinThreads);
+            merges(hub_bucket_merge<LpMode::Refine, 0>, hub_bucket_merge<LpMode::Refine, 1>, hub_bucket_merge<LpMode::Refine, 2>);
             decide(hub_decide<LpMode::Refine>);
         }
     }

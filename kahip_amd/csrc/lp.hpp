@@ -133,9 +133,11 @@ private:
     void fetch(hipStream_t s);  // host_ctl_ of the last run
     Mail mail_;
     // Counters of a run: {traversed edges in 64 spread 64-bit counters, moves per round, lengths
-    // of the hub merges' big task queues and of the long moved rows per sub-round, error flag}
+    // of the hub merges' big and mid-size task queues and of the long moved rows per sub-round,
+    // error flag}
     static constexpr int kCtlMoves = 128, kCtlBig = kCtlMoves + kMaxRounds,
-                         kCtlLong = kCtlBig + kMaxSub * kMaxRounds,
+                         kCtlMid = kCtlBig + kMaxSub * kMaxRounds,
+                         kCtlLong = kCtlMid + kMaxSub * kMaxRounds,
                          kCtlErr = kCtlLong + kMaxSub * kMaxRounds, kCtlInts = kCtlErr + 1;
     DevBuf<int> ctl_;
     int host_ctl_[kCtlBig + 1] = {};  // the traversed edges, the moves, the error flag
@@ -172,7 +174,7 @@ private:
     DevBuf<int> ct_base_, cnt_t_, pos_t_;
     DevBuf<char> scan_tmp_;
     DevBuf<long long> offm_base_;
-    DevBuf<int> offm_, task_prefix_, bown_, big_tasks_;
+    DevBuf<int> offm_, task_prefix_, bown_, big_tasks_, mid_tasks_;
     DevBuf<int4> bres_, big_;
     DevBuf<int4> cmap_, tmap_, mmap_;  // hub-chunk, (hub, bucket) task, mid-size hub descriptors
     DevBuf<int> midpos_;
