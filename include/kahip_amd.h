@@ -114,8 +114,9 @@ int kahip_partition(kahip_graph_t g, const kahip_params* params, int* part, kahi
 
 /* The entry points that run on the GPU keep their device workspaces, the device copies of host
  * arrays and the stream per device between calls, so that repeated calls do not allocate them
- * again; this frees those of the engines no call is using. No counterpart in the reference (its
- * kaffpa keeps no state between calls). */
+ * again; this frees those of the engines no call is using. A call that runs out of device memory
+ * gives them back and runs once more by itself. No counterpart in the reference (its kaffpa keeps
+ * no state between calls). */
 int kahip_release_workspaces(void);
 /* JSON object {name: {launches, ms, bytes, edges}} of the last profiled call on this thread. */
 int kahip_profile_json(char* buf, int len);

@@ -11,9 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <exception>
-#include <map>
 #include <memory>
-#include <mutex>
 #include <optional>
 #include <queue>
 #include <sstream>
@@ -24,6 +22,7 @@
 #include "driver.hpp"
 #include "fm_refine.hpp"
 #include "gen.hpp"
+#include "lease.hpp"
 #include "rebalance.hpp"
 #include "kahip_amd.h"
 
@@ -46,7 +45,7 @@ thread_local std::string g_last_profile = "{}";
 template <class F>
 int guarded(F&& f) {
     try {
-        f();
+        run_giving_back<Engine>(f);
         g_last_error.clear();
         return 0;
     } catch (const std::exception& e) {
@@ -57,62 +56,12 @@ int guarded(F&& f) {
     return 1;
 }
 
-// The entry points run on a cached engine of the current device, so that a repeated call reuses
-// the device workspaces sized by the previous ones instead of allocating (and freeing) them inside
-// the call (a stream, about 35 buffers and 6 of the 22 ms of kahip_contract on R-MAT 2^19); every
-// workspace is
-// re-initialised by the kernels that use it, exactly as between two levels of one call. A call
-// that finds the device's engine held by another thread runs on an engine of its own, and a call
-// that fails drops the cached engine. The cache is never destroyed at exit (its memory goes with
-// the process); kahip_release_workspaces frees the idle engines.
-struct CachedEngine {
-    std::mutex mu;
-    std::unique_ptr<Engine> eng;
-};
-std::mutex g_cache_mu;
-std::map<int, CachedEngine*>& engine_cache() {
-    static auto* cache = new std::map<int, CachedEngine*>();  // left to the process exit
-    return *cache;
-}
-
-class EngineLease {
-public:
-    EngineLease() : unwinding_(std::uncaught_exceptions()) {
-        int dev = 0;
-        KH_CHECK(hipGetDevice(&dev));
-        CachedEngine* c;
-        {
-            std::lock_guard<std::mutex> g(g_cache_mu);
-            CachedEngine*& slot = engine_cache()[dev];
-            if (!slot) slot = new CachedEngine();
-            c = slot;
-        }
-        std::unique_lock<std::mutex> lk(c->mu, std::try_to_lock);
-        if (lk.owns_lock()) {
-            if (!c->eng) c->eng.reset(new Engine());
-            cached_ = c;
-            e_ = c->eng.get();
-            lk_ = std::move(lk);
-        } else {
-            own_.reset(new Engine());
-            e_ = own_.get();
-        }
-    }
-    ~EngineLease() {
-        if (cached_ && std::uncaught_exceptions() > unwinding_) cached_->eng.reset();
-    }
-    EngineLease(const EngineLease&) = delete;
-    EngineLease& operator=(const EngineLease&) = delete;
-    Engine& operator*() { return *e_; }
-    Engine* operator->() { return e_; }
-
-private:
-    int unwinding_;
-    CachedEngine* cached_ = nullptr;
-    Engine* e_ = nullptr;
-    std::unique_ptr<Engine> own_;
-    std::unique_lock<std::mutex> lk_;
-};
+// The entry points run on a kept engine of the current device, so that a repeated call reuses the
+// device workspaces sized by the previous ones instead of allocating (and freeing) them inside the
+// call (a stream, about 35 buffers and 6 of the 22 ms of kahip_contract on R-MAT 2^19); every
+// workspace is re-initialised by the kernels that use it, exactly as between two levels of one
+// call. kahip_release_workspaces frees the idle engines.
+using EngineLease = Lease<Engine>;
 
 PartitionParams to_params(const kahip_params* q) {
     kahip_params d;
@@ -478,13 +427,7 @@ int kahip_graph_to_host(kahip_graph_t g, int* xadj, int* adjncy, int* vwgt, int*
 void kahip_graph_free(kahip_graph_t g) { delete g; }
 
 int kahip_release_workspaces(void) {
-    return guarded([&] {
-        std::lock_guard<std::mutex> g(g_cache_mu);
-        for (auto& kv : engine_cache()) {
-            std::unique_lock<std::mutex> lk(kv.second->mu, std::try_to_lock);
-            if (lk.owns_lock()) kv.second->eng.reset();  // an engine in use stays
-        }
-    });
+    return guarded([&] { (void)EngineLease::release_idle(); });
 }
 
 int kahip_partition(kahip_graph_t g, const kahip_params* params, int* part, kahip_stats* stats) {
@@ -493,12 +436,9 @@ int kahip_partition(kahip_graph_t g, const kahip_params* params, int* part, kahi
         PartitionParams p = to_params(params);
         EngineLease eng;
         std::vector<int> tmp;
-        if (!part) {
-            tmp.resize(std::max(g->og.g.n, 1));
-            part = tmp.data();
-        }
+        if (!part) tmp.resize(std::max(g->og.g.n, 1));
         PartitionStats st;
-        eng->partition(g->og.g, p, part, &st);
+        eng->partition(g->og.g, p, part ? part : tmp.data(), &st);
         if (p.profile) g_last_profile = profile_json(eng->prof);
         fill_stats(st, stats);
     });
@@ -934,13 +874,11 @@ int kahip_batch_partition(kahip_batch_t b, const kahip_params* params, int use_g
         PartitionParams p = to_params(params);
         EngineLease eng;
         std::vector<int> tmp;
-        if (!part) {
-            tmp.resize(std::max(b->og.g.n, 1));
-            part = tmp.data();
-        }
+        if (!part) tmp.resize(std::max(b->og.g.n, 1));
         BatchStats st;
         const int G = (int)b->node_off.size() - 1;
-        partition_batch(*eng, b->og.g, G, b->node_off.data(), p, part, &st, use_graph != 0);
+        partition_batch(*eng, b->og.g, G, b->node_off.data(), p, part ? part : tmp.data(), &st,
+                        use_graph != 0);
         for (int g = 0; g < G; ++g) {
             if (cuts) cuts[g] = st.cut[g];
             if (max_block_weights) max_block_weights[g] = st.max_block_weight[g];

@@ -14,6 +14,9 @@ namespace kahip {
 struct Error : std::runtime_error {
     using std::runtime_error::runtime_error;
 };
+struct OutOfMemory : Error {  // of the device
+    using Error::Error;
+};
 
 #define KH_CHECK(expr)                                                                         \
     do {                                                                                       \

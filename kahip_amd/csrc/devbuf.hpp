@@ -32,16 +32,18 @@ struct DevBuf {
     }
     ~DevBuf() { free(); }
     // Ensures room for n elements (contents are not preserved on growth). A buffer that has to
-    // grow gets an eighth more than asked for: calls on graphs of about one size differ by a few
-    // percent in their edges, and without it most of them would free and allocate every buffer
-    // again (about 0.1 ms each).
+    // grow gets an eighth more than asked for, if there is room: calls on graphs of about one size
+    // differ by a few percent in their edges, and without it most of them would free and allocate
+    // every buffer again (about 0.1 ms each).
     T* reserve(long long n) {
         if (n < 1) n = 1;
         if (n > cap) {
-            const long long room = cap > 0 ? n + n / 8 : n;
+            const bool grows = cap > 0;
             free();
-            KH_CHECK(hipMalloc((void**)&p, sizeof(T) * room));
-            cap = room;
+            if (!(grows && alloc(n + n / 8)) && !alloc(n))
+                throw OutOfMemory("HIP error out of memory: no " +
+                                  std::to_string(sizeof(T) * (unsigned long long)n) +
+                                  " bytes of device memory");
         }
         return p;
     }
@@ -51,6 +53,20 @@ struct DevBuf {
         cap = 0;
     }
     operator T*() const { return p; }
+
+private:
+    // false: not enough memory (the error is not left to the next call's check)
+    bool alloc(long long n) {
+        const hipError_t e = hipMalloc((void**)&p, sizeof(T) * n);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        KH_CHECK(e);
+        cap = n;
+        return true;
+    }
 };
 
 // Kernel-launch profiler. Each record brackets one launch (or one fused phase) on a stream with a
