@@ -8,9 +8,9 @@ partitioning of the coarsest graph, GPU projection + LP refinement for every lev
 metric value = GTEPS of the LP path as the metric defines it = (2m per LP clustering round,
 per contraction, per LP refinement round and per cut pass, summed over the levels) / (GPU time
 of coarsening + refinement + cut, hipEvents on the library's stream). value_edges_read divides
-the same time into the edges actually read (the refinement rounds work on a frontier, and hubs
-decide from kept per-block counters without reading their rows); `phases` splits time, edges and
-algorithmic bytes per phase. The CPU initial partitioning is outside the metric; its time is in
+the same time into the edges actually read (later clustering rounds of large meshes skip settled
+nodes, the refinement rounds work on a frontier, and hubs decide from kept per-block counters
+without reading their rows); `phases` splits time, edges and algorithmic bytes per phase. The CPU initial partitioning is outside the metric; its time is in
 ms_per_step (wall clock per full step) and reported separately.
 
 roofline: the dominant kernel (largest share of the timed LP launches), with algorithmic bytes
@@ -185,18 +185,22 @@ def make_graph(K, w):
     raise ValueError(w["kind"])
 
 
-def algorithmic_bytes(st, cluster_rounds=10):
-    """Algorithmic HBM bytes of the whole path from the per-level stats: LP clustering rounds
-    12 B per traversed edge + 16 B per node; contraction 12 B per fine edge + 16 B per fine node
-    + 8 B per coarse edge and node; LP refinement 12 B per traversed edge; cut 12 B per edge and
-    node."""
-    b = 0.0
+def clustering_read(prof, steps):
+    """(edges read, algorithmic bytes) of the clustering of a step, from the profile: 12 B per edge
+    read and 16 B per node of the rounds that look at every node."""
+    v = prof["lp_cluster_total"]
+    return v["edges"] // steps, v["bytes"] / steps
+
+
+def algorithmic_bytes(st, cluster_bytes):
+    """Algorithmic HBM bytes of the whole path: the clustering's (clustering_read); contraction 12 B
+    per fine edge + 16 B per fine node + 8 B per coarse edge and node; LP refinement 12 B per
+    traversed edge; cut 12 B per edge and node."""
+    b = cluster_bytes
     for lvl in range(st["levels"]):
         n, m2 = st["level_n"][lvl], st["level_m2"][lvl]
         nc, mc = st["level_n"][lvl + 1], st["level_m2"][lvl + 1]
-        b += 16.0 * n * cluster_rounds
         b += 12.0 * m2 + 16.0 * n + 8.0 * mc + 8.0 * nc
-    b += 12.0 * st["edges_cluster"]
     b += 12.0 * st["edges_refine"]
     b += 12.0 * st["edges_cut"] + 12.0 * st["level_n"][0]
     return b
@@ -242,22 +246,22 @@ def host_cpu():
     return {"host_cpu": model, "nproc": os.cpu_count(), "usable_cores": usable}
 
 
-def phase_breakdown(stats, prof, steps, cluster_rounds=10):
+def phase_breakdown(stats, prof, steps):
     """Per-phase GPU time, edges and algorithmic bytes per step: clustering (the lp_cluster_total
     profiler scope of every level), contraction (remap + contract), refinement
-    (kahip_stats.ms_refine; edges = the rows actually read), cut. Algorithmic bytes as in
+    (kahip_stats.ms_refine), cut. Edges are those actually read, algorithmic bytes as in
     algorithmic_bytes()."""
     st = stats[-1]
     ms = lambda pred: sum(v["ms"] for k, v in prof.items() if pred(k)) / steps
     levels = range(st["levels"])
-    cl_bytes = sum(16.0 * st["level_n"][l] * cluster_rounds for l in levels) + 12.0 * st["edges_cluster"]
+    cl_edges, cl_bytes = clustering_read(prof, steps)
     ct_bytes = sum(12.0 * st["level_m2"][l] + 16.0 * st["level_n"][l] + 8.0 * st["level_m2"][l + 1]
                    + 8.0 * st["level_n"][l + 1] for l in levels)
     rf_bytes = 12.0 * st["edges_refine"]
     cut_bytes = 12.0 * st["edges_cut"] + 12.0 * st["level_n"][0]
     out = {}
     for name, t, edges, b in (
-            ("clustering", ms(lambda k: k == "lp_cluster_total"), st["edges_cluster"], cl_bytes),
+            ("clustering", ms(lambda k: k == "lp_cluster_total"), cl_edges, cl_bytes),
             ("contraction", ms(lambda k: k in ("contract", "remap")), st["edges_contract"], ct_bytes),
             ("refinement", sum(s["ms_refine"] for s in stats) / len(stats), st["edges_refine"], rf_bytes),
             ("cut", sum(s["ms_cut"] for s in stats) / len(stats), st["edges_cut"], cut_bytes)):
@@ -265,6 +269,7 @@ def phase_breakdown(stats, prof, steps, cluster_rounds=10):
                      "gteps": round(edges / (t / 1e3) / 1e9, 2) if t > 0 else None,
                      "alg_gbs": round(b / (t / 1e3) / 1e9, 1) if t > 0 else None}
     out["reorder"] = {"ms": round(ms(lambda k: k == "reorder"), 2)}
+    out["clustering"]["edges_per_definition"] = st["edges_cluster"]
     out["refinement"]["edges_per_definition"] = refine_edges_per_round(st)
     out["refinement"]["note"] = ("edges = rows read by the refinement kernels (hubs deciding "
                                  "from their kept per-block counters read none) and rows of "
@@ -361,19 +366,19 @@ def main():
 
     gpu_ms = [s["ms_coarsen"] + s["ms_refine"] + s["ms_cut"] for s in stats]
     # value: GTEPS as the metric defines it (2m per LP clustering round, per contraction, per LP
-    # refinement round and per cut pass); beside it the same time with the refinement counting
-    # only the edges its kernels actually read (its rounds work on a frontier and hubs decide from
-    # kept per-block counters)
+    # refinement round and per cut pass); beside it the same time with the clustering and the
+    # refinement counting only the edges their kernels actually read
     edges = [s["edges_cluster"] + s["edges_contract"] + refine_edges_per_round(s) + s["edges_cut"]
              for s in stats]
-    edges_read = [s["edges_cluster"] + s["edges_contract"] + s["edges_refine"] + s["edges_cut"]
+    cluster_edges, cluster_bytes = clustering_read(prof, args.steps)
+    edges_read = [cluster_edges + s["edges_contract"] + s["edges_refine"] + s["edges_cut"]
                   for s in stats]
     gteps = sum(edges) / (sum(gpu_ms) / 1e3) / 1e9
     gteps_read = sum(edges_read) / (sum(gpu_ms) / 1e3) / 1e9
-    path_bytes = algorithmic_bytes(stats[-1])
+    path_bytes = algorithmic_bytes(stats[-1], cluster_bytes)
     path_gbs = path_bytes / (gpu_ms[-1] / 1e3) / 1e9
 
-    timed = {k: v for k, v in prof.items() if v["bytes"] > 0}
+    timed = {k: v for k, v in prof.items() if v["bytes"] > 0 and k != "lp_cluster_total"}
     dom_name = max(timed, key=lambda k: timed[k]["ms"]) if timed else None
     roofline = None
     if dom_name:

@@ -75,6 +75,9 @@ typedef struct {
     int level_n[KAHIP_MAX_LEVELS + 1];
     long long level_m2[KAHIP_MAX_LEVELS + 1];
     double ms_coarsen, ms_initial, ms_refine, ms_cut;
+    /* directed edges: of every clustering round (2m a round, also where settled nodes are skipped:
+     * the edges read are those of "lp_cluster_total" in the profile), contracted, read by the
+     * refinement, and of the cut */
     long long edges_cluster, edges_contract, edges_refine, edges_cut;
     long long max_block_weight;
     double ms_rating; /* rating time, part of ms_coarsen */

@@ -149,6 +149,12 @@ struct ProfScope {
               hipStream_t st)
         : p(prof), idx(prof ? prof->begin(name, bytes, edges, st) : -1), s(st) {}
     ~ProfScope() { close(); }
+    // What only its end knows.
+    void book(double bytes, long long edges) {
+        if (!p || idx < 0) return;
+        p->recs[idx].bytes = bytes;
+        p->recs[idx].edges = edges;
+    }
     // Ends the timed range early (idempotent).
     void close() {
         if (p) p->end(idx, s);

@@ -291,9 +291,14 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
         lp.run(LpMode::Cluster, rated, label.p, size.p, (int)B, p.cluster_rounds, cseed, s, prof,
                "lp_cluster");
         lp.check(s);
-        long long edges_round = 0;
-        for (int i = 0; i < p.subrounds * kNumBins; ++i) edges_round += lp.host_edges[i];
+        long long edges_round = 0, nodes_round = 0;
+        for (int i = 0; i < p.subrounds * kNumBins; ++i) {
+            edges_round += lp.host_edges[i];
+            nodes_round += lp.host_counts[i];
+        }
         S.edges_cluster += edges_round * p.cluster_rounds;
+        long long edges_read = lp.book_edges(s, prof);
+        long long nodes_read = nodes_round * lp.whole_rounds();
         for (int run = 1; run < p.ensemble; ++run) {
             // another clustering with its own seed and cluster factor, overlaid on the result
             const uint32_t eseed = ensemble_seed(p.seed, level, run);
@@ -304,9 +309,13 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
             lp.run(LpMode::Cluster, rated, elabel.p, size.p, eb, p.cluster_rounds, eseed, s, prof,
                    "lp_cluster");
             lp.check(s);
+            edges_read += lp.book_edges(s, prof);
+            nodes_read += nodes_round * lp.whole_rounds();
             S.edges_cluster += edges_round * p.cluster_rounds;
             overlay(fine.n, label.p, elabel.p, s);
         }
+        // edges read, and 12 B for each and 16 B per node of a whole round
+        ps_cluster.book(12.0 * (double)edges_read + 16.0 * (double)nodes_read, edges_read);
         ps_cluster.close();
         if ((int)maps.size() <= level) maps.emplace_back();
         if ((int)coarse.size() <= level) coarse.emplace_back(new OwnedGraph());

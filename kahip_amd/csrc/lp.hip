@@ -388,7 +388,7 @@ __device__ __attribute__((always_inline)) inline void scan_wave_table(
 // dependent loads (list, offsets, targets, labels, label weights) are issued together, so each
 // wave has that many chains in flight.
 // One virtual block (IT x kBlock / W nodes of the list); every thread of the workgroup calls it
-// (it synchronises the workgroup). `edges` adds up the traversed edges (refinement).
+// (it synchronises the workgroup). `edges` adds up the traversed edges (refinement and SETTLE).
 // SETTLE: also flags the nodes that are not settled (kSettleRound).
 template <LpMode M, int W, int E, int IT, bool SETTLE = false>
 __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
@@ -511,7 +511,7 @@ __device__ __attribute__((always_inline)) inline void group_vb(const LpArgs& a,
         const int tag = h_tag[i];
         if (tag >= 0) add_contrib(a, Contrib{tag >> 1, h_w[i], h_key[i], (tag & 1) != 0});
     }
-    if (M == LpMode::Refine) {
+    if (M == LpMode::Refine || SETTLE) {
 #pragma unroll
         for (int i = 0; i < IT; ++i)
             if (valid[i] && gl == 0) edges += (unsigned long long)deg[i];
@@ -623,7 +623,7 @@ __device__ __attribute__((always_inline)) inline void wave_vb(const LpArgs& a,
     else
         wave_node<M, DENSE, kWaveEdges, SETTLE>(a, base + gi, v, beg, deg, num_labels, lane,
                                                 skey[wave], sval[wave]);
-    if (M == LpMode::Refine && lane == 0) edges += (unsigned long long)deg;
+    if ((M == LpMode::Refine || SETTLE) && lane == 0) edges += (unsigned long long)deg;
 }
 
 // Clustering: the proposals of a sub-round's lists in one launch, the longest rows first, one
@@ -689,6 +689,7 @@ __global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F
                                                           edges);
         }
     }
+    if (SETTLE && F.dcount) count_traversed(a, edges);  // (whole lists: known to the host)
 }
 
 // ---------------------------------------------------------------- clustering: settled nodes
@@ -2644,6 +2645,8 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     const int S = subrounds_;
     const bool cl = mode == LpMode::Cluster;
     KH_REQUIRE(cl || !(dense_wave_ || dense_hub_) || num_labels_ > 0, "prepare() not called");
+    whole_rounds_ = rounds;
+    settled_rec_ = -1;
     fill_async(ctl_.p, kCtlErr, 0, s);  // the error flag is cleared by prepare()
     fetched_ = false;
     if (rounds == 0) return;
@@ -2719,6 +2722,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
     }
     const bool settle = cl && hubs == 0 && rounds > kSettleRound + 1 && g.m2 > kSettleEdges;
     if (settle) {
+        whole_rounds_ = kSettleRound + 1;
         active_.reserve(g.n);
         clists_.reserve(g.n);
         ccount_.reserve(rounds * nseg);  // list lengths per round
@@ -2780,7 +2784,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
             ProfScope ps(prof, base + "_settled", 0.0, 0, s);
             a.next_active = act;
             for (int sr = 0; sr < S; ++sr)
-                settled_subround(a, sr, r == kSettleRound ? nullptr : ccount_.p + r * nseg + sr * kNumBins, s);
+                settled_subround(a, sr, r == kSettleRound ? nullptr : ccount_.p + r * nseg + sr * kNumBins, s, prof, base);
             ++r;
             continue;
         }
@@ -3041,16 +3045,26 @@ void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, const int* d
 
 // Sub-round sr of a clustering from round kSettleRound on: over the whole lists (dcount nullptr)
 // or over their nodes that are not settled (dcount: their lengths, zero on entry).
-void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s) {
+void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s,
+                                   Profiler* prof, const std::string& base) {
     const int l0 = sr * kNumBins;
     int total = 0;
-    for (int b = 0; b < kNumBins; ++b) total += host_counts[l0 + b];
+    long long edges = 0;  // of the whole lists
+    for (int b = 0; b < kNumBins; ++b) {
+        total += host_counts[l0 + b];
+        edges += host_edges[l0 + b];
+    }
     if (total == 0) return;
     if (dcount)
         hipLaunchKernelGGL(compact_active, dim3(grid_for(total, 256 * kCompactItems)), dim3(256), 0,
                            s, lists_.p, offsets_.p + l0, kNumBins, host_offsets[l0], total,
                            a.next_active, 1, nullptr, dcount, clists_.p);
-    launch_lists(a, sr, 1, dcount, true, Turnover{}, s);
+    {
+        ProfScope ps(prof, base + "_propose_settled", dcount ? 0.0 : 12.0 * (double)edges + 16.0 * total,
+                     dcount ? 0 : edges, s);
+        if (dcount && settled_rec_ < 0) settled_rec_ = ps.idx;  // (booked by book_edges())
+        launch_lists(a, sr, 1, dcount, true, Turnover{}, s);
+    }
     SubLists L{};
     for (int b = 0; b < kNumBins; ++b) {
         L.list[b] = (dcount ? clists_.p : lists_.p) + host_offsets[l0 + b];
@@ -3104,6 +3118,17 @@ long long LpWorkspace::traversed(hipStream_t s) {
     long long t = 0;
     for (int i = 0; i < 64; ++i) t += (long long)h[i];
     return t;
+}
+
+long long LpWorkspace::book_edges(hipStream_t s, Profiler* prof) {
+    const long long compacted = traversed(s);
+    if (prof && settled_rec_ >= 0) {
+        prof->recs[settled_rec_].edges = compacted;
+        prof->recs[settled_rec_].bytes = 12.0 * (double)compacted;
+    }
+    long long edges = 0;
+    for (int l = 0; l < subrounds_ * kNumBins; ++l) edges += host_edges[l];
+    return edges * whole_rounds_ + compacted;
 }
 
 void LpWorkspace::border(const DGraph& g, const int* part, uint8_t* flags, hipStream_t s) {

@@ -109,8 +109,14 @@ public:
     void read_moves(int rounds, int* out, hipStream_t s);
     // Directed edges read by the last refinement run (waits for it): the rows scanned
     // by the proposal kernels (hubs deciding from their kept counters read none) and the rows of
-    // moved nodes scanned to mark their neighbours and update hub counters.
+    // moved nodes scanned to mark their neighbours and update hub counters. Clustering: the rows
+    // of the rounds that skip settled nodes.
     long long traversed(hipStream_t s);
+    // Directed edges read by the proposals of the last clustering run (waits for it); books those
+    // of the rounds that skip settled nodes on their first profile record.
+    long long book_edges(hipStream_t s, Profiler* prof);
+    // Rounds of the last clustering run that looked at every listed node.
+    int whole_rounds() const { return whole_rounds_; }
     // Throws if a kernel of a run() since the last prepare() set the device error flag (waits for
     // the last run).
     void check(hipStream_t s);
@@ -126,7 +132,8 @@ private:
                      const uint8_t* include, int copies);
     void launch_lists(const LpArgs& a, int sr, int copies, const int* dcount, bool settle,
                       const Turnover& T, hipStream_t s);
-    void settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s);
+    void settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s, Profiler* prof,
+                          const std::string& base);
     void propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool incremental, hipStream_t s,
                       Profiler* prof, const std::string& base);
     int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
@@ -142,6 +149,8 @@ private:
     DevBuf<int> ctl_;
     int host_ctl_[kCtlBig + 1] = {};  // the traversed edges, the moves, the error flag
     bool fetched_ = false;
+    int whole_rounds_ = 0;
+    int settled_rec_ = -1;  // profile record of the first proposals over compacted lists
     bool keep_err_ = false, clear_err_ = false;
     bool small_ = false;  // refinement that starts in refine_tail, without lists
     void build_chunk_maps(hipStream_t s);  // cmap_ of every sub-round (after chunk_prefix_)
