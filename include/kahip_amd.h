@@ -74,6 +74,8 @@ typedef struct {
     int levels;             /* number of contractions */
     int level_n[KAHIP_MAX_LEVELS + 1];
     long long level_m2[KAHIP_MAX_LEVELS + 1];
+    /* GPU time of coarsening, refinement and cut by events; ms_initial: the CPU's time from the
+     * coarsest graph on the host to its partition on the way to the GPU */
     double ms_coarsen, ms_initial, ms_refine, ms_cut;
     /* directed edges: of every clustering round (2m a round, also where settled nodes are skipped:
      * the edges read are those of "lp_cluster_total" in the profile), contracted, read by the

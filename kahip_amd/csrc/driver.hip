@@ -337,9 +337,9 @@ void Engine::partition(const DGraph& input, const PartitionParams& p, int* part_
 
     // ------------------------------------------------------------------ initial partitioning
     const DGraph& cg = level_graph(level);
-    const auto t0 = std::chrono::steady_clock::now();
     HostGraph hg;
-    download_graph(cg, hg, s, &mw.mail);
+    download_graph(cg, hg, s, &mw.mail);  // waits for the coarsening, whose time is ev_coarsen's
+    const auto t0 = std::chrono::steady_clock::now();
     std::vector<int> hpart;
     IpParams ip;
     ip.k = p.k;
