@@ -21,6 +21,7 @@
 #include <future>
 #include <numeric>
 #include <queue>
+#include <system_error>
 #include <thread>
 
 namespace kahip {
@@ -589,22 +590,22 @@ void recurse(const Graph& g, int lb, int ub, RecCtx& ctx, std::vector<int>& part
     Graph half[2];
     extract(g, side, half, ids);
     std::vector<int> p0, p1;
-    bool spawned = false;
     std::future<void> fut;
     if (k1 > 1 && k2 > 1 && g.n > kSpawnNodes && take_thread(*ctx.idle)) {
-        fut = std::async(std::launch::async, [&] {
-            struct Back {  // the thread is idle again, also after an exception
-                std::atomic<int>* idle;
-                ~Back() { ++*idle; }
-            } back{ctx.idle};
-            recurse(half[0], lb, mid, ctx, p0);
-        });
-        spawned = true;
-    } else {
-        recurse(half[0], lb, mid, ctx, p0);
+        try {
+            fut = std::async(std::launch::async, [&] {
+                struct Back {  // the thread is idle again, also after an exception
+                    std::atomic<int>* idle;
+                    ~Back() { ++*idle; }
+                } back{ctx.idle};
+                recurse(half[0], lb, mid, ctx, p0);
+            });
+        } catch (const std::system_error&) {  // the system has no thread to give: go on without
+        }
     }
+    if (!fut.valid()) recurse(half[0], lb, mid, ctx, p0);
     recurse(half[1], mid + 1, ub, ctx, p1);
-    if (spawned) fut.get();
+    if (fut.valid()) fut.get();
     for (size_t i = 0; i < ids[0].size(); ++i) part[ids[0][i]] = p0[i];
     for (size_t i = 0; i < ids[1].size(); ++i) part[ids[1][i]] = p1[i];
 }
@@ -726,15 +727,22 @@ void initial_partition(const HostGraph& g, const IpParams& p, std::vector<int>& 
         // an exception (e.g. bad_alloc) is rethrown here, not left to end the process
         std::vector<std::exception_ptr> err(reps);
         std::vector<std::thread> pool;
-        for (int r = 0; r < reps; ++r)
-            pool.emplace_back([&, r] {
-                try {
-                    run_rep(r);
-                } catch (...) {
-                    err[r] = std::current_exception();
-                }
-                ++idle;
-            });
+        const auto rep = [&](int r) {
+            try {
+                run_rep(r);
+            } catch (...) {
+                err[r] = std::current_exception();
+            }
+            ++idle;
+        };
+        pool.reserve(reps);
+        for (int r = 0; r < reps; ++r) {
+            try {
+                pool.emplace_back(rep, r);
+            } catch (const std::system_error&) {  // no thread to be had: on this one
+                rep(r);
+            }
+        }
         for (auto& t : pool) t.join();
         for (auto& e : err)
             if (e) std::rethrow_exception(e);
