@@ -16,7 +16,7 @@
 //               their places and the coarse weights.
 //   rows_thread one thread per row of fd <= 8 (rows of fd = 0 need no work);
 //   rows_few    one wave per row of 128 < fd <= 4096 where the clusters have many members: a small
-//               table, rows with more neighbours are left to rows_block;
+//               table, rows with more neighbours are left early to rows_block;
 //   rows_wave   one wave per row of fd <= 128 / <= 512: LDS hash (q -> w, min t), a stage
 //               indexed by t that marks each entry at its first appearance, one ordered pass;
 //   rows_block  the same with one workgroup per row of fd <= 1024 (256 threads) / <= 4096 (1024);
@@ -469,11 +469,14 @@ __global__ __launch_bounds__(THREADS) void rows_block(
 
 // One wave per row of fd <= kTierFd[3] with at most kFewMax distinct neighbours: K / V / M as in
 // rows_wave, in a table of kFewCap slots; the entries are ranked by their first appearances
-// against each other. Rows with more are appended to `over`. For levels whose clusters
-// have many members (kFewMembers): most of their edges stay inside (RGG 2^22: 22 members, 317 edges and
-// 6 neighbours a row), and the tables of rows_wave / rows_block, sized for fd distinct neighbours,
-// took the time to clear and to scan and left 11 waves on a CU. Measured there, rows of
-// 128 < fd <= 4096: 950 -> 320 us.
+// against each other. For levels whose clusters have many members (kFewMembers): on meshes most of
+// their edges stay inside (RGG 2^22: 22 members, 317 edges and 6 neighbours a row), and the tables of
+// rows_wave / rows_block, sized for fd distinct neighbours, took the time to clear and to scan and
+// left 11 waves on a CU. Measured there, rows of 128 < fd <= 4096: 950 -> 320 us.
+// Rows with more neighbours are left as soon as they have them and appended to `over`, by size for the
+// two rows_block kernels. Measured, kahip_contract of R-MAT 2^14 by clusters of 30 consecutive nodes:
+// 1.35 ms when a full table was probed to the row's end and all such rows took 1024 threads, now 0.60
+// (1.10 without rows_few and with the buffers of every call its own).
 constexpr int kFewMembers = 8;  // fine nodes per coarse node
 constexpr int kFewCap = 128;
 constexpr int kFewMax = 64;
@@ -483,9 +486,10 @@ __global__ __launch_bounds__(64 * kFewWaves) void rows_few(
     const int* __restrict__ adjncy, const int* __restrict__ adjwgt, const int* __restrict__ map,
     const int* __restrict__ moff, const int* __restrict__ members, const int* __restrict__ tpos,
     int* __restrict__ cdeg, int* __restrict__ tq, int* __restrict__ tw, int* __restrict__ over,
-    int* __restrict__ n_over) {
+    int* __restrict__ n_over, int* __restrict__ err) {
     constexpr int kEpl = 4;
     static_assert(kFewCap == 128 && kFewMax == 64, "two slots and one entry per lane");
+    static_assert(kFewMax + 64 <= kFewCap, "64 edges always find a slot");
     __shared__ int sk[kFewWaves][kFewCap], sv[kFewWaves][kFewCap], sm[kFewWaves][kFewCap];
     __shared__ int spre[kFewWaves][64], sstart[kFewWaves][64];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -504,9 +508,8 @@ __global__ __launch_bounds__(64 * kFewWaves) void rows_few(
         M[i] = 0x7fffffff;
     }
     const int mb = moff[p], me = moff[p + 1];
-    int tbase = 0;
-    bool full = false;
-    for (int base = mb; base < me && !__any(full); base += 64) {
+    int tbase = 0, cnt = 0;  // cnt: entries of the table (uniform)
+    for (int base = mb; base < me && cnt <= kFewMax; base += 64) {
         const int mi = base + lane;
         int b = 0, d = 0;
         if (mi < me) {
@@ -524,7 +527,7 @@ __global__ __launch_bounds__(64 * kFewWaves) void rows_few(
         mpre[lane] = incl;
         mstart[lane] = b;
         wave_lds_order();
-        for (int t0 = 0; t0 < total; t0 += 64 * kEpl) {
+        for (int t0 = 0; t0 < total && cnt <= kFewMax; t0 += 64 * kEpl) {
             int es[kEpl], qs[kEpl], ws[kEpl];
 #pragma unroll
             for (int j = 0; j < kEpl; ++j) {
@@ -549,27 +552,31 @@ __global__ __launch_bounds__(64 * kFewWaves) void rows_few(
                 if (es[j] >= 0) qs[j] = map[qs[j]];
 #pragma unroll
             for (int j = 0; j < kEpl; ++j) {
+                if (cnt > kFewMax) break;  // uniform
                 const int q = qs[j];
-                if (es[j] < 0 || q == p) continue;
-                const int h = probe_claim(K, kFewCap, q);
-                if (h < 0) {
-                    full = true;
-                    continue;
+                bool fresh = false;
+                if (es[j] >= 0 && q != p) {
+                    const int h = probe_claim(K, kFewCap, q, fresh);  // <= kFewMax + 64 entries
+                    if (h < 0) {
+                        *err = kErrProbe;
+                    } else {
+                        atomicAdd(&V[h], ws[j]);
+                        atomicMin(&M[h], tbase + t0 + lane + 64 * j);
+                    }
                 }
-                atomicAdd(&V[h], ws[j]);
-                atomicMin(&M[h], tbase + t0 + lane + 64 * j);
+                cnt += __popcll(__ballot(fresh));
             }
         }
         tbase += total;
         wave_lds_order();  // mpre / mstart are rewritten by the next batch
     }
-    const int k0 = K[lane], k1 = K[lane + 64];
-    const unsigned long long u0 = __ballot(k0 >= 0), u1 = __ballot(k1 >= 0);
-    const int n0 = __popcll(u0), cnt = n0 + __popcll(u1);
-    if (__any(full) || cnt > kFewMax) {
+    if (cnt > kFewMax) {
         if (lane == 0) over[atomicAdd(n_over, 1)] = p;
         return;
     }
+    const int k0 = K[lane], k1 = K[lane + 64];
+    const unsigned long long u0 = __ballot(k0 >= 0), u1 = __ballot(k1 >= 0);
+    const int n0 = __popcll(u0);
     const unsigned long long below = (1ull << lane) - 1;
     const int m0 = M[lane], m1 = M[lane + 64];
     int* const first = mpre;  // first appearances of the entries
@@ -1121,8 +1128,8 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
     mrec_.reserve((long long)n + 1);
     mpre_.reserve((long long)n + 1);
     // ctl_: lengths of the five LDS tiers' row lists, of the global tier's and of the rows left
-    // over by rows_few, error flag
-    constexpr int kCtlGlobal = 5, kCtlOver = 6, kCtlErr = 7, kCtlInts = 8;
+    // over by rows_few (of the tiers up to fd = kTierFd[2], and of the largest), error flag
+    constexpr int kCtlGlobal = 5, kCtlOver = 6, kCtlErr = 8, kCtlInts = 9;
     ctl_.reserve(kCtlInts);
     int* const err = ctl_.p + kCtlErr;
     fill_async(ctl_.p, kCtlInts, 0, s);
@@ -1176,13 +1183,15 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
         {
             ProfScope ps(prof, "contract_rows_lds", bytes, m2, s);
             if (few) {
-                over_.reserve(nc);
+                over_[0].reserve(rc[2] + rc[3]);
+                over_[1].reserve(rc[4]);
                 for (int t = 2; t < 5; ++t)
                     if (rc[t] > 0)
                         hipLaunchKernelGGL(rows_few, dim3(grid_for(rc[t], kFewWaves)),
                                            dim3(64 * kFewWaves), 0, s, rlist_[t].p, rc[t], g.xadj,
                                            g.adjncy, g.adjwgt, map, moff_.p, members_.p, tpos_.p,
-                                           cdeg_.p, tq_.p, tw_.p, over_.p, ctl_.p + kCtlOver);
+                                           cdeg_.p, tq_.p, tw_.p, over_[t / 4].p,
+                                           ctl_.p + kCtlOver + t / 4, err);
             }
             if (rc[0] > 0)
                 hipLaunchKernelGGL(rows_thread, dim3(grid_for(rc[0], 256)), dim3(256), 0, s,
@@ -1201,17 +1210,17 @@ void ContractWorkspace::contract(const DGraph& g, const int* map, int nc, OwnedG
             // grid-stride over the device-side counts: five 256-thread workgroups per CU, one
             // 1024-thread workgroup per CU
             ProfScope ps(prof, "contract_rows_lds_big", 0.0, 0, s);
-            if (rc[3] > 0 && !few)
-                hipLaunchKernelGGL((rows_block<kMidThreads, kMidCap>), dim3(std::min(rc[3], 256 * 5)),
-                               dim3(kMidThreads), 0, s, rlist_[3].p, ctl_.p + 3, g.xadj,
-                               g.adjncy, g.adjwgt, map, moff_.p, members_.p, fdeg_.p, tpos_.p,
-                               cdeg_.p, tq_.p, tw_.p, err);
-            const int big = few ? rc[2] + rc[3] + rc[4] : rc[4];  // at most
-            if (big > 0)
-                hipLaunchKernelGGL((rows_block<kBigThreads, kBigCap>), dim3(std::min(big, 256)), dim3(kBigThreads),
-                               0, s, few ? over_.p : rlist_[4].p, ctl_.p + (few ? kCtlOver : 4), g.xadj, g.adjncy, g.adjwgt, map,
-                               moff_.p, members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p,
-                               err);
+            const int mid = few ? rc[2] + rc[3] : rc[3];  // at most
+            if (mid > 0)
+                hipLaunchKernelGGL((rows_block<kMidThreads, kMidCap>), dim3(std::min(mid, 256 * 5)),
+                               dim3(kMidThreads), 0, s, few ? over_[0].p : rlist_[3].p,
+                               ctl_.p + (few ? kCtlOver : 3), g.xadj, g.adjncy, g.adjwgt, map, moff_.p,
+                               members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p, err);
+            if (rc[4] > 0)
+                hipLaunchKernelGGL((rows_block<kBigThreads, kBigCap>), dim3(std::min(rc[4], 256)),
+                               dim3(kBigThreads), 0, s, few ? over_[1].p : rlist_[4].p,
+                               ctl_.p + (few ? kCtlOver + 1 : 4), g.xadj, g.adjncy, g.adjwgt, map, moff_.p,
+                               members_.p, fdeg_.p, tpos_.p, cdeg_.p, tq_.p, tw_.p, err);
         }
     }
     if (novl > 0) {

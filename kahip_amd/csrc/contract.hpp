@@ -40,7 +40,7 @@ private:
     DevBuf<int> fdeg_, moff_, tpos_, cdeg_, members_, tq_, tw_;
     DevBuf<int> mkeys_;                      // sorted clusters of the members
     DevBuf<unsigned long long> mrec_, mpre_; // members' {degree, weight} and their scan
-    DevBuf<int> over_;                       // rows left over by rows_few
+    DevBuf<int> over_[2];                    // rows left over by rows_few
     DevBuf<int> rlist_[5];                   // rows of the thread tier and the four LDS tiers
     DevBuf<int> ovl2_list_, ctl_;            // rows of the global tier; list lengths, error flag
     Mail mail_;
