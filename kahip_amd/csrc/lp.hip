@@ -1624,18 +1624,22 @@ __global__ void set_hub_slots(const int* __restrict__ list, const int* __restric
 // workgroup and not a grid with device-wide barriers: a barrier across the XCDs' L2s costs about
 // as much as a launch. The limits keep it to frontiers for which one CU is faster than the grid:
 // a pass of 64 nodes of <= 16 edges takes about 2 us, so kTailNodes / 4 nodes of a sub-round
-// stay at the cost of its launches. Larger frontiers (or labels beyond the LDS, or hubs among
-// the nodes) are left to the grid. Graphs within the limits start here without node lists.
-// Measured, calls of kahip_partition: RGG 2^10 k = 2 5.1 -> 2.2 ms (refinement 3.0 -> 0.3), RGG
+// stay at the cost of its launches; with fewer than four sub-rounds the frontier's limits are that
+// much lower (tail_nodes, tail_edges: one sub-round, 2040 nodes of 16 edges, k = 500: kahip_lp_refine
+// 3.40 ms with the limits of four, 1.02 with these, 1.32 before refine_tail). Larger frontiers (or
+// labels beyond the LDS, or hubs among the nodes) are left to the grid. Graphs within the limits start
+// here without node lists. Measured, calls of kahip_partition: RGG 2^10 k = 2 5.1 -> 2.2 ms (refinement 3.0 -> 0.3), RGG
 // 2^22 k = 2 32.3 -> 26.1 ms, R-MAT 2^17 k = 8 39.1 -> 36.8 ms (its coarse levels settle early).
 constexpr int kTailThreads = 1024;
-constexpr int kTailNodes = 2048;     // frontier nodes
-constexpr int kTailEdges = 1 << 15;  // edges of the frontier's rows
+constexpr int kTailNodes = 2048;     // frontier nodes, at most
+constexpr int kTailEdges = 1 << 15;  // edges of the frontier's rows, at most
 constexpr int kTailLabels = 512;     // labels (blocks) held in LDS
 constexpr int kTailHash = 2 * kTailNodes;
 constexpr int kTailWaves = kTailThreads / 64;
 constexpr int kTailDegree = 512;     // largest degree (8 edges per lane of a wave)
 constexpr int kTailGroup = 16;       // lanes per node of degree <= 16
+inline int tail_nodes(int S) { return std::min(kTailNodes, S * (kTailNodes / 4)); }
+inline int tail_edges(int S) { return std::min(kTailEdges, S * (kTailEdges / 4)); }
 
 // Runs rounds a.round.. while the frontier is small; *state receives the round to go on with
 // (`rounds`: all done), whose frontier is then flagged in a.next_active, or compacted already if
@@ -1682,7 +1686,7 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
     for (int b = tid; b < k; b += kTailThreads)
         if (a.size[b] > bound_of(a, b)) over = 1;
     if (t.clists) {
-        if (nfront <= kTailNodes)
+        if (nfront <= t.max_nodes)
             for (int i = tid; i < nfront; i += kTailThreads) {
                 int lo = 0, hi = t.nseg - 1;  // last list starting at or before i
                 while (lo < hi) {
@@ -1691,13 +1695,13 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
                 }
                 raw[i] = t.clists[t.offsets[lo] + (i - pre[lo])];
             }
-    } else {  // round 0 of a graph of at most kTailNodes nodes (host)
+    } else {  // round 0 of a graph of at most t.max_nodes nodes (host)
         for (int v = tid; v < t.n; v += kTailThreads)
             if (a.xadj[v + 1] > a.xadj[v]) raw[atomicAdd(&nfront, 1)] = v;
     }
     __syncthreads();
     int r = t.round;
-    bool fits = nfront <= kTailNodes && k <= kTailLabels && !t.hubs;  // uniform
+    bool fits = nfront <= t.max_nodes && k <= kTailLabels && !t.hubs;  // uniform
     if (fits) {
         for (int i = tid; i < nfront; i += kTailThreads) {
             const int d = a.xadj[raw[i] + 1] - a.xadj[raw[i]];
@@ -1705,7 +1709,7 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
             if (d > kTailDegree) bad = 1;
         }
         __syncthreads();
-        fits = nedges <= kTailEdges && !bad;
+        fits = nedges <= t.max_edges && !bad;
     }
     if (fits && nfront > 0 && r < t.rounds) {
         for (int b = tid; b < k; b += kTailThreads) {
@@ -1911,7 +1915,7 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
                         a.next_active[u] = 1;
                         bool fresh = false;
                         if (!spill && probe_claim(hash, kTailHash, u, fresh) < 0) spill = 1;
-                        if (fresh && atomicAdd(&nnext, 1) >= kTailNodes) spill = 1;
+                        if (fresh && atomicAdd(&nnext, 1) >= t.max_nodes) spill = 1;
                     }
                 }
                 if (tid == 0) nmoves += nm;
@@ -1927,13 +1931,13 @@ __global__ __launch_bounds__(kTailThreads) void refine_tail(LpArgs a, TailArgs t
             for (int i = tid; i < kTailHash; i += kTailThreads) {
                 const int u = hash[i];
                 if (u < 0) continue;
-                raw[atomicAdd(&nfront, 1)] = u;  // nnext <= kTailNodes
+                raw[atomicAdd(&nfront, 1)] = u;  // nnext <= t.max_nodes
                 const int d = a.xadj[u + 1] - a.xadj[u];
                 atomicAdd(&nedges, min(d, kTailEdges));
                 if (d > kTailDegree) bad = 1;
             }
             __syncthreads();
-            if (nfront == 0 || nedges > kTailEdges || bad || r == t.rounds) break;
+            if (nfront == 0 || nedges > t.max_edges || bad || r == t.rounds) break;
             for (int i = tid; i < kTailHash; i += kTailThreads) {
                 if (hash[i] >= 0) a.next_active[hash[i]] = 0;
                 hash[i] = -1;
@@ -2327,8 +2331,8 @@ void LpWorkspace::prepare(LpMode mode, const DGraph& g, int num_labels, int S, u
         next_active_.reserve(g.n);
     }
     // a graph that refine_tail takes from round 0 needs no lists
-    small_ = mode == LpMode::Refine && !include && g.n <= kTailNodes && g.m2 <= kTailEdges &&
-             num_labels <= kTailLabels;
+    small_ = mode == LpMode::Refine && !include && g.n <= tail_nodes(S) &&
+             g.m2 <= tail_edges(S) && num_labels <= kTailLabels;
     if (!small_) build_lists(mode, g, seed, s, include, copies);
     else if (clear_err_) fill_async(ctl_.p + kCtlErr, 1, 0, s);
     clear_err_ = false;  // (run() may build the lists later on)
@@ -3081,6 +3085,8 @@ void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStre
 int LpWorkspace::run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded) {
     t.num_labels = num_labels_;
     t.S = subrounds_;
+    t.max_nodes = tail_nodes(subrounds_);
+    t.max_edges = tail_edges(subrounds_);
     t.moves = ctl_.p + kCtlMoves;
     t.state = mail_.box();
     t.seq = mail_.next();

@@ -60,6 +60,7 @@ struct TailArgs {
     int* cnext;          // cleared for the next compaction (nseg entries)
     int nseg, n, num_labels, S, round, rounds;
     uint32_t seed;
+    int max_nodes, max_edges;  // of a frontier that it takes
     int hubs;            // nodes of more than the wave bin's degree exist: never run here
     int* moves;          // per round
     int* state;          // mail: {number, next round, overloaded block exists}
