@@ -701,12 +701,23 @@ __global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F
 // nodes and those neighbours, and from the round after it a sub-round first compacts its lists to
 // the flagged nodes (right before it, as the earlier sub-rounds' moves unsettle nodes of this one).
 // Earlier, most nodes move and flag all of their neighbours: measured, RGG 2^22, k = 2, coarsening
-// from round 1 9.3, from 2 8.9, from 3 9.0 ms, without 10.1 ms. For large graphs only: at
-// kSettleEdges edges and below a sub-round is bound by its launches, and the compaction is one
-// more (RGG of 60 001 nodes: 0.80 -> 1.12 ms, of 1 000 003: 3.8 -> 3.2 ms). Not for graphs
-// with hubs: on R-MAT graphs 14 to 18 % of the nodes settle and hardly fewer edges are read.
+// from round 1 9.3, from 2 8.9, from 3 9.0 ms, without 10.1 ms. For graphs of more than kSettleEdges
+// edges only: below, a sub-round is bound by its launches, and the compaction is one more (RGG of
+// 60 001 nodes: 0.80 -> 1.12 ms, of 1 000 003: 3.8 -> 3.2 ms). Not for graphs with hubs: on R-MAT
+// graphs 14 to 18 % of the nodes settle and hardly fewer edges are read. Not for a single sub-round:
+// whole rounds of simultaneous moves leave 72 to 100 % of the edges with nodes that are not settled.
+// And the graph has to settle: the flags cost the marking of every mover's row, so the first
+// sub-round with flags is asked how much it has left, and if that is more than kSettleShare of its
+// lists' edges, nothing is skipped. Left with 4 (8) sub-rounds, and clustering and contraction with
+// all flags over those without any: RGG 0.32 to 0.35 (0.20), 4 194 304 nodes 0.80 (0.82); rings with
+// rewired edges 0.36 (0.20), 400 000 nodes 0.89 (0.99); dense communities 0.00 to 0.06, 0.62 to 0.93
+// (0.67 to 0.86); grid 2000 x 2000 0.47 (0.36), 0.96 (0.95); 160^3 0.59 (0.45), 1.05 (1.08); random
+// and regular graphs of degree 8 to 500 0.70 to 1.00, 1.10 to 2.0 (1.12 to 2.1); RGG of average
+// degree 247 0.85 (0.65), 1.24 (1.39); communities of 300 that the cluster bound splits 0.96, 2.1
+// (2.9). With the answer no, 1.00 to 1.15.
 constexpr int kSettleRound = 2;
 constexpr long long kSettleEdges = 1LL << 21;
+constexpr double kSettleShare = 0.5;
 
 // Refinement: the proposals of all degree lists of a sub-round in one launch. The lists are the
 // round's compacted frontier (lengths on the device); the workgroups stride over the virtual
@@ -2724,7 +2735,7 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         hipLaunchKernelGGL(init_frontier, dim3(grid_for(std::max(nf, 2 * nseg), 256)), dim3(256),
                            0, s, nf, act, (uint8_t)(keep_flags ? 1 : 0), map, start, nxt, 2 * nseg, ccount_.p);
     }
-    const bool settle = cl && hubs == 0 && rounds > kSettleRound + 1 && g.m2 > kSettleEdges;
+    bool settle = cl && hubs == 0 && S > 1 && rounds > kSettleRound + 1 && g.m2 > kSettleEdges;
     if (settle) {
         whole_rounds_ = kSettleRound + 1;
         active_.reserve(g.n);
@@ -2784,15 +2795,25 @@ void LpWorkspace::run(LpMode mode, const DGraph& g, int* label, int* size, int b
         a.moves = ctl_.p + kCtlMoves + r;
         a.active = cl ? nullptr : act;
         a.next_active = cl ? nullptr : nxt;
+        int sr0 = 0;  // sub-rounds run with flags
         if (settle && r >= kSettleRound) {
             ProfScope ps(prof, base + "_settled", 0.0, 0, s);
             a.next_active = act;
-            for (int sr = 0; sr < S; ++sr)
-                settled_subround(a, sr, r == kSettleRound ? nullptr : ccount_.p + r * nseg + sr * kNumBins, s, prof, base);
-            ++r;
-            continue;
+            bool asked = r > kSettleRound;
+            for (; sr0 < S && settle; ++sr0) {
+                int* dcount = ccount_.p + r * nseg + sr0 * kNumBins;
+                if (!settled_subround(a, sr0, r == kSettleRound ? nullptr : dcount, s, prof, base) || asked) continue;
+                asked = true;
+                settle = few_unsettled(act, sr0, dcount, s);
+            }
+            if (settle) {
+                ++r;
+                continue;
+            }
+            whole_rounds_ = rounds;
+            a.next_active = nullptr;
         }
-        for (int sr = 0; sr < S; ++sr) {
+        for (int sr = sr0; sr < S; ++sr) {
             int sub_total = 0;
             if (!cl) {
                 if (from_start) {
@@ -3048,8 +3069,9 @@ void LpWorkspace::launch_lists(const LpArgs& a, int sr, int copies, const int* d
 }
 
 // Sub-round sr of a clustering from round kSettleRound on: over the whole lists (dcount nullptr)
-// or over their nodes that are not settled (dcount: their lengths, zero on entry).
-void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s,
+// or over their nodes that are not settled (dcount: their lengths, zero on entry). False if it has
+// no nodes.
+bool LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s,
                                    Profiler* prof, const std::string& base) {
     const int l0 = sr * kNumBins;
     int total = 0;
@@ -3058,7 +3080,7 @@ void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStre
         total += host_counts[l0 + b];
         edges += host_edges[l0 + b];
     }
-    if (total == 0) return;
+    if (total == 0) return false;
     if (dcount)
         hipLaunchKernelGGL(compact_active, dim3(grid_for(total, 256 * kCompactItems)), dim3(256), 0,
                            s, lists_.p, offsets_.p + l0, kNumBins, host_offsets[l0], total,
@@ -3078,6 +3100,27 @@ void LpWorkspace::settled_subround(const LpArgs& a, int sr, int* dcount, hipStre
     const int gs = std::min(grid_for(total, 256), 1024);
     hipLaunchKernelGGL(admit_moves_sub, dim3(gs), dim3(256), 0, s, a, L);
     hipLaunchKernelGGL(apply_moves_sub<LpMode::Cluster>, dim3(gs), dim3(kBlock), 0, s, a, L);
+    return true;
+}
+
+// Whether the nodes of sub-round sr that are not settled hold few of its lists' edges. count:
+// kNumBins counters, zero on entry.
+bool LpWorkspace::few_unsettled(uint8_t* flags, int sr, int* count, hipStream_t s) {
+    const int l0 = sr * kNumBins;
+    int total = 0;
+    for (int b = 0; b < kNumBins; ++b) total += host_counts[l0 + b];
+    hipLaunchKernelGGL(compact_active, dim3(grid_for(total, 256 * kCompactItems)), dim3(256), 0, s,
+                       lists_.p, offsets_.p + l0, kNumBins, host_offsets[l0], total, flags, 0,
+                       nullptr, count, clists_.p);
+    mail_.post(s, {count, kNumBins});
+    const int* left = mail_.wait(s);
+    double edges = 0.0, read = 0.0;
+    for (int b = 0; b < kNumBins; ++b) {
+        const int l = l0 + b;
+        edges += (double)host_edges[l];
+        if (host_counts[l] > 0) read += (double)host_edges[l] * left[b] / host_counts[l];
+    }
+    return read <= kSettleShare * edges;
 }
 
 // Launches refine_tail and waits for its answer: the round to go on with, and whether a block is

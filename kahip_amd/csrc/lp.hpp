@@ -133,8 +133,9 @@ private:
                      const uint8_t* include, int copies);
     void launch_lists(const LpArgs& a, int sr, int copies, const int* dcount, bool settle,
                       const Turnover& T, hipStream_t s);
-    void settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s, Profiler* prof,
+    bool settled_subround(const LpArgs& a, int sr, int* dcount, hipStream_t s, Profiler* prof,
                           const std::string& base);
+    bool few_unsettled(uint8_t* flags, int sr, int* count, hipStream_t s);
     void propose_hubs(LpMode mode, LpArgs a, int r, int sr, bool incremental, hipStream_t s,
                       Profiler* prof, const std::string& base);
     int run_tail(const LpArgs& a, TailArgs& t, hipStream_t s, bool* overloaded);
