@@ -703,9 +703,12 @@ __global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F
 // Earlier, most nodes move and flag all of their neighbours: measured, RGG 2^22, k = 2, coarsening
 // from round 1 9.3, from 2 8.9, from 3 9.0 ms, without 10.1 ms. For graphs of more than kSettleEdges
 // edges only: below, a sub-round is bound by its launches, and the compaction is one more (RGG of
-// 60 001 nodes: 0.80 -> 1.12 ms, of 1 000 003: 3.8 -> 3.2 ms). Not for graphs with hubs: on R-MAT
-// graphs 14 to 18 % of the nodes settle and hardly fewer edges are read. Not for a single sub-round:
-// whole rounds of simultaneous moves leave 72 to 100 % of the edges with nodes that are not settled.
+// 60 001 nodes: 0.80 -> 1.12 ms). That still holds some way above the line: clustering and
+// contraction of an RGG, k = 4, without flags and with them, 200 003 nodes 0.94 and 1.34, 400 003
+// nodes 2.05 and 2.18, 1 000 003 nodes 2.98 and 2.83, 4 194 304 nodes 9.0 and 7.2 ms. Not for graphs
+// with hubs: on R-MAT graphs 14 to 18 % of the nodes settle and hardly fewer edges are read. Not for
+// a single sub-round: whole rounds of simultaneous moves leave 72 to 100 % of the edges with nodes
+// that are not settled (dense communities alone gained, 0.75 to 0.93 of the time).
 // And the graph has to settle: the flags cost the marking of every mover's row, so the first
 // sub-round with flags is asked how much it has left, and if that is more than kSettleShare of its
 // lists' edges, nothing is skipped. Left with 4 (8) sub-rounds, and clustering and contraction with
@@ -714,7 +717,7 @@ __global__ __launch_bounds__(kBlock) void propose_lists(LpArgs a, ClusterLists F
 // (0.67 to 0.86); grid 2000 x 2000 0.47 (0.36), 0.96 (0.95); 160^3 0.59 (0.45), 1.05 (1.08); random
 // and regular graphs of degree 8 to 500 0.70 to 1.00, 1.10 to 2.0 (1.12 to 2.1); RGG of average
 // degree 247 0.85 (0.65), 1.24 (1.39); communities of 300 that the cluster bound splits 0.96, 2.1
-// (2.9). With the answer no, 1.00 to 1.15.
+// (2.9). With the answer no, 1.00 to 1.2.
 constexpr int kSettleRound = 2;
 constexpr long long kSettleEdges = 1LL << 21;
 constexpr double kSettleShare = 0.5;
